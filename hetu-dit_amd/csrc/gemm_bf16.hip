@@ -42,6 +42,7 @@
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <type_traits>
 
 #include "hdit_common.h"
@@ -146,7 +147,7 @@ constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0f70; }
 // All tiles of one shape that this workgroup owns.
 template <class C>
 __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles, int tiles_per_xcd, int wgs_per_xcd,
-                                          unsigned char* lds) {
+                                          int wg_in_xcd, unsigned char* lds) {
   constexpr int TM = C::TM, TN = C::TN;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -160,7 +161,7 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
   const int xcd = blockIdx.x % NUM_XCD;
   const int xcd_begin = xcd * tiles_per_xcd;
   const int xcd_end = min(xcd_begin + tiles_per_xcd, total_tiles);
-  int lid = xcd_begin + blockIdx.x / NUM_XCD;
+  int lid = xcd_begin + wg_in_xcd;
   if (lid >= xcd_end) return;
 
   // ---- producer: the slab stream, two slabs ahead of the MFMAs ------------------
@@ -664,7 +665,7 @@ template <class C>
 __global__ void __launch_bounds__(NT) gemm_kernel(const GemmTable tab, int total_tiles, int tiles_per_xcd,
                                                   int wgs_per_xcd) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-  run_tiles<C>(tab, total_tiles, tiles_per_xcd, wgs_per_xcd, lds);
+  run_tiles<C>(tab, total_tiles, tiles_per_xcd, wgs_per_xcd, blockIdx.x / NUM_XCD, lds);
 }
 
 // Two tile shapes in one launch: the large tiles of the tall problems first, then the small tiles of the
@@ -674,9 +675,14 @@ template <class C1, class C2>
 __global__ void __launch_bounds__(NT) gemm_kernel2(const GemmTable tab1, int total1, int per_xcd1, const GemmTable tab2,
                                                    int total2, int per_xcd2, int wgs_per_xcd) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-  run_tiles<C1>(tab1, total1, per_xcd1, wgs_per_xcd, lds);
+  const int wg = blockIdx.x / NUM_XCD;
+  run_tiles<C1>(tab1, total1, per_xcd1, wgs_per_xcd, wg, lds);
   __syncthreads();  // the second phase reuses the LDS of the first
-  run_tiles<C2>(tab2, total2, per_xcd2, wgs_per_xcd, lds);
+  // the small tiles are dealt from the first workgroup on that has no tile in the last round of large ones
+  const int xcd = blockIdx.x % NUM_XCD;
+  const int own1 = max(min(per_xcd1, total1 - xcd * per_xcd1), 0);
+  const int first = own1 % wgs_per_xcd;
+  run_tiles<C2>(tab2, total2, per_xcd2, wgs_per_xcd, wg >= first ? wg - first : wg - first + wgs_per_xcd, lds);
 }
 
 std::atomic<int> g_num_cus{0};
@@ -748,7 +754,7 @@ int launch2(const hdit_gemm_problem* p1, int n1, const hdit_gemm_problem* p2, in
   const int total1 = fill_table<C1>(t1, p1, n1), total2 = fill_table<C2>(t2, p2, n2);
   const int per1 = (total1 + NUM_XCD - 1) / NUM_XCD, per2 = (total2 + NUM_XCD - 1) / NUM_XCD;
   int wgs_per_xcd = max_wgs / NUM_XCD;
-  const int need = per1 > per2 ? per1 : per2;
+  const int need = per1 + per2;  // a workgroup of its own for every tile, while there are CUs
   if (wgs_per_xcd > need) wgs_per_xcd = need;
   hipLaunchKernelGGL((gemm_kernel2<C1, C2>), dim3(wgs_per_xcd * NUM_XCD), dim3(NT), LDS, stream, t1, total1, per1, t2,
                      total2, per2, wgs_per_xcd);
@@ -780,38 +786,74 @@ using Cfg128x192 = Cfg<2, 3>;
 std::atomic<int> g_force_cfg{-1};
 
 // ---- launch planning ---------------------------------------------------------
-// A launch runs ceil(tiles / CUs) rounds of tiles; a tile costs (k / 64) slab times plus an epilogue.
-// Problems of very different heights (the 8192-row image stream and the 666-row text stream of a joint
-// block) are badly served by one tile shape: the small problem's few large tiles add a nearly empty
-// round.  The planner therefore gives every problem the shape that is cheapest for it alone, launches
-// one kernel per shape, and falls back to a single shape when that is cheaper.
+// A launch deals its tiles to 256 workgroups (one per CU) in rounds; a tile costs (k / 64) slab times plus an epilogue.
+// A slab takes `lo` microseconds while at most half of the CUs work and `hi` while all do (the chip's power budget is
+// shared), in between in between.  All figures measured on MI355X with weights that come from HBM: single problems of
+// 32 - 1024 tiles, K = 1536 and 6144; the model below reproduces those launches within 4 %.
+//
+// What a plan has to get right is the last round.  One tile shape for everything wastes most of it: the 666-row text
+// stream of a joint block on the image stream's 256-row tiles adds a nearly empty round, and 17 550 rows x 3072 columns
+// are 828 tiles of 256 x 256, three rounds and 60 tiles (K = 12288: 1249 us on the 128 x 256 tiles that a model without
+// `lo` preferred, 1076 us on 256 x 256, 1004 us on 768 tiles of 256 x 256 and 240 of 128 x 128).  So besides every single shape the planner prices launches of two shapes, the large tiles
+// first: problems dealt to the shape that suits them, and the whole call on large tiles except the rows at the end of
+// its tallest problem that would open another round; those take the small shape.
+// Results do not depend on any of this (every shape forms the same sums in the same order).
+struct Shape {
+  int bm, bn;
+  double lo, hi, epi;
+};
 constexpr int NCFG = 5;
-constexpr int kBM[NCFG] = {256, 128, 128, 256, 128};
-constexpr int kBN[NCFG] = {192, 256, 128, 256, 192};
-// measured on MI355X: microseconds per 64-wide slab and per epilogue of one tile
-constexpr double kSlabUs[NCFG] = {1.21, 0.72, 0.44, 1.40, 0.68};
-constexpr double kEpiUs[NCFG] = {13.0, 12.4, 8.0, 16.0, 7.1};  // epilogue plus the pipeline fill of a tile
-constexpr double kLaunchUs = 3.0;
+constexpr Shape kShape[NCFG] = {
+    {256, 192, 0.95, 1.19, 7.7}, {128, 256, 0.80, 0.92, 5.6}, {128, 128, 0.54, 0.57, 4.0},
+    {256, 256, 1.11, 1.50, 8.0}, {128, 192, 0.67, 0.77, 4.1},
+};
+constexpr double kLaunchUs = 4.0;
 constexpr int kSlots = 256;
 
-int tiles_of(const hdit_gemm_problem& p, int c) { return ((p.m + kBM[c] - 1) / kBM[c]) * ((p.n + kBN[c] - 1) / kBN[c]); }
-
-// time of all tiles of `ps` under shape c, without launch overhead
-double tiles_time(const hdit_gemm_problem* const* ps, int count, int c) {
-  int tiles = 0;
-  double work = 0;
-  for (int i = 0; i < count; i++) {
-    const int t = tiles_of(*ps[i], c);
-    tiles += t;
-    work += t * ((ps[i]->k / BK) * kSlabUs[c] + kEpiUs[c]);
-  }
-  if (tiles == 0) return 0;
-  const int rounds = (tiles + kSlots - 1) / kSlots;
-  return rounds * (work / tiles);
+int tiles_of(const hdit_gemm_problem& p, int c) {
+  return ((p.m + kShape[c].bm - 1) / kShape[c].bm) * ((p.n + kShape[c].bn - 1) / kShape[c].bn);
 }
 
-double launch_time(const hdit_gemm_problem* const* ps, int count, int c) {
-  return count == 0 ? 0.0 : kLaunchUs + tiles_time(ps, count, c);
+struct Load {  // the tiles of some problems under one shape
+  int tiles = 0;
+  double slabs = 0;  // per tile, on average
+};
+
+Load load_of(const hdit_gemm_problem* ps, int count, int c) {
+  Load l;
+  for (int i = 0; i < count; i++) {
+    const int t = tiles_of(ps[i], c);
+    l.tiles += t;
+    l.slabs += (double)t * (ps[i].k / BK);
+  }
+  if (l.tiles) l.slabs /= l.tiles;
+  return l;
+}
+
+// one tile of shape c while `busy` of the 256 CUs work on such tiles
+double tile_us(int c, double slabs, int busy) {
+  const double f = busy >= kSlots ? 1.0 : busy > kSlots / 2 ? 2.0 * busy / kSlots - 1.0 : 0.0;
+  return slabs * (kShape[c].lo + (kShape[c].hi - kShape[c].lo) * f) + kShape[c].epi;
+}
+
+double single_us(const Load& l, int c) {
+  const int full = l.tiles / kSlots, rem = l.tiles % kSlots;
+  return full * tile_us(c, l.slabs, kSlots) + (rem ? tile_us(c, l.slabs, rem) : 0.0);
+}
+
+// Tiles of c1, then tiles of c2 in the same launch: the small tiles go first to the workgroups that have one large tile
+// fewer (see gemm_kernel2).
+double two_us(const Load& l1, int c1, const Load& l2, int c2) {
+  if (l1.tiles == 0) return single_us(l2, c2);
+  if (l2.tiles == 0) return single_us(l1, c1);
+  const int full = l1.tiles / kSlots, rem = l1.tiles % kSlots;
+  const int idle = rem ? kSlots - rem : 0;  // workgroups without a tile of the last large round
+  const int base = l2.tiles / kSlots, extra = l2.tiles % kSlots;
+  const double t1 = full * tile_us(c1, l1.slabs, kSlots), t1_last = rem ? tile_us(c1, l1.slabs, rem) : 0.0;
+  const double t2 = tile_us(c2, l2.slabs, base ? kSlots : extra);
+  const double of_idle = t1 + (base + (extra > 0 ? 1 : 0)) * t2;
+  const double of_rest = t1 + t1_last + (base + (extra > idle ? 1 : 0)) * t2;
+  return idle && of_idle > of_rest ? of_idle : of_rest;
 }
 
 int launch_cfg(int cfg, const hdit_gemm_problem* problems, int count, hipStream_t s) {
@@ -861,52 +903,76 @@ extern "C" __attribute__((visibility("default"))) int hdit_gemm_bf16(const hdit_
   const int forced = g_force_cfg.load(std::memory_order_relaxed);
   if (forced >= 0) return launch_cfg(forced, live, nlive, s);
 
-  // every problem's own best shape
-  int own[HDIT_GEMM_MAX_PROBLEMS];
-  const hdit_gemm_problem* ptr[HDIT_GEMM_MAX_PROBLEMS];
-  for (int i = 0; i < nlive; i++) {
-    const hdit_gemm_problem* one = &live[i];
-    own[i] = 0;
-    double best = launch_time(&one, 1, 0);
-    for (int c = 1; c < NCFG; c++) {
-      const double t = launch_time(&one, 1, c);
-      if (t < best) best = t, own[i] = c;
-    }
-  }
-  // plan A: one shape for everything
-  for (int i = 0; i < nlive; i++) ptr[i] = &live[i];
+  // one shape for everything
   int single = 0;
-  double single_cost = launch_time(ptr, nlive, 0);
-  for (int c = 1; c < NCFG; c++) {
-    const double t = launch_time(ptr, nlive, c);
+  double single_cost = 1e30;
+  for (int c = 0; c < NCFG; c++) {
+    const double t = single_us(load_of(live, nlive, c), c);
     if (t < single_cost) single_cost = t, single = c;
   }
-  // plan B: one launch, two shapes -- the problems that want 256-row tiles on the better of the two large
-  // shapes, the others on the better of the two 128-row shapes
-  hdit_gemm_problem big[HDIT_GEMM_MAX_PROBLEMS], small[HDIT_GEMM_MAX_PROBLEMS];
-  const hdit_gemm_problem* pb[HDIT_GEMM_MAX_PROBLEMS];
-  const hdit_gemm_problem* psm[HDIT_GEMM_MAX_PROBLEMS];
-  int nb = 0, ns = 0;
-  for (int i = 0; i < nlive; i++) {
-    if (own[i] == 0 || own[i] == 3) big[nb] = live[i], pb[nb] = &live[i], nb++;
-    else small[ns] = live[i], psm[ns] = &live[i], ns++;
-  }
+  // two shapes, large tiles of 256 rows (c1) and small ones of 128 (c2)
+  hdit_gemm_problem big[HDIT_GEMM_MAX_PROBLEMS + 1], small[HDIT_GEMM_MAX_PROBLEMS + 1];
+  int nb = 0, ns = 0, big_cfg = 3, small_cfg = 2;
   double two_cost = 1e30;
-  int big_cfg = 0, small_cfg = 2;
-  if (nb > 0 && ns > 0) {
-    const double t0 = tiles_time(pb, nb, 0), t3 = tiles_time(pb, nb, 3);
-    big_cfg = t3 < t0 ? 3 : 0;
-    // the short problems on 128x128 or, when that needs a second round, on 128x256
-    const double s2 = tiles_time(psm, ns, 2), s1 = tiles_time(psm, ns, 1);
-    small_cfg = s1 < s2 ? 1 : 2;
-    two_cost = kLaunchUs + (t3 < t0 ? t3 : t0) + (s1 < s2 ? s1 : s2);
+  for (const int c1 : {3, 0}) {
+    for (const int c2 : {2, 1}) {
+      // (a) every problem where it is cheaper on its own
+      hdit_gemm_problem b[HDIT_GEMM_MAX_PROBLEMS + 1], m[HDIT_GEMM_MAX_PROBLEMS + 1];
+      int kb = 0, km = 0;
+      for (int i = 0; i < nlive; i++) {
+        const bool large = single_us(load_of(&live[i], 1, c1), c1) <= single_us(load_of(&live[i], 1, c2), c2);
+        (large ? b[kb++] : m[km++]) = live[i];
+      }
+      double t = two_us(load_of(b, kb, c1), c1, load_of(m, km, c2), c2);
+      if (kb && km && t < two_cost) {
+        two_cost = t, big_cfg = c1, small_cfg = c2, nb = kb, ns = km;
+        memcpy(big, b, kb * sizeof(*b));
+        memcpy(small, m, km * sizeof(*m));
+      }
+      // (b) and (c): the problems that (a) gives large tiles, or all of them, except the rows that open another round
+      for (int all = 0; all < 2; all++) {
+        if (all) {
+          for (int i = 0; i < km; i++) b[kb++] = m[i];
+          km = 0;
+        }
+        const int excess = load_of(b, kb, c1).tiles % kSlots;
+        int tall = 0;
+        for (int i = 1; i < kb; i++)
+          if (b[i].m > b[tall].m) tall = i;
+        if (kb == 0 || excess == 0 || load_of(b, kb, c1).tiles < kSlots) continue;
+        if (km >= HDIT_GEMM_MAX_PROBLEMS) continue;  // the table of the small tiles is full
+        const int tiles_n = (b[tall].n + kShape[c1].bn - 1) / kShape[c1].bn;
+        const int blocks = (b[tall].m + kShape[c1].bm - 1) / kShape[c1].bm;
+        const int keep = blocks - (excess + tiles_n - 1) / tiles_n;
+        // a gate per batch element is looked up by the row within the problem: only one batch element can be split
+        const bool gated = (b[tall].epilogue & HDIT_EPI_MODE_MASK) == HDIT_EPI_GATE_RESIDUAL;
+        if (keep <= 0 || (gated && b[tall].m > b[tall].rows_per_batch)) continue;
+        const hdit_gemm_problem whole = b[tall];
+        const int64_t r0 = (int64_t)keep * kShape[c1].bm;
+        hdit_gemm_problem rest = whole;
+        rest.m = whole.m - (int)r0;
+        rest.a = (const char*)whole.a + r0 * whole.lda * 2;
+        rest.c = (char*)whole.c + r0 * whole.ldc * ((whole.epilogue & HDIT_EPI_OUT_F32) ? 4 : 2);
+        if (gated) rest.resid = (const char*)whole.resid + r0 * whole.ldr * ((whole.epilogue & HDIT_EPI_RESID_F32) ? 4 : 2);
+        b[tall].m = (int)r0;
+        m[km] = rest;
+        t = two_us(load_of(b, kb, c1), c1, load_of(m, km + 1, c2), c2);
+        if (t < two_cost) {
+          two_cost = t, big_cfg = c1, small_cfg = c2, nb = kb, ns = km + 1;
+          memcpy(big, b, kb * sizeof(*b));
+          memcpy(small, m, (km + 1) * sizeof(*m));
+        }
+        b[tall] = whole;
+      }
+    }
   }
   static const bool debug = getenv("HDIT_GEMM_DEBUG") != nullptr;
   if (debug) {
     fprintf(stderr, "hdit_gemm_bf16 plan:");
-    for (int i = 0; i < nlive; i++) fprintf(stderr, " [%dx%dx%d epi%d own%d]", live[i].m, live[i].n, live[i].k, live[i].epilogue, own[i]);
-    fprintf(stderr, " single cfg%d %.1f us, two-shape(big cfg%d, small cfg%d) %.1f us\n", single, single_cost, big_cfg,
-            small_cfg, two_cost);
+    for (int i = 0; i < nlive; i++) fprintf(stderr, " [%dx%dx%d epi%d]", live[i].m, live[i].n, live[i].k, live[i].epilogue);
+    fprintf(stderr, " single cfg%d %.1f us, two-shape(big cfg%d %d tiles, small cfg%d %d tiles) %.1f us\n", single,
+            single_cost + kLaunchUs, big_cfg, load_of(big, nb, big_cfg).tiles, small_cfg, load_of(small, ns, small_cfg).tiles,
+            two_cost + kLaunchUs);
   }
   if (two_cost < single_cost) {
     if (big_cfg == 0 && small_cfg == 2) return launch2<Cfg256x192, Cfg128x128>(big, nb, small, ns, s);

@@ -85,6 +85,43 @@ def test_gemm_result_does_not_depend_on_the_tile_shape(hdit, epi):
         assert torch.equal(out, outs[0]), f"shape {cfg} differs from shape 0"
 
 
+@pytest.mark.parametrize("n", [3072, 3080])
+@pytest.mark.parametrize("epi", ["bias", "gelu", "gate", "gate_two_batches"])
+def test_gemm_rows_that_open_another_round_take_the_small_shape(hdit, epi, n):
+    """5700 x 3072 is 276 tiles of 256 x 256: the plan keeps 252 of them and gives the rows behind to 128-row tiles in
+    the same launch (a problem whose gate differs between batch elements is not divided).  Bits of one shape."""
+    print(f"gemm divided rows epi={epi} n={n}", flush=True)
+    ops, lib = hdit.ops, hdit._lib.lib()
+    k, ms = 512, (5700, 226)
+    batches = 2 if epi == "gate_two_batches" else 1
+    a = [g(rnd(m, k, seed=41 + i)) for i, m in enumerate(ms)]
+    w = [g(rnd(n, k, scale=0.05, seed=43 + i)) for i in range(2)]
+    b = [g(rnd(n, seed=45 + i)) for i in range(2)]
+    res = [torch.randn(m, n, generator=torch.Generator(device=DEV).manual_seed(47 + i), device=DEV) for i, m in enumerate(ms)]
+    gate = torch.randn(batches, n, generator=torch.Generator(device=DEV).manual_seed(49), device=DEV)
+
+    def launch(cfg):
+        outs, probs = [], []
+        for i, m in enumerate(ms):
+            if epi.startswith("gate"):
+                outs.append(torch.empty(m, n, dtype=torch.float32, device=DEV))
+                probs.append(ops.gemm_problem(a[i], w[i], outs[i], b[i], ops.EPI_GATE_RESIDUAL, resid=res[i], gate=gate,
+                                              rows_per_batch=m // batches))
+            else:
+                outs.append(torch.empty(m, n, dtype=torch.bfloat16, device=DEV))
+                probs.append(ops.gemm_problem(a[i], w[i], outs[i], b[i], ops.EPI_BIAS_GELU if epi == "gelu" else ops.EPI_BIAS))
+        lib.hdit_gemm_force_config(cfg)
+        try:
+            ops.gemm_launch(probs)
+        finally:
+            lib.hdit_gemm_force_config(-1)
+        torch.cuda.synchronize()
+        return outs
+
+    for got, want in zip(launch(-1), launch(2)):
+        assert torch.equal(got, want)
+
+
 def test_gemm_gelu_and_gate_residual_grouped(hdit):
     B, T1, T2, D, F = 2, 320, 77, 256, 512
     x1, x2 = rnd(B, T1, D), rnd(B, T2, D)
