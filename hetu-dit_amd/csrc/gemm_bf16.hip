@@ -24,16 +24,24 @@
 //    behind the barrier that ends slab g, the B rows of slab g+2 go into the B
 //    slot just vacated.  Requests retire in order, so the wait in front of the
 //    barrier leaves exactly the newest A requests in flight.
-//  * 128-row shapes: two LDS stages, register-staged.  While slab h is
+//  * 128x256: two LDS stages, register-staged.  While slab h is
 //    multiplied out of stage h&1, the registers holding slab h+1 are written
 //    to the other stage and immediately refilled with the global loads of slab
 //    h+2, one write+load pair every few MFMAs.
+//  * ring shapes (64x64 to 128x192), for the launches that do not fill the chip: a slab is 4 to 24 MFMAs per wave,
+//    and what bounds it is the operands' way to the CU: time per slab is proportional to its bytes, 25 - 40 B/clk/CU,
+//    whatever its MFMAs.  Direct to LDS through a ring of 3 to 8 stages; the fragments of a whole slab are
+//    double-buffered in registers, so a slab has one barrier and no wait for LDS inside, and its stage is free for
+//    the request of the slab NS ahead as soon as it begins.  Measured (warm weights, microseconds per slab): 128x128
+//    0.36 - 0.39, 0.54 before with four stages and fragments one k-step ahead; 128x192 0.45, 0.67 before
+//    (register-staged); 64x128 0.27; 64x64 0.19.  Small tiles are what short problems need: 333 x 1536 x 6144 is 36
+//    tiles of 128x128 (61 us at first), 144 of 64x64 (27 us).
 //
 // Epilogue.  A lane's accumulator holds one output row m and runs of 4
 // consecutive n; lanes l and l^32 swap halves (v_permlane32_swap) to own 8
 // consecutive n.  bias / GELU-tanh are applied there, the bf16 result is staged
 // through a wave-private 8 KiB window inside the LDS stage (the A slot) the last
-// slab just vacated and written back with 16 lanes covering 256 contiguous bytes of a row
+// slab just vacated (ring shapes: behind the stages) and written back with 16 lanes covering 256 contiguous bytes of a row
 // (gate and residual are applied in that coalesced layout, in fp32).
 //
 // One launch covers up to HDIT_GEMM_MAX_PROBLEMS problems.  Tiles are dealt to
@@ -63,6 +71,8 @@ struct GemmTable {
   hdit_gemm_problem p[HDIT_GEMM_MAX_PROBLEMS];
 };
 
+constexpr int RING_MAX_MMA = 6;  // MFMAs per k-step of the shapes that take their slabs through a ring
+
 template <int TM_, int TN_>
 struct Cfg {
   static constexpr int TM = TM_, TN = TN_;
@@ -82,17 +92,18 @@ struct Cfg {
   static constexpr int A_SLOTS = 3, B_SLOTS = 2;
   static constexpr int B_OFF = A_SLOTS * A_BYTES;
   static constexpr int DMA_BYTES = A_SLOTS * A_BYTES + B_SLOTS * B_BYTES;
-  // RING: the 128x128 shape takes its slabs the same way into a ring of four stages (A then B, 32 KiB each),
-  // requested three slabs ahead: its slabs are short (16 MFMAs per wave), and only a lead of several of them
-  // covers the latency of operands that come from HBM.  The epilogue windows alias the stage the tile's last slab
-  // vacated.
-  static constexpr bool RING = TM == 2 && TN == 2;
-  static constexpr int NS = RING ? 4 : 2;
+  // RING: the shapes with short slabs (4 to 24 MFMAs per wave) take them the same way into a ring of NS stages
+  // (A then B), as many as fit beside the epilogue windows: only a lead of several slabs covers the latency of
+  // operands that come from HBM.
+  static constexpr bool RING = TM * TN <= RING_MAX_MMA;
+  static constexpr int EPI_OFF = 160 * 1024 - NW * EPI_WAVE_BYTES;  // ring shapes: windows of their own behind the stages
+  static constexpr int NS = RING ? (EPI_OFF / STAGE_BYTES < 8 ? EPI_OFF / STAGE_BYTES : 8) : 2;
   static constexpr bool DIRECT = DMA || RING;
-  static constexpr int LDS_BYTES = DMA ? DMA_BYTES : NS * STAGE_BYTES;
+  static constexpr int LDS_BYTES = DMA ? DMA_BYTES : RING ? 160 * 1024 : NS * STAGE_BYTES;
   static_assert(LDS_BYTES <= 160 * 1024, "tile does not fit the LDS");
-  static_assert(DMA ? NW * EPI_WAVE_BYTES <= A_BYTES : NW * EPI_WAVE_BYTES <= STAGE_BYTES,
+  static_assert(RING || (DMA ? NW * EPI_WAVE_BYTES <= A_BYTES : NW * EPI_WAVE_BYTES <= STAGE_BYTES),
                 "the epilogue windows live inside one stage (one A slot)");
+  static_assert(!RING || NS >= 3, "a ring holds the slab being read and at least one on its way");
   static_assert(TN <= 4, "epilogue staging window is 128 columns wide");
 };
 
@@ -250,6 +261,15 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
   const int a_row = (wm0 + l32) * ROW_BYTES;
   const int b_row = (wn0 + l32) * ROW_BYTES;
   bf16x8 fa[2][TM], fb[2][TN];
+  // ring shapes: the fragments of whole slabs, the one being multiplied and the next
+  constexpr int SK = C::RING ? BK / 16 : 1;
+  bf16x8 sfa[2][SK][TM], sfb[2][SK][TN];
+  auto read_slab_frag = [&](const unsigned char* sbase, int buf, int r) {  // r-th fragment in the order of use
+    const int ks = r / (TM + TN), f = r % (TM + TN);
+    const int ch = ((ks * 2 + lh) ^ swz) << 4;
+    if (f < TN) sfb[buf][ks][f] = *(const bf16x8*)(sbase + C::A_BYTES + b_row + ch + f * 32 * ROW_BYTES);
+    else sfa[buf][ks][f - TN] = *(const bf16x8*)(sbase + a_row + ch + (f - TN) * 32 * ROW_BYTES);
+  };
   auto read_frags2 = [&](const unsigned char* abase, const unsigned char* bbase, int ks, int buf) {
     const int ch = ((ks * 2 + lh) ^ swz) << 4;
 #pragma unroll
@@ -297,16 +317,17 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
     __syncthreads();
     read_frags2(lds, lds + C::B_OFF, 0, 0);
   } else if constexpr (C::RING) {
-    // slabs 0 .. NS-2 into stages 0 .. NS-2; slab 0 has landed before the first fragment read
+    // slabs 0 .. NS-1 into stages 0 .. NS-1; slab 0 has landed before the first fragment read
 #pragma unroll
-    for (int s = 0; s < C::NS - 1; s++) {
+    for (int s = 0; s < C::NS; s++) {
 #pragma unroll
       for (int i = 0; i < C::LOADS; i++) dma_ring(s, i);
       p_advance();
     }
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm((C::NS - 2) * C::LOADS));
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm((C::NS - 1) * C::LOADS));
     __syncthreads();
-    read_frags(lds, 0, 0);
+#pragma unroll
+    for (int r = 0; r < SK * (TM + TN); r++) read_slab_frag(lds, 0, r);
   } else {
 #pragma unroll
     for (int i = 0; i < C::LOADS; i++) g_load(i);
@@ -325,7 +346,7 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
   constexpr int RD_MFMA = (NRD + 1) / 2;  // MFMAs that are followed by two fragment reads
   constexpr int SLOTS = NMMA - RD_MFMA;   // MFMAs per k-step that can carry a write+load pair
   constexpr int CP = (C::LOADS + 2) / 3;  // pairs per k-step (k-steps 0..2 of a slab)
-  static_assert(RD_MFMA < NMMA, "not enough MFMAs to place the fragment reads");
+  static_assert(C::RING || RD_MFMA < NMMA, "not enough MFMAs to place the fragment reads");
 
   bool first_tile = true;
   while (true) {
@@ -409,8 +430,7 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
           for (int j = 0; j < C::LOADS; j++)
             if (j < n && RD_MFMA + (j * SLOTS) / (n > 0 ? n : 1) == t) {
               if (kind == 0) dma_a(slot, first + j);
-              else if (kind == 1) dma_b(slot, first + j);
-              else dma_ring(slot, first + j);
+              else dma_b(slot, first + j);
             }
           SCHED_FENCE();
         }
@@ -438,23 +458,48 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
         p_advance();
       }
     } else if constexpr (C::RING) {
-      constexpr int RQ = C::LOADS / 4;  // requests per k-step
-      static_assert(C::LOADS % 4 == 0, "ring requests are dealt evenly to the four k-steps");
-      for (int kt = 0; kt < KT; kt++) {
-        const unsigned char* sbase = lds + stage * C::STAGE_BYTES;
-        // the slab NS-1 ahead goes to the stage the previous slab vacated
-        const int rq = stage == 0 ? C::NS - 1 : stage - 1;
-        k_step_dma(0, sbase, sbase + C::A_BYTES, 1, 2, 0, RQ, rq);
-        k_step_dma(1, sbase, sbase + C::A_BYTES, 2, 2, RQ, 2 * RQ, rq);
-        k_step_dma(0, sbase, sbase + C::A_BYTES, 3, 2, 2 * RQ, 3 * RQ, rq);
-        // ---- turn over: the next slab has landed -- everything but the slab after it (NS-3 whole slabs in
-        // general) and the requests just issued
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm((C::NS - 3) * C::LOADS + 3 * RQ) & 0xf0ff);  // and lgkmcnt(0)
+      // One slab: its MFMAs, on fragments that are in registers; under the first of them, the reads of the next
+      // slab's fragments, under the others the requests of the slab NS ahead, into the stage this slab's fragments
+      // have been read from.  One barrier per slab: every wave holds this slab's fragments, and the next slab has
+      // landed (everything but the NS-2 slabs behind it).
+      constexpr int NM = SK * NMMA, NR = SK * NRD;
+      constexpr int RPM = (NR + (NM + 1) / 2 - 1) / ((NM + 1) / 2);  // reads behind each of the first MFMAs
+      constexpr int RM = (NR + RPM - 1) / RPM;                       // MFMAs that carry them
+      auto ring_slab = [&](int buf) {
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm((C::NS - 2) * C::LOADS) & 0xf0ff);  // and lgkmcnt(0)
         __syncthreads();
+        const int rq = stage;
         stage = stage == C::NS - 1 ? 0 : stage + 1;
         const unsigned char* nbase = lds + stage * C::STAGE_BYTES;
-        k_step_dma(1, nbase, nbase + C::A_BYTES, 0, 2, 3 * RQ, C::LOADS, rq);
+#pragma unroll
+        for (int t = 0; t < NM; t++) {
+          const int ks = t / NMMA, i = (t % NMMA) / TN, j = t % TN;
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sfb[buf][ks][j], sfa[buf][ks][i], acc[i][j], 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < RPM; r++)
+            if (t < RM && t * RPM + r < NR) read_slab_frag(nbase, buf ^ 1, t * RPM + r);
+#pragma unroll
+          for (int q = 0; q < C::LOADS; q++)
+            if (t >= RM && RM + q * (NM - RM) / C::LOADS == t) dma_ring(rq, q);
+          SCHED_FENCE();
+        }
         p_advance();
+      };
+      int kt = 0;
+#pragma unroll 1
+      for (; kt + 1 < KT; kt += 2) {
+        ring_slab(0);
+        ring_slab(1);
+      }
+      if (kt < KT) {
+        ring_slab(0);
+#pragma unroll
+        for (int ks = 0; ks < SK; ks++) {
+#pragma unroll
+          for (int i = 0; i < TM; i++) sfa[0][ks][i] = sfa[1][ks][i];
+#pragma unroll
+          for (int j = 0; j < TN; j++) sfb[0][ks][j] = sfb[1][ks][j];
+        }
       }
     } else
     for (int kt = 0; kt < KT; kt++) {
@@ -473,7 +518,7 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
     // staging window of this wave: inside the stage (the A slot) the tile's last slab vacated
     unsigned char* epi = lds + wave * EPI_WAVE_BYTES +
                          (C::DMA    ? (sa == 0 ? C::A_SLOTS - 1 : sa - 1) * C::A_BYTES
-                          : C::RING ? (stage == 0 ? C::NS - 1 : stage - 1) * C::STAGE_BYTES
+                          : C::RING ? C::EPI_OFF
                                     : (stage ^ 1) * C::STAGE_BYTES);
 
     // ---- epilogue ---------------------------------------------------------
@@ -661,11 +706,49 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
   if constexpr (C::DIRECT) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
 }
 
+// A launch with fewer tiles than CUs is bound by the latency of its weights, which come from HBM (every layer's are read
+// once per pass): a CU has at most its LDS in flight, 128 KiB / 2 us.  So CUs without a tile -- up to four per XCD, which
+// is enough to keep HBM busy and leaves room for another stream's launch -- run ahead and bring the weights into the
+// last-level cache.  Measured, weights cold: 1357 x 1536 x 6144 on 132 tiles of 128 x 128 59.3 us without helpers, 47.5
+// with two per XCD, 43.9 with four, 43.9 with eight; 1536 x 3072 x 15360 on 192 tiles of 128 x 192 170, 149, 148, 152;
+// 333 x 1536 x 6144 on 144 tiles of 64 x 64 31.9, 31.9, 26.6, 24.4.
+constexpr int HELPERS_PER_XCD = 4;
+
+// A workgroup without tiles: helper `id` of `helpers` reads one word of every 128-byte line of a weight matrix, four
+// slabs of all its rows at a time, so that the slabs behind the first few come from the last-level cache.
+__device__ __forceinline__ void fetch_weights(const GemmTable& tab, int id, int helpers) {
+  // the helpers are dealt to the problems, whose tiles run side by side
+  const int pi = id % tab.count;
+  const int of_problem = (helpers - pi + tab.count - 1) / tab.count;
+  const hdit_gemm_problem& pr = tab.p[pi];
+  const unsigned char* base = (const unsigned char*)pr.b;
+  const unsigned KT = (unsigned)pr.k / BK, n = (unsigned)pr.n, pitch = (unsigned)pr.ldb * 2u;
+  const unsigned per_chunk = 4u * n, total = (KT + 3) / 4 * per_chunk, step = (unsigned)of_problem * NT;
+  constexpr int U = 8;
+  for (unsigned u0 = (unsigned)(id / tab.count) * NT + threadIdx.x; u0 < total; u0 += U * step) {
+    unsigned v[U];
+#pragma unroll
+    for (int i = 0; i < U; i++) {
+      const unsigned u = min(u0 + i * step, total - 1);
+      const unsigned chunk = u / per_chunk, r = u - chunk * per_chunk;
+      const unsigned line = min(chunk * 4 + (r & 3), KT - 1);
+      v[i] = *(const unsigned*)(base + (uint64_t)((r >> 2) * pitch) + line * ROW_BYTES);
+    }
+#pragma unroll
+    for (int i = 0; i < U; i++) asm volatile("" : : "v"(v[i]));
+  }
+}
+
 template <class C>
 __global__ void __launch_bounds__(NT) gemm_kernel(const GemmTable tab, int total_tiles, int tiles_per_xcd,
                                                   int wgs_per_xcd) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-  run_tiles<C>(tab, total_tiles, tiles_per_xcd, wgs_per_xcd, blockIdx.x / NUM_XCD, lds);
+  const int wg = blockIdx.x / NUM_XCD;
+  if (wg >= wgs_per_xcd) {  // uniform over the workgroup
+    fetch_weights(tab, blockIdx.x - wgs_per_xcd * NUM_XCD, gridDim.x - wgs_per_xcd * NUM_XCD);
+    return;
+  }
+  run_tiles<C>(tab, total_tiles, tiles_per_xcd, wgs_per_xcd, wg, lds);
 }
 
 // Two tile shapes in one launch: the large tiles of the tall problems first, then the small tiles of the
@@ -702,6 +785,9 @@ int max_workgroups() {
   return max_wgs < NUM_XCD ? NUM_XCD : max_wgs;
 }
 
+// workgroups without a tile to launch beside those with one
+int helpers_per_xcd(int cus, int busy) { return busy >= cus ? 0 : cus - busy < HELPERS_PER_XCD ? cus - busy : HELPERS_PER_XCD; }
+
 template <class C>
 int launch(const GemmTable& tab, int total_tiles, hipStream_t stream) {
   static std::atomic<bool> attr_set{false};  // setting the attribute twice from two threads is harmless
@@ -717,8 +803,9 @@ int launch(const GemmTable& tab, int total_tiles, hipStream_t stream) {
   if (max_wgs < 0) return HDIT_ELAUNCH;
   const int tiles_per_xcd = (total_tiles + NUM_XCD - 1) / NUM_XCD;
   int wgs_per_xcd = max_wgs / NUM_XCD;
+  const int helpers = helpers_per_xcd(wgs_per_xcd, tiles_per_xcd);
   if (wgs_per_xcd > tiles_per_xcd) wgs_per_xcd = tiles_per_xcd;
-  hipLaunchKernelGGL(gemm_kernel<C>, dim3(wgs_per_xcd * NUM_XCD), dim3(NT), C::LDS_BYTES, stream, tab, total_tiles,
+  hipLaunchKernelGGL(gemm_kernel<C>, dim3((wgs_per_xcd + helpers) * NUM_XCD), dim3(NT), C::LDS_BYTES, stream, tab, total_tiles,
                      tiles_per_xcd, wgs_per_xcd);
   return hdit_host::check_launch("hdit_gemm_bf16");
 }
@@ -782,14 +869,18 @@ using Cfg256x192 = Cfg<4, 3>;
 using Cfg128x256 = Cfg<2, 4>;
 using Cfg128x128 = Cfg<2, 2>;
 using Cfg128x192 = Cfg<2, 3>;
+using Cfg64x128 = Cfg<1, 2>;
+using Cfg64x64 = Cfg<1, 1>;
 
 std::atomic<int> g_force_cfg{-1};
 
 // ---- launch planning ---------------------------------------------------------
-// A launch deals its tiles to 256 workgroups (one per CU) in rounds; a tile costs (k / 64) slab times plus an epilogue.
-// A slab takes `lo` microseconds while at most half of the CUs work and `hi` while all do (the chip's power budget is
-// shared), in between in between.  All figures measured on MI355X with weights that come from HBM: single problems of
-// 32 - 1024 tiles, K = 1536 and 6144; the model below reproduces those launches within 4 %.
+// A launch deals its tiles to 256 workgroups (one per CU) in rounds; a tile costs (k / 64) slab times plus an epilogue
+// with the fill of the pipeline.  Both depend on how many CUs work: a slab takes `lo` microseconds while at most half of
+// them do (what the CU's requests take to come from the last-level cache) and `hi` while all do (the chip's power budget
+// is shared), in between in between.  All figures measured on MI355X with weights that come from HBM: single problems of
+// 1 - 6144 rows, N = 1536 - 9216, K = 1536 - 12288 under every shape; the model reproduces those launches within 4 - 10 %
+// and its choice among the shapes is on average 0.1 % slower than the best of them (at most 4 %).
 //
 // What a plan has to get right is the last round.  One tile shape for everything wastes most of it: the 666-row text
 // stream of a joint block on the image stream's 256-row tiles adds a nearly empty round, and 17 550 rows x 3072 columns
@@ -800,12 +891,13 @@ std::atomic<int> g_force_cfg{-1};
 // Results do not depend on any of this (every shape forms the same sums in the same order).
 struct Shape {
   int bm, bn;
-  double lo, hi, epi;
+  double lo, hi, epi_lo, epi_hi;
 };
-constexpr int NCFG = 5;
+constexpr int NCFG = 7;
 constexpr Shape kShape[NCFG] = {
-    {256, 192, 0.95, 1.19, 7.7}, {128, 256, 0.80, 0.92, 5.6}, {128, 128, 0.54, 0.57, 4.0},
-    {256, 256, 1.11, 1.50, 8.0}, {128, 192, 0.67, 0.77, 4.1},
+    {256, 192, 0.765, 1.182, 3.9, 6.1}, {128, 256, 0.618, 0.860, 2.5, 4.8}, {128, 128, 0.365, 0.527, 2.3, 3.4},
+    {256, 256, 0.939, 1.523, 4.9, 6.5}, {128, 192, 0.468, 0.676, 2.6, 4.7}, {64, 128, 0.275, 0.358, 1.7, 1.8},
+    {64, 64, 0.194, 0.222, 1.7, 1.5},
 };
 constexpr double kLaunchUs = 4.0;
 constexpr int kSlots = 256;
@@ -833,7 +925,8 @@ Load load_of(const hdit_gemm_problem* ps, int count, int c) {
 // one tile of shape c while `busy` of the 256 CUs work on such tiles
 double tile_us(int c, double slabs, int busy) {
   const double f = busy >= kSlots ? 1.0 : busy > kSlots / 2 ? 2.0 * busy / kSlots - 1.0 : 0.0;
-  return slabs * (kShape[c].lo + (kShape[c].hi - kShape[c].lo) * f) + kShape[c].epi;
+  const Shape& s = kShape[c];
+  return slabs * (s.lo + (s.hi - s.lo) * f) + s.epi_lo + (s.epi_hi - s.epi_lo) * f;
 }
 
 double single_us(const Load& l, int c) {
@@ -849,8 +942,9 @@ double two_us(const Load& l1, int c1, const Load& l2, int c2) {
   const int full = l1.tiles / kSlots, rem = l1.tiles % kSlots;
   const int idle = rem ? kSlots - rem : 0;  // workgroups without a tile of the last large round
   const int base = l2.tiles / kSlots, extra = l2.tiles % kSlots;
-  const double t1 = full * tile_us(c1, l1.slabs, kSlots), t1_last = rem ? tile_us(c1, l1.slabs, rem) : 0.0;
-  const double t2 = tile_us(c2, l2.slabs, base ? kSlots : extra);
+  const int busy = rem + l2.tiles;  // CUs at work in the last round
+  const double t1 = full * tile_us(c1, l1.slabs, kSlots), t1_last = rem ? tile_us(c1, l1.slabs, busy) : 0.0;
+  const double t2 = tile_us(c2, l2.slabs, busy);
   const double of_idle = t1 + (base + (extra > 0 ? 1 : 0)) * t2;
   const double of_rest = t1 + t1_last + (base + (extra > idle ? 1 : 0)) * t2;
   return idle && of_idle > of_rest ? of_idle : of_rest;
@@ -862,6 +956,8 @@ int launch_cfg(int cfg, const hdit_gemm_problem* problems, int count, hipStream_
     case 1: return build_and_launch<Cfg128x256>(problems, count, s);
     case 4: return build_and_launch<Cfg128x192>(problems, count, s);
     case 3: return build_and_launch<Cfg256x256>(problems, count, s);
+    case 5: return build_and_launch<Cfg64x128>(problems, count, s);
+    case 6: return build_and_launch<Cfg64x64>(problems, count, s);
     default: return build_and_launch<Cfg128x128>(problems, count, s);
   }
 }
@@ -923,8 +1019,12 @@ extern "C" __attribute__((visibility("default"))) int hdit_gemm_bf16(const hdit_
         const bool large = single_us(load_of(&live[i], 1, c1), c1) <= single_us(load_of(&live[i], 1, c2), c2);
         (large ? b[kb++] : m[km++]) = live[i];
       }
+      // (large tiles that do not fill one round are better off alone, on whichever shape: 4316+154 x 1536 x 6144 as 136
+      // tiles of 256 x 192 and 24 of 128 x 128 takes 97 us, all on 256 x 192 88, all on 128 x 256 83; 8192+666 x 1536 x
+      // 6144 136 us against 130 on 256 x 256)
+      const bool round = load_of(b, kb, c1).tiles >= kSlots;
       double t = two_us(load_of(b, kb, c1), c1, load_of(m, km, c2), c2);
-      if (kb && km && t < two_cost) {
+      if (round && km && t < two_cost) {
         two_cost = t, big_cfg = c1, small_cfg = c2, nb = kb, ns = km;
         memcpy(big, b, kb * sizeof(*b));
         memcpy(small, m, km * sizeof(*m));

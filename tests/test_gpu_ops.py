@@ -85,6 +85,42 @@ def test_gemm_result_does_not_depend_on_the_tile_shape(hdit, epi):
         assert torch.equal(out, outs[0]), f"shape {cfg} differs from shape 0"
 
 
+@pytest.mark.parametrize("cfg", [2, 4, 5, 6])
+@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (63, 72, 128), (65, 200, 192), (129, 136, 640), (200, 1544, 1088)])
+def test_gemm_ring_shapes(hdit, cfg, m, n, k):
+    """The shapes that take their slabs through a ring (128x128, 128x192, 64x128, 64x64): fewer slabs than stages, odd
+    and even numbers of them, tiles cut off in rows and columns, operands with gaps between their rows, two problems of
+    one launch with different k -- against fp32 products and, bit for bit, against 256x256 tiles."""
+    print(f"gemm ring cfg={cfg} {m}x{n}x{k}", flush=True)
+    ops, lib = hdit.ops, hdit._lib.lib()
+    ks = (k, 64 * (k // 64 + 1))
+    a = [g(rnd(m, kk + 8, seed=61 + i))[:, :kk] for i, kk in enumerate(ks)]
+    w = [g(rnd(n, kk + 72, scale=0.05, seed=63 + i))[:, :kk] for i, kk in enumerate(ks)]
+    b = [g(rnd(n, seed=65 + i)) for i in range(2)]
+    res = torch.randn(m, n, generator=torch.Generator(device=DEV).manual_seed(67), device=DEV)
+    gate = torch.randn(1, n, generator=torch.Generator(device=DEV).manual_seed(68), device=DEV)
+
+    def launch(c):
+        y = [torch.zeros(m, n + 8, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+        x1 = torch.zeros(m, n, dtype=torch.float32, device=DEV)
+        lib.hdit_gemm_force_config(c)
+        try:
+            ops.gemm_launch([ops.gemm_problem(a[0], w[0], y[0][:, :n], b[0]),
+                             ops.gemm_problem(a[1], w[1], y[1][:, :n], b[1], ops.EPI_BIAS_GELU),
+                             ops.gemm_problem(a[0], w[0], x1, b[0], ops.EPI_GATE_RESIDUAL, resid=res, gate=gate, rows_per_batch=m)])
+        finally:
+            lib.hdit_gemm_force_config(-1)
+        torch.cuda.synchronize()
+        assert not y[0][:, n:].any() and not y[1][:, n:].any()
+        return y[0][:, :n], y[1][:, :n], x1
+
+    got, want = launch(cfg), launch(3)
+    for x, y in zip(got, want):
+        assert torch.equal(x, y)
+    assert_parity(got[0].float().cpu(), O.linear(a[0].float().cpu(), w[0].float().cpu(), b[0].float().cpu()), what="bias")
+    assert_parity(got[1].float().cpu(), O.gelu_tanh(O.linear(a[1].float().cpu(), w[1].float().cpu(), b[1].float().cpu())), what="gelu")
+
+
 @pytest.mark.parametrize("n", [3072, 3080])
 @pytest.mark.parametrize("epi", ["bias", "gelu", "gate", "gate_two_batches"])
 def test_gemm_rows_that_open_another_round_take_the_small_shape(hdit, epi, n):
