@@ -134,7 +134,7 @@ class SD3TransformerBlocks(nn.Module):
         the previous block of this chain of blocks left to this one's first normalisation (``_Chain``); updated
         with what this block leaves to the next.  ``batch0``: index of the
         first batch element of ``hidden`` within the ``temb`` the modulation ``mods`` was computed for.
-        ``defer``: a list -- the call is prepared and appended to it instead of launched (``_launch_front``).
+        ``defer``: a list -- the call is prepared and appended to it, with what has to live until its launch, instead of launched.
         ``patch``: index of the pipeline patch in patch mode.  The later patches of a step are fed the text states
         the first one stored (``transformer_sd3.py:131-146``), so the text stream's keys and values are the same
         numbers for all of them: the first patch's call leaves them in a buffer and the later ones take them from
@@ -184,8 +184,10 @@ class SD3TransformerBlocks(nn.Module):
             calls[i].launch()
             del ws  # stream-ordered reuse: the workspace may be freed as soon as the launches are queued
         else:
-            # the struct is filled, the launch is the caller's (merged with the other blocks of its front)
-            defer.append((calls[i], ws))
+            # the struct is filled, the launch is the caller's (merged with the other blocks of its front): until
+            # then the streams it reads stay alive too, or another block of the front is given their memory for its
+            # outputs and writes it in the very launch that reads it
+            defer.append((calls[i], (ws, hidden, encoder, temb)))
         return encoder_out, hidden_new
 
     def _kv_buffer(self, i: int, hidden: torch.Tensor):
@@ -405,7 +407,7 @@ class SD3TransformerBlocks(nn.Module):
                             i, calls, mods, hidden[p], cache[i], temb, skip_text_output=True, kv_buffer=kv[0],
                             kv_row0=kv[1], patch=p, defer=group, chain=chains[p])
                 ops.sd3_blocks_launch([c for c, _ in group])
-                del group  # the workspaces: stream-ordered reuse once the launches are queued
+                del group  # workspaces and inputs: stream-ordered reuse once the launches are queued
         finally:
             rs.pipeline_patch_idx = 0
         return hidden

@@ -120,6 +120,46 @@ def test_pipefusion_patch_graph_replay_from_restored_buffers(hdit):
         torch.cuda.synchronize()
 
 
+def test_pipefusion_front_writes_no_memory_it_reads(hdit, monkeypatch):
+    """The blocks of a front run as one merged call, so no block's outputs or workspace may lie where another one's
+    inputs do (a stream that a block has been prepared with must outlive the merged launch)."""
+    from hetu_dit_amd import synthetic, transformer
+    from hetu_dit_amd.runtime_state import get_runtime_state
+
+    B, Ni, Nt, D, H, P, L = 2, 768, 77, 256, 4, 3, 5
+    with torch.device(DEV):
+        stack = transformer.SD3TransformerBlocks(L, D, H, 64)
+    synthetic.init_module_(stack, 31)
+    e, t = dev_randn((B, Nt, D), 32), dev_randn((B, D), 33)
+    rs = get_runtime_state()
+    rs.set_token_patches([Ni // P * i for i in range(P + 1)])
+    rs.set_patched_mode(False)
+    stack(dev_randn((B, Ni, D), 34), e, t)
+    rs.set_patched_mode(True)
+    launch, fronts = hdit.ops.sd3_blocks_launch, []
+
+    def checked(calls):
+        reads, writes = [], []
+        for n, c in enumerate(calls):
+            a = c.args
+            img, txt = B * a.n_img * D, B * a.n_txt * D
+            reads += [(n, q, size) for q, size in ((a.hidden, img * (4 if a.hidden_f32 else 2)), (a.encoder, txt * (4 if a.encoder_f32 else 2)),
+                                                  (a.pending_img, img * 2), (a.pending_txt, txt * 2)) if q]
+            writes += [(n, q, size) for q, size in ((a.hidden_out, img * (4 if a.out_f32 else 2)), (a.encoder_out, txt * (4 if a.out_f32 else 2)),
+                                                   (a.defer_img, img * 2), (a.defer_txt, txt * 2), (a.workspace, a.workspace_bytes)) if q]
+        for n, q, size in writes:
+            for n2, q2, size2 in reads + [w for w in writes if w[0] != n]:
+                assert q + size <= q2 or q2 + size2 <= q, f"front {len(fronts)}: block {n} writes what block {n2} uses"
+        fronts.append(len(calls))
+        launch(calls)
+
+    monkeypatch.setattr(hdit.ops, "sd3_blocks_launch", checked)
+    for _ in range(2):
+        stack.forward_patches([dev_randn((B, Ni // P, D), 35 + p) for p in range(P)], e, t, num_streams=1)
+    torch.cuda.synchronize()
+    assert max(fronts) == P and len(fronts) == 2 * (L + P - 1)
+
+
 def test_pipefusion_grouped_fronts_graph_replay(hdit):
     """``forward_patches(num_streams=1)``: every front of independent (patch, layer) blocks is one merged
     ``hdit_block_sd3_multi`` call on the caller's stream, so the whole PipeFusion step can be recorded into a graph.
