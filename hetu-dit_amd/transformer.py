@@ -62,6 +62,14 @@ class _Chain:
             self.txt = left[1] if left is not None else None
 
 
+# Rows (image + text) per chain from which a pass of several batch elements runs as chains on side streams.  Below, one
+# chain of all elements is faster: half the launches and half the host time, weights fetched once, launches that fill
+# more of the GPU.  SD3 step at B = 2 on two streams / one, ms: 256+77 rows per element 4.4 / 3.4, 784+333 6.7 / 5.4,
+# 1024+333 6.6 / 6.5, 2112+333 11.4 / 10.1, 3364+333 16.6 / 15.8, 3600+333 17.0 / 16.8, 3844+333 18.5 / 19.2, 4096+333
+# 19.3 / 19.9, 4356+333 21.1 / 21.1.
+LANE_ROWS = 4096
+
+
 class SD3TransformerBlocks(nn.Module):
     """The 24 joint blocks of the SD3 transformer with the reference's block loop.
 
@@ -72,7 +80,7 @@ class SD3TransformerBlocks(nn.Module):
 
     * ``batch_streams``: a full-sequence pass of B >= 2 batch elements (the CFG pair) runs the elements as
       independent chains on that many side streams, blocks issued alternately -- one chain's launches fill the
-      CUs another's partial last round of tiles leaves idle (about 5 % of the SD3 step at B = 2);
+      CUs another's partial last round of tiles leaves idle (``LANE_ROWS`` says from which size on);
     * ``forward_patches``: the patches of a PipeFusion step, one block apart.
 
     Neither is recorded into a HIP graph: under capture, and whenever a per-launch timer is installed, the pass
@@ -225,6 +233,8 @@ class SD3TransformerBlocks(nn.Module):
             temb = temb.contiguous()
             mods = self.modulation.precompute_by_module(temb)
             lanes = min(self.batch_streams, hidden_states.shape[0])
+            if hidden_states.shape[0] * (hidden_states.shape[1] + encoder_hidden_states.shape[1]) < lanes * LANE_ROWS:
+                lanes = 1
             if not rs.patch_mode and lanes > 1 and not torch.cuda.is_current_stream_capturing():
                 return self._forward_batch_lanes(calls, mods, hidden_states, encoder_hidden_states, temb, lanes)
         chain = _Chain() if self.defer_residuals else None

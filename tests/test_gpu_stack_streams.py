@@ -74,10 +74,12 @@ def run_step_sequence(stack, B, Ni, Nt, D, P, entry_points, batch_streams, patch
 
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("B", [1, 2, 3])
-def test_entry_point_blocks_lanes_and_overlapped_patches_give_the_same_bits(hdit, B, fp8):
+def test_entry_point_blocks_lanes_and_overlapped_patches_give_the_same_bits(hdit, B, fp8, monkeypatch):
+    from hetu_dit_amd import transformer
     from hetu_dit_amd.runtime_state import reset_runtime_state
 
     Ni, Nt, D, H, P, L = 1024, 77, 256, 4, 4, 5
+    monkeypatch.setattr(transformer, "LANE_ROWS", 0)  # batch lanes at any size
     stack = make_stack(L, D, H, 31)
     for block in stack.transformer_blocks:
         block.attn.fp8_attention = fp8  # the attention of every form on the fp8-e4m3 path
@@ -124,6 +126,38 @@ def test_forward_patches_refuses_what_it_cannot_run(hdit):
     with pytest.raises(ValueError):
         stack.forward_patches(xs, e, t, num_streams=0)
     assert len(stack.forward_patches(xs, e, t)) == P
+
+
+def test_prefilled_calls_follow_swapped_weights(hdit):
+    """The whole-block calls re-read the weights' addresses per pass: a re-assigned ``.data``, a replaced parameter, a
+    replaced feed-forward and a switched flag each take effect in the next pass, as kernel by kernel."""
+    D, H, L = 256, 4, 3
+    stack = make_stack(L, D, H, 91)
+    x, e, t = dev_randn((2, 512, D), 92), dev_randn((2, 40, D), 93), dev_randn((2, D), 94)
+
+    def both():
+        stack.use_block_entry_points, stack.batch_streams = False, 1
+        want = stack(x, e, t).clone()
+        stack.use_block_entry_points, stack.batch_streams = True, 2
+        got = stack(x, e, t)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        return want
+
+    seen = [both()]
+    b = stack.transformer_blocks[1]
+    swaps = [
+        lambda: setattr(b.ff.module.net[2].weight, "data", b.ff.module.net[2].weight.data * 0.5),
+        lambda: setattr(b.attn.module.to_k.weight, "data", b.attn.module.to_k.weight.data * 0.5),
+        lambda: setattr(b.attn.module.add_v_proj.bias, "data", b.attn.module.add_v_proj.bias.data + 1.0),
+        lambda: setattr(b.attn, "output_bias", torch.nn.Parameter(b.attn.output_bias.data + 1.0, requires_grad=False)),
+        lambda: setattr(b, "ff_context", make_stack(2, D, H, 96).transformer_blocks[0].ff_context),
+        lambda: setattr(b.attn, "fp8_attention", True),
+    ]
+    for n, swap in enumerate(swaps):
+        swap()
+        seen.append(both())
+        assert not torch.equal(seen[-1], seen[-2]), f"swap {n} changed nothing"
 
 
 def test_stack_takes_changing_batch_and_sequence_sizes(hdit):
