@@ -601,8 +601,9 @@ constexpr int PIPE_MIN_TILES = 3;
 
 #define SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
 
+// true: the fixed reference did not hold, nothing has been written, the whole workgroup starts over
 template <int HD>
-__device__ __forceinline__ void attn_pipe_body(const AttnParams& P, int q_tiles, unsigned char* lds, int block_id, int nblocks) {
+__device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles, unsigned char* lds, int block_id, int nblocks) {
   using PL = PipeLds<HD>;
   constexpr int KS = HD / 16, DB = HD / 32, CPR = HD / 8, NCH = BKV * CPR / 256, RPI = 64 / CPR, ROW = PL::ROW;
   constexpr int PIPE_TILE = PL::TILE, PIPE_V_OFF = PL::V_OFF, PIPE_FLAG_OFF = PL::FLAG_OFF;
@@ -748,8 +749,7 @@ __device__ __forceinline__ void attn_pipe_body(const AttnParams& P, int q_tiles,
     }
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
     __syncthreads();  // the flag barrier
-    if (*(volatile lds_int*)flag) attn_tracked_body<HD>(P, q_tiles, lds, block_id, nblocks);
-    return;
+    return *(volatile lds_int*)flag != 0;
   }
 
   // ---- Q fragments, softmax scale folded in: lane holds q row (qb*32 + l32), d = 16*ks + 8*lh .. +7
@@ -991,10 +991,7 @@ __device__ __forceinline__ void attn_pipe_body(const AttnParams& P, int q_tiles,
     if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *flag = 1;
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
     __syncthreads();
-    if (*(volatile lds_int*)flag) {
-      attn_tracked_body<HD>(P, q_tiles, lds, block_id, nblocks);
-      return;
-    }
+    if (*(volatile lds_int*)flag) return true;
   }
 
   // ---- normalise and write O[q][d]: lane owns q = qb*32 + l32, d = 32*db + 8*(v/4) + 4*lh + v%4
@@ -1015,13 +1012,37 @@ __device__ __forceinline__ void attn_pipe_body(const AttnParams& P, int q_tiles,
         *(i32x2*)(op + db * 32 + g * 8 + lh * 4) = out;
       }
   }
+  return false;
 }
 
+// The second pass.  It takes its arguments from the kernel's parameter block again, through an address the compiler
+// cannot connect with the first pass: whatever the two passes would share -- segment addresses, strides, positions --
+// would otherwise be held in scalar registers, or spilled, all through the first pass (83 of them), and its loop is
+// scheduled around that.  A second pass inlined twice (waves with and without query rows), arguments shared -> this
+// form: d = 128, 24 heads, 16896 x 16896 3444 -> 3336 us (1.02 -> 1.05 PFLOP/s), 4608 x 4608 274 -> 267, 1536 x 1536
+// 55.3 -> 52.2; d = 64, 1357 x 1357 28.9 -> 27.9, 333 x 333 13.4 -> 12.8.  Without any second pass the same d = 128
+// times, 26.5 and 12.6.
+template <int HD>
+__device__ __forceinline__ void attn_second_pass(size_t params_at, int q_tiles, unsigned char* lds, int block_id, int nblocks) {
+  typedef const __attribute__((address_space(4))) int64_t* const_ptr;
+  uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr() + params_at;
+  asm volatile("" : "+s"(at), "+s"(q_tiles), "+s"(block_id), "+s"(nblocks));
+  static_assert(sizeof(AttnParams) % 8 == 0, "copied in 8-byte pieces");
+  struct Raw {
+    int64_t v[sizeof(AttnParams) / 8];
+  } raw;
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(AttnParams) / 8; i++) raw.v[i] = ((const_ptr)at)[i];
+  const AttnParams P = __builtin_bit_cast(AttnParams, raw);
+  __syncthreads();  // every wave has read the flag, whose bytes this pass may overwrite
+  attn_tracked_body<HD>(P, q_tiles, lds, block_id, nblocks);
+}
 
 template <int HD>
 __global__ void __launch_bounds__(256, 1) attn_fwd_pipe_kernel(const AttnParams P, int q_tiles) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  attn_pipe_body<HD>(P, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x);
+  if (attn_pipe_body<HD>(P, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x))
+    attn_second_pass<HD>(0, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x);
 }
 
 template <int HD>
@@ -1032,7 +1053,8 @@ __global__ void __launch_bounds__(256, 1) attn_fwd_pipe_multi_kernel(const AttnM
   while (i + 1 < M.count && (int)blockIdx.x >= M.start[i + 1]) i++;
   const int local = (int)blockIdx.x - M.start[i];
   if (local >= M.nblocks[i]) return;
-  attn_pipe_body<HD>(M.p[i], M.q_tiles[i], lds, local, M.nblocks[i]);
+  if (attn_pipe_body<HD>(M.p[i], M.q_tiles[i], lds, local, M.nblocks[i]))
+    attn_second_pass<HD>(offsetof(AttnMulti, p) + i * sizeof(AttnParams), M.q_tiles[i], lds, local, M.nblocks[i]);
 }
 
 // Host side of a multi launch: the table of `count` problems, ranges padded to multiples of 8 workgroups.
