@@ -25,6 +25,7 @@ HIPCC_FLAGS = [
 # those without a copy per score.  In the VGPR form the allocator decides per value.
 EXTRA_FLAGS = {
     "attention_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "attention_bf16_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

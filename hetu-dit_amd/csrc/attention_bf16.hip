@@ -104,21 +104,68 @@ bool to_params(const hdit_attn_args* a, AttnParams& P, int& q_tiles, unsigned& g
 namespace {
 // Which kernel serves a problem: decided from the problem alone, so that it gets the same kernel -- and the same
 // bits -- launched on its own or merged with others.
-// d = 64: one wave per SIMD (the pipelined kernel) pays off while every workgroup has a CU to itself and some to
-// spare (measured: 68 against 81 us for 144 workgroups); from about 5/8 of the CUs upwards, and for grids of
-// several rounds, two workgroups per CU hiding each other's stalls serve better (SD3 step shape, 864
-// workgroups: 288 against 273 us), and a merged launch of such problems wants the two-per-CU kernel anyway.
 // d = 128: the tracked kernel runs one wave per SIMD as well, so the pipelined one serves every grid.
-// HDIT_ATTN_PIPE=0 keeps every launch on the tracked-reference kernels, =1 puts every eligible launch on the
+// d = 64: what decides is how the workgroups fill the CUs, in microseconds per tile of 64 keys (measured on MI355X for
+// one and two batch elements of 24 heads and 333 - 4470 rows, less a fixed 4.5 us):
+//   small      (128 query rows, three workgroups per CU)   0.75 with one per CU, 1.10 with two, 1.60 with three
+//   tracked    (256 rows, two per CU)                       1.16, 1.95
+//   pipelined  (256 rows, one per CU)                       1.05 a round (1.0 while it is the only one)
+// So the small tiles serve grids that would leave CUs idle (333 rows 12.8 -> 9.2 us, 1117 rows 23.5 -> 18.0, 1024 of
+// 4429 rows 68 -> 54) or half idle in the last round (2 x 1357 rows 45 -> 39, 4000 rows 118 -> 108), the pipelined
+// kernel one full round (2445 rows 49.6 -> 43.4), the tracked kernel everything larger: per row it does the least.
+// A problem with fewer query than key rows is a patch of a pipeline, which shares its launch with the other patches of
+// the step or runs alone, and with or without text queries: its kernel must not depend on its query rows (the image
+// rows keep their bits), so it is decided by the whole sequence.  Small tiles serve both uses well (24 heads, 1024 of
+// 4429 rows: alone 54 us, pipelined 68, tracked 78) until
+// the patches of a step make more than two full rounds of the tracked kernel's.
+// HDIT_ATTN_PIPE=0 keeps every launch on the tracked-reference kernel with 256 rows, =1 puts every eligible launch on the
 // pipelined ones (for A/B timing).
-bool wants_pipelined(const hdit_attn_args* a, const AttnParams& P, unsigned grid) {
+enum Kind { TRACKED, PIPELINED, SMALL, KINDS };
+constexpr int SMALL_BQ = 128;
+
+double fill_cost(Kind kind, int64_t workgroups, int cus) {
+  const int64_t per_cu = (workgroups + cus - 1) / cus;
+  if (kind == PIPELINED) return 1.05 * (double)per_cu;
+  if (kind == TRACKED) return 1.95 * (double)(per_cu / 2) + (per_cu % 2 ? 1.16 : 0.0);
+  const int rest = (int)(per_cu % 3);
+  if (per_cu < 3) return rest == 1 ? 0.75 : 1.10;
+  return 1.60 * (double)(per_cu / 3) + 0.55 * rest;
+}
+
+// the kernel of a problem, with its grid in that kernel's tiles
+Kind choose(const hdit_attn_args* a, const AttnParams& P, int& q_tiles, unsigned& grid) {
   static const char* pipe_env = getenv("HDIT_ATTN_PIPE");
   const bool pipe_off = pipe_env && pipe_env[0] == '0', pipe_force = pipe_env && pipe_env[0] == '1';
   const bool strides_ok = a->k[0].stride_s < (1 << 22) && a->k[1].stride_s < (1 << 22) && a->v[0].stride_s < (1 << 22) &&
                           a->v[1].stride_s < (1 << 22);  // a tile step (64 rows, in bytes) fits 32 bits
-  if (pipe_off || !strides_ok || (P.skv + BKV - 1) / BKV < PIPE_MIN_TILES) return false;
-  if (a->head_dim == 128 || pipe_force) return true;
-  return (int)grid * 8 <= hdit_host::num_cus() * 5;
+  const bool can_pipe = !pipe_off && strides_ok && (P.skv + BKV - 1) / BKV >= PIPE_MIN_TILES;
+  if (a->head_dim == 128 || pipe_off || pipe_force) return can_pipe ? PIPELINED : TRACKED;
+  const int cus = hdit_host::num_cus(), tiles_small = (P.sq + SMALL_BQ - 1) / SMALL_BQ;
+  const int64_t bh = (int64_t)a->batch * a->heads;
+  bool small;
+  Kind large;
+  if (P.sq < P.skv) {
+    small = bh * ((P.skv + BQ - 1) / BQ) <= 4 * (int64_t)cus;
+    large = can_pipe && bh * q_tiles * 8 <= (int64_t)cus * 5 ? PIPELINED : TRACKED;
+  } else {
+    const double tracked = fill_cost(TRACKED, bh * q_tiles, cus), cost = fill_cost(SMALL, bh * tiles_small, cus);
+    const double piped = can_pipe ? fill_cost(PIPELINED, bh * q_tiles, cus) : 1e30;
+    // (a few per cent are less than the model resolves: 2 x 4429 rows 264.7 us on small tiles, 264.1 tracked)
+    small = cost < 0.93 * tracked && cost < piped;
+    large = piped < tracked ? PIPELINED : TRACKED;
+  }
+  if (small) {
+    q_tiles = tiles_small;
+    grid = (unsigned)(bh * tiles_small);
+    return SMALL;
+  }
+  return large;
+}
+
+int launch_one(int head_dim, const AttnParams& P, int q_tiles, unsigned grid, Kind kind, hipStream_t s) {
+  if (kind == SMALL) return hdit_attn::launch_d64_small(P, q_tiles, grid, s);
+  return head_dim == 64 ? hdit_attn::launch_d64(P, q_tiles, grid, kind == PIPELINED, s)
+                        : hdit_attn::launch_d128(P, q_tiles, grid, kind == PIPELINED, s);
 }
 }  // namespace
 
@@ -129,9 +176,8 @@ extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16(const h
   int q_tiles;
   unsigned grid;
   if (!to_params(a, P, q_tiles, grid)) return HDIT_OK;
-  hipStream_t s = (hipStream_t)stream;
-  const bool pipelined = wants_pipelined(a, P, grid);
-  rc = a->head_dim == 64 ? hdit_attn::launch_d64(P, q_tiles, grid, pipelined, s) : hdit_attn::launch_d128(P, q_tiles, grid, pipelined, s);
+  const Kind kind = choose(a, P, q_tiles, grid);
+  rc = launch_one(a->head_dim, P, q_tiles, grid, kind, (hipStream_t)stream);
   if (rc != HDIT_OK) return rc;
   return hdit_host::check_launch("hdit_attn_fwd_bf16");
 }
@@ -145,24 +191,23 @@ extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16_multi(c
     if (args[i].head_dim != args[0].head_dim) return HDIT_EINVAL;
   }
   // one merged launch per kind of kernel the problems want
-  for (int kind = 0; kind < 2; kind++) {
+  for (int kind = 0; kind < KINDS; kind++) {
     AttnParams P[HDIT_ATTN_MAX_MULTI];
     int q_tiles[HDIT_ATTN_MAX_MULTI], nblocks[HDIT_ATTN_MAX_MULTI], n = 0;
     for (int i = 0; i < count; i++) {
       unsigned grid;
       if (!to_params(&args[i], P[n], q_tiles[n], grid)) continue;
-      if ((int)wants_pipelined(&args[i], P[n], grid) != kind) continue;
+      if ((int)choose(&args[i], P[n], q_tiles[n], grid) != kind) continue;
       nblocks[n++] = (int)grid;
     }
     if (n == 0) continue;
     hipStream_t s = (hipStream_t)stream;
     int rc;
-    if (n == 1)
-      rc = args[0].head_dim == 64 ? hdit_attn::launch_d64(P[0], q_tiles[0], (unsigned)nblocks[0], kind != 0, s)
-                                  : hdit_attn::launch_d128(P[0], q_tiles[0], (unsigned)nblocks[0], kind != 0, s);
+    if (n == 1) rc = launch_one(args[0].head_dim, P[0], q_tiles[0], (unsigned)nblocks[0], (Kind)kind, s);
+    else if (kind == SMALL) rc = hdit_attn::launch_multi_d64_small(P, q_tiles, nblocks, n, s);
     else
-      rc = args[0].head_dim == 64 ? hdit_attn::launch_multi_d64(P, q_tiles, nblocks, n, kind != 0, s)
-                                  : hdit_attn::launch_multi_d128(P, q_tiles, nblocks, n, kind != 0, s);
+      rc = args[0].head_dim == 64 ? hdit_attn::launch_multi_d64(P, q_tiles, nblocks, n, kind == PIPELINED, s)
+                                  : hdit_attn::launch_multi_d128(P, q_tiles, nblocks, n, kind == PIPELINED, s);
     if (rc != HDIT_OK) return rc;
     if ((rc = hdit_host::check_launch("hdit_attn_fwd_bf16_multi")) != HDIT_OK) return rc;
   }

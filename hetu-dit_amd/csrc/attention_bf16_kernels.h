@@ -5,7 +5,8 @@
 // Joint (image + text) flash attention forward for gfx950, bf16 in/out.
 //
 // Work split: one workgroup = 4 waves = 256 query rows of one (batch, head);
-// each wave owns 64 query rows (two 32-row MFMA column blocks) and walks the
+// each wave owns 64 query rows (two 32-row MFMA column blocks; one block and
+// 128 rows per workgroup in attention_bf16_small.hip) and walks the
 // keys in tiles of 64.  K and V tiles go straight from global memory into two
 // LDS buffers (direct-to-LDS loads, one barrier per tile).
 //
@@ -59,6 +60,9 @@ struct AttnParams {
 // pipelined: take the software-pipelined kernel (the caller has checked that the problem qualifies).
 int launch_d64(const AttnParams& P, int q_tiles, unsigned grid, bool pipelined, hipStream_t stream);
 int launch_d128(const AttnParams& P, int q_tiles, unsigned grid, bool pipelined, hipStream_t stream);
+// head dim 64, one query block per wave: q_tiles of 128 query rows
+int launch_d64_small(const AttnParams& P, int q_tiles, unsigned grid, hipStream_t stream);
+int launch_multi_d64_small(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
 // `count` problems of one head dim as one grid of the tracked or of the pipelined kernel
 int launch_multi_d64(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, bool pipelined, hipStream_t stream);
 int launch_multi_d128(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, bool pipelined, hipStream_t stream);
@@ -71,7 +75,11 @@ using hdit_attn::AttnParams;
 using hdit_attn::Seg2;
 
 constexpr int BKV = 64;   // keys per tile
-constexpr int WQ = 64;    // query rows per wave
+#ifndef HDIT_ATTN_QUERY_BLOCKS
+#define HDIT_ATTN_QUERY_BLOCKS 2  // 32-row query blocks per wave (attention_bf16_small.hip: 1)
+#endif
+constexpr int QB = HDIT_ATTN_QUERY_BLOCKS;
+constexpr int WQ = 32 * QB;  // query rows per wave
 constexpr int NWAVE = 4;
 constexpr int BQ = WQ * NWAVE;
 
@@ -196,7 +204,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
   const bool active = __builtin_amdgcn_readfirstlane(q0 < P.sq);
 
   // ---- Q fragments: lane holds q row (qb*32 + l32), d = 16*ks + 8*lh .. +7
-  bf16x8 qf[2][L::Q_IN_LDS ? 1 : KS];
+  bf16x8 qf[QB][L::Q_IN_LDS ? 1 : KS];
   unsigned char* qlds = lds + L::Q_OFF + wave * L::Q_WAVE_BYTES;
   if constexpr (L::Q_IN_LDS) {
     // the wave's 64 query rows, 16 lanes per row (coalesced 256-byte rows), into its private LDS region;
@@ -211,7 +219,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
     }
   } else
 #pragma unroll
-  for (int qb = 0; qb < 2; qb++) {
+  for (int qb = 0; qb < QB; qb++) {
     int r = min(q0 + qb * 32 + l32, P.sq - 1);
     const __bf16* rp = row_ptr(P.q, b, h, r);
 #pragma unroll
@@ -283,23 +291,24 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
       }
     }
   };
-  f32x16 oacc[DB][2];
+  f32x16 oacc[DB][QB];
 #pragma unroll
   for (int i = 0; i < DB; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int j = 0; j < QB; j++)
 #pragma unroll
       for (int v = 0; v < 16; v++) oacc[i][j][v] = 0.f;
   // running reference m of the online softmax (log2 units) and running sum per query column.  With FOLD the
   // accumulators of a score block start from negm = -m (the same value in all 16 entries: a lane owns one
   // query column per qb) and m starts at 0 until the first tile sets it to that tile's column maxima.
-  float m_run[2] = {FOLD ? 0.f : -INFINITY, FOLD ? 0.f : -INFINITY};
-  float l_run[2] = {0.f, 0.f};
-  f32x16 negm[2];
+  float m_run[QB], l_run[QB];
+  f32x16 negm[QB];
 #pragma unroll
-  for (int qb = 0; qb < 2; qb++)
+  for (int qb = 0; qb < QB; qb++) {
+    m_run[qb] = FOLD ? 0.f : -INFINITY, l_run[qb] = 0.f;
 #pragma unroll
     for (int v = 0; v < 16; v++) negm[qb][v] = 0.f;
+  }
   bool first = true;
 
   // lane-constant part of the V^T transpose-read address:
@@ -316,7 +325,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
     constexpr bool MASK = decltype(mask_tag)::value;
     const unsigned char* sv = sk + L::K_BYTES;
     // ---- S^T[kb][qb] = K_tile . Q^T (first k-step starts from a zero accumulator operand)
-    f32x16 sacc[2][2];
+    f32x16 sacc[2][QB];
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if constexpr (L::Q_IN_LDS) {
 #pragma unroll
@@ -342,8 +351,8 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
           for (int v = 0; v < 16; v++) {
             int key = kb * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
             if (key >= valid) {
-              sacc[kb][0][v] = -INFINITY;
-              sacc[kb][1][v] = -INFINITY;
+#pragma unroll
+              for (int qb = 0; qb < QB; qb++) sacc[kb][qb][v] = -INFINITY;
             }
           }
       }
@@ -356,7 +365,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
           bf16x8 kf = *(const bf16x8*)(sk + k_off + kb * 32 * L::K_ROW +
                                        (((ks * 2 + lh) ^ k_swz) << 4));
 #pragma unroll
-          for (int qb = 0; qb < 2; qb++)
+          for (int qb = 0; qb < QB; qb++)
             sacc[kb][qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[qb][L::Q_IN_LDS ? 0 : ks], ks == 0 ? (FOLD ? negm[qb] : zero16) : sacc[kb][qb], 0, 0, 0);
         }
       }
@@ -368,16 +377,16 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
       // Both key blocks start from the reference vectors.  Reading them once more here keeps them alive past the
       // second block's first MFMA, which the compiler otherwise ties to a copy of them (16 v_mov_b64 per tile)
       // instead of naming them as its addend the way the first block's does.
-      asm volatile("" : : "v"(negm[0]), "v"(negm[1]));
+      asm volatile("" : : "v"(negm[0]), "v"(negm[QB - 1]));
     }
 
     // ---- online softmax in the log2 domain.  A lane owns one query column per qb and 32 of its 64 keys;
     // the other 32 live in lane^32.
-    bf16x8 pf[2][4];  // [qb][u], u = 2*kb + half: the 16 keys of PV k-step u
+    bf16x8 pf[QB][4];  // [qb][u], u = 2*kb + half: the 16 keys of PV k-step u
     if constexpr (FOLD) {
-      float mrel[2];  // column maxima relative to the running reference
+      float mrel[QB];  // column maxima relative to the running reference
 #pragma unroll
-      for (int qb = 0; qb < 2; qb++) {
+      for (int qb = 0; qb < QB; qb++) {
         float mx = fmaxf(sacc[0][qb][0], sacc[1][qb][0]);
 #pragma unroll
         for (int v = 1; v < 16; v++) mx = fmaxf(fmaxf(mx, sacc[0][qb][v]), sacc[1][qb][v]);  // one v_max3 per step
@@ -385,10 +394,10 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
         mrel[qb] = fmaxf(__int_as_float(sw[0]), __int_as_float(sw[1]));
       }
       // move the reference (and rescale) only if some column outgrew the threshold: wave-uniform branch
-      const bool grow = first || mrel[0] > RESCALE_THRESHOLD || mrel[1] > RESCALE_THRESHOLD;
+      const bool grow = first || mrel[0] > RESCALE_THRESHOLD || mrel[QB - 1] > RESCALE_THRESHOLD;
       if (__builtin_amdgcn_ballot_w64(grow) != 0) {
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) {
+        for (int qb = 0; qb < QB; qb++) {
           const float d = first ? mrel[qb] : fmaxf(mrel[qb], 0.f);
           m_run[qb] += d;
           if (!first) {
@@ -435,7 +444,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
       }
     }
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
+    for (int qb = 0; qb < QB; qb++) {
       const float m = m_run[qb];
       float rs = l_run[qb];
 #pragma unroll
@@ -472,7 +481,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
         s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         bf16x8 vf = __builtin_bit_cast(bf16x8, both);
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++)
+        for (int qb = 0; qb < QB; qb++)
           oacc[db][qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[qb][u], oacc[db][qb], 0, 0, 0);
       }
     }
@@ -510,7 +519,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
 
   // ---- normalise and write O[q][d]: lane owns q = qb*32 + l32, d = 32*db + 8*(v/4) + 4*lh + v%4
 #pragma unroll
-  for (int qb = 0; qb < 2; qb++) {
+  for (int qb = 0; qb < QB; qb++) {
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(l_run[qb]), __float_as_int(l_run[qb]), false, false);
     const float inv = 1.0f / (__int_as_float(sw[0]) + __int_as_float(sw[1]));
     const int r = q0 + qb * 32 + l32;
@@ -529,7 +538,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
 }
 
 template <int HD>
-__global__ void __launch_bounds__(256, (HD == 64 ? 2 : 1)) attn_fwd_kernel(const AttnParams P, int q_tiles) {
+__global__ void __launch_bounds__(256, (HD == 64 ? (QB == 1 ? 3 : 2) : 1)) attn_fwd_kernel(const AttnParams P, int q_tiles) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   attn_tracked_body<HD>(P, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x);
 }
@@ -547,7 +556,7 @@ struct AttnMulti {
 };
 
 template <int HD>
-__global__ void __launch_bounds__(256, (HD == 64 ? 2 : 1)) attn_fwd_multi_kernel(const AttnMulti M) {
+__global__ void __launch_bounds__(256, (HD == 64 ? (QB == 1 ? 3 : 2) : 1)) attn_fwd_multi_kernel(const AttnMulti M) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   int i = 0;
 #pragma unroll 1
@@ -604,6 +613,7 @@ constexpr int PIPE_MIN_TILES = 3;
 // true: the fixed reference did not hold, nothing has been written, the whole workgroup starts over
 template <int HD>
 __device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles, unsigned char* lds, int block_id, int nblocks) {
+  static_assert(QB == 2, "written for two query blocks per wave");
   using PL = PipeLds<HD>;
   constexpr int KS = HD / 16, DB = HD / 32, CPR = HD / 8, NCH = BKV * CPR / 256, RPI = 64 / CPR, ROW = PL::ROW;
   constexpr int PIPE_TILE = PL::TILE, PIPE_V_OFF = PL::V_OFF, PIPE_FLAG_OFF = PL::FLAG_OFF;

@@ -337,6 +337,29 @@ def test_attention_logits_outgrow_the_first_tile(hdit, gain, skv):
         assert_parity(o[:, :, h], want[:, :, h], what=f"attention, logits outgrow the first tile, head {h}")
 
 
+@pytest.mark.parametrize("gain", [0.0, 40.0])
+@pytest.mark.parametrize("B,H,sq,skv", [
+    (1, 96, 320, 256), (1, 96, 320, 300),                       # one round of 256-row workgroups: pipelined
+    (4, 100, 200, 65), (4, 100, 200, 128), (4, 100, 256, 200),  # between one and two: tracked, 256 rows
+    (1, 2, 1, 1), (2, 2, 31, 64), (1, 3, 33, 63), (1, 2, 127, 65), (2, 1, 128, 300), (1, 2, 129, 130), (1, 2, 257, 577),  # 128 rows
+])
+def test_attention_d64_kernels(hdit, B, H, sq, skv, gain):
+    """The three kernels of head dim 64, each at sizes that the choice gives to it (on 256 CUs): cut-off query and key
+    tiles, joint sequences of two buffers whose boundary lies inside a tile, logits that outgrow the first tile's."""
+    print(f"attention d64 B={B} H={H} {sq}x{skv} gain={gain}", flush=True)
+    q, k, v = rnd(B, sq, H, 64, seed=71), rnd(B, skv, H, 64, seed=72), rnd(B, skv, H, 64, seed=73)
+    if gain:
+        k[:, skv - 1, 0] = gain * q[:, :, 0].mean(1) * 2.0
+        k[:, skv // 2, H - 1] = gain * q[:, 0, H - 1] / 8.0
+    q, k = bf16_round(q), bf16_round(k)
+    cut = lambda t, n: [g(t[:, :n].contiguous()), g(t[:, n:].contiguous())] if 0 < n < t.shape[1] else [g(t)]
+    nq, nk = sq * 2 // 3, skv * 3 // 5
+    out = hdit.ops.attention(cut(q, nq), cut(k, nk), cut(v, nk))
+    torch.cuda.synchronize()
+    want = O.attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)).transpose(1, 2)
+    assert_parity(torch.cat(out, 1), want, what="attention d64")
+
+
 @pytest.mark.parametrize("dim", [64, 1536, 3072, 4096 + 8])
 def test_layernorm_modulate(hdit, dim):
     B, T = 2, 37
