@@ -116,7 +116,7 @@ namespace {
 // A problem with fewer query than key rows is a patch of a pipeline, which shares its launch with the other patches of
 // the step or runs alone, and with or without text queries: its kernel must not depend on its query rows (the image
 // rows keep their bits), so it is decided by the whole sequence.  Small tiles serve both uses well (24 heads, 1024 of
-// 4429 rows: alone 54 us, pipelined 68, tracked 78) until
+// 4429 rows: alone 54 us, pipelined 68, tracked 78; four in one launch, one with 333 text queries, 164, pipelined 170) until
 // the patches of a step make more than two full rounds of the tracked kernel's.
 // HDIT_ATTN_PIPE=0 keeps every launch on the tracked-reference kernel with 256 rows, =1 puts every eligible launch on the
 // pipelined ones (for A/B timing).
