@@ -393,12 +393,14 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
         auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(mx), __float_as_int(mx), false, false);
         mrel[qb] = fmaxf(__int_as_float(sw[0]), __int_as_float(sw[1]));
       }
-      // move the reference (and rescale) only if some column outgrew the threshold: wave-uniform branch
+      // Move the reference (and rescale) where a column outgrew the threshold; the branch is wave-uniform, the decision
+      // every column's own (the others move by 0, which changes no bit): a query row's result does not depend on the
+      // rows it shares a wave with, so workgroups of 128 and of 256 rows give the same bits.
       const bool grow = first || mrel[0] > RESCALE_THRESHOLD || mrel[QB - 1] > RESCALE_THRESHOLD;
       if (__builtin_amdgcn_ballot_w64(grow) != 0) {
 #pragma unroll
         for (int qb = 0; qb < QB; qb++) {
-          const float d = first ? mrel[qb] : fmaxf(mrel[qb], 0.f);
+          const float d = first || mrel[qb] > RESCALE_THRESHOLD ? mrel[qb] : 0.f;
           m_run[qb] += d;
           if (!first) {
             const float alpha = __builtin_amdgcn_exp2f(-d);

@@ -360,6 +360,35 @@ def test_attention_d64_kernels(hdit, B, H, sq, skv, gain):
     assert_parity(torch.cat(out, 1), want, what="attention d64")
 
 
+@pytest.mark.parametrize("B,ni,nk,nt", [
+    (1, 4096, 4096, 333),  # whole sequence: 256-row workgroups with the text queries
+    (1, 1000, 4096, 333),  # patch whose last image rows share their wave with text rows
+    (2, 5184, 5184, 333),  # other workgroups for one batch element than for two
+    (2, 1024, 4096, 77),
+])
+def test_attention_image_rows_do_not_depend_on_the_text_queries(hdit, B, ni, nk, nt):
+    """Dropping the text queries of a joint problem, or a batch element, leaves the image rows' bits alone, whatever
+    workgroups the problem is then given -- with logits that outgrow the first tile's at different tiles for
+    neighbouring rows, so that the softmax reference of some columns of a wave moves and that of others does not."""
+    H = 24
+    print(f"attention text queries B={B} {ni}+{nt} x {nk}+{nt}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(81)
+    r = lambda n: torch.randn(B, n, H, 64, generator=gen, device=DEV)
+    q, k, v, qt, kt, vt = r(ni), r(nk), r(nk), r(nt), r(nt), r(nt)
+    q[:, ::3] *= 4.0
+    qt *= 6.0
+    q, k, v, qt, kt, vt = (t.to(torch.bfloat16) for t in (q, k, v, qt, kt, vt))
+    both = hdit.ops.attention([q, qt], [k, kt], [v, vt])[0]
+    image = hdit.ops.attention([q], [k, kt], [v, vt])[0]
+    assert torch.equal(image, both), "image rows changed with the text queries"
+    for b in range(B):
+        one = hdit.ops.attention([q[b:b + 1]], [k[b:b + 1], kt[b:b + 1]], [v[b:b + 1], vt[b:b + 1]])[0]
+        assert torch.equal(one, both[b:b + 1]), "image rows changed with the batch"
+    want = O.attention(q[:1, :200].float().transpose(1, 2).cpu(), torch.cat([k, kt], 1)[:1].float().transpose(1, 2).cpu(),
+                       torch.cat([v, vt], 1)[:1].float().transpose(1, 2).cpu()).transpose(1, 2)
+    assert_parity(both[:1, :200], want, what="attention")
+
+
 @pytest.mark.parametrize("dim", [64, 1536, 3072, 4096 + 8])
 def test_layernorm_modulate(hdit, dim):
     B, T = 2, 37
