@@ -141,6 +141,7 @@ Kind choose(const hdit_attn_args* a, const AttnParams& P, int& q_tiles, unsigned
   const bool can_pipe = !pipe_off && strides_ok && (P.skv + BKV - 1) / BKV >= PIPE_MIN_TILES;
   if (a->head_dim == 128 || pipe_off || pipe_force) return can_pipe ? PIPELINED : TRACKED;
   const int cus = hdit_host::num_cus(), tiles_small = (P.sq + SMALL_BQ - 1) / SMALL_BQ;
+  if (cus <= 0) return TRACKED;  // no device to ask: the launch reports it
   const int64_t bh = (int64_t)a->batch * a->heads;
   bool small;
   Kind large;

@@ -127,6 +127,32 @@ def test_entry_points_reject_bad_arguments_without_a_gpu(library):
     assert lib.hdit_qk_norm_rope(None, 1, 1, 1, 64, 1e-6, None) == -1
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_attention_without_a_device_returns_an_error(head_dim):
+    """The choice of the attention kernel asks for the number of CUs: with no device to ask, the call still ends with
+    an error code (in a process of its own: what it must not do is end the process)."""
+    import subprocess
+    import sys
+
+    import torch
+
+    if torch.cuda.is_available():
+        pytest.skip("there is a device")
+    code = f"""
+import ctypes
+from hetu_dit_amd import _lib
+buf = ctypes.create_string_buffer(1 << 16)
+a = _lib.AttnArgs()
+a.batch, a.heads, a.head_dim = 1, 2, {head_dim}
+for name in "qkvo":
+    s = getattr(a, name)[0]
+    s.ptr, s.stride_s, s.stride_h, s.len = (ctypes.addressof(buf) + 255) // 256 * 256, 2 * {head_dim}, {head_dim}, 32
+print(_lib.lib().hdit_attn_fwd_bf16(ctypes.byref(a), None))
+"""
+    done = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert done.returncode == 0 and done.stdout.split()[-1] == "-3", (done.returncode, done.stdout, done.stderr[-500:])
+
+
 def test_library_exports_nothing_the_header_does_not_declare(library):
     import shutil
     import subprocess
