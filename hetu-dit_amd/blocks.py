@@ -173,7 +173,9 @@ class JointTransformerBlock(nn.Module):
         """``skip_text_output``: the caller drops this block's text output (the SD3 block loop does for every
         pipeline patch after the first, ``transformer_sd3.py:131-146``), so the text stream stops after its
         q|k|v projection -- no out-projection, ``norm2_context`` or ``ff_context`` -- and ``None`` is returned
-        for it.  The image output is unchanged bit for bit.
+        for it.  The image output is unchanged bit for bit -- for a patch always; for a whole sequence of at most one
+        round of attention workgroups except in rows that share a workgroup with a text row whose logits outgrow those
+        of its first 64 keys by more than 44.
 
         ``pending`` / ``defer`` (block stacks, f32 streams): the launches of ``hdit_block_sd3`` with
         ``lazy_residual`` -- see ``_forward_lazy``."""

@@ -102,22 +102,28 @@ bool to_params(const hdit_attn_args* a, AttnParams& P, int& q_tiles, unsigned& g
 }  // namespace
 
 namespace {
-// Which kernel serves a problem: decided from the problem alone, so that it gets the same kernel -- and the same
-// bits -- launched on its own or merged with others.
+// Which kernel serves a problem.
 // d = 128: the tracked kernel runs one wave per SIMD as well, so the pipelined one serves every grid.
-// d = 64: what decides is how the workgroups fill the CUs, in microseconds per tile of 64 keys (measured on MI355X for
-// one and two batch elements of 24 heads and 333 - 4470 rows, less a fixed 4.5 us):
+// d = 64: the small and the tracked kernel give the same bits; the pipelined one, whose softmax reference is fixed, does
+// not.  So whether a problem gets the pipelined kernel is decided from the problem alone (launched on its own or merged
+// with others, it keeps its bits), and in the same way with and without the text queries of a joint sequence, whose
+// image rows keep their bits: a query segment that is left out counts as if it were there (`rows_with_text`), and query
+// patches of joint sequences never get that kernel.  (Exception: image rows in a workgroup of the pipelined kernel that
+// also holds text rows.  If a text row outgrows the fixed reference by 2^64, the tracked kernel computes the workgroup.)
+// What decides is how the workgroups fill the CUs, in microseconds per tile of 64 keys (measured on MI355X for one and
+// two batch elements of 24 heads and 333 - 4470 rows, less a fixed 4.5 us):
 //   small      (128 query rows, three workgroups per CU)   0.75 with one per CU, 1.10 with two, 1.60 with three
 //   tracked    (256 rows, two per CU)                       1.16, 1.95
-//   pipelined  (256 rows, one per CU)                       1.05 a round (1.0 while it is the only one)
+//   pipelined  (256 rows, one per CU)                       1.05 a round
 // So the small tiles serve grids that would leave CUs idle (333 rows 12.8 -> 9.2 us, 1117 rows 23.5 -> 18.0, 1024 of
 // 4429 rows 68 -> 54) or half idle in the last round (2 x 1357 rows 45 -> 39, 4000 rows 118 -> 108), the pipelined
 // kernel one full round (2445 rows 49.6 -> 43.4), the tracked kernel everything larger: per row it does the least.
 // A problem with fewer query than key rows is a patch of a pipeline, which shares its launch with the other patches of
-// the step or runs alone, and with or without text queries: its kernel must not depend on its query rows (the image
-// rows keep their bits), so it is decided by the whole sequence.  Small tiles serve both uses well (24 heads, 1024 of
+// the step or runs alone: it is decided by the whole sequence.  Small tiles serve both uses well (24 heads, 1024 of
 // 4429 rows: alone 54 us, pipelined 68, tracked 78; four in one launch, one with 333 text queries, 164, pipelined 170) until
-// the patches of a step make more than two full rounds of the tracked kernel's.
+// the patches of a step make more than two full rounds of the tracked kernel's.  The pipelined kernel serves patches of
+// longer sequences only where the keys are one segment, so that no text queries can be left out (648 of 5517 rows, two
+// batch elements: 84 us, tracked 96).
 // HDIT_ATTN_PIPE=0 keeps every launch on the tracked-reference kernel with 256 rows, =1 puts every eligible launch on the
 // pipelined ones (for A/B timing).
 enum Kind { TRACKED, PIPELINED, SMALL, KINDS };
@@ -132,6 +138,15 @@ double fill_cost(Kind kind, int64_t workgroups, int cus) {
   return 1.60 * (double)(per_cu / 3) + 0.55 * rest;
 }
 
+// The query rows of a problem, a segment counted with its key rows where its queries were left out: one that is empty
+// while the other one lies within the key segment of its own.
+int rows_with_text(const hdit_attn_args* a) {
+  int rows = a->q[0].len + a->q[1].len;
+  for (int s = 0; s < 2; s++)
+    if (a->q[s].len == 0 && a->q[1 - s].len <= a->k[1 - s].len) rows += a->k[s].len;
+  return rows;
+}
+
 // the kernel of a problem, with its grid in that kernel's tiles
 Kind choose(const hdit_attn_args* a, const AttnParams& P, int& q_tiles, unsigned& grid) {
   static const char* pipe_env = getenv("HDIT_ATTN_PIPE");
@@ -143,14 +158,17 @@ Kind choose(const hdit_attn_args* a, const AttnParams& P, int& q_tiles, unsigned
   const int cus = hdit_host::num_cus(), tiles_small = (P.sq + SMALL_BQ - 1) / SMALL_BQ;
   if (cus <= 0) return TRACKED;  // no device to ask: the launch reports it
   const int64_t bh = (int64_t)a->batch * a->heads;
+  const int rows = rows_with_text(a);
   bool small;
   Kind large;
-  if (P.sq < P.skv) {
+  if (rows < P.skv) {
     small = bh * ((P.skv + BQ - 1) / BQ) <= 4 * (int64_t)cus;
-    large = can_pipe && bh * q_tiles * 8 <= (int64_t)cus * 5 ? PIPELINED : TRACKED;
+    const bool joint = a->k[0].len > 0 && a->k[1].len > 0;
+    large = can_pipe && !joint && bh * q_tiles * 8 <= (int64_t)cus * 5 ? PIPELINED : TRACKED;
   } else {
-    const double tracked = fill_cost(TRACKED, bh * q_tiles, cus), cost = fill_cost(SMALL, bh * tiles_small, cus);
-    const double piped = can_pipe ? fill_cost(PIPELINED, bh * q_tiles, cus) : 1e30;
+    const int64_t grid_large = bh * ((rows + BQ - 1) / BQ), grid_small = bh * ((rows + SMALL_BQ - 1) / SMALL_BQ);
+    const double tracked = fill_cost(TRACKED, grid_large, cus), cost = fill_cost(SMALL, grid_small, cus);
+    const double piped = can_pipe ? fill_cost(PIPELINED, grid_large, cus) : 1e30;
     // (a few per cent are less than the model resolves: 2 x 4429 rows 264.7 us on small tiles, 264.1 tracked)
     small = cost < 0.93 * tracked && cost < piped;
     large = piped < tracked ? PIPELINED : TRACKED;

@@ -365,6 +365,9 @@ def test_attention_d64_kernels(hdit, B, H, sq, skv, gain):
     (1, 1000, 4096, 333),  # patch whose last image rows share their wave with text rows
     (2, 5184, 5184, 333),  # other workgroups for one batch element than for two
     (2, 1024, 4096, 77),
+    (2, 648, 5184, 333),   # few workgroups without the text queries, on a long sequence
+    (1, 1024, 1024, 333),  # pipelined with the text queries
+    (1, 512, 512, 50),
 ])
 def test_attention_image_rows_do_not_depend_on_the_text_queries(hdit, B, ni, nk, nt):
     """Dropping the text queries of a joint problem, or a batch element, leaves the image rows' bits alone, whatever
