@@ -118,15 +118,16 @@ namespace {
 // So the small tiles serve grids that would leave CUs idle (333 rows 12.8 -> 9.2 us, 1117 rows 23.5 -> 18.0, 1024 of
 // 4429 rows 68 -> 54) or half idle in the last round (2 x 1357 rows 45 -> 39, 4000 rows 118 -> 108), the pipelined
 // kernel one full round (2445 rows 49.6 -> 43.4), the tracked kernel everything larger: per row it does the least.
-// A problem with fewer query than key rows is a patch of a pipeline, which shares its launch with the other patches of
-// the step or runs alone: it is decided by the whole sequence.  Small tiles serve both uses well (24 heads, 1024 of
-// 4429 rows: alone 54 us, pipelined 68, tracked 78; four in one launch, one with 333 text queries, 164, pipelined 170) until
-// the patches of a step make more than two full rounds of the tracked kernel's.  The pipelined kernel serves patches of
-// longer sequences only where the keys are one segment, so that no text queries can be left out (648 of 5517 rows, two
-// batch elements: 84 us, tracked 96).
+// Between small and tracked the whole launch decides (`small_tiles_serve`), with all problems that are merged in it: the
+// same model holds for the patches of a step.  24 heads, image rows + 333 of text, us on tracked / small tiles:
+//   4096 in two patches 137 / 159, in four 149 / 164; two batch elements of 4600 in two 307 / 335, of 2304 + 154 in two
+//   116 / 92, of 5184 in eight (four per launch) 263 / 234; one patch of 1024 alone 79 / 58, with the text queries 82 / 79
+// Patches of sequences up to 4 * CUs workgroups are never pipelined (1024 of 4429 rows alone 54 us small, 68 pipelined),
+// those of longer ones only where the keys are one segment, so that no text queries can be left out (648 of 5517 rows,
+// two batch elements: 84 us, small 92, tracked 96).
 // HDIT_ATTN_PIPE=0 keeps every launch on the tracked-reference kernel with 256 rows, =1 puts every eligible launch on the
 // pipelined ones (for A/B timing).
-enum Kind { TRACKED, PIPELINED, SMALL, KINDS };
+enum Kind { TRACKED, PIPELINED, SMALL };
 constexpr int SMALL_BQ = 128;
 
 double fill_cost(Kind kind, int64_t workgroups, int cus) {
@@ -147,38 +148,41 @@ int rows_with_text(const hdit_attn_args* a) {
   return rows;
 }
 
-// the kernel of a problem, with its grid in that kernel's tiles
-Kind choose(const hdit_attn_args* a, const AttnParams& P, int& q_tiles, unsigned& grid) {
+int64_t workgroups(const hdit_attn_args* a, int rows, int rows_per_workgroup) {
+  return (int64_t)a->batch * a->heads * ((rows + rows_per_workgroup - 1) / rows_per_workgroup);
+}
+
+bool pipe_off() {
   static const char* pipe_env = getenv("HDIT_ATTN_PIPE");
-  const bool pipe_off = pipe_env && pipe_env[0] == '0', pipe_force = pipe_env && pipe_env[0] == '1';
+  return pipe_env && pipe_env[0] == '0';
+}
+
+bool wants_pipelined(const hdit_attn_args* a, const AttnParams& P) {
+  static const char* pipe_env = getenv("HDIT_ATTN_PIPE");
+  const bool pipe_force = pipe_env && pipe_env[0] == '1';
   const bool strides_ok = a->k[0].stride_s < (1 << 22) && a->k[1].stride_s < (1 << 22) && a->v[0].stride_s < (1 << 22) &&
                           a->v[1].stride_s < (1 << 22);  // a tile step (64 rows, in bytes) fits 32 bits
-  const bool can_pipe = !pipe_off && strides_ok && (P.skv + BKV - 1) / BKV >= PIPE_MIN_TILES;
-  if (a->head_dim == 128 || pipe_off || pipe_force) return can_pipe ? PIPELINED : TRACKED;
-  const int cus = hdit_host::num_cus(), tiles_small = (P.sq + SMALL_BQ - 1) / SMALL_BQ;
-  if (cus <= 0) return TRACKED;  // no device to ask: the launch reports it
-  const int64_t bh = (int64_t)a->batch * a->heads;
+  if (pipe_off() || !strides_ok || (P.skv + BKV - 1) / BKV < PIPE_MIN_TILES) return false;
+  if (a->head_dim == 128 || pipe_force) return true;
+  const int cus = hdit_host::num_cus();
+  if (cus <= 0) return false;  // no device to ask: the launch reports it
   const int rows = rows_with_text(a);
-  bool small;
-  Kind large;
   if (rows < P.skv) {
-    small = bh * ((P.skv + BQ - 1) / BQ) <= 4 * (int64_t)cus;
     const bool joint = a->k[0].len > 0 && a->k[1].len > 0;
-    large = can_pipe && !joint && bh * q_tiles * 8 <= (int64_t)cus * 5 ? PIPELINED : TRACKED;
-  } else {
-    const int64_t grid_large = bh * ((rows + BQ - 1) / BQ), grid_small = bh * ((rows + SMALL_BQ - 1) / SMALL_BQ);
-    const double tracked = fill_cost(TRACKED, grid_large, cus), cost = fill_cost(SMALL, grid_small, cus);
-    const double piped = can_pipe ? fill_cost(PIPELINED, grid_large, cus) : 1e30;
-    // (a few per cent are less than the model resolves: 2 x 4429 rows 264.7 us on small tiles, 264.1 tracked)
-    small = cost < 0.93 * tracked && cost < piped;
-    large = piped < tracked ? PIPELINED : TRACKED;
+    return !joint && workgroups(a, P.skv, BQ) > 4 * (int64_t)cus && workgroups(a, rows, BQ) * 8 <= (int64_t)cus * 5;
   }
-  if (small) {
-    q_tiles = tiles_small;
-    grid = (unsigned)(bh * tiles_small);
-    return SMALL;
-  }
-  return large;
+  const double tracked = fill_cost(TRACKED, workgroups(a, rows, BQ), cus), small = fill_cost(SMALL, workgroups(a, rows, SMALL_BQ), cus);
+  const double piped = fill_cost(PIPELINED, workgroups(a, rows, BQ), cus);
+  return piped < tracked && !(small < 0.93 * tracked && small < piped);
+}
+
+// Whether a launch of these many workgroups is better off with small tiles.  Where every workgroup of 256 rows has a CU
+// to itself it is (no more than two small ones then share a CU); above, the fill decides, by more than the few per cent
+// that the model resolves (2 x 4429 rows: 264.7 us on small tiles, 264.1 tracked).
+bool small_tiles_serve(int64_t grid_tracked, int64_t grid_small) {
+  const int cus = hdit_host::num_cus();
+  if (pipe_off() || cus <= 0) return false;
+  return grid_tracked <= cus || fill_cost(SMALL, grid_small, cus) < 0.93 * fill_cost(TRACKED, grid_tracked, cus);
 }
 
 int launch_one(int head_dim, const AttnParams& P, int q_tiles, unsigned grid, Kind kind, hipStream_t s) {
@@ -195,7 +199,12 @@ extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16(const h
   int q_tiles;
   unsigned grid;
   if (!to_params(a, P, q_tiles, grid)) return HDIT_OK;
-  const Kind kind = choose(a, P, q_tiles, grid);
+  Kind kind = wants_pipelined(a, P) ? PIPELINED : TRACKED;
+  if (kind == TRACKED && a->head_dim == 64 && small_tiles_serve(grid, workgroups(a, P.sq, SMALL_BQ))) {
+    kind = SMALL;
+    q_tiles = (P.sq + SMALL_BQ - 1) / SMALL_BQ;
+    grid = (unsigned)workgroups(a, P.sq, SMALL_BQ);
+  }
   rc = launch_one(a->head_dim, P, q_tiles, grid, kind, (hipStream_t)stream);
   if (rc != HDIT_OK) return rc;
   return hdit_host::check_launch("hdit_attn_fwd_bf16");
@@ -209,20 +218,33 @@ extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16_multi(c
     if (rc != HDIT_OK) return rc;
     if (args[i].head_dim != args[0].head_dim) return HDIT_EINVAL;
   }
-  // one merged launch per kind of kernel the problems want
-  for (int kind = 0; kind < KINDS; kind++) {
+  // one merged launch of the problems for the pipelined kernel, one of the others
+  for (int pass = 0; pass < 2; pass++) {
     AttnParams P[HDIT_ATTN_MAX_MULTI];
+    const hdit_attn_args* of[HDIT_ATTN_MAX_MULTI];
     int q_tiles[HDIT_ATTN_MAX_MULTI], nblocks[HDIT_ATTN_MAX_MULTI], n = 0;
+    int64_t grid_tracked = 0, grid_small = 0;
     for (int i = 0; i < count; i++) {
       unsigned grid;
       if (!to_params(&args[i], P[n], q_tiles[n], grid)) continue;
-      if ((int)choose(&args[i], P[n], q_tiles[n], grid) != kind) continue;
+      if (wants_pipelined(&args[i], P[n]) != (pass == 0)) continue;
+      grid_tracked += grid;
+      grid_small += workgroups(&args[i], P[n].sq, SMALL_BQ);
+      of[n] = &args[i];
       nblocks[n++] = (int)grid;
+    }
+    Kind kind = pass == 0 ? PIPELINED : TRACKED;
+    if (kind == TRACKED && args[0].head_dim == 64 && n > 0 && small_tiles_serve(grid_tracked, grid_small)) {
+      kind = SMALL;
+      for (int i = 0; i < n; i++) {
+        q_tiles[i] = (P[i].sq + SMALL_BQ - 1) / SMALL_BQ;
+        nblocks[i] = (int)workgroups(of[i], P[i].sq, SMALL_BQ);
+      }
     }
     if (n == 0) continue;
     hipStream_t s = (hipStream_t)stream;
     int rc;
-    if (n == 1) rc = launch_one(args[0].head_dim, P[0], q_tiles[0], (unsigned)nblocks[0], (Kind)kind, s);
+    if (n == 1) rc = launch_one(args[0].head_dim, P[0], q_tiles[0], (unsigned)nblocks[0], kind, s);
     else if (kind == SMALL) rc = hdit_attn::launch_multi_d64_small(P, q_tiles, nblocks, n, s);
     else
       rc = args[0].head_dim == 64 ? hdit_attn::launch_multi_d64(P, q_tiles, nblocks, n, kind == PIPELINED, s)
