@@ -392,6 +392,42 @@ def test_attention_image_rows_do_not_depend_on_the_text_queries(hdit, B, ni, nk,
     assert_parity(both[:1, :200], want, what="attention")
 
 
+# (batch, heads, query rows, key rows, key rows in the second buffer, gap between heads, outgrowing query rows)
+@pytest.mark.parametrize("hd,problems", [
+    (128, [(1, 3, 300, 200, 0, 0, ()), (2, 2, 64, 333, 133, 0, (0, 63)), (1, 5, 513, 1000, 77, 64, (512,)), (2, 1, 1, 129, 64, 8, (0,))]),
+    (128, [(1, 2, 256, 193, 0, 0, (255,)), (1, 2, 40, 100, 0, 0, (3,))]),  # the second: two key tiles, tracked
+    # one round of 256-row workgroups that small tiles would overfill: pipelined
+    (64, [(1, 96, 320, 256, 0, 0, ()), (1, 100, 300, 260, 60, 8, (299, 5)), (2, 45, 513, 513, 13, 0, (512,))]),
+    (64, [(4, 100, 200, 65, 0, 0, (1,)), (4, 100, 255, 130, 2, 8, (0, 254))]),  # between one and two rounds: 256 rows, tracked
+    (64, [(1, 2, 31, 64, 0, 0, (30,)), (2, 3, 200, 333, 77, 8, (0, 199)), (1, 1, 1, 1, 0, 0, ()), (1, 96, 320, 256, 56, 0, (319,))]),
+])
+def test_attention_merged_launches(hdit, hd, problems):
+    """Problems of one call with different sizes and strides, on every kernel that merged launches use: the bits of one
+    launch per problem, and the oracle's numbers -- also where a row's logits outgrow the pipelined kernel's fixed
+    reference (by more than 2^64), so that its workgroup, of a later problem too, starts over with arguments read again."""
+    print(f"attention merged d={hd} {problems}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(83)
+    args, outs, want = [], [], []
+    for B, H, sq, skv, second, gap, grown in problems:
+        r = lambda n: torch.randn(B, n, H, hd + gap, generator=gen, device=DEV).to(torch.bfloat16)[..., :hd]
+        q, k, v = r(sq), r(skv), r(skv)
+        for i, row in enumerate(grown):  # a late key along the row: its logit is 12 |q|^2 / sqrt(d), about 96 at d = 64
+            k[:, skv - 1 - i] = 12.0 * q[:, row]
+        cut = lambda t: [t[:, :skv - second], t[:, skv - second:].clone(memory_format=torch.contiguous_format)] if second else [t]
+        got, alone = (torch.zeros(B, sq, H, hd, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+        args.append(hdit.ops.attention_args([q], cut(k), cut(v), [got], 0.0))
+        hdit.ops.attention([q], cut(k), cut(v), out=[alone])
+        outs.append((got, alone))
+        want.append(O.attention(*(t.float().cpu().transpose(1, 2) for t in (q, k, v))).transpose(1, 2))
+    arr = (hdit._lib.AttnArgs * len(args))(*args)
+    rc = hdit._lib.lib().hdit_attn_fwd_bf16_multi(arr, len(args), hdit.ops._stream())
+    torch.cuda.synchronize()
+    assert rc == 0
+    for i, ((got, alone), w) in enumerate(zip(outs, want)):
+        assert torch.equal(got, alone), f"problem {i}: merged and single launch differ"
+        assert_parity(got, w, what=f"attention merged, problem {i}")
+
+
 @pytest.mark.parametrize("dim", [64, 1536, 3072, 4096 + 8])
 def test_layernorm_modulate(hdit, dim):
     B, T = 2, 37
