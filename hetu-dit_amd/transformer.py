@@ -62,11 +62,13 @@ class _Chain:
             self.txt = left[1] if left is not None else None
 
 
-# Rows (image + text) per chain from which a pass of several batch elements runs as chains on side streams.  Below, one
-# chain of all elements is faster: half the launches and half the host time, weights fetched once, launches that fill
-# more of the GPU.  SD3 step at B = 2 on two streams / one, ms: 256+77 rows per element 4.4 / 3.4, 784+333 6.7 / 5.4,
-# 1024+333 6.6 / 6.5, 2112+333 11.4 / 10.1, 3364+333 16.6 / 15.8, 3600+333 17.0 / 16.8, 3844+333 18.5 / 19.2, 4096+333
-# 19.3 / 19.9, 4356+333 21.1 / 21.1.
+# Rows (image + text) per chain, on average over the chains, from which a pass of several batch elements runs as chains
+# on side streams: the default of ``SD3TransformerBlocks.lane_rows``.  Below, one chain of all elements is faster: half
+# the launches and half the host time, weights fetched once, launches that fill more of the GPU.  SD3 step at B = 2 on
+# two streams / one, ms: 256+77 rows per element 4.4 / 3.4, 784+333 6.7 / 5.4, 1024+333 6.6 / 6.5, 2112+333 11.4 / 10.1,
+# 3364+333 16.6 / 15.8, 3600+333 17.0 / 16.8, 3844+333 18.5 / 19.2, 4096+333 19.3 / 19.9, 4356+333 21.1 / 21.1.  At B = 3
+# (chains of one and two): 576+333 6.7 / 5.8, 2048+333 14.4 / 12.9, 2398+333 16.5 / 17.1, 3136+333 21.5 / 20.4, 3600+333
+# 24.8 / 25.7; at B = 4: 784+333 9.2 / 8.6, 1444+333 13.9 / 12.7, 2704+333 23.7 / 24.6, 4096+333 36.1 / 37.0.
 LANE_ROWS = 4096
 
 
@@ -80,7 +82,8 @@ class SD3TransformerBlocks(nn.Module):
 
     * ``batch_streams``: a full-sequence pass of B >= 2 batch elements (the CFG pair) runs the elements as
       independent chains on that many side streams, blocks issued alternately -- one chain's launches fill the
-      CUs another's partial last round of tiles leaves idle (``LANE_ROWS`` says from which size on);
+      CUs another's partial last round of tiles leaves idle.  ``lane_rows``: how many rows (image + text) a chain has to
+      have, on average, for a pass to be divided (0: any size);
     * ``forward_patches``: the patches of a PipeFusion step, one block apart.
 
     Neither is recorded into a HIP graph: under capture, and whenever a per-launch timer is installed, the pass
@@ -101,6 +104,7 @@ class SD3TransformerBlocks(nn.Module):
         use_fp32_residual_stream(self.transformer_blocks)
         self.use_block_entry_points = True
         self.batch_streams = 2
+        self.lane_rows = LANE_ROWS
         self.reuse_text_kv = True  # patch mode: later patches take the text keys / values the first patch projected
         self.group_fronts = True   # forward_patches on one stream: one merged call per front of independent blocks
         # entry-point passes: a block leaves its MLP residual to the next block's norm1 (HDIT_DEFER_RESIDUALS=0: fused
@@ -233,7 +237,7 @@ class SD3TransformerBlocks(nn.Module):
             temb = temb.contiguous()
             mods = self.modulation.precompute_by_module(temb)
             lanes = min(self.batch_streams, hidden_states.shape[0])
-            if hidden_states.shape[0] * (hidden_states.shape[1] + encoder_hidden_states.shape[1]) < lanes * LANE_ROWS:
+            if hidden_states.shape[0] * (hidden_states.shape[1] + encoder_hidden_states.shape[1]) < lanes * self.lane_rows:
                 lanes = 1
             if not rs.patch_mode and lanes > 1 and not torch.cuda.is_current_stream_capturing():
                 return self._forward_batch_lanes(calls, mods, hidden_states, encoder_hidden_states, temb, lanes)

@@ -128,11 +128,66 @@ def test_forward_patches_refuses_what_it_cannot_run(hdit):
     assert len(stack.forward_patches(xs, e, t)) == P
 
 
-def test_prefilled_calls_follow_swapped_weights(hdit):
+def count_lanes(stack, monkeypatch):
+    """The numbers of chains of the passes that ran as several."""
+    seen, inner = [], stack._forward_batch_lanes
+    monkeypatch.setattr(stack, "_forward_batch_lanes", lambda *a: (seen.append(a[-1]), inner(*a))[1])
+    return seen
+
+
+@pytest.mark.parametrize("B,rows,lane_rows,chains", [
+    (2, 340, 340, 2), (2, 339, 340, 1), (2, 40, 0, 2),
+    (3, 340, 510, 2), (3, 339, 510, 1), (4, 170, 340, 2), (1, 340, 0, 1),
+    (2, 340, None, 1), (2, 4096, None, 2), (3, 2731, None, 2), (3, 2730, None, 1),
+])
+def test_batch_lanes_from_lane_rows_on(hdit, monkeypatch, B, rows, lane_rows, chains):
+    """Which passes are divided into chains -- from ``lane_rows`` rows per chain on, uneven chains counted by their
+    average, 4096 where nothing is set -- and that dividing them changes no bits."""
+    D, H = 128, 2
+    stack = make_stack(2, D, H, 41)
+    if lane_rows is not None:
+        stack.lane_rows = lane_rows
+    seen = count_lanes(stack, monkeypatch)
+    x, e, t = dev_randn((B, rows - 13, D), 42), dev_randn((B, 13, D), 43), dev_randn((B, D), 44)
+    got = stack(x, e, t).clone()
+    torch.cuda.synchronize()
+    assert seen == ([chains] if chains > 1 else [])
+    stack.batch_streams = 1
+    want = stack(x, e, t)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
+def test_batch_lanes_keep_the_bits_where_one_element_fills_the_chip_otherwise(hdit, monkeypatch):
+    """5184 + 333 rows of 24 heads: one batch element alone and two at once get attention workgroups of different sizes.
+    With weights that make logits outgrow those of the first key tile, an eager pass in chains and the undivided pass
+    (what a captured graph records) still agree bit for bit."""
+    D, H = 1536, 24
+    stack = make_stack(2, D, H, 45)
+    for block in stack.transformer_blocks:
+        m = block.attn.module
+        m.to_q.weight.data *= 6.0
+        m.to_k.weight.data *= 6.0
+    seen = count_lanes(stack, monkeypatch)
+    x, e, t = dev_randn((2, 5184, D), 46), dev_randn((2, 333, D), 47), dev_randn((2, D), 48)
+    got = stack(x, e, t).clone()
+    torch.cuda.synchronize()
+    assert seen == [2]
+    stack.batch_streams = 1
+    want = stack(x, e, t)
+    torch.cuda.synchronize()
+    assert seen == [2] and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("lane_rows", [0, None])
+def test_prefilled_calls_follow_swapped_weights(hdit, monkeypatch, lane_rows):
     """The whole-block calls re-read the weights' addresses per pass: a re-assigned ``.data``, a replaced parameter, a
     replaced feed-forward and a switched flag each take effect in the next pass, as kernel by kernel."""
     D, H, L = 256, 4, 3
     stack = make_stack(L, D, H, 91)
+    if lane_rows is not None:
+        stack.lane_rows = lane_rows
+    seen_lanes = count_lanes(stack, monkeypatch)
     x, e, t = dev_randn((2, 512, D), 92), dev_randn((2, 40, D), 93), dev_randn((2, D), 94)
 
     def both():
@@ -158,14 +213,19 @@ def test_prefilled_calls_follow_swapped_weights(hdit):
         swap()
         seen.append(both())
         assert not torch.equal(seen[-1], seen[-2]), f"swap {n} changed nothing"
+    assert seen_lanes == ([2] * (len(swaps) + 1) if lane_rows == 0 else [])
 
 
-def test_stack_takes_changing_batch_and_sequence_sizes(hdit):
+@pytest.mark.parametrize("lane_rows", [0, None])
+def test_stack_takes_changing_batch_and_sequence_sizes(hdit, monkeypatch, lane_rows):
     """One stack, passes of different batch sizes, token counts and stream element types one after the other: the
     prefilled whole-block calls, the modulation regrouping and the side streams hold nothing that is tied to the
     first shape they saw.  Every pass is compared with the kernel-by-kernel pass on one stream."""
     D, H, L = 256, 4, 3
     stack = make_stack(L, D, H, 77)
+    if lane_rows is not None:
+        stack.lane_rows = lane_rows
+    seen_lanes = count_lanes(stack, monkeypatch)
     for k, (B, Ni, Nt, f32) in enumerate([(2, 512, 77, False), (1, 300, 40, False), (3, 1024, 8, True), (2, 512, 77, False)]):
         x, e, t = dev_randn((B, Ni, D), 100 + k), dev_randn((B, Nt, D), 200 + k), dev_randn((B, D), 300 + k)
         if f32:
@@ -177,3 +237,4 @@ def test_stack_takes_changing_batch_and_sequence_sizes(hdit):
         got = stack(x, e, t)
         torch.cuda.synchronize()
         assert got.dtype == want.dtype and torch.equal(got, want), f"pass {k}: B {B}, {Ni}+{Nt} tokens"
+    assert seen_lanes == ([2, 2, 2] if lane_rows == 0 else [])  # three of the passes have several elements
