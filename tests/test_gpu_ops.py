@@ -21,7 +21,7 @@ def rnd(*shape, scale=1.0, seed=None):
     return bf16_round(torch.randn(*shape, generator=gen) * scale)
 
 
-@pytest.mark.parametrize("cfg", [-1, 0, 1, 2, 3, 4])
+@pytest.mark.parametrize("cfg", [-1, 0, 1, 2, 3, 4, 5, 6])
 @pytest.mark.parametrize("m,n,k", [(256, 256, 64), (300, 384, 128), (666, 1536, 1536), (1, 128, 64), (1024, 512, 256)])
 def test_gemm_bias(hdit, m, n, k, cfg):
     print(f"gemm_bias m={m} n={n} k={k} cfg={cfg}", flush=True)
@@ -35,7 +35,7 @@ def test_gemm_bias(hdit, m, n, k, cfg):
         hdit._lib.lib().hdit_gemm_force_config(-1)
 
 
-@pytest.mark.parametrize("cfg", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("cfg", [0, 1, 2, 3, 4, 5, 6])
 @pytest.mark.parametrize("m", [666, 154, 40])
 def test_gemm_ragged_tile_with_operands_out_of_the_caches(hdit, m, cfg):
     """The out-of-range rows of a ragged tile all read the problem's last row.  Served from the CU's L1, such
@@ -72,7 +72,7 @@ def test_gemm_result_does_not_depend_on_the_tile_shape(hdit, epi):
     a, w, b = g(rnd(m, k, seed=1)), g(rnd(n, k, scale=0.05, seed=2)), g(rnd(n, seed=3))
     outs = []
     try:
-        for cfg in (0, 1, 2, 3, 4):
+        for cfg in (0, 1, 2, 3, 4, 5, 6):
             lib.hdit_gemm_force_config(cfg)
             out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
             hdit.ops.gemm_launch([hdit.ops.gemm_problem(a, w, out, None if epi == "nobias" else b,
@@ -188,13 +188,15 @@ def test_gemm_gelu_and_gate_residual_grouped(hdit):
     assert_parity(res, want, what="gate residual")
 
 
-@pytest.mark.parametrize("cfg", [0, 3])
+@pytest.mark.parametrize("cfg", [0, 2, 3, 4, 5, 6])
 @pytest.mark.parametrize("m,n,k", [(4096, 4608, 64), (2500, 3000, 192), (5000, 2056, 320)])
 @pytest.mark.parametrize("epi", ["bias", "nobias", "gate"])
 def test_gemm_many_short_tiles_per_workgroup(hdit, m, n, k, cfg, epi):
     """More tiles than workgroups with one, three and five slabs per tile: the operand stream of the 256-row
     shapes runs two slabs ahead of the MFMAs across tile boundaries, through three A slots and two B slots, so
-    the slot a tile ends on (and the one its epilogue stages through) differs from tile to tile."""
+    the slot a tile ends on (and the one its epilogue stages through) differs from tile to tile.  The ring shapes
+    read the first fragments of a tile during the previous one, and a tile with an odd number of slabs leaves them in
+    the other set of registers."""
     print(f"gemm short tiles m={m} n={n} k={k} cfg={cfg} epi={epi}", flush=True)
     ops = hdit.ops
     a, w, b = rnd(m, k, seed=31), rnd(n, k, scale=0.05, seed=32), rnd(n, seed=33)
@@ -719,7 +721,7 @@ def test_attention_random_shapes(hdit):
 # fp32 residual stream: gated-residual epilogue with f32 residual and / or f32 output, LayerNorm on f32 rows
 # ---------------------------------------------------------------------------
 
-@pytest.mark.parametrize("cfg", [-1, 0, 1, 2, 3, 4])
+@pytest.mark.parametrize("cfg", [-1, 0, 1, 2, 3, 4, 5, 6])
 @pytest.mark.parametrize("resid_f32,out_f32", [(True, True), (False, True), (True, False)])
 @pytest.mark.parametrize("m,n,k", [(666, 1536, 128), (1000, 520, 64), (4100, 1536, 192)])
 def test_gemm_gate_residual_fp32_stream(hdit, m, n, k, resid_f32, out_f32, cfg):
