@@ -711,7 +711,8 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
 // is enough to keep HBM busy and leaves room for another stream's launch -- run ahead and bring the weights into the
 // last-level cache.  Measured, weights cold: 1357 x 1536 x 6144 on 132 tiles of 128 x 128 59.3 us without helpers, 47.5
 // with two per XCD, 43.9 with four, 43.9 with eight; 1536 x 3072 x 15360 on 192 tiles of 128 x 192 170, 149, 148, 152;
-// 333 x 1536 x 6144 on 144 tiles of 64 x 64 31.9, 31.9, 26.6, 24.4.
+// 333 x 1536 x 6144 on 144 tiles of 64 x 64 31.9, 31.9, 26.6, 24.4.  Only where they are done before the tiles
+// (`build_and_launch`).
 constexpr int HELPERS_PER_XCD = 4;
 
 // A workgroup without tiles: helper `id` of `helpers` reads one word of every 128-byte line of a weight matrix, four
@@ -785,11 +786,9 @@ int max_workgroups() {
   return max_wgs < NUM_XCD ? NUM_XCD : max_wgs;
 }
 
-// workgroups without a tile to launch beside those with one
-int helpers_per_xcd(int cus, int busy) { return busy >= cus ? 0 : cus - busy < HELPERS_PER_XCD ? cus - busy : HELPERS_PER_XCD; }
-
+// helper_us: how long each helper of an XCD's `n` works, n = 1 .. HELPERS_PER_XCD; tiles_us: how long the tiles take
 template <class C>
-int launch(const GemmTable& tab, int total_tiles, hipStream_t stream) {
+int launch(const GemmTable& tab, int total_tiles, const double* helper_us, double tiles_us, hipStream_t stream) {
   static std::atomic<bool> attr_set{false};  // setting the attribute twice from two threads is harmless
   if (!attr_set.load(std::memory_order_acquire)) {
     hipError_t e = hipFuncSetAttribute((const void*)gemm_kernel<C>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES);
@@ -803,7 +802,10 @@ int launch(const GemmTable& tab, int total_tiles, hipStream_t stream) {
   if (max_wgs < 0) return HDIT_ELAUNCH;
   const int tiles_per_xcd = (total_tiles + NUM_XCD - 1) / NUM_XCD;
   int wgs_per_xcd = max_wgs / NUM_XCD;
-  const int helpers = helpers_per_xcd(wgs_per_xcd, tiles_per_xcd);
+  // workgroups without a tile beside those with one, if they are done before the tiles
+  int helpers = wgs_per_xcd - tiles_per_xcd;
+  if (helpers > HELPERS_PER_XCD) helpers = HELPERS_PER_XCD;
+  if (helpers <= 0 || helper_us[helpers - 1] > tiles_us) helpers = 0;
   if (wgs_per_xcd > tiles_per_xcd) wgs_per_xcd = tiles_per_xcd;
   hipLaunchKernelGGL(gemm_kernel<C>, dim3((wgs_per_xcd + helpers) * NUM_XCD), dim3(NT), C::LDS_BYTES, stream, tab, total_tiles,
                      tiles_per_xcd, wgs_per_xcd);
@@ -846,22 +848,6 @@ int launch2(const hdit_gemm_problem* p1, int n1, const hdit_gemm_problem* p2, in
   hipLaunchKernelGGL((gemm_kernel2<C1, C2>), dim3(wgs_per_xcd * NUM_XCD), dim3(NT), LDS, stream, t1, total1, per1, t2,
                      total2, per2, wgs_per_xcd);
   return hdit_host::check_launch("hdit_gemm_bf16");
-}
-
-template <class C>
-int count_tiles(const hdit_gemm_problem* problems, int count) {
-  int total = 0;
-  for (int i = 0; i < count; i++)
-    total += ((problems[i].m + C::BM - 1) / C::BM) * ((problems[i].n + C::BN - 1) / C::BN);
-  return total;
-}
-
-template <class C>
-int build_and_launch(const hdit_gemm_problem* problems, int count, hipStream_t stream) {
-  GemmTable tab;
-  const int total = fill_table<C>(tab, problems, count);
-  if (total == 0) return HDIT_OK;
-  return launch<C>(tab, total, stream);
 }
 
 using Cfg256x256 = Cfg<4, 4>;
@@ -950,15 +936,37 @@ double two_us(const Load& l1, int c1, const Load& l2, int c2) {
   return idle && of_idle > of_rest ? of_idle : of_rest;
 }
 
+// One shape for all problems.  A helper that is still fetching when the last tile is done holds the launch up: on 240
+// tiles two per XCD are left, which bring in 80 GB/s each (75 - 98 measured).  649 + 430 rows x 12288 x 3072, 151 MB of
+// weights: 126 us with them, 76 without; 883 + 183 x 9216 x 3072 86 and 60; 250 + 292 x 6144 x 1536 28 and 22.
+constexpr double kHelperBytesPerUs = 80e3;
+
+template <class C>
+int build_and_launch(int cfg, const hdit_gemm_problem* problems, int count, hipStream_t stream) {
+  GemmTable tab;
+  const int total = fill_table<C>(tab, problems, count);
+  if (total == 0) return HDIT_OK;
+  double helper_us[HELPERS_PER_XCD] = {}, slabs = 0;
+  for (int i = 0; i < count; i++) {
+    if (problems[i].k / BK > slabs) slabs = problems[i].k / BK;
+    for (int h = 1; h <= HELPERS_PER_XCD; h++) {
+      const int of_problem = (h * NUM_XCD - i + count - 1) / count;  // as fetch_weights deals them
+      const double us = of_problem > 0 ? 2.0 * problems[i].n * problems[i].k / (of_problem * kHelperBytesPerUs) : 0.0;
+      if (us > helper_us[h - 1]) helper_us[h - 1] = us;
+    }
+  }
+  return launch<C>(tab, total, helper_us, tile_us(cfg, slabs, total), stream);
+}
+
 int launch_cfg(int cfg, const hdit_gemm_problem* problems, int count, hipStream_t s) {
   switch (cfg) {
-    case 0: return build_and_launch<Cfg256x192>(problems, count, s);
-    case 1: return build_and_launch<Cfg128x256>(problems, count, s);
-    case 4: return build_and_launch<Cfg128x192>(problems, count, s);
-    case 3: return build_and_launch<Cfg256x256>(problems, count, s);
-    case 5: return build_and_launch<Cfg64x128>(problems, count, s);
-    case 6: return build_and_launch<Cfg64x64>(problems, count, s);
-    default: return build_and_launch<Cfg128x128>(problems, count, s);
+    case 0: return build_and_launch<Cfg256x192>(cfg, problems, count, s);
+    case 1: return build_and_launch<Cfg128x256>(cfg, problems, count, s);
+    case 4: return build_and_launch<Cfg128x192>(cfg, problems, count, s);
+    case 3: return build_and_launch<Cfg256x256>(cfg, problems, count, s);
+    case 5: return build_and_launch<Cfg64x128>(cfg, problems, count, s);
+    case 6: return build_and_launch<Cfg64x64>(cfg, problems, count, s);
+    default: return build_and_launch<Cfg128x128>(2, problems, count, s);
   }
 }
 

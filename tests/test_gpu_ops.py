@@ -158,6 +158,36 @@ def test_gemm_rows_that_open_another_round_take_the_small_shape(hdit, epi, n):
         assert torch.equal(got, want)
 
 
+def test_gemm_helpers_do_not_outlast_the_tiles(hdit):
+    """Two problems on 240 tiles with 151 MB of weights that come from HBM: what the CUs without a tile do meanwhile must
+    not make the call take longer than its problems one after the other (126 us against 100 when it did, 76 without)."""
+    ops = hdit.ops
+    ms, n, k, copies = (649, 430), 12288, 3072, 4  # four times the weights: more than the last-level cache holds
+    a = [torch.randn(m, k, device=DEV).to(torch.bfloat16) for m in ms]
+    y = [torch.empty(m, n, dtype=torch.bfloat16, device=DEV) for m in ms]
+    w = [[(torch.randn(n, k, device=DEV) * 0.02).to(torch.bfloat16) for _ in ms] for _ in range(copies)]
+    together = [[[ops.gemm_problem(a[i], w[c][i], y[i]) for i in range(2)]] for c in range(copies)]
+    apart = [[[p] for p in calls[0]] for calls in together]
+
+    def us(calls):
+        best = 1e30
+        for _ in range(5):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            torch.cuda.synchronize()
+            start.record()
+            for c in calls:
+                for problems in c:
+                    ops.gemm_launch(problems)
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, start.elapsed_time(end) / copies * 1e3)
+        return best
+
+    us(together), us(apart)
+    one, two = us(together), us(apart)
+    assert one < 1.1 * two, f"one call {one:.1f} us, one call per problem {two:.1f} us"
+
+
 def test_gemm_gelu_and_gate_residual_grouped(hdit):
     B, T1, T2, D, F = 2, 320, 77, 256, 512
     x1, x2 = rnd(B, T1, D), rnd(B, T2, D)
