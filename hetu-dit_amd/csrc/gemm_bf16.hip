@@ -915,9 +915,12 @@ double tile_us(int c, double slabs, int busy) {
   return slabs * (s.lo + (s.hi - s.lo) * f) + s.epi_lo + (s.epi_hi - s.epi_lo) * f;
 }
 
+// A partial round behind full ones has no helpers beside it, and without them the slabs of the ring shapes take as long as
+// on a full chip (274 + 295 rows x 12288 x 3072: 384 tiles of 128 x 192 76 us, priced at 66 with `lo`; 256 of 256 x 192 61).
 double single_us(const Load& l, int c) {
   const int full = l.tiles / kSlots, rem = l.tiles % kSlots;
-  return full * tile_us(c, l.slabs, kSlots) + (rem ? tile_us(c, l.slabs, rem) : 0.0);
+  const bool ring = kShape[c].bm * kShape[c].bn <= RING_MAX_MMA * 64 * 64;
+  return full * tile_us(c, l.slabs, kSlots) + (rem ? tile_us(c, l.slabs, full && ring ? kSlots : rem) : 0.0);
 }
 
 // Tiles of c1, then tiles of c2 in the same launch: the small tiles go first to the workgroups that have one large tile
