@@ -297,7 +297,8 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
   };
   fetch_bias(locate<C>(tab, lid));
 
-  // prologue: slab 0 into stage 0, slab 1 into the registers
+  // prologue: the first slabs of the stream -- two into the slots of the 256-row shapes, NS into the stages of the ring
+  // shapes; register-staged: slab 0 into stage 0, slab 1 into the registers
   p_setup();
   int stage = 0;
   int sa = 0, sb = 0;  // DMA: the A and B slots of the slab being multiplied
