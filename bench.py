@@ -1,7 +1,7 @@
 """Benchmark of the one-GPU DiT denoise-step hot path.
 
 ``python bench.py [--gpus 1] [--steps K] [--warmup W]`` times K passes of the
-24-block SD3-shape MMDiT stack (bf16, batch 2 = CFG
+24-block SD3-shape MMDiT stack (a 1024 x 1024 image: bf16, batch 2 = CFG
 pair, 4096 image + 333 text tokens, hidden 1536, 24 x 64 heads, last block
 context_pre_only) on synthetic inputs already resident in HBM, and prints one
 JSON line.  ``roofline`` describes the dominant kernel (the grouped MFMA GEMM):
@@ -78,9 +78,9 @@ WORKLOADS = ("sd3_1024", "sd3_1024_transformer", "sd3_pipefusion", "sd3_pipefusi
 
 
 def make_workload(name, dev):
-    """(step callable, description, gemm flops, attention flops, blocks per step, attention kernel name) of one of
-    BASELINE.json's configs.  sd3_1024 is the headline workload; the others are the shapes of
-    configs[3], [2] and [4], selectable for profiling."""
+    """(step callable, description, gemm flops, attention flops, blocks per step, attention kernel name) of a named
+    workload.  sd3_1024 is the headline; the others are the PipeFusion, Flux and CogVideoX shapes, selectable for
+    profiling."""
     import torch
 
     from hetu_dit_amd import synthetic, transformer
@@ -113,7 +113,7 @@ def make_workload(name, dev):
         gemm, attn = algorithmic_flops(cfg)
         D, T, Nt = cfg["dim"], cfg["n_img"], cfg["n_txt"]
         gemm += 2.0 * 2 * (T * 64 * D * 2 + Nt * 4096 * D + 256 * D + D * D + 2048 * D + D * D)
-        desc = ("configs[1] inside the whole SD3 transformer: patch embedding + position table, timestep/text conditioning, "
+        desc = ("the sd3_1024 stack inside the whole SD3 transformer: patch embedding + position table, timestep/text conditioning, "
                 "context projection, 24 joint blocks, norm_out + proj_out + unpatchify, guidance 7.0 and the Euler update")
 
         def step():
@@ -123,8 +123,8 @@ def make_workload(name, dev):
         step.set_single_stream = lambda on: setattr(model._runner, "batch_streams", 1 if on else 2)
         return step, desc, gemm, attn, cfg["layers"], "attn_fwd_kernel<64>"
     if name in ("flux_1024_step", "cogvideox_5b_step"):
-        # the whole block stacks of the two models at the shapes of configs[2] / configs[4]: 19 double + 38 single
-        # Flux blocks (the 1024^2 step BASELINE.md quotes 0.84 s for on the reference's hardware), 42 CogVideoX-5B
+        # the whole block stacks of the two models at 1024 x 1024 pixels and 49 frames of 480 x 720: 19 double + 38
+        # single Flux blocks (0.84 s per step published for the reference on its hardware), 42 CogVideoX-5B
         # blocks; every block one call of its whole-block entry point
         cfg = synthetic.CONFIGS[name[:-5]]
         B, Ni, Nt, D = cfg["batch"], cfg["n_img"], cfg["n_txt"], cfg["dim"]
@@ -140,7 +140,7 @@ def make_workload(name, dev):
             rope, t = (cos.to(dev), sin.to(dev)), rnd(B, D)
             gemm = 24.0 * S * D * D * B * (L2 + L1)
             attn = 4.0 * S * S * D * B * (L2 + L1)
-            desc = ("configs[2] as a whole step: Flux-shape, 19 double-stream + 38 single-stream blocks, B1, 4096 image + 512 "
+            desc = ("Flux-shape step, 19 double-stream + 38 single-stream blocks, B1, 4096 image + 512 "
                     "text tokens, D3072, 24x128 heads")
             return (lambda: stack(x, e, t, rope)[0]), desc, gemm, attn, L2 + L1, "attn_fwd_pipe_kernel<128>"
         L = 42
@@ -149,7 +149,7 @@ def make_workload(name, dev):
         randomize_(stack, dev)
         cos, sin = synthetic.rope_table(synthetic.cogvideox_positions(*cfg["grid"]), (16, 24, 24))
         rope, t = (cos.to(dev), sin.to(dev)), rnd(B, cfg["temb_dim"])
-        desc = "configs[4] as a whole step: CogVideoX-5B-shape, 42 blocks, B1, 226 text + 17550 video tokens, D3072, 48x64 heads"
+        desc = "CogVideoX-5B-shape step, 42 blocks, B1, 226 text + 17550 video tokens, D3072, 48x64 heads"
         return (lambda: stack(x, e, t, rope)[0]), desc, 24.0 * S * D * D * B * L, 4.0 * S * S * D * B * L, L, "attn_fwd_kernel<64>"
     cfg = synthetic.CONFIGS[name]
     B, Ni, Nt, D = cfg["batch"], cfg["n_img"], cfg["n_txt"], cfg["dim"]
@@ -160,7 +160,7 @@ def make_workload(name, dev):
         if name == "sd3_1024":
             x = rnd(B, Ni, D)
             gemm, attn = algorithmic_flops(cfg)
-            desc = ("configs[1]: SD3-shape denoise step, 24 joint blocks, B2 (CFG pair), 4096 image + 333 text "
+            desc = ("SD3-shape denoise step, 24 joint blocks, B2 (CFG pair), 4096 image + 333 text "
                     "tokens, D1536, 24x64 heads, last block context_pre_only")
             def step():
                 return stack(x, e, t)
@@ -209,7 +209,7 @@ def make_workload(name, dev):
         # stream only supplies keys and values (k|v projection, no query rows, no out-projection, no MLP)
         gemm = (24.0 * Sq * D * D * B * L - 18.0 * Nt * D * D * B) + (P - 1) * (24.0 * Np + 4.0 * Nt) * D * D * B * L
         attn = 4.0 * Sq * S * D * B * L + (P - 1) * 4.0 * Np * S * D * B * L
-        desc = (f"configs[3]: SD3 PipeFusion shard, 24 joint blocks x 4 patches, B{B}, query 1024 image + 333 text tokens "
+        desc = (f"SD3 PipeFusion shard, 24 joint blocks x 4 patches, B{B}, query 1024 image + 333 text tokens "
                 "against the 4096 + 333 stale K/V buffer")
         return step, desc, gemm, attn, L * P, "attn_fwd_kernel<64>"
     if name == "flux_1024":
@@ -222,7 +222,7 @@ def make_workload(name, dev):
         x, e, t = rnd(B, Ni, D), rnd(B, Nt, D), rnd(B, D)
         gemm = 24.0 * S * D * D * B * 2
         attn = 4.0 * S * S * D * B * 2
-        desc = "configs[2]: Flux-shape, one double-stream + one single-stream block, B1, 4096 image + 512 text tokens, D3072, 24x128 heads"
+        desc = "Flux-shape, one double-stream + one single-stream block, B1, 4096 image + 512 text tokens, D3072, 24x128 heads"
         return (lambda: stack(x, e, t, rope)[0]), desc, gemm, attn, 2, "attn_fwd_pipe_kernel<128>"
     with torch.device(dev):
         stack = transformer.CogVideoXTransformerBlocks(1, D, cfg["heads"], cfg["head_dim"], cfg["temb_dim"])
@@ -232,14 +232,14 @@ def make_workload(name, dev):
     x, e, t = rnd(B, Ni, D), rnd(B, Nt, D), rnd(B, cfg["temb_dim"])
     gemm = 24.0 * S * D * D * B
     attn = 4.0 * S * S * D * B
-    desc = "configs[4]: CogVideoX-5B-shape block, B1, 226 text + 17550 video tokens, D3072, 48x64 heads"
+    desc = "CogVideoX-5B-shape block, B1, 226 text + 17550 video tokens, D3072, 48x64 heads"
     return (lambda: stack(x, e, t, rope)[0]), desc, gemm, attn, 1, "attn_fwd_kernel<64>"
 
 
 def cpu_baseline(runs=3):
     """fp32 oracle of one joint block on the host cores (a reported baseline, not a target): at the headline
-    shape (configs[1]: B2, 4096 + 333 tokens; about 10 s of CPU work for a warm-up and `runs` timed blocks,
-    scaled to the 24 blocks of a step) and at configs[0] (B1, 1024 + 333 tokens, the CPU-sized case)."""
+    shape (B2, 4096 + 333 tokens; about 10 s of CPU work for a warm-up and `runs` timed blocks,
+    scaled to the 24 blocks of a step) and at 512 x 512 (B1, 1024 + 333 tokens, the CPU-sized case)."""
     import torch
 
     import oracle
@@ -271,9 +271,9 @@ def cpu_baseline(runs=3):
         "unit": "ms",
         "cores": torch.get_num_threads(),
         "kind": "port",
-        "sample": f"fp32 oracle, one SD3 joint block at the headline shape (configs[1]: B2, 4096+333 tokens, D1536): "
+        "sample": f"fp32 oracle, one SD3 joint block at the headline shape (B2, 4096+333 tokens, D1536): "
                   f"median of {runs} runs = {ms_block:.0f} ms/block, value = 24 x block (the step has 24 blocks; the "
-                  f"last one's shorter text path is not discounted); configs[0] (B1, 1024+333 tokens): "
+                  f"last one's shorter text path is not discounted); 512 x 512 (B1, 1024+333 tokens): "
                   f"{ms_small:.1f} ms/block; os.cpu_count()={os.cpu_count()}",
     }
 
@@ -318,7 +318,7 @@ def main():
                     help="sd3_1024: time the pass on one stream (a HIP-graph replay unless --no-graph) instead of the "
                          "eager form that runs the batch elements as independent chains on two streams")
     ap.add_argument("--workload", choices=WORKLOADS, default="sd3_1024",
-                    help="sd3_1024 (BASELINE.json configs[1]) is the headline metric; the others are for profiling")
+                    help="sd3_1024 is the headline metric; the others are for profiling")
     ap.add_argument("--probe", choices=["coissue"], default=None,
                     help="instead of a workload, run a hardware probe and print its table: coissue = do the matrix "
                          "pipe and the vector ALU of a SIMD work side by side (hdit_probe_coissue)")

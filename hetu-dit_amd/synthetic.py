@@ -57,7 +57,7 @@ def cogvideox_positions(frames: int, height: int, width: int) -> torch.Tensor:
     return torch.stack([t, h, w], dim=-1).reshape(-1, 3)
 
 
-# name -> shape parameters of BASELINE.json's configs
+# name -> shape parameters of the benchmark's workloads
 CONFIGS: Dict[str, dict] = {
     "sd3_512": dict(family="sd3", batch=1, n_img=1024, n_txt=333, dim=1536, heads=24, head_dim=64),
     "sd3_1024": dict(family="sd3", batch=2, n_img=4096, n_txt=333, dim=1536, heads=24, head_dim=64, layers=24),

@@ -48,7 +48,7 @@ def test_sd3_joint_block(hdit, pre_only):
 
 
 def test_sd3_block_config0_shape(hdit):
-    """B1, 1024 image + 333 text tokens, hidden 1536, 24 x 64 heads."""
+    """A 512 x 512 image: B1, 1024 image + 333 text tokens, hidden 1536, 24 x 64 heads."""
     from hetu_dit_amd import blocks, synthetic
 
     B, N, Nt, D, H = 1, 1024, 333, 1536, 24
@@ -257,8 +257,8 @@ def test_sd3_pipefusion_patches_stale_kv(hdit):
 
 @pytest.mark.parametrize("family", ["sd3", "cogvideox"])
 def test_block_with_fp8_attention(hdit, family):
-    """The fp8-e4m3 attention path inside a block, against the fp32 oracle at the tolerance BASELINE.json
-    states for it: relative L2 <= 3e-2 on the block outputs."""
+    """The fp8-e4m3 attention path inside a block, against the fp32 oracle at the tolerance
+    stated for it: relative L2 <= 3e-2 on the block outputs."""
     from hetu_dit_amd import blocks, synthetic
 
     if family == "sd3":

@@ -1,6 +1,6 @@
 """Parity after the whole 24-block stack: the HIP path against the fp32 oracle applied 24 times to the same
-bf16-rounded weights and inputs, at the tolerance BASELINE.json states for bf16 (cosine >= 0.9995 and relative
-L2 <= 1e-2) -- the full configs[1] shape, and the PipeFusion order of configs[3] (a full-sequence pass, then
+bf16-rounded weights and inputs, at the tolerance stated for bf16 (cosine >= 0.9995 and relative
+L2 <= 1e-2) -- the full 1024 x 1024 shape, and the PipeFusion order (a full-sequence pass, then
 four patches over stale K/V buffers) with 24 layers at hidden 1536."""
 import pytest
 import torch
@@ -43,7 +43,7 @@ def build_stack(L, D, H, hd, seed):
 
 @pytest.mark.timeout(600)
 def test_sd3_24_blocks_config1_against_oracle(hdit):
-    """B2 (CFG pair), 4096 image + 333 text tokens, D1536, 24 x 64 heads, 24 joint
+    """The headline shape: B2 (CFG pair), 4096 image + 333 text tokens, D1536, 24 x 64 heads, 24 joint
     blocks, the last one context_pre_only.  The oracle carries its own fp32 residual stream through all 24
     blocks; only the final hidden states are compared (plus, for the record, the drift after each block)."""
     torch.set_num_threads(16)
@@ -65,13 +65,13 @@ def test_sd3_24_blocks_config1_against_oracle(hdit):
         print(f"block {i:2d}: hidden rel_l2={rel_l2(gxc, ox):.3e} cos={cosine(gxc, ox):.6f}", flush=True)
         del params
     assert torch.equal(gx, got), "block-by-block calls and the stack runner disagree"
-    r, c = assert_parity(got, ox, what="24-block stack, configs[1]")
+    r, c = assert_parity(got, ox, what="24-block stack, 1024 x 1024")
     print(f"24 blocks: rel_l2={r:.3e} cos={c:.6f}", flush=True)
 
 
 @pytest.mark.timeout(600)
 def test_sd3_24_blocks_pipefusion_against_stale_kv_oracle(hdit):
-    """configs[3]'s order of calls with 24 layers at D1536 and configs[0]'s token counts (1024 image tokens in
+    """The PipeFusion order of calls with 24 layers at D1536 and the token counts of a 512 x 512 image (1024 image tokens in
     four patches of 256, 333 text tokens; B2): a full-sequence pass of a different hidden state fills the K/V
     buffers, then patch k attends to a buffer whose patches < k are fresh and > k stale.  The oracle keeps one
     brute-force StaleKVBuffer per layer."""

@@ -1,4 +1,4 @@
-"""Parity at the full sizes of BASELINE.json's configs, where the fp32 oracle of the whole problem would
+"""Parity at the full sizes of the benchmark's workloads, where the fp32 oracle of the whole problem would
 take minutes: sampled rows against the oracle (a row of a GEMM or of an attention output only needs that
 row of the left operand), and properties that hold at any size -- softmax of a constant V returns V, the
 order of the key/value segments does not matter, adaLN-Zero with a zero modulation projection is the
@@ -38,10 +38,10 @@ def sample_rows(m, count, seed):
     return idx
 
 
-# (image rows, text rows, n, k, epilogue): the four GEMM calls of an SD3 joint block at configs[1], the
-# out-projection and second MLP call of a PipeFusion patch at configs[3] (2048 image rows: the planner gives them the
-# 128x128 ring alone, with 24 and 96 slabs per tile), the QKV+MLP call of a Flux single block at configs[2], the FF1
-# call of a CogVideoX block at configs[4]
+# (image rows, text rows, n, k, epilogue): the four GEMM calls of an SD3 joint block at 1024 x 1024, the
+# out-projection and second MLP call of a PipeFusion patch (2048 image rows: the planner gives them the
+# 128x128 ring alone, with 24 and 96 slabs per tile), the QKV+MLP call of a Flux single block at 1024 x 1024, the FF1
+# call of a CogVideoX block at 49 frames of 480 x 720
 GEMM_CASES = [
     (8192, 666, 4608, 1536, "bias"),
     (8192, 666, 1536, 1536, "gate"),
@@ -88,7 +88,7 @@ def test_gemm_full_size_sampled_rows(hdit, m_img, m_txt, n, k, epi):
 
 
 # One launch per case, a list of problems (rows, n, k, epilogue, f32 stream?, problems that share the left operand
-# with the first one): the launches of the Flux (configs[2]) and CogVideoX (configs[4]) blocks whose tile shapes and
+# with the first one): the launches of the Flux and CogVideoX blocks whose tile shapes and
 # two-phase plans differ from the SD3 ones -- the Flux single block's [q|k|v] + GELU(proj_mlp) call on one operand,
 # its proj_out (k = 15360, gated onto the fp32 stream), the Flux double block's QKV and FF2 (k = 12288, gated fp32)
 # over image + text rows, and CogVideoX's QKV / out-projection / FF2 over 226 text + 17550 video rows.
@@ -174,7 +174,7 @@ def test_qk_norm_rope_full_size_sampled_rows(hdit, S, n_txt, H, hd, kind, axes):
 
 
 def test_flux_blocks_full_size_against_oracle(hdit):
-    """configs[2] at its real size -- B1, 512 text + 4096 image tokens (64 x 64 grid), D 3072, 24 heads of 128 --
+    """Flux at 1024 x 1024 -- B1, 512 text + 4096 image tokens (64 x 64 grid), D 3072, 24 heads of 128 --
     one double-stream block and one single-stream block, each against the fp32 oracle (about 1.3 TFLOP of CPU
     work apiece).  At this width the planner picks tile shapes and two-phase launches the small-width block tests
     never see."""
@@ -218,7 +218,7 @@ def test_flux_blocks_full_size_against_oracle(hdit):
     assert torch.equal(out2, out)
 
 
-# (batch, heads, image tokens, text tokens, head dim): configs[1], [2], [4]
+# (batch, heads, image tokens, text tokens, head dim): SD3 and Flux at 1024 x 1024, CogVideoX
 ATTN_CASES = [(2, 24, 4096, 333, 64), (1, 24, 4096, 512, 128), (1, 48, 17550, 226, 64)]
 
 
@@ -256,7 +256,7 @@ def test_attention_full_size(hdit, B, H, n_img, n_txt, hd):
 
 
 def test_sd3_stack_full_size_properties(hdit):
-    """configs[1] and configs[3] at full size (24 blocks, B2, 4096 + 333 tokens)."""
+    """The SD3 step and its PipeFusion form at full size (24 blocks, B2, 4096 + 333 tokens)."""
     from hetu_dit_amd import synthetic, transformer
     from hetu_dit_amd.layers.modules import AdaLayerNormContinuous, AdaLayerNormZero
     from hetu_dit_amd.runtime_state import get_runtime_state
@@ -317,7 +317,7 @@ def test_sd3_stack_full_size_properties(hdit):
 
 
 def test_attention_fp8_full_size_cogvideox(hdit):
-    """configs[4]'s fp8 leg at its real length: 48 heads, 226 text + 17550 video tokens (17776 keys).  Sampled
+    """CogVideoX on the fp8 path at its real length: 48 heads, 226 text + 17550 video tokens (17776 keys).  Sampled
     query rows against the fp32 oracle at the kernel-level fp8 bound (zero-mean random V: nothing averages the
     e4m3 rounding of V and P away relative to the signal), and a V that is the same for every key and exactly
     representable in e4m3: the output must then be V itself, which holds only if the row sum is taken over the

@@ -554,7 +554,7 @@ def test_copy_rows_into_slice(hdit):
 
 # Kernel-level bound for the fp8 path on zero-mean random V with diffuse attention: nothing averages the
 # e4m3 rounding noise of V and P away relative to the (equally averaged) signal, so the output carries
-# about sqrt(2) * 2^-4 / sqrt(3) ~ 5e-2 relative noise.  The tolerance BASELINE.json states for the fp8
+# about sqrt(2) * 2^-4 / sqrt(3) ~ 5e-2 relative noise.  The tolerance stated for the fp8
 # path (relative L2 <= 3e-2) is on BLOCK outputs and is checked in tests/test_gpu_blocks.py.
 FP8_KERNEL_REL = 6e-2
 

@@ -12,7 +12,7 @@ def cosine(a: torch.Tensor, b: torch.Tensor) -> float:
 
 
 def assert_parity(got: torch.Tensor, want: torch.Tensor, rel=1e-2, cos=0.9995, what=""):
-    """The tolerance BASELINE.json states for bf16: cosine >= 0.9995 and
+    """The tolerance stated for bf16: cosine >= 0.9995 and
     relative L2 <= 1e-2 against the fp32 oracle (3e-2 for the fp8 path)."""
     got = got.detach().float().cpu()
     want = want.detach().float().cpu()
