@@ -238,3 +238,30 @@ def test_stack_takes_changing_batch_and_sequence_sizes(hdit, monkeypatch, lane_r
         torch.cuda.synchronize()
         assert got.dtype == want.dtype and torch.equal(got, want), f"pass {k}: B {B}, {Ni}+{Nt} tokens"
     assert seen_lanes == ([2, 2, 2] if lane_rows == 0 else [])  # three of the passes have several elements
+
+
+@pytest.mark.parametrize("B", [1, 2])
+def test_patch_steps_with_unchanged_inputs_repeat_the_whole_pass(hdit, B):
+    """PipeFusion steps whose patches are those of the whole-sequence pass before them: every key and value row is written
+    again with what the buffer holds, so the outputs are the rows of the whole pass and stay so step after step -- bit for
+    bit, although rows share waves and workgroups with other rows than in the whole pass, and with weights that make
+    logits outgrow those of the first key tile.  (384 rows and more per patch, 24 heads: no pipelined kernel on either side.)"""
+    from hetu_dit_amd.runtime_state import get_runtime_state
+
+    D, H, L, Nt = 1536, 24, 2, 77
+    starts = [0, 1000, 1700, 2900]
+    stack = make_stack(L, D, H, 51)
+    for block in stack.transformer_blocks:
+        block.attn.module.to_q.weight.data *= 6.0
+        block.attn.module.to_k.weight.data *= 6.0
+    rs = get_runtime_state()
+    rs.set_token_patches(starts)
+    rs.set_patched_mode(False)
+    x, e, t = dev_randn((B, starts[-1], D), 52), dev_randn((B, Nt, D), 53), dev_randn((B, D), 54)
+    want = stack(x, e, t).clone()
+    torch.cuda.synchronize()
+    rs.set_patched_mode(True)
+    for step in range(2):
+        got = stack.forward_patches([x[:, a:b].contiguous() for a, b in zip(starts, starts[1:])], e, t, num_streams=1)
+        torch.cuda.synchronize()
+        assert torch.equal(torch.cat(got, 1), want), f"step {step}"
