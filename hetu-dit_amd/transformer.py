@@ -76,8 +76,9 @@ class SD3TransformerBlocks(nn.Module):
     """The 24 joint blocks of the SD3 transformer with the reference's block loop.
 
     ``use_block_entry_points``: run every block through ``hdit_block_sd3`` (one foreign call per block, the
-    same launches on the same operands as the Python block: results are bit for bit the same) instead of one
-    foreign call per kernel.  An eager pass is then bound by the GPU and not by the interpreter, which is what
+    same launches on the same operands as the Python block: results are bit for bit the same; chains of a pass that is
+    divided below the default ``lane_rows`` may get the pipelined attention kernel where the undivided batch does not)
+    instead of one foreign call per kernel.  An eager pass is then bound by the GPU and not by the interpreter, which is what
     lets independent work run side by side on several streams:
 
     * ``batch_streams``: a full-sequence pass of B >= 2 batch elements (the CFG pair) runs the elements as
