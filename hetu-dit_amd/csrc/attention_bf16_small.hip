@@ -1,5 +1,5 @@
 // Joint flash attention, head dim 64, with one 32-row query block per wave: workgroups of 128 query rows, three per CU
-// (device code and its description: attention_bf16_kernels.h).  Which problems it serves: `choose` in attention_bf16.hip.
+// (device code and its description: attention_bf16_kernels.h).  Which launches it serves: `small_tiles_serve` in attention_bf16.hip.
 // A wave does half the MFMAs and softmax of a 64-row wave on the same fragment reads (LDS busy for about half of the
 // time, no longer a quarter), which costs 8 % per row on a full chip, and needs 168 registers instead of 256.
 #define HDIT_ATTN_QUERY_BLOCKS 1
