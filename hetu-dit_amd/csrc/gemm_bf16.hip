@@ -2,7 +2,15 @@
 //
 // Persistent kernel, one 256-thread workgroup (2x2 waves) per CU, walking a
 // static list of output tiles of (64*TM) x (64*TN) elements; a wave owns a
-// (32*TM) x (32*TN) sub-tile in accumulators (v_mfma_f32_32x32x16_bf16).
+// (32*TM) x (32*TN) sub-tile in accumulators (v_mfma_f32_16x16x32_bf16).
+//
+// What bounds the large shapes is the board's power: the main loop holds 1.9 - 2.0 of 2.4 GHz.  The 16x16x32 MFMA moves
+// half the accumulator bytes per flop of the 32x32x16 one and costs less energy: bare loops of either on random operands,
+// all CUs, run at 2.00 and 1.73 PFLOP/s (1.89 where no operand is shared by consecutive MFMAs, 2.00 where one is).  Bias
+// epilogue, 32x32x16 -> 16x16x32 on one box: 8192 x 2048 x 6144 149.9 -> 138.3 us, 8192 x 1536 x 6144 116.7 -> 109.0,
+// 8192 x 4608 x 1536 99.2 -> 94.2, 4608 x 3072 x 15360 327 -> 312, 8192^3 762 -> 709 (1.55 PFLOP/s); with GELU 8192 x 6144 x
+// 1536 140.6 -> 131.6.  The shapes that do not fill the chip are bound otherwise (below) and stay level.  Both
+// instructions give the same bits.
 //
 // Staging.  Both operands are k-contiguous, so A and B tiles are staged the
 // same way, in slabs of 64 k (128 bytes per row).  A wave-wide request fetches
@@ -14,13 +22,14 @@
 //
 // Pipeline.  The k slabs of all tiles of a workgroup form one flat stream; tile
 // boundaries are invisible to it, so a tile's first slabs arrive during the
-// previous tile's last slab and epilogue.  Fragments are double-buffered in
-// registers one k-step ahead; the workgroup barrier sits before the last k-step
-// of a slab, whose fragments are already in registers, so that the first
-// fragments of the next slab are read under that k-step's MFMAs.
+// previous tile's last slab and epilogue.  A slab is worked on in eight quarters
+// (two k-steps of 32 times four quarters of the wave's tile), whose fragments are
+// read two quarters ahead; the workgroup barrier sits before the last two
+// quarters of a slab, whose fragments are already in registers, so that the first
+// fragments of the next slab are read under their MFMAs.
 //  * 256-row shapes: direct to LDS (global_load_lds_dwordx4, swizzle applied on
 //    the source side), three A slots and two B slots.  During slab g the A rows
-//    of slab g+2 are requested (k-steps 0..2) into the slot slab g-1 vacated;
+//    of slab g+2 are requested (quarters 0..5) into the slot slab g-1 vacated;
 //    behind the barrier that ends slab g, the B rows of slab g+2 go into the B
 //    slot just vacated.  Requests retire in order, so the wait in front of the
 //    barrier leaves exactly the newest A requests in flight.
@@ -28,18 +37,20 @@
 //    multiplied out of stage h&1, the registers holding slab h+1 are written
 //    to the other stage and immediately refilled with the global loads of slab
 //    h+2, one write+load pair every few MFMAs.
-//  * ring shapes (64x64 to 128x192), for the launches that do not fill the chip: a slab is 4 to 24 MFMAs per wave,
+//  * ring shapes (64x64 to 128x192), for the launches that do not fill the chip: a slab is 8 to 48 MFMAs per wave,
 //    and what bounds it is the operands' way to the CU: time per slab is proportional to its bytes, 25 - 40 B/clk/CU,
-//    whatever its MFMAs.  Direct to LDS through a ring of 3 to 8 stages; the fragments of a whole slab are
+//    whatever its MFMAs.  (The requests alone, no arithmetic, take the same time: 85 - 90 GB/s per CU whether 64 or 248 CUs
+//    of the chip work, whatever the stages, the waves, the row pitch or the order of the rows; 135 only where everything
+//    is in the XCD's L2 already.)  Direct to LDS through a ring of 3 to 8 stages; the fragments of a whole slab are
 //    double-buffered in registers, so a slab has one barrier and no wait for LDS inside, and its stage is free for
 //    the request of the slab NS ahead as soon as it begins.  Measured (warm weights, microseconds per slab): 128x128
 //    0.36 - 0.39, 0.54 before with four stages and fragments one k-step ahead; 128x192 0.45, 0.67 before
 //    (register-staged); 64x128 0.27; 64x64 0.19.  Small tiles are what short problems need: 333 x 1536 x 6144 is 36
 //    tiles of 128x128 (61 us at first), 144 of 64x64 (27 us).
 //
-// Epilogue.  A lane's accumulator holds one output row m and runs of 4
-// consecutive n; lanes l and l^32 swap halves (v_permlane32_swap) to own 8
-// consecutive n.  bias / GELU-tanh are applied there, the bf16 result is staged
+// Epilogue.  A lane's accumulator holds one output row m and 4 consecutive n of
+// a 16-column block; lanes l and l^16 swap runs of two neighbouring blocks
+// (v_permlane16_swap) to own 8 consecutive n.  bias / GELU-tanh are applied there, the bf16 result is staged
 // through a wave-private 8 KiB window inside the LDS stage (the A slot) the last
 // slab just vacated (ring shapes: behind the stages) and written back with 16 lanes covering 256 contiguous bytes of a row
 // (gate and residual are applied in that coalesced layout, in fp32).
@@ -71,7 +82,7 @@ struct GemmTable {
   hdit_gemm_problem p[HDIT_GEMM_MAX_PROBLEMS];
 };
 
-constexpr int RING_MAX_MMA = 6;  // MFMAs per k-step of the shapes that take their slabs through a ring
+constexpr int RING_MAX_MMA = 6;  // TM * TN of the shapes that take their slabs through a ring
 
 template <int TM_, int TN_>
 struct Cfg {
@@ -92,7 +103,7 @@ struct Cfg {
   static constexpr int A_SLOTS = 3, B_SLOTS = 2;
   static constexpr int B_OFF = A_SLOTS * A_BYTES;
   static constexpr int DMA_BYTES = A_SLOTS * A_BYTES + B_SLOTS * B_BYTES;
-  // RING: the shapes with short slabs (4 to 24 MFMAs per wave) take them the same way into a ring of NS stages
+  // RING: the shapes with short slabs (8 to 48 MFMAs per wave) take them the same way into a ring of NS stages
   // (A then B), as many as fit beside the epilogue windows: only a lead of several slabs covers the latency of
   // operands that come from HBM.
   static constexpr bool RING = TM * TN <= RING_MAX_MMA;
@@ -163,7 +174,7 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, lh = lane >> 5;
+  const int l16 = lane & 15, lg = lane >> 4;
   const int wm0 = (wave >> 1) * C::WM;
   const int wn0 = (wave & 1) * C::WN;
 
@@ -256,43 +267,50 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
 
   // ---- consumer ------------------------------------------------------------
   // fragment read offsets: row r, logical chunk c -> r*128 + ((c ^ ((r>>1)&7)) << 4); fragment rows are
-  // l32 plus a multiple of 32, so (r>>1)&7 == (l32>>1)&7.  k-step ks uses chunk 2*ks + lh.
-  const int swz = (l32 >> 1) & 7;
-  const int a_row = (wm0 + l32) * ROW_BYTES;
-  const int b_row = (wn0 + l32) * ROW_BYTES;
-  bf16x8 fa[2][TM], fb[2][TN];
+  // l16 plus a multiple of 16, so (r>>1)&7 == (l16>>1)&7.  k-step ks (32 k) uses chunk 4*ks + lg.
+  const int swz = (l16 >> 1) & 7;
+  const int a_row = (wm0 + l16) * ROW_BYTES;
+  const int b_row = (wn0 + l16) * ROW_BYTES;
+  // fragments of half of the wave's rows and half of its columns, two slots each
+  bf16x8 fa[2][TM], fb[4][TN];
   // ring shapes: the fragments of whole slabs, the one being multiplied and the next
-  constexpr int SK = C::RING ? BK / 16 : 1;
-  bf16x8 sfa[2][SK][TM], sfb[2][SK][TN];
+  constexpr int SK = C::RING ? BK / 32 : 1;
+  bf16x8 sfa[2][SK][2 * TM], sfb[2][SK][2 * TN];
   auto read_slab_frag = [&](const unsigned char* sbase, int buf, int r) {  // r-th fragment in the order of use
-    const int ks = r / (TM + TN), f = r % (TM + TN);
-    const int ch = ((ks * 2 + lh) ^ swz) << 4;
-    if (f < TN) sfb[buf][ks][f] = *(const bf16x8*)(sbase + C::A_BYTES + b_row + ch + f * 32 * ROW_BYTES);
-    else sfa[buf][ks][f - TN] = *(const bf16x8*)(sbase + a_row + ch + (f - TN) * 32 * ROW_BYTES);
+    const int ks = r / (2 * TM + 2 * TN), f = r % (2 * TM + 2 * TN);
+    const int ch = ((ks * 4 + lg) ^ swz) << 4;
+    if (f < 2 * TN) sfb[buf][ks][f] = *(const bf16x8*)(sbase + C::A_BYTES + b_row + ch + f * 16 * ROW_BYTES);
+    else sfa[buf][ks][f - 2 * TN] = *(const bf16x8*)(sbase + a_row + ch + (f - 2 * TN) * 16 * ROW_BYTES);
   };
-  auto read_frags2 = [&](const unsigned char* abase, const unsigned char* bbase, int ks, int buf) {
-    const int ch = ((ks * 2 + lh) ^ swz) << 4;
-#pragma unroll
-    for (int i = 0; i < TM; i++) fa[buf][i] = *(const bf16x8*)(abase + a_row + ch + i * 32 * ROW_BYTES);
-#pragma unroll
-    for (int j = 0; j < TN; j++) fb[buf][j] = *(const bf16x8*)(bbase + b_row + ch + j * 32 * ROW_BYTES);
+  auto read_a = [&](const unsigned char* abase, int ks, int half, int slot, int i) {
+    fa[slot][i] = *(const bf16x8*)(abase + a_row + (((ks * 4 + lg) ^ swz) << 4) + (half * TM + i) * 16 * ROW_BYTES);
   };
-  auto read_frags = [&](const unsigned char* sbase, int ks, int buf) { read_frags2(sbase, sbase + C::A_BYTES, ks, buf); };
+  auto read_b = [&](const unsigned char* bbase, int ks, int half, int slot, int j) {
+    fb[slot][j] = *(const bf16x8*)(bbase + b_row + (((ks * 4 + lg) ^ swz) << 4) + (half * TN + j) * 16 * ROW_BYTES);
+  };
+  auto read_first = [&](const unsigned char* abase, const unsigned char* bbase) {  // rows and columns of a slab's first quarter
+#pragma unroll
+    for (int i = 0; i < TM; i++) read_a(abase, 0, 0, 0, i);
+#pragma unroll
+    for (int j = 0; j < TN; j++) read_b(bbase, 0, 0, 0, j);
+#pragma unroll
+    for (int j = 0; j < TN; j++) read_b(bbase, 0, 1, 1, j);
+  };
 
-  // The bias enters through the accumulators: a tile's accumulators start as bias (x) ones -- one MFMA per 32-column
+  // The bias enters through the accumulators: a tile's accumulators start as bias (x) ones -- one MFMA per 16-column
   // block, whose A operand holds bias[n] at k = 0 and whose B operand holds 1 at k = 0 -- instead of zero.  The
   // epilogue then needs neither bias registers (the 256 x 256 shape could only find its 32 by spilling accumulators)
   // nor an LDS slot, and every shape forms bias + sum of products in the same order, so results do not depend on the
-  // shape a problem is given.  Lane l < 32 fetches the bias of column l of each of the wave's column blocks; the
+  // shape a problem is given.  Lane l < 16 fetches the bias of column l of each of the wave's column blocks; the
   // values of the next tile are requested at the start of the current tile's epilogue, in front of its stores.
-  unsigned short bnext[TN];
+  unsigned short bnext[2 * TN];
   auto fetch_bias = [&](const TileCoord& tc) {
     const hdit_gemm_problem& pr = tab.p[tc.pi];
     const unsigned short* bsrc = (const unsigned short*)pr.bias;
 #pragma unroll
-    for (int j = 0; j < TN; j++) {
+    for (int j = 0; j < 2 * TN; j++) {
       bnext[j] = 0;
-      if (bsrc) bnext[j] = bsrc[min(tc.n0 + wn0 + j * 32 + l32, pr.n - 1)];
+      if (bsrc) bnext[j] = bsrc[min(tc.n0 + wn0 + j * 16 + l16, pr.n - 1)];
     }
   };
   fetch_bias(locate<C>(tab, lid));
@@ -316,7 +334,7 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
     p_advance();
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(C::LOADS));
     __syncthreads();
-    read_frags2(lds, lds + C::B_OFF, 0, 0);
+    read_first(lds, lds + C::B_OFF);
   } else if constexpr (C::RING) {
     // slabs 0 .. NS-1 into stages 0 .. NS-1; slab 0 has landed before the first fragment read
 #pragma unroll
@@ -328,7 +346,7 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
     __builtin_amdgcn_s_waitcnt(waitcnt_vm((C::NS - 1) * C::LOADS));
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < SK * (TM + TN); r++) read_slab_frag(lds, 0, r);
+    for (int r = 0; r < SK * 2 * (TM + TN); r++) read_slab_frag(lds, 0, r);
   } else {
 #pragma unroll
     for (int i = 0; i < C::LOADS; i++) g_load(i);
@@ -339,15 +357,10 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
     for (int i = 0; i < C::LOADS; i++) g_load(i);
     p_advance();
     __syncthreads();
-    read_frags(lds, 0, 0);
+    read_first(lds, lds + C::A_BYTES);
   }
 
-  constexpr int NMMA = TM * TN;
-  constexpr int NRD = TM + TN;            // fragment reads per k-step
-  constexpr int RD_MFMA = (NRD + 1) / 2;  // MFMAs that are followed by two fragment reads
-  constexpr int SLOTS = NMMA - RD_MFMA;   // MFMAs per k-step that can carry a write+load pair
-  constexpr int CP = (C::LOADS + 2) / 3;  // pairs per k-step (k-steps 0..2 of a slab)
-  static_assert(C::RING || RD_MFMA < NMMA, "not enough MFMAs to place the fragment reads");
+  constexpr int NQ = TM * TN;  // MFMAs of a quarter of the wave's tile
 
   bool first_tile = true;
   while (true) {
@@ -359,85 +372,47 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
     }
     first_tile = false;
 
-    f32x16 acc[TM][TN];
+    f32x4 acc[2 * TM][2 * TN];
     {
-      const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      i32x4 ones_bits = {lh == 0 ? 0x3f80 : 0, 0, 0, 0};  // bf16 1.0 at k = 0 (lanes < 32 hold k = 0..7)
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+      i32x4 ones_bits = {lg == 0 ? 0x3f80 : 0, 0, 0, 0};  // bf16 1.0 at k = 0 (lanes < 16 hold k = 0..7)
       bf16x8 ones;
       __builtin_memcpy(&ones, &ones_bits, 16);
 #pragma unroll
-      for (int j = 0; j < TN; j++) {
-        i32x4 bb = {lh == 0 ? (int)bnext[j] : 0, 0, 0, 0};
+      for (int j = 0; j < 2 * TN; j++) {
+        i32x4 bb = {lg == 0 ? (int)bnext[j] : 0, 0, 0, 0};
         bf16x8 bfr;
         __builtin_memcpy(&bfr, &bb, 16);
 #pragma unroll
-        for (int i = 0; i < TM; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr, ones, zero, 0, 0, 0);
+        for (int i = 0; i < 2 * TM; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr, ones, zero, 0, 0, 0);
       }
     }
 
-    // One k-step: the MFMAs on fragment buffer `buf`.  Under them, pinned in this order: two reads per MFMA
-    // of the fragments the next k-step needs (an MFMA goes first, so that its wait for its own fragments
-    // is placed while no younger read is outstanding), then the write+load pairs [cp_first, cp_last)
-    // spread over the remaining MFMAs: registers of slab h+1 to LDS stage `wstage`, then the same
-    // registers refilled with slab h+2.
-    auto k_step = [&](int buf, const unsigned char* rd_base, int rd_ks, int wstage, int cp_first, int cp_last) {
-      read_frags(rd_base, rd_ks, buf ^ 1);
+    // A slab is two k-steps of 32 k, a k-step four quarters of the wave's tile -- rows half a0 or a1, columns half b0 or
+    // b1 -- in the order (a0,b0) (a0,b1) (a1,b1) (a1,b0): each needs one half that the one before did not.  A half is
+    // read two quarters ahead, behind the first MFMAs of a quarter: a1 in quarter 0, b0 of the second k-step in 1, its
+    // a0 in 2, its b1 in 3, its a1 in 4; behind the barrier (after 5) the next slab's a0 and b0 in 6 and b1 in 7.
+    // The rows have two slots, the columns four (k-step, half).  Consecutive MFMAs share an operand.
+    // `carry(t)`: what else is issued behind MFMA t.
+    auto quarter = [&](int h, const unsigned char* rd_a, const unsigned char* rd_b, auto&& carry) {
+      const int q = h & 3, ks = h >> 2, ah = q >> 1, bh = (q == 1 || q == 2) ? 1 : 0;
 #pragma unroll
-      for (int t = 0; t < NMMA; t++) {
-        acc[t / TN][t % TN] =
-            __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[buf][t % TN], fa[buf][t / TN], acc[t / TN][t % TN], 0, 0, 0);
-        if (t == RD_MFMA - 1) {
-#pragma unroll
-          for (int u = 0; u < RD_MFMA; u++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                        // MFMA
-            if (2 * u + 2 <= NRD) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // DS reads
-            else __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          }
-          SCHED_FENCE();
-        }
-        if (t >= RD_MFMA) {
-#pragma unroll
-          for (int j = 0; j < CP; j++)
-            if (RD_MFMA + (j * SLOTS) / CP == t && cp_first + j < cp_last) {
-              l_store(wstage, cp_first + j);
-              g_load(cp_first + j);
-            }
-          SCHED_FENCE();
-        }
+      for (int t = 0; t < NQ; t++) {
+        const int j = t / TM, i = (j & 1) ? TM - 1 - t % TM : t % TM;
+        f32x4& c = acc[ah * TM + i][bh * TN + j];
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[2 * ks + bh][j], fa[ah][i], c, 0, 0, 0);
+        if (h == 0 && t < TM) read_a(rd_a, 0, 1, 1, t);
+        if (h == 1 && t < TN) read_b(rd_b, 1, 0, 2, t);
+        if (h == 2 && t < TM) read_a(rd_a, 1, 0, 0, t);
+        if (h == 3 && t < TN) read_b(rd_b, 1, 1, 3, t);
+        if (h == 4 && t < TM) read_a(rd_a, 1, 1, 1, t);
+        if (h == 6 && t < TM) read_a(rd_a, 0, 0, 0, t);
+        if (h == 6 && t < TN) read_b(rd_b, 0, 0, 0, t);
+        if (h == 7 && t < TN) read_b(rd_b, 0, 1, 1, t);
+        carry(t);
+        SCHED_FENCE();
       }
     };
-
-    // The same k-step for the direct-to-LDS shapes: under the MFMAs that carry no fragment reads, requests
-    // [first, last) of the slab at the cursor -- A rows (kind 0) or B rows (kind 1) -- into slot `slot`.
-    auto k_step_dma = [&](int buf, const unsigned char* rd_a, const unsigned char* rd_b, int rd_ks, int kind, int first,
-                          int last, int slot) {
-      read_frags2(rd_a, rd_b, rd_ks, buf ^ 1);
-#pragma unroll
-      for (int t = 0; t < NMMA; t++) {
-        acc[t / TN][t % TN] =
-            __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[buf][t % TN], fa[buf][t / TN], acc[t / TN][t % TN], 0, 0, 0);
-        if (t == RD_MFMA - 1) {
-#pragma unroll
-          for (int u = 0; u < RD_MFMA; u++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                        // MFMA
-            if (2 * u + 2 <= NRD) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // DS reads
-            else __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          }
-          SCHED_FENCE();
-        }
-        if (t >= RD_MFMA) {
-          const int n = last - first;
-#pragma unroll
-          for (int j = 0; j < C::LOADS; j++)
-            if (j < n && RD_MFMA + (j * SLOTS) / (n > 0 ? n : 1) == t) {
-              if (kind == 0) dma_a(slot, first + j);
-              else dma_b(slot, first + j);
-            }
-          SCHED_FENCE();
-        }
-      }
-    };
-    constexpr int CPA = (C::A_LOADS + 2) / 3;  // A requests per k-step (k-steps 0..2 of a slab)
 
     if constexpr (C::DMA) {
       for (int kt = 0; kt < KT; kt++) {
@@ -445,17 +420,30 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
         const unsigned char* bb = lds + C::B_OFF + sb * C::B_BYTES;
         // A rows of the slab after next go to the slot the previous slab vacated
         const int sa_req = sa == 0 ? C::A_SLOTS - 1 : sa - 1;
-        k_step_dma(0, ab, bb, 1, 0, 0, CPA, sa_req);
-        k_step_dma(1, ab, bb, 2, 0, CPA, 2 * CPA, sa_req);
-        k_step_dma(0, ab, bb, 3, 0, 2 * CPA, C::A_LOADS, sa_req);
+        constexpr int APQ = (C::A_LOADS + 5) / 6;  // A requests per quarter
+#pragma unroll
+        for (int h = 0; h < 6; h++) {
+          quarter(h, ab, bb, [&](int t) {
+#pragma unroll
+            for (int r = 0; r < APQ; r++)
+              if (h * APQ + r < C::A_LOADS && t == NQ - 1 - 3 * (APQ - 1 - r)) dma_a(sa_req, h * APQ + r);
+          });
+        }
         // ---- turn over: everything but the A requests just issued has landed (the next slab is complete),
-        // and the fragments of the last k-step are in registers
+        // and the last fragments of this slab are in registers
         __builtin_amdgcn_s_waitcnt(waitcnt_vm(C::A_LOADS) & 0xf0ff);  // and lgkmcnt(0)
         __syncthreads();
         const int sb_req = sb;  // the B slot this slab vacates takes the B rows of the slab after next
         sa = sa == C::A_SLOTS - 1 ? 0 : sa + 1;
         sb ^= 1;
-        k_step_dma(1, lds + sa * C::A_BYTES, lds + C::B_OFF + sb * C::B_BYTES, 0, 1, 0, C::B_LOADS, sb_req);
+        constexpr int BPQ = (C::B_LOADS + 1) / 2;
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+          quarter(6 + h, lds + sa * C::A_BYTES, lds + C::B_OFF + sb * C::B_BYTES, [&](int t) {
+#pragma unroll
+            for (int r = 0; r < BPQ; r++)
+              if (h * BPQ + r < C::B_LOADS && t == NQ - 1 - 2 * (BPQ - 1 - r)) dma_b(sb_req, h * BPQ + r);
+          });
         p_advance();
       }
     } else if constexpr (C::RING) {
@@ -463,7 +451,7 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
       // slab's fragments, under the others the requests of the slab NS ahead, into the stage this slab's fragments
       // have been read from.  One barrier per slab: every wave holds this slab's fragments, and the next slab has
       // landed (everything but the NS-2 slabs behind it).
-      constexpr int NM = SK * NMMA, NR = SK * NRD;
+      constexpr int NM = SK * 4 * NQ, NR = SK * 2 * (TM + TN);
       constexpr int RPM = (NR + (NM + 1) / 2 - 1) / ((NM + 1) / 2);  // reads behind each of the first MFMAs
       constexpr int RM = (NR + RPM - 1) / RPM;                       // MFMAs that carry them
       auto ring_slab = [&](int buf) {
@@ -474,8 +462,8 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
         const unsigned char* nbase = lds + stage * C::STAGE_BYTES;
 #pragma unroll
         for (int t = 0; t < NM; t++) {
-          const int ks = t / NMMA, i = (t % NMMA) / TN, j = t % TN;
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sfb[buf][ks][j], sfa[buf][ks][i], acc[i][j], 0, 0, 0);
+          const int ks = t / (4 * NQ), j = (t % (4 * NQ)) / (2 * TM), i0 = t % (2 * TM), i = (j & 1) ? 2 * TM - 1 - i0 : i0;
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sfb[buf][ks][j], sfa[buf][ks][i], acc[i][j], 0, 0, 0);
 #pragma unroll
           for (int r = 0; r < RPM; r++)
             if (t < RM && t * RPM + r < NR) read_slab_frag(nbase, buf ^ 1, t * RPM + r);
@@ -497,24 +485,36 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
 #pragma unroll
         for (int ks = 0; ks < SK; ks++) {
 #pragma unroll
-          for (int i = 0; i < TM; i++) sfa[0][ks][i] = sfa[1][ks][i];
+          for (int i = 0; i < 2 * TM; i++) sfa[0][ks][i] = sfa[1][ks][i];
 #pragma unroll
-          for (int j = 0; j < TN; j++) sfb[0][ks][j] = sfb[1][ks][j];
+          for (int j = 0; j < 2 * TN; j++) sfb[0][ks][j] = sfb[1][ks][j];
         }
       }
     } else
     for (int kt = 0; kt < KT; kt++) {
       const unsigned char* sbase = lds + stage * C::STAGE_BYTES;
       const int wstage = stage ^ 1;  // held slab h-1; every wave passed the barrier of that slab
-      k_step(0, sbase, 1, wstage, 0, CP);
-      k_step(1, sbase, 2, wstage, CP, 2 * CP);
-      k_step(0, sbase, 3, wstage, 2 * CP, C::LOADS);
+      // registers of slab h+1 to LDS stage `wstage`, then the same registers refilled with slab h+2
+      constexpr int LPQ = (C::LOADS + 5) / 6;
+#pragma unroll
+      for (int h = 0; h < 6; h++) {
+        quarter(h, sbase, sbase + C::A_BYTES, [&](int t) {
+#pragma unroll
+          for (int r = 0; r < LPQ; r++)
+            if (h * LPQ + r < C::LOADS && t == NQ - 1 - 2 * (LPQ - 1 - r)) {
+              l_store(wstage, h * LPQ + r);
+              g_load(h * LPQ + r);
+            }
+        });
+      }
       p_advance();
-      // ---- turn the stages over: the fragments of the last k-step are in registers, slab h+1 is written
+      // ---- turn the stages over: the last fragments of this slab are in registers, slab h+1 is written
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
       __syncthreads();
       stage ^= 1;
-      k_step(1, lds + stage * C::STAGE_BYTES, 0, wstage, 0, 0);
+      const unsigned char* nbase = lds + stage * C::STAGE_BYTES;
+#pragma unroll
+      for (int h = 0; h < 2; h++) quarter(6 + h, nbase, nbase + C::A_BYTES, [](int) {});
     }
     // staging window of this wave: inside the stage (the A slot) the tile's last slab vacated
     unsigned char* epi = lds + wave * EPI_WAVE_BYTES +
@@ -531,7 +531,7 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
       // to spare, spills them around it -- reloads that wait for every operand request in flight.
       int lane_e = lane;
       asm volatile("" : "+v"(lane_e));
-      const int l32 = lane_e & 31, lh = lane_e >> 5;
+      const int l16 = lane_e & 15, lg = lane_e >> 4;
       // all addressing below is a uniform base plus a 32-bit byte offset per lane (checked on the host)
       unsigned char* __restrict__ Cb = (unsigned char*)pr.c;
       const unsigned char* __restrict__ Rb = (const unsigned char*)pr.resid;
@@ -597,29 +597,30 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
         // base, so slot (chunk ^ (row & 15)) of a row is (row base + ((row & 15) << 4)) ^ (chunk << 4): one register
         // and one v_xor per access, made opaque per block so that the sixteen write and eight read addresses are not
         // computed ahead and spilled.
-        unsigned wa = lds_address(epi) + l32 * 256 + ((l32 & 15) << 4);
+        unsigned wa = lds_address(epi) + l16 * 256 + (l16 << 4);
         unsigned ra = lds_address(epi) + wr_row * 256 + ((rchunk ^ wr_row) << 4);
         asm volatile("" : "+v"(wa), "+v"(ra));
 #pragma unroll
         for (int j = 0; j < TN; j++) {
 #pragma unroll
-          for (int gp = 0; gp < 2; gp++) {
-            // accumulator groups g = 2gp (even) and 2gp+1 (odd) hold columns 8g + 4*lh + e.  After the swap
-            // lanes < 32 own the 8 columns of the even group, lanes >= 32 those of the odd group.
+          for (int mi = 0; mi < 2; mi++) {
+            // The accumulators of column blocks 2j (even) and 2j+1 (odd) hold columns 4*lg + e.  The swap exchanges
+            // the odd 16-lane rows of the first with the even ones of the second: lanes of group 0 and 2 then own
+            // columns 0..7 and 8..15 of the even block, those of group 1 and 3 the same columns of the odd one.
             float v[8];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-              auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(acc[i][j][(2 * gp) * 4 + e]),
-                                                         __float_as_int(acc[i][j][(2 * gp + 1) * 4 + e]), false, false);
+              auto sw = __builtin_amdgcn_permlane16_swap(__float_as_int(acc[2 * i + mi][2 * j][e]),
+                                                         __float_as_int(acc[2 * i + mi][2 * j + 1][e]), false, false);
               v[e] = __int_as_float(sw[0]);
               v[4 + e] = __int_as_float(sw[1]);
             }
-            const int chunk = j * 4 + 2 * gp + lh;  // 16-byte chunk inside the wave's 256-byte row
+            const int chunk = j * 4 + ((lg & 1) << 1) + (lg >> 1);  // 16-byte chunk inside the wave's 256-byte row
             if (MODE == HDIT_EPI_BIAS_GELU) {
 #pragma unroll
               for (int e = 0; e < 8; e++) v[e] = hdit::gelu_tanh_f(v[e]);
             }
-            *(lds_i32x4*)(uintptr_t)(wa ^ (unsigned)(chunk << 4)) = hdit::pack8(v);
+            *(lds_i32x4*)(uintptr_t)((wa ^ (unsigned)(chunk << 4)) + mi * 16 * 256) = hdit::pack8(v);
           }
           SCHED_FENCE();  // keeps the scheduler from pulling whole accumulator tiles into VGPRs at once
         }
@@ -865,9 +866,10 @@ std::atomic<int> g_force_cfg{-1};
 // A launch deals its tiles to 256 workgroups (one per CU) in rounds; a tile costs (k / 64) slab times plus an epilogue
 // with the fill of the pipeline.  Both depend on how many CUs work: a slab takes `lo` microseconds while at most half of
 // them do (what the CU's requests take to come from the last-level cache) and `hi` while all do (the chip's power budget
-// is shared), in between in between.  All figures measured on MI355X with weights that come from HBM: single problems of
-// 1 - 6144 rows, N = 1536 - 9216, K = 1536 - 12288 under every shape; the model reproduces those launches within 4 - 10 %
-// and its choice among the shapes is on average 0.1 % slower than the best of them (at most 4 %).
+// is shared), in between in between.  All figures fitted to MI355X times with weights that come from HBM: 260 random launches
+// of the models' sizes (one or two problems, 64 - 17000 rows, N = 1536 - 21504, K = 1536 - 15360) under every shape; the
+// model reproduces those launches within 4 - 10 % and its choice among the shapes is on average 0.04 % slower than the best
+// of them (at most 3 %).
 //
 // What a plan has to get right is the last round.  One tile shape for everything wastes most of it: the 666-row text
 // stream of a joint block on the image stream's 256-row tiles adds a nearly empty round, and 17 550 rows x 3072 columns
@@ -882,9 +884,9 @@ struct Shape {
 };
 constexpr int NCFG = 7;
 constexpr Shape kShape[NCFG] = {
-    {256, 192, 0.765, 1.182, 3.9, 6.1}, {128, 256, 0.618, 0.860, 2.5, 4.8}, {128, 128, 0.365, 0.527, 2.3, 3.4},
-    {256, 256, 0.939, 1.523, 4.9, 6.5}, {128, 192, 0.468, 0.676, 2.6, 4.7}, {64, 128, 0.275, 0.358, 1.7, 1.8},
-    {64, 64, 0.194, 0.222, 1.7, 1.5},
+    {256, 192, 0.762, 1.076, 5.1, 5.0}, {128, 256, 0.640, 0.847, 4.1, 4.0}, {128, 128, 0.354, 0.465, 3.1, 3.3},
+    {256, 256, 0.975, 1.357, 5.7, 6.6}, {128, 192, 0.445, 0.617, 4.5, 4.1}, {64, 128, 0.262, 0.323, 1.8, 2.3},
+    {64, 64, 0.195, 0.218, 0.7, 1.3},
 };
 constexpr double kLaunchUs = 4.0;
 constexpr int kSlots = 256;
