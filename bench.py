@@ -99,7 +99,7 @@ def make_workload(name, dev):
                 for m in obj.modules():
                     if isinstance(m, hetuDiTAttentionWrapper):
                         m.fp8_attention = True
-        return step, desc + "; attention on the fp8-e4m3 path", gemm, attn, blocks, kernel.replace("attn_fwd_kernel", "attn_fp8_kernel")
+        return step, desc + "; attention on the fp8-e4m3 path", gemm, attn, blocks, kernel.replace("attn_fwd_pipe_kernel", "attn_fp8_kernel")
     if name == "sd3_1024_transformer":
         # the same 24 blocks inside the whole transformer: latent in, guided and Euler-updated latent out
         from hetu_dit_amd.transformer_sd3 import SD3Transformer2DModel
@@ -121,7 +121,7 @@ def make_workload(name, dev):
 
         step.multi_stream = "eager, the two batch elements as independent block chains on two streams"
         step.set_single_stream = lambda on: setattr(model._runner, "batch_streams", 1 if on else 2)
-        return step, desc, gemm, attn, cfg["layers"], "attn_fwd_kernel<64>"
+        return step, desc, gemm, attn, cfg["layers"], "attn_fwd_pipe_kernel<64>"
     if name in ("flux_1024_step", "cogvideox_5b_step"):
         # the whole block stacks of the two models at 1024 x 1024 pixels and 49 frames of 480 x 720: 19 double + 38
         # single Flux blocks (0.84 s per step published for the reference on its hardware), 42 CogVideoX-5B
@@ -150,7 +150,7 @@ def make_workload(name, dev):
         cos, sin = synthetic.rope_table(synthetic.cogvideox_positions(*cfg["grid"]), (16, 24, 24))
         rope, t = (cos.to(dev), sin.to(dev)), rnd(B, cfg["temb_dim"])
         desc = "CogVideoX-5B-shape step, 42 blocks, B1, 226 text + 17550 video tokens, D3072, 48x64 heads"
-        return (lambda: stack(x, e, t, rope)[0]), desc, 24.0 * S * D * D * B * L, 4.0 * S * S * D * B * L, L, "attn_fwd_kernel<64>"
+        return (lambda: stack(x, e, t, rope)[0]), desc, 24.0 * S * D * D * B * L, 4.0 * S * S * D * B * L, L, "attn_fwd_pipe_kernel<64>"
     cfg = synthetic.CONFIGS[name]
     B, Ni, Nt, D = cfg["batch"], cfg["n_img"], cfg["n_txt"], cfg["dim"]
     S = Ni + Nt
@@ -168,7 +168,7 @@ def make_workload(name, dev):
             # launched eagerly the stack runs the two batch elements as independent chains on two streams
             step.multi_stream = "eager, the two batch elements as independent block chains on two streams"
             step.set_single_stream = lambda on: setattr(stack, "batch_streams", 1 if on else 2)
-            return step, desc, gemm, attn, cfg["layers"], "attn_fwd_kernel<64>"
+            return step, desc, gemm, attn, cfg["layers"], "attn_fwd_pipe_kernel<64>"
         # PipeFusion shard: a full-sequence pass fills the K/V buffers ("previous step"), then one step is
         # four patch passes of 1024 image tokens each against the stale full-length buffers
         P = cfg["patches"]
@@ -211,7 +211,7 @@ def make_workload(name, dev):
         attn = 4.0 * Sq * S * D * B * L + (P - 1) * 4.0 * Np * S * D * B * L
         desc = (f"SD3 PipeFusion shard, 24 joint blocks x 4 patches, B{B}, query 1024 image + 333 text tokens "
                 "against the 4096 + 333 stale K/V buffer")
-        return step, desc, gemm, attn, L * P, "attn_fwd_kernel<64>"
+        return step, desc, gemm, attn, L * P, "attn_fwd_pipe_kernel<64>"
     if name == "flux_1024":
         with torch.device(dev):
             stack = transformer.FluxTransformerBlocks(1, 1, D, cfg["heads"], cfg["head_dim"])
@@ -233,7 +233,7 @@ def make_workload(name, dev):
     gemm = 24.0 * S * D * D * B
     attn = 4.0 * S * S * D * B
     desc = "CogVideoX-5B-shape block, B1, 226 text + 17550 video tokens, D3072, 48x64 heads"
-    return (lambda: stack(x, e, t, rope)[0]), desc, gemm, attn, 1, "attn_fwd_kernel<64>"
+    return (lambda: stack(x, e, t, rope)[0]), desc, gemm, attn, 1, "attn_fwd_pipe_kernel<64>"
 
 
 def cpu_baseline(runs=3):

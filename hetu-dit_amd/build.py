@@ -20,12 +20,13 @@ HIPCC_FLAGS = [
 ]
 
 
-# Per-file additions.  attention_bf16.hip: its pipelined kernel runs one wave per SIMD with 512 registers, where
-# the compiler would otherwise keep every MFMA accumulator in the AGPR half -- and the softmax (VALU) cannot read
-# those without a copy per score.  In the VGPR form the allocator decides per value.
+# Per-file additions.  The attention kernels of one or two waves per SIMD: left alone the compiler keeps every MFMA
+# accumulator in the AGPR half, and the softmax (VALU) cannot read those without a copy per score.  In the VGPR form the
+# allocator decides per value.
 EXTRA_FLAGS = {
     "attention_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-    "attention_bf16_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "attention_bf16_pipe4.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "attention_bf16_pipe8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

@@ -31,40 +31,7 @@ Seg2 make_seg(const hdit_seq_segment* s) {
 }  // namespace
 
 namespace hdit_attn {
-int launch_d64(const AttnParams& P, int q_tiles, unsigned grid, bool pipelined, hipStream_t stream) {
-  if (pipelined) {
-    static std::atomic<bool> attr{false};  // setting the attribute twice from two threads is harmless
-    if (!attr.load(std::memory_order_acquire)) {
-      if (hipFuncSetAttribute((const void*)attn_fwd_pipe_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              PipeLds<64>::TOTAL) != hipSuccess)
-        return HDIT_ELAUNCH;
-      attr.store(true, std::memory_order_release);
-    }
-    hipLaunchKernelGGL(attn_fwd_pipe_kernel<64>, dim3(grid), dim3(256), PipeLds<64>::TOTAL, stream, P, q_tiles);
-  } else {
-    hipLaunchKernelGGL(attn_fwd_kernel<64>, dim3(grid), dim3(256), Lds<64>::TOTAL, stream, P, q_tiles);
-  }
-  return HDIT_OK;
-}
-
-int launch_multi_d64(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, bool pipelined, hipStream_t stream) {
-  AttnMulti M;
-  const int grid = fill_multi(M, P, q_tiles, nblocks, count);
-  static std::atomic<bool> attr{false};  // setting the attributes twice from two threads is harmless
-  if (!attr.load(std::memory_order_acquire)) {
-    if (hipFuncSetAttribute((const void*)attn_fwd_pipe_multi_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            PipeLds<64>::TOTAL) != hipSuccess ||
-        hipFuncSetAttribute((const void*)attn_fwd_multi_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            Lds<64>::TOTAL) != hipSuccess)
-      return HDIT_ELAUNCH;
-    attr.store(true, std::memory_order_release);
-  }
-  if (pipelined)
-    hipLaunchKernelGGL(attn_fwd_pipe_multi_kernel<64>, dim3((unsigned)grid), dim3(256), PipeLds<64>::TOTAL, stream, M);
-  else
-    hipLaunchKernelGGL(attn_fwd_multi_kernel<64>, dim3((unsigned)grid), dim3(256), Lds<64>::TOTAL, stream, M);
-  return HDIT_OK;
-}
+HDIT_ATTN_LAUNCH(launch_tracked_d64, 64, attn_fwd_kernel, attn_fwd_multi_kernel, Lds)
 }  // namespace hdit_attn
 
 namespace hdit_host {
@@ -84,7 +51,7 @@ int attn_validate(const hdit_attn_args* a) {
 
 namespace {
 // validated arguments -> kernel parameters; false: no query rows, nothing to do
-bool to_params(const hdit_attn_args* a, AttnParams& P, int& q_tiles, unsigned& grid) {
+bool to_params(const hdit_attn_args* a, AttnParams& P) {
   P.q = make_seg(a->q);
   P.k = make_seg(a->k);
   P.v = make_seg(a->v);
@@ -95,100 +62,66 @@ bool to_params(const hdit_attn_args* a, AttnParams& P, int& q_tiles, unsigned& g
   if (P.sq == 0) return false;
   const float scale = a->scale > 0.f ? a->scale : 1.0f / sqrtf((float)a->head_dim);
   P.scale_log2 = scale * 1.4426950408889634f;
-  q_tiles = (P.sq + BQ - 1) / BQ;
-  grid = (unsigned)(q_tiles * a->batch * a->heads);
   return true;
 }
-}  // namespace
 
-namespace {
-// Which kernel serves a problem.
-// d = 128: the tracked kernel runs one wave per SIMD as well, so the pipelined one serves every grid.
-// d = 64: the small and the tracked kernel give the same bits; the pipelined one, whose softmax reference is fixed, does
-// not.  So whether a problem gets the pipelined kernel is decided from the problem alone (launched on its own or merged
-// with others, it keeps its bits), and in the same way with and without the text queries of a joint sequence, whose
-// image rows keep their bits: a query segment that is left out counts as if it were there (`rows_with_text`), and query
-// patches of joint sequences never get that kernel.  (Exception: image rows in a workgroup of the pipelined kernel that
-// also holds text rows.  If a text row outgrows the fixed reference by 2^64, the tracked kernel computes the workgroup.)
-// What decides is how the workgroups fill the CUs, in microseconds per tile of 64 keys (measured on MI355X for one and
-// two batch elements of 24 heads and 333 - 4470 rows, less a fixed 4.5 us):
-//   small      (128 query rows, three workgroups per CU)   0.75 with one per CU, 1.10 with two, 1.60 with three
-//   tracked    (256 rows, two per CU)                       1.16, 1.95
-//   pipelined  (256 rows, one per CU)                       1.05 a round
-// So the small tiles serve grids that would leave CUs idle (333 rows 12.8 -> 9.2 us, 1117 rows 23.5 -> 18.0, 1024 of
-// 4429 rows 68 -> 54) or half idle in the last round (2 x 1357 rows 45 -> 39, 4000 rows 118 -> 108), the pipelined
-// kernel one full round (2445 rows 49.6 -> 43.4), the tracked kernel everything larger: per row it does the least.
-// Between small and tracked the whole launch decides (`small_tiles_serve`), with all problems that are merged in it: the
-// same model holds for the patches of a step.  24 heads, image rows + 333 of text, us on tracked / small tiles:
-//   4096 in two patches 137 / 159, in four 149 / 164; two batch elements of 4600 in two 307 / 335, of 2304 + 154 in two
-//   116 / 92, of 5184 in eight (four per launch) 263 / 234; one patch of 1024 alone 79 / 58, with the text queries 82 / 79
-// Patches of sequences up to 4 * CUs workgroups are never pipelined (1024 of 4429 rows alone 54 us small, 68 pipelined),
-// those of longer ones only where the keys are one segment, so that no text queries can be left out (648 of 5517 rows,
-// two batch elements: 84 us, small 92, tracked 96).
-// HDIT_ATTN_PIPE=0 keeps every launch on the tracked-reference kernel with 256 rows, =1 puts every eligible launch on the
-// pipelined ones (for A/B timing).
-enum Kind { TRACKED, PIPELINED, SMALL };
-constexpr int SMALL_BQ = 128;
-
-double fill_cost(Kind kind, int64_t workgroups, int cus) {
-  const int64_t per_cu = (workgroups + cus - 1) / cus;
-  if (kind == PIPELINED) return 1.05 * (double)per_cu;
-  if (kind == TRACKED) return 1.95 * (double)(per_cu / 2) + (per_cu % 2 ? 1.16 : 0.0);
-  const int rest = (int)(per_cu % 3);
-  if (per_cu < 3) return rest == 1 ? 0.75 : 1.10;
-  return 1.60 * (double)(per_cu / 3) + 0.55 * rest;
+// Which kernel serves a problem.  The pipelined ones where there are at least three tiles of keys and a tile's step fits
+// 32 bits; the tracked one otherwise.  That is decided from keys and strides alone, and a row's result depends on the row
+// and the keys alone: neither rows that are left out (the text queries of a joint sequence) nor other problems of the
+// launch change a bit.
+// HDIT_ATTN_PIPE=0 keeps every launch on the tracked kernel, =4 and =8 every other one of head dim 64 on workgroups of four
+// or eight waves (for A/B timing).
+char pipe_env() {
+  static const char* env = getenv("HDIT_ATTN_PIPE");
+  return env ? env[0] : 0;
 }
 
-// The query rows of a problem, a segment counted with its key rows where its queries were left out: one that is empty
-// while the other one lies within the key segment of its own.
-int rows_with_text(const hdit_attn_args* a) {
-  int rows = a->q[0].len + a->q[1].len;
-  for (int s = 0; s < 2; s++)
-    if (a->q[s].len == 0 && a->q[1 - s].len <= a->k[1 - s].len) rows += a->k[s].len;
-  return rows;
+bool is_pipelined(const hdit_attn_args* a, const AttnParams& P) {
+  const bool strides_ok = a->k[0].stride_s < (1 << 22) && a->k[1].stride_s < (1 << 22) && a->v[0].stride_s < (1 << 22) &&
+                          a->v[1].stride_s < (1 << 22);  // a tile step (64 rows, in bytes) fits 32 bits
+  return pipe_env() != '0' && strides_ok && (P.skv + BKV - 1) / BKV >= PIPE_MIN_TILES;
 }
 
-int64_t workgroups(const hdit_attn_args* a, int rows, int rows_per_workgroup) {
+int64_t workgroups(const hdit_attn_args* a, int rows_per_workgroup) {
+  const int rows = a->q[0].len + a->q[1].len;
   return (int64_t)a->batch * a->heads * ((rows + rows_per_workgroup - 1) / rows_per_workgroup);
 }
 
-bool pipe_off() {
-  static const char* pipe_env = getenv("HDIT_ATTN_PIPE");
-  return pipe_env && pipe_env[0] == '0';
-}
-
-bool wants_pipelined(const hdit_attn_args* a, const AttnParams& P) {
-  static const char* pipe_env = getenv("HDIT_ATTN_PIPE");
-  const bool pipe_force = pipe_env && pipe_env[0] == '1';
-  const bool strides_ok = a->k[0].stride_s < (1 << 22) && a->k[1].stride_s < (1 << 22) && a->v[0].stride_s < (1 << 22) &&
-                          a->v[1].stride_s < (1 << 22);  // a tile step (64 rows, in bytes) fits 32 bits
-  if (pipe_off() || !strides_ok || (P.skv + BKV - 1) / BKV < PIPE_MIN_TILES) return false;
-  if (a->head_dim == 128 || pipe_force) return true;
-  const int cus = hdit_host::num_cus();
-  if (cus <= 0) return false;  // no device to ask: the launch reports it
-  const int rows = rows_with_text(a);
-  if (rows < P.skv) {
-    const bool joint = a->k[0].len > 0 && a->k[1].len > 0;
-    return !joint && workgroups(a, P.skv, BQ) > 4 * (int64_t)cus && workgroups(a, rows, BQ) * 8 <= (int64_t)cus * 5;
+// Query rows per workgroup of a pipelined launch at head dim 64, by how the workgroups fill the CUs.  Measured on MI355X,
+// 24 heads and more, microseconds per tile of 64 keys:
+//   128 rows, four waves, two workgroups per CU   0.55 where a CU has one, 0.90 where it has two
+//   256 rows, eight waves, one per CU             0.86, and 1 us more until it has begun (five tiles ahead, no neighbour)
+// Per row the same, so the last round decides, and small workgroups where CUs would be idle.  128 / 256 rows: 333 rows
+// 8.6 / 11.4 us, 2 x 666 15.0 / 16.1, 2 x 1357 37.1 / 39.3, 1024 of 4429 rows 41.0 / 57.5, two of them 63.3 / 60.1, 4470
+// rows 127.9 / 122.4, 2 x 4429 227 / 247, 17776 rows with 48 heads 3443 / 3378.
+int pipe_rows(const hdit_attn_args* const* of, int count) {
+  if (pipe_env() == '4') return 128;
+  if (pipe_env() == '8') return 256;
+  int64_t small = 0, large = 0, tiles = 0;
+  for (int i = 0; i < count; i++) {
+    small += workgroups(of[i], 128), large += workgroups(of[i], 256);
+    const int64_t t = (of[i]->k[0].len + of[i]->k[1].len + BKV - 1) / BKV;
+    if (t > tiles) tiles = t;
   }
-  const double tracked = fill_cost(TRACKED, workgroups(a, rows, BQ), cus), small = fill_cost(SMALL, workgroups(a, rows, SMALL_BQ), cus);
-  const double piped = fill_cost(PIPELINED, workgroups(a, rows, BQ), cus);
-  return piped < tracked && !(small < 0.93 * tracked && small < piped);
-}
-
-// Whether a launch of these many workgroups is better off with small tiles.  Where every workgroup of 256 rows has a CU
-// to itself it is (no more than two small ones then share a CU); above, the fill decides, by more than the few per cent
-// that the model resolves (2 x 4429 rows: 264.7 us on small tiles, 264.1 tracked).
-bool small_tiles_serve(int64_t grid_tracked, int64_t grid_small) {
   const int cus = hdit_host::num_cus();
-  if (pipe_off() || cus <= 0) return false;
-  return grid_tracked <= cus || fill_cost(SMALL, grid_small, cus) < 0.93 * fill_cost(TRACKED, grid_tracked, cus);
+  if (cus <= 0) return 256;  // no device to ask: the launch reports it
+  small = (small + cus - 1) / cus, large = (large + cus - 1) / cus;
+  const double cost_small = tiles * (0.90 * (double)(small / 2) + 0.55 * (double)(small % 2));
+  return cost_small <= tiles * 0.86 * (double)large + 1.0 ? 128 : 256;
 }
 
-int launch_one(int head_dim, const AttnParams& P, int q_tiles, unsigned grid, Kind kind, hipStream_t s) {
-  if (kind == SMALL) return hdit_attn::launch_d64_small(P, q_tiles, grid, s);
-  return head_dim == 64 ? hdit_attn::launch_d64(P, q_tiles, grid, kind == PIPELINED, s)
-                        : hdit_attn::launch_d128(P, q_tiles, grid, kind == PIPELINED, s);
+// The problems of one call that one kernel serves, as one launch.
+int launch_some(const hdit_attn_args* const* of, const AttnParams* P, int count, bool pipelined, hipStream_t s) {
+  const int hd = of[0]->head_dim;
+  const int rows = pipelined && hd == 64 ? pipe_rows(of, count) : 256;
+  int q_tiles[HDIT_ATTN_MAX_MULTI], nblocks[HDIT_ATTN_MAX_MULTI];
+  for (int i = 0; i < count; i++) {
+    q_tiles[i] = (P[i].sq + rows - 1) / rows;
+    nblocks[i] = (int)workgroups(of[i], rows);
+  }
+  if (!pipelined) return hd == 64 ? hdit_attn::launch_tracked_d64(P, q_tiles, nblocks, count, s) : hdit_attn::launch_tracked_d128(P, q_tiles, nblocks, count, s);
+  if (hd == 128) return hdit_attn::launch_pipe8_d128(P, q_tiles, nblocks, count, s);
+  return rows == 128 ? hdit_attn::launch_pipe4_d64(P, q_tiles, nblocks, count, s) : hdit_attn::launch_pipe8_d64(P, q_tiles, nblocks, count, s);
 }
 }  // namespace
 
@@ -196,16 +129,8 @@ extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16(const h
   int rc = hdit_host::attn_validate(a);
   if (rc != HDIT_OK) return rc;
   AttnParams P;
-  int q_tiles;
-  unsigned grid;
-  if (!to_params(a, P, q_tiles, grid)) return HDIT_OK;
-  Kind kind = wants_pipelined(a, P) ? PIPELINED : TRACKED;
-  if (kind == TRACKED && a->head_dim == 64 && small_tiles_serve(grid, workgroups(a, P.sq, SMALL_BQ))) {
-    kind = SMALL;
-    q_tiles = (P.sq + SMALL_BQ - 1) / SMALL_BQ;
-    grid = (unsigned)workgroups(a, P.sq, SMALL_BQ);
-  }
-  rc = launch_one(a->head_dim, P, q_tiles, grid, kind, (hipStream_t)stream);
+  if (!to_params(a, P)) return HDIT_OK;
+  rc = launch_some(&a, &P, 1, is_pipelined(a, P), (hipStream_t)stream);
   if (rc != HDIT_OK) return rc;
   return hdit_host::check_launch("hdit_attn_fwd_bf16");
 }
@@ -218,37 +143,17 @@ extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16_multi(c
     if (rc != HDIT_OK) return rc;
     if (args[i].head_dim != args[0].head_dim) return HDIT_EINVAL;
   }
-  // one merged launch of the problems for the pipelined kernel, one of the others
+  // one merged launch of the problems for the pipelined kernels, one of the others
   for (int pass = 0; pass < 2; pass++) {
     AttnParams P[HDIT_ATTN_MAX_MULTI];
     const hdit_attn_args* of[HDIT_ATTN_MAX_MULTI];
-    int q_tiles[HDIT_ATTN_MAX_MULTI], nblocks[HDIT_ATTN_MAX_MULTI], n = 0;
-    int64_t grid_tracked = 0, grid_small = 0;
+    int n = 0;
     for (int i = 0; i < count; i++) {
-      unsigned grid;
-      if (!to_params(&args[i], P[n], q_tiles[n], grid)) continue;
-      if (wants_pipelined(&args[i], P[n]) != (pass == 0)) continue;
-      grid_tracked += grid;
-      grid_small += workgroups(&args[i], P[n].sq, SMALL_BQ);
-      of[n] = &args[i];
-      nblocks[n++] = (int)grid;
-    }
-    Kind kind = pass == 0 ? PIPELINED : TRACKED;
-    if (kind == TRACKED && args[0].head_dim == 64 && n > 0 && small_tiles_serve(grid_tracked, grid_small)) {
-      kind = SMALL;
-      for (int i = 0; i < n; i++) {
-        q_tiles[i] = (P[i].sq + SMALL_BQ - 1) / SMALL_BQ;
-        nblocks[i] = (int)workgroups(of[i], P[i].sq, SMALL_BQ);
-      }
+      if (!to_params(&args[i], P[n]) || is_pipelined(&args[i], P[n]) != (pass == 0)) continue;
+      of[n++] = &args[i];
     }
     if (n == 0) continue;
-    hipStream_t s = (hipStream_t)stream;
-    int rc;
-    if (n == 1) rc = launch_one(args[0].head_dim, P[0], q_tiles[0], (unsigned)nblocks[0], kind, s);
-    else if (kind == SMALL) rc = hdit_attn::launch_multi_d64_small(P, q_tiles, nblocks, n, s);
-    else
-      rc = args[0].head_dim == 64 ? hdit_attn::launch_multi_d64(P, q_tiles, nblocks, n, kind == PIPELINED, s)
-                                  : hdit_attn::launch_multi_d128(P, q_tiles, nblocks, n, kind == PIPELINED, s);
+    int rc = launch_some(of, P, n, pass == 0, (hipStream_t)stream);
     if (rc != HDIT_OK) return rc;
     if ((rc = hdit_host::check_launch("hdit_attn_fwd_bf16_multi")) != HDIT_OK) return rc;
   }

@@ -4,10 +4,13 @@
 //
 // Joint (image + text) flash attention forward for gfx950, bf16 in/out.
 //
+// Two kernels: the pipelined one further down serves everything that has three
+// tiles of keys; the one described here ("tracked") the rest, and the rows for
+// which the pipelined kernel's fixed softmax reference does not hold.
+//
 // Work split: one workgroup = 4 waves = 256 query rows of one (batch, head);
-// each wave owns 64 query rows (two 32-row MFMA column blocks; one block and
-// 128 rows per workgroup in attention_bf16_small.hip) and walks the
-// keys in tiles of 64.  K and V tiles go straight from global memory into two
+// each wave owns 64 query rows (two 32-row MFMA column blocks; one block inside
+// the pipelined kernels) and walks the keys in tiles of 64.  K and V tiles go straight from global memory into two
 // LDS buffers (direct-to-LDS loads, one barrier per tile).
 //
 // The scores are produced transposed, S^T = K . Q^T, with K rows as the MFMA
@@ -28,6 +31,7 @@
 #include <atomic>
 #include <cstdlib>
 #include <type_traits>
+#include <utility>
 
 #include "hdit_common.h"
 
@@ -56,16 +60,14 @@ struct AttnParams {
   float scale_log2;
 };
 
-// Launch of the kernels for one head dim on an argument block the entry point has validated and converted.
-// pipelined: take the software-pipelined kernel (the caller has checked that the problem qualifies).
-int launch_d64(const AttnParams& P, int q_tiles, unsigned grid, bool pipelined, hipStream_t stream);
-int launch_d128(const AttnParams& P, int q_tiles, unsigned grid, bool pipelined, hipStream_t stream);
-// head dim 64, one query block per wave: q_tiles of 128 query rows
-int launch_d64_small(const AttnParams& P, int q_tiles, unsigned grid, hipStream_t stream);
-int launch_multi_d64_small(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
-// `count` problems of one head dim as one grid of the tracked or of the pipelined kernel
-int launch_multi_d64(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, bool pipelined, hipStream_t stream);
-int launch_multi_d128(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, bool pipelined, hipStream_t stream);
+// Launch of `count` problems of one head dim, on argument blocks the entry point has validated and converted, as one grid:
+// the tracked kernel (256 query rows per workgroup), the pipelined ones of 128 and 256 rows.  q_tiles and nblocks count
+// workgroups of those rows.
+int launch_tracked_d64(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
+int launch_tracked_d128(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
+int launch_pipe4_d64(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
+int launch_pipe8_d64(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
+int launch_pipe8_d128(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
 
 }  // namespace hdit_attn
 
@@ -76,11 +78,15 @@ using hdit_attn::Seg2;
 
 constexpr int BKV = 64;   // keys per tile
 #ifndef HDIT_ATTN_QUERY_BLOCKS
-#define HDIT_ATTN_QUERY_BLOCKS 2  // 32-row query blocks per wave (attention_bf16_small.hip: 1)
+#define HDIT_ATTN_QUERY_BLOCKS 2  // 32-row query blocks per wave (the pipelined kernels' units: 1)
 #endif
 constexpr int QB = HDIT_ATTN_QUERY_BLOCKS;
 constexpr int WQ = 32 * QB;  // query rows per wave
-constexpr int NWAVE = 4;
+#ifndef HDIT_ATTN_WAVES
+#define HDIT_ATTN_WAVES 4  // waves per workgroup (attention_bf16_pipe8.hip: 8)
+#endif
+constexpr int NWAVE = HDIT_ATTN_WAVES;
+constexpr int NTHR = 64 * NWAVE;
 constexpr int BQ = WQ * NWAVE;
 
 template <int HD>
@@ -105,7 +111,7 @@ struct Lds {
   static constexpr int Q_ROW = HD * 2 + 16;
   static constexpr int Q_OFF = 2 * STAGE;
   static constexpr int Q_WAVE_BYTES = WQ * Q_ROW;
-  static constexpr int TOTAL = 2 * STAGE + (Q_IN_LDS ? 4 * Q_WAVE_BYTES : 0);
+  static constexpr int TOTAL = 2 * STAGE + (Q_IN_LDS ? NWAVE * Q_WAVE_BYTES : 0);
   static_assert(TOTAL <= 160 * 1024, "attention tiles do not fit the LDS");
 };
 
@@ -161,15 +167,16 @@ constexpr int waitcnt_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0
 constexpr float RESCALE_THRESHOLD = 8.0f;
 
 // The whole kernel for one workgroup: the online softmax with a running reference that follows the column
-// maxima.  Also the second pass of the pipelined d = 64 kernel when its fixed reference overflowed.
+// maxima.  Also the second pass of the pipelined kernels, for the rows whose fixed reference did not hold: bit l of
+// `rows` (one query block per wave) stands for the wave's row l, the others have been written.
 template <int HD>
 __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_tiles, unsigned char* lds, int block_id,
-                                                  int nblocks) {
+                                                  int nblocks, unsigned rows = ~0u) {
   using L = Lds<HD>;
   constexpr int KS = HD / 16;       // k-steps of the S^T MFMA (over head dim)
   constexpr int DB = HD / 32;       // 32-wide d blocks of O^T
   constexpr int CPR = HD / 8;       // 16-byte chunks per row
-  constexpr int NCH = BKV * CPR / 256;  // chunks per thread per tile (K and V each)
+  constexpr int NCH = BKV * CPR / NTHR;  // chunks per thread per tile (K and V each)
   // FOLD: the softmax scale is multiplied into Q once and the running reference m is subtracted inside the
   // score MFMA (its first k-step accumulates onto -m), so the accumulators feed exp2 directly: one FMA less
   // per score in a loop that is bound by the VALU.  Costs 32 registers; the d = 128 kernel has none to spare.
@@ -241,7 +248,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
   // (wave-uniform base) + (loop-invariant per-thread offset); the tile that straddles the segment boundary
   // and the last, clamped tile take the per-row path.
   unsigned koff[2][NCH], voff[2][NCH];
-  // direct-to-LDS (d = 64): request i of a wave covers rows 8*(wave + 4*i) .. +7, lane -> (row, slot lane%8);
+  // direct-to-LDS (d = 64): request i of a wave covers rows 8*(wave + NWAVE*i) .. +7, lane -> (row, slot lane%8);
   // the chunk fetched for a slot is the slot index XORed with the row's swizzle (the same for every i)
   constexpr int RPI = 64 / CPR;  // rows per request
   const int dma_row = wave * RPI + lane / CPR;
@@ -250,7 +257,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
   const unsigned lds_base_addr = __builtin_amdgcn_readfirstlane(lds_address(lds));
 #pragma unroll
   for (int i = 0; i < NCH; i++) {
-    const int row = dma_row + 4 * RPI * i;
+    const int row = dma_row + NWAVE * RPI * i;
     koff[0][i] = (unsigned)((row * P.k.ss0 + dma_kc * 8) * 2);
     koff[1][i] = (unsigned)((row * P.k.ss1 + dma_kc * 8) * 2);
     voff[0][i] = (unsigned)((row * P.v.ss0 + dma_vc * 8) * 2);
@@ -271,23 +278,23 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
       const unsigned char* vb = vb0 + (int64_t)r0 * P.v.ss0 * 2;
 #pragma unroll
       for (int i = 0; i < NCH; i++) {
-        lds_dma16<false>(kb, koff[0][i], kdst + i * 4096);
-        lds_dma16<false>(vb, voff[0][i], vdst + i * 4096);
+        lds_dma16<false>(kb, koff[0][i], kdst + i * (NWAVE * 1024));
+        lds_dma16<false>(vb, voff[0][i], vdst + i * (NWAVE * 1024));
       }
     } else if (r0 >= len0 && r0 + BKV <= P.skv) {
       const unsigned char* kb = kb1 + (int64_t)(r0 - len0) * P.k.ss1 * 2;
       const unsigned char* vb = vb1 + (int64_t)(r0 - len0) * P.v.ss1 * 2;
 #pragma unroll
       for (int i = 0; i < NCH; i++) {
-        lds_dma16<false>(kb, koff[1][i], kdst + i * 4096);
-        lds_dma16<false>(vb, voff[1][i], vdst + i * 4096);
+        lds_dma16<false>(kb, koff[1][i], kdst + i * (NWAVE * 1024));
+        lds_dma16<false>(vb, voff[1][i], vdst + i * (NWAVE * 1024));
       }
     } else {
 #pragma unroll
       for (int i = 0; i < NCH; i++) {
-        const int r = min(r0 + dma_row + 4 * RPI * i, P.skv - 1);
-        lds_dma16_ptr<false>((const unsigned char*)(row_ptr(P.k, b, h, r) + dma_kc * 8), kdst + i * 4096);
-        lds_dma16_ptr<false>((const unsigned char*)(row_ptr(P.v, b, h, r) + dma_vc * 8), vdst + i * 4096);
+        const int r = min(r0 + dma_row + NWAVE * RPI * i, P.skv - 1);
+        lds_dma16_ptr<false>((const unsigned char*)(row_ptr(P.k, b, h, r) + dma_kc * 8), kdst + i * (NWAVE * 1024));
+        lds_dma16_ptr<false>((const unsigned char*)(row_ptr(P.v, b, h, r) + dma_vc * 8), vdst + i * (NWAVE * 1024));
       }
     }
   };
@@ -330,16 +337,16 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
     if constexpr (L::Q_IN_LDS) {
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) {
-        bf16x8 qk[2], kf[2];
+        bf16x8 qk[QB], kf[2];
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) qk[qb] = *(const bf16x8*)(qlds + (qb * 32 + l32) * L::Q_ROW + lh * 16 + ks * 32);
+        for (int qb = 0; qb < QB; qb++) qk[qb] = *(const bf16x8*)(qlds + (qb * 32 + l32) * L::Q_ROW + lh * 16 + ks * 32);
 #pragma unroll
         for (int kb = 0; kb < 2; kb++)
           kf[kb] = *(const bf16x8*)(sk + k_off + kb * 32 * L::K_ROW + (((ks * 2 + lh) ^ k_swz) << 4));
 #pragma unroll
         for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-          for (int qb = 0; qb < 2; qb++)
+          for (int qb = 0; qb < QB; qb++)
             sacc[kb][qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kb], qk[qb], ks == 0 ? zero16 : sacc[kb][qb], 0, 0, 0);
       }
     }
@@ -420,9 +427,9 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
         first = false;
       }
     } else {
-      float mcand[2];
+      float mcand[QB];
 #pragma unroll
-      for (int qb = 0; qb < 2; qb++) {
+      for (int qb = 0; qb < QB; qb++) {
         float mx = fmaxf(sacc[0][qb][0], sacc[1][qb][0]);
 #pragma unroll
         for (int v = 1; v < 16; v++) mx = fmaxf(fmaxf(mx, sacc[0][qb][v]), sacc[1][qb][v]);  // one v_max3 per step
@@ -431,10 +438,10 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
         mcand[qb] = fmaxf(m_run[qb], mx * P.scale_log2);
       }
       // raise the running maxima (and rescale) only if some row outgrew the threshold: wave-uniform branch
-      const bool grow = (mcand[0] - m_run[0] > RESCALE_THRESHOLD) || (mcand[1] - m_run[1] > RESCALE_THRESHOLD);
+      const bool grow = (mcand[0] - m_run[0] > RESCALE_THRESHOLD) || (mcand[QB - 1] - m_run[QB - 1] > RESCALE_THRESHOLD);
       if (__builtin_amdgcn_ballot_w64(grow) != 0) {
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) {
+        for (int qb = 0; qb < QB; qb++) {
           const float alpha = __builtin_amdgcn_exp2f(m_run[qb] - mcand[qb]);
           m_run[qb] = mcand[qb];
           l_run[qb] *= alpha;
@@ -525,7 +532,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(l_run[qb]), __float_as_int(l_run[qb]), false, false);
     const float inv = 1.0f / (__int_as_float(sw[0]) + __int_as_float(sw[1]));
     const int r = q0 + qb * 32 + l32;
-    if (r >= P.sq) continue;
+    if (r >= P.sq || (QB == 1 && !((rows >> l32) & 1))) continue;
     __bf16* op = (__bf16*)row_ptr(P.o, b, h, r);
 #pragma unroll
     for (int db = 0; db < DB; db++)
@@ -540,7 +547,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
 }
 
 template <int HD>
-__global__ void __launch_bounds__(256, (HD == 64 ? (QB == 1 ? 3 : 2) : 1)) attn_fwd_kernel(const AttnParams P, int q_tiles) {
+__global__ void __launch_bounds__(NTHR, HD == 64 ? 2 : 1) attn_fwd_kernel(const AttnParams P, int q_tiles) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   attn_tracked_body<HD>(P, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x);
 }
@@ -558,7 +565,7 @@ struct AttnMulti {
 };
 
 template <int HD>
-__global__ void __launch_bounds__(256, (HD == 64 ? (QB == 1 ? 3 : 2) : 1)) attn_fwd_multi_kernel(const AttnMulti M) {
+__global__ void __launch_bounds__(NTHR, HD == 64 ? 2 : 1) attn_fwd_multi_kernel(const AttnMulti M) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   int i = 0;
 #pragma unroll 1
@@ -569,67 +576,97 @@ __global__ void __launch_bounds__(256, (HD == 64 ? (QB == 1 ? 3 : 2) : 1)) attn_
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Software-pipelined inside the wave (both head sizes).
+// The pipelined kernels.
 //
-// On this chip the matrix pipe and the vector ALU of a SIMD overlap only inside ONE wave's instruction stream
-// (an MFMA executes for 32 cycles after it issued, and independent VALU instructions of the same wave issue
-// under it); two waves do not overlap each other.  A tile's work is half MFMA and half VALU (exponentials,
-// packs, row sums), so the kernel above, whose waves alternate between an MFMA phase and a VALU phase, pays
-// the sum.  Here a wave owns its SIMD alone (512 registers) and every instruction between two tile barriers
-// is one basic block in which the score MFMAs of tile t+1 and the PV MFMAs of tile t are dealt between the
-// softmax instructions of tile t:
+// What bounds a tile is the sum of what the vector ALU has to issue (the exponentials, packs, and about 8 cycles for
+// every MFMA) and, beside it, the matrix pipe -- and where the whole chip works, the board's power.  An MFMA runs beside
+// vector instructions of its own wave and of the SIMD's other waves (measured: 32 MFMAs of 32 cycles in one wave, 256
+// additions, exponentials, maxima or packs in the other: the longer of the two plus 8 cycles per MFMA).  The exceptions
+// are the dot products (v_dot2*): they wait for the matrix pipe, 256 of them beside those MFMAs take the sum of both.  The
+// row sums of the kernel above are dot products; here they are 4x4x4 MFMAs, which add four of a lane's own values.
 //
-//   segment A   P.V step 3 of tile t-1 (4 MFMAs) + scores of tile t, keys 32-63, k-steps 0-1 (4)  |  exp/pack/sum of keys  0-15
-//   segment B   scores of tile t, keys 32-63, k-steps 2-3 (4) + P.V step 0 of tile t (4)          |  keys 16-31
-//   segment C   scores of tile t+1, keys 0-31 (8), into the registers keys 0-31 of tile t vacated  |  keys 32-47
-//   segment D   P.V steps 1, 2 of tile t (8)                                                      |  keys 48-63
+// So a wave's instruction stream is laid out so that both always have work: between two barriers it is one basic block in
+// which every MFMA is followed by its share of everything else, pinned there (`sched_barrier`):
+//
+//   slots [0, F)        P.V of keys 32-63 of tile t-1, scores of keys 32-63 of tile t     | softmax of keys  0-31 of tile t
+//   slots [F, 2F)       P.V of keys  0-31 of tile t,   scores of keys  0-31 of tile t+1   | softmax of keys 32-63 of tile t
+//
+// F = HD / 4.  A wave owns 32 query rows in 256 registers, so that a SIMD has two waves: one alone issues an instruction
+// every 4.5 cycles at best (165 of them per tile at d = 64).  The MFMAs are 16x16x32: less energy per flop (see
+// gemm_bf16.hip).  A lane owns one query column of each of two 16-row blocks and 4 of every 16 keys.
+// Operands: fragment f (two MFMAs) is read FRAG_LEAD fragments ahead, across the barrier too; the tile requests are
+// dealt over the slots and have a pointer per lane that moves on from tile to tile.
+//
+// Measured on one box, the better of the kernel above and a former pipelined one (64 rows per wave, one wave per SIMD, dot
+// products, 32x32x16 MFMAs, requests in one piece) -> this one.  d = 64, 24 heads: 333 rows 8.9 -> 8.6 us, 2 x 666 18.1 ->
+// 15.0, 1357 27.2 -> 24.0, 4470 130 -> 122, 1024 of 4429 rows 52.3 -> 41.0, two of them 75 -> 60, 2 x 4429 255 -> 227; 17776 rows
+// with 48 heads 3573 -> 3378 (1.15 PFLOP/s).  d = 128, 24 heads: 1536 rows 50.5 -> 42.1, 4608 258 -> 214, 9728 1062 -> 903 (1.29
+// PFLOP/s), 16896 3420 -> 2880.  Of the steps, at 2 x 4429 rows: this layout 244, the loop unrolled over the ring 241 (a
+// fragment's address needs no addition), one exponential per MFMA in place of two in turn with none 235, the query rows
+// requested in front of the tiles 1 us (at 333 rows 9.3 -> 8.6).  With 32x32x16 MFMAs a SIMD's tile takes fewer cycles (each
+// MFMA holds the issue port) but the clock falls by more: 2 x 4429 rows 244 us at 1.92 GHz against 244 at 2.15.
 //
 // For the block to have no branch the reference of the online softmax is fixed after the first tile (its column
 // maxima plus a margin: p = 2^(s - m) may then grow to PIPE_LIMIT and shrink to nothing without any loss
-// of relative precision in fp32 / bf16): no maxima, no rescale in the loop.  A row whose sum ends at or above
-// the limit (infinity and NaN included) makes the whole workgroup run the tracked kernel above from the start.
-// K tiles are staged one tile ahead of V tiles (the scores run half a tile ahead of P.V), in rings of four LDS slots
-// each, requested two tiles before they are read.
-constexpr int PIPE_RING = 4;  // LDS slots per operand
-// iteration t requests K tile t + PIPE_LEAD and V tile t + PIPE_LEAD - 1 (rings of 8 with leads of 5 and 7 tiles
-// were measured: no difference, the requests arrive in time)
-constexpr int PIPE_LEAD = 3;
-static_assert(PIPE_LEAD >= 3 && PIPE_LEAD < PIPE_RING, "a requested tile must not land in a slot still being read");
-constexpr int PIPE_MASK = PIPE_RING - 1;
+// of relative precision in fp32 / bf16): no maxima, no rescale in the loop.  (The key that holds the maximum has a p that
+// bf16 represents exactly.  With the maxima of 32 keys instead of the tile's 64, as the kernel above has them, results with
+// peaked logits were up to 1.2 % further from 64 bits.)  Rows whose sum ends at or above
+// the limit (infinity and NaN included) are left to the body of the kernel above, which the workgroup then runs for them.
+// So a row's result depends on that row and the keys alone, whatever rows it shares a wave or workgroup with.
 template <int HD>
 struct PipeLds {
-  static constexpr int ROW = HD * 2;         // bytes of a K or V row
-  static constexpr int TILE = BKV * ROW;     // bytes of one K or V tile
-  static constexpr int V_OFF = PIPE_RING * TILE;
-  static constexpr int FLAG_OFF = 2 * PIPE_RING * TILE;
+  // tiles between two barriers: eight waves wait for each other half as often where twice the slots fit (17776 keys,
+  // 48 heads, d = 64: 3800 us with one, 3658 with two)
+  static constexpr int SYNC = HD == 64 && NWAVE == 8 ? 2 : 1;
+  static constexpr int RING = SYNC == 2 ? 8 : 4;  // LDS slots per operand
+  // Iteration t requests K tile t + LEAD and V tile t + LEAD - 1.  It reads K tiles t and t + 1 and V tiles t - 1 and t: a
+  // slot is requested again at the earliest when every wave has passed a barrier behind its last use.
+  static constexpr int LEAD = SYNC == 2 ? 5 : 3;
+  static constexpr int MASK = RING - 1;
+  static constexpr int ROW = HD * 2;      // bytes of a K or V row
+  static constexpr int TILE = BKV * ROW;  // bytes of one K or V tile
+  static constexpr int V_OFF = RING * TILE;
+  static constexpr int FLAG_OFF = 2 * RING * TILE;
   // the launch also covers the tracked kernel's layout, which a workgroup falls back to
   static constexpr int TOTAL = FLAG_OFF + 16 > Lds<HD>::TOTAL ? FLAG_OFF + 16 : Lds<HD>::TOTAL;
   static_assert(TOTAL <= 160 * 1024, "rings do not fit the LDS");
+  static_assert(NWAVE != 4 || HD != 64 || TOTAL <= 80 * 1024, "two workgroups per CU");
 };
-constexpr float PIPE_MARGIN = 24.0f;
+constexpr float PIPE_MARGIN = 24.0f;  // an integer: the exact p's stay exact
 constexpr float PIPE_LIMIT = 0x1p40f;
 constexpr int PIPE_MIN_TILES = 3;
+constexpr int FRAG_LEAD = 3;
 
-#define SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
+template <int... I, class F>
+__device__ __forceinline__ void static_for_seq(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_seq(std::make_integer_sequence<int, N>{}, f);
+}
 
-// true: the fixed reference did not hold, nothing has been written, the whole workgroup starts over
+constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0f70; }
+
+// true: the fixed reference did not hold for some row of the workgroup; those of this wave are set in `rows`
 template <int HD>
-__device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles, unsigned char* lds, int block_id, int nblocks) {
-  static_assert(QB == 2, "written for two query blocks per wave");
+__device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles, unsigned char* lds, int block_id, int nblocks,
+                                               unsigned& rows) {
   using PL = PipeLds<HD>;
-  constexpr int KS = HD / 16, DB = HD / 32, CPR = HD / 8, NCH = BKV * CPR / 256, RPI = 64 / CPR, ROW = PL::ROW;
-  constexpr int PIPE_TILE = PL::TILE, PIPE_V_OFF = PL::V_OFF, PIPE_FLAG_OFF = PL::FLAG_OFF;
-  constexpr int NMFMA = 4 * KS + 8 * DB;  // per iteration: two key blocks of scores, four P.V steps
-  constexpr int VALU_PER_MFMA = (160 + NMFMA - 1) / NMFMA;
+  constexpr int KS = HD / 32, DB = HD / 16, CPR = HD / 8, NCH = BKV * CPR / NTHR, RPI = 64 / CPR, ROW = PL::ROW;
+  constexpr int TILE = PL::TILE, V_OFF = PL::V_OFF, LEAD = PL::LEAD, MASK = PL::MASK, SYNC = PL::SYNC;
+  constexpr int F = 2 * DB + 4 * KS;  // fragments per iteration, two MFMAs each
+  constexpr int PER = F / 8;          // MFMAs per pair of scores (16 pairs)
+  constexpr int ROWS = 32 * NWAVE;    // query rows per workgroup
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int l32 = lane & 31, lh = lane >> 5;
+  const int l16 = lane & 15, lg = lane >> 4;
   // same placement of (batch, head, query tile) on workgroups as the kernel above
   const int nbh = nblocks / q_tiles;
   const bool by_xcd = nbh % 8 == 0;
   const int slot = by_xcd ? (block_id >> 3) : block_id;
   const int nbh_loc = by_xcd ? nbh / 8 : nbh;
   int qt = slot % q_tiles, bhl = slot / q_tiles;
-  if (q_tiles > 1 && P.sq % BQ != 0) {
+  if (q_tiles > 1 && P.sq % ROWS != 0) {
     const int heavy = nbh_loc * (q_tiles - 1);
     if (slot < heavy) {
       qt = slot % (q_tiles - 1);
@@ -641,390 +678,379 @@ __device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles,
   }
   const int bh = by_xcd ? bhl * 8 + (block_id & 7) : bhl;
   const int b = bh / P.heads, h = bh % P.heads;
-  const int q0 = qt * BQ + wave * WQ;
+  const int q0 = qt * ROWS + wave * 32;
   const bool active = __builtin_amdgcn_readfirstlane(q0 < P.sq);
   const int NT = (P.skv + BKV - 1) / BKV;  // >= PIPE_MIN_TILES (host)
+  rows = 0;
 
   typedef __attribute__((address_space(3))) int lds_int;
-  lds_int* const flag = (lds_int*)(uintptr_t)(lds_address(lds) + PIPE_FLAG_OFF);
+  lds_int* const flag = (lds_int*)(uintptr_t)(lds_address(lds) + PL::FLAG_OFF);
 
-  // ---- K / V tile requests, straight into LDS (same source-side swizzles as the kernel above)
+  // ---- K / V tile requests, straight into LDS.  Slot p of K row r holds chunk p ^ ((r>>1)&7) (d = 64) or p ^ (r&15), as
+  // in the kernel above: a fragment read covers 16 rows.  A transpose read takes 32 bytes of each of 16 V rows: slot p of
+  // V row r holds chunk p ^ 2*((r>>1)&3) (d = 64) or p ^ 2*(r&7), which spreads eight rows over the banks.
   const int dma_row = wave * RPI + lane / CPR;
   const int dma_kc = (lane % CPR) ^ (HD == 64 ? ((dma_row >> 1) & 7) : (dma_row & 15));
-  const int dma_vc = (lane % CPR) ^ (4 * (HD == 64 ? ((dma_row >> 1) & 1) : (dma_row & 3)));
+  const int dma_vc = (lane % CPR) ^ (2 * (HD == 64 ? ((dma_row >> 1) & 3) : (dma_row & 7)));
   const unsigned lds_base_addr = __builtin_amdgcn_readfirstlane(lds_address(lds));
-  // lane offsets of request 0 inside a tile of segment 0 / 1; request i lies 4 * RPI * i rows further down, a
-  // scalar step that goes into the request's scalar base
-  unsigned koff[2], voff[2];
-  koff[0] = (unsigned)((dma_row * P.k.ss0 + dma_kc * 8) * 2);
-  koff[1] = (unsigned)((dma_row * P.k.ss1 + dma_kc * 8) * 2);
-  voff[0] = (unsigned)((dma_row * P.v.ss0 + dma_vc * 8) * 2);
-  voff[1] = (unsigned)((dma_row * P.v.ss1 + dma_vc * 8) * 2);
-  // A tile that lies inside one segment is (scalar base of the segment + tile * bytes per tile) + a loop-invariant
-  // lane offset: four scalar instructions for the address (the host has checked that a tile step fits 32 bits).
-  // The tile that straddles the segment boundary and the clamped last tile take the per-row path.
   const int len0 = P.k.len0;
-  const int full0 = len0 / BKV;              // tiles [0, full0) lie in segment 0
-  const int first1 = (len0 + BKV - 1) / BKV; // tiles [first1, full_all) lie in segment 1
+  const int full0 = len0 / BKV;               // tiles [0, full0) lie in segment 0
+  const int first1 = (len0 + BKV - 1) / BKV;  // tiles [first1, full_all) lie in segment 1
   const int full_all = P.skv / BKV;
-  const unsigned span1 = full_all > first1 ? (unsigned)(full_all - first1) : 0u;
   const uint64_t kb0 = (uint64_t)(P.k.p0 + b * P.k.sb0 + h * P.k.sh0);
   const uint64_t vb0 = (uint64_t)(P.v.p0 + b * P.v.sb0 + h * P.v.sh0);
-  // segment 1 bases moved back by the rows of segment 0, so that they too are indexed by the tile number
+  // segment 1 bases moved back by the rows of segment 0, so that they too are indexed by the row number
   const uint64_t kb1 = (uint64_t)(P.k.p1 + b * P.k.sb1 + h * P.k.sh1) - (uint64_t)((int64_t)len0 * P.k.ss1 * 2);
   const uint64_t vb1 = (uint64_t)(P.v.p1 + b * P.v.sb1 + h * P.v.sh1) - (uint64_t)((int64_t)len0 * P.v.ss1 * 2);
   const unsigned krow0 = (unsigned)(P.k.ss0 * 2), krow1 = (unsigned)(P.k.ss1 * 2);  // bytes per row
   const unsigned vrow0 = (unsigned)(P.v.ss0 * 2), vrow1 = (unsigned)(P.v.ss1 * 2);
-  const unsigned kstep0 = krow0 * BKV, kstep1 = krow1 * BKV, vstep0 = vrow0 * BKV, vstep1 = vrow1 * BKV;
   const unsigned wave_dst = lds_base_addr + __builtin_amdgcn_readfirstlane(wave) * 1024;
-  // tile t (clamped to the last one) into the LDS bytes at dst (this wave's share: two requests 4 KiB apart)
-  auto dma_k = [&](int t, unsigned dst) __attribute__((always_inline)) {
-    if (t < full0) {
-      const unsigned char* kb = (const unsigned char*)(kb0 + (uint64_t)(unsigned)t * kstep0);
+  // A pointer per lane and request.  It moves on by one tile (a uniform step that fits 32 bits: host) while the tiles lie
+  // inside one segment; where one straddles the boundary, begins a segment or is the clamped last one, the pointers are
+  // formed row by row, outside of the block that holds the arithmetic.  Past the end the last tile is requested again
+  // (into a slot nobody reads any more): every iteration issues the same number of requests.
+  uint64_t kp[NCH], vp[NCH];
+  auto k_ptrs = [&](int t) __attribute__((always_inline)) {
+    const int r0 = min(t, NT - 1) * BKV;
 #pragma unroll
-      for (int i = 0; i < NCH; i++) lds_dma16<true>(kb + i * (4 * RPI) * krow0, koff[0], dst + i * 4096);
-    } else if ((unsigned)(t - first1) < span1) {
-      const unsigned char* kb = (const unsigned char*)(kb1 + (uint64_t)(unsigned)t * kstep1);
-#pragma unroll
-      for (int i = 0; i < NCH; i++) lds_dma16<true>(kb + i * (4 * RPI) * krow1, koff[1], dst + i * 4096);
-    } else {
-      const int r0 = min(t, NT - 1) * BKV;
-#pragma unroll
-      for (int i = 0; i < NCH; i++) {
-        const int r = min(r0 + dma_row + 4 * RPI * i, P.skv - 1);
-        const bool in0 = r < len0;
-        const uint64_t a = (in0 ? kb0 : kb1) + (uint64_t)(unsigned)r * (in0 ? krow0 : krow1) + dma_kc * 16;
-        lds_dma16_ptr<true>((const unsigned char*)a, dst + i * 4096);
-      }
+    for (int i = 0; i < NCH; i++) {
+      const int r = min(r0 + dma_row + NWAVE * RPI * i, P.skv - 1);
+      const bool in0 = r < len0;
+      kp[i] = (in0 ? kb0 : kb1) + (uint64_t)(unsigned)r * (in0 ? krow0 : krow1) + dma_kc * 16;
     }
   };
-  auto dma_v = [&](int t, unsigned dst) __attribute__((always_inline)) {
-    if (t < full0) {
-      const unsigned char* vb = (const unsigned char*)(vb0 + (uint64_t)(unsigned)t * vstep0);
+  auto v_ptrs = [&](int t) __attribute__((always_inline)) {
+    const int r0 = min(t, NT - 1) * BKV;
 #pragma unroll
-      for (int i = 0; i < NCH; i++) lds_dma16<true>(vb + i * (4 * RPI) * vrow0, voff[0], dst + i * 4096);
-    } else if ((unsigned)(t - first1) < span1) {
-      const unsigned char* vb = (const unsigned char*)(vb1 + (uint64_t)(unsigned)t * vstep1);
-#pragma unroll
-      for (int i = 0; i < NCH; i++) lds_dma16<true>(vb + i * (4 * RPI) * vrow1, voff[1], dst + i * 4096);
-    } else {
-      const int r0 = min(t, NT - 1) * BKV;
-#pragma unroll
-      for (int i = 0; i < NCH; i++) {
-        const int r = min(r0 + dma_row + 4 * RPI * i, P.skv - 1);
-        const bool in0 = r < len0;
-        const uint64_t a = (in0 ? vb0 : vb1) + (uint64_t)(unsigned)r * (in0 ? vrow0 : vrow1) + dma_vc * 16;
-        lds_dma16_ptr<true>((const unsigned char*)a, dst + i * 4096);
-      }
+    for (int i = 0; i < NCH; i++) {
+      const int r = min(r0 + dma_row + NWAVE * RPI * i, P.skv - 1);
+      const bool in0 = r < len0;
+      vp[i] = (in0 ? vb0 : vb1) + (uint64_t)(unsigned)r * (in0 ? vrow0 : vrow1) + dma_vc * 16;
     }
   };
-  // Iteration t works on the scores of tiles t (keys 32-63) and t+1 (keys 0-31) and the probabilities of tile t.
-  // It requests K tile t+3 and V tile t+2 first and, at its end, waits for everything older than those requests
-  // (a wave's requests complete in order): K tile t+2 and V tile t+1, which the barrier then publishes.
-  // Past the end the last tile is simply requested again (into a slot nobody reads any more): every iteration
-  // then issues the same number of requests, its closing wait is one immediate, and the block that holds the
-  // arithmetic ends at the barrier without a branch the compiler could sink instructions behind.
-  auto stage_begin = [&](int t) __attribute__((always_inline)) {
-    dma_k(t + PIPE_LEAD, wave_dst + ((t + PIPE_LEAD) & PIPE_MASK) * PIPE_TILE);
-    dma_v(t + PIPE_LEAD - 1, wave_dst + PIPE_V_OFF + ((t + PIPE_LEAD - 1) & PIPE_MASK) * PIPE_TILE);
+  // request i of the tile the pointers stand at, into the slot at dst (this wave's share of it)
+  auto dma_k = [&](int i, unsigned dst) __attribute__((always_inline)) {
+    lds_dma16_ptr<true>((const unsigned char*)kp[i], dst + i * (NWAVE * 1024));
   };
-  auto stage_end = [&]() {
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(2 * NCH * (PIPE_LEAD - 2)));
-    __syncthreads();
+  auto dma_v = [&](int i, unsigned dst) __attribute__((always_inline)) {
+    lds_dma16_ptr<true>((const unsigned char*)vp[i], dst + i * (NWAVE * 1024));
+  };
+  auto tile_k = [&](int t) __attribute__((always_inline)) {
+    k_ptrs(t);
+#pragma unroll
+    for (int i = 0; i < NCH; i++) dma_k(i, wave_dst + (unsigned)(t & MASK) * TILE);
+  };
+  auto tile_v = [&](int t) __attribute__((always_inline)) {
+    v_ptrs(t);
+#pragma unroll
+    for (int i = 0; i < NCH; i++) dma_v(i, wave_dst + V_OFF + (unsigned)(t & MASK) * TILE);
+  };
+  // The end of SYNC iterations: everything older than the requests of the newest LEAD - 1 - SYNC iterations has landed (a
+  // wave's requests complete in order), which the barrier publishes.  Fragment reads may be in flight over it.
+  auto stage_end = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * NCH * (LEAD - 1 - SYNC)));
+    asm volatile("" : : : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" : : : "memory");
   };
 
   // ---- prologue: flag, a zero V tile in the last slot (the lagged P.V of iteration 0 multiplies it by P = 0),
-  // tiles K0 | K1 V0 | K2 V1 in request order
+  // tiles K0 | K1 V0 | K2 V1 .. in request order
   if (tid == 0) *flag = 0;
   {
     const i32x4 z = {0, 0, 0, 0};
 #pragma unroll
-    for (int i = 0; i < PIPE_TILE / 4096; i++) *(i32x4*)(lds + PIPE_V_OFF + PIPE_MASK * PIPE_TILE + i * 4096 + tid * 16) = z;
+    for (int i = 0; i < TILE / (16 * NTHR); i++) *(i32x4*)(lds + V_OFF + MASK * TILE + i * (16 * NTHR) + tid * 16) = z;
   }
-  dma_k(0, wave_dst);
+  // the query rows, requested in front of the tiles: they arrive with the first
+  i32x4 qraw[2][KS];
 #pragma unroll
-  for (int j = 1; j < PIPE_LEAD; j++) {
-    dma_k(j, wave_dst + j * PIPE_TILE);
-    dma_v(j - 1, wave_dst + PIPE_V_OFF + (j - 1) * PIPE_TILE);
+  for (int qb = 0; qb < 2; qb++) {
+    const __bf16* rp = row_ptr(P.q, b, h, min(q0 + qb * 16 + l16, P.sq - 1));
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) qraw[qb][ks] = *(const i32x4*)(rp + ks * 32 + lg * 8);
   }
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(2 * NCH * (PIPE_LEAD - 1)));  // K0 has landed
+  __builtin_amdgcn_sched_barrier(0);
+  tile_k(0);
+#pragma unroll
+  for (int j = 1; j < LEAD; j++) {
+    tile_k(j);
+    tile_v(j - 1);
+  }
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(2 * NCH * (LEAD - 1)));  // K0 has landed
   __syncthreads();
 
   const int nb = NT - 1;  // pipelined iterations
   if (!active) {
     // no query rows: this wave's share of every tile and the same barriers, nothing else
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(2 * NCH * (PIPE_LEAD - 2)));
-    __syncthreads();
+    stage_end();
     for (int t = 0; t < nb; t++) {
-      stage_begin(t);
-      stage_end();
+      tile_k(t + LEAD);
+      tile_v(t + LEAD - 1);
+      if (SYNC == 1 || (t & 1)) stage_end();
     }
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
-    __syncthreads();  // the flag barrier
+    if (SYNC == 2) __syncthreads();  // the last tile is published
+    __syncthreads();                 // the flag barrier
     return *(volatile lds_int*)flag != 0;
   }
 
-  // ---- Q fragments, softmax scale folded in: lane holds q row (qb*32 + l32), d = 16*ks + 8*lh .. +7
+  // ---- Q fragments, softmax scale folded in: lane holds q row (qb*16 + l16), d = 32*ks + 8*lg .. +7
   bf16x8 qf[2][KS];
 #pragma unroll
-  for (int qb = 0; qb < 2; qb++) {
-    const int r = min(q0 + qb * 32 + l32, P.sq - 1);
-    const __bf16* rp = row_ptr(P.q, b, h, r);
+  for (int qb = 0; qb < 2; qb++)
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      const i32x4 raw = *(const i32x4*)(rp + ks * 16 + lh * 8);
       float f[8];
-      hdit::unpack8(raw, f);
+      hdit::unpack8(qraw[qb][ks], f);
 #pragma unroll
       for (int e = 0; e < 8; e++) f[e] *= P.scale_log2;
       qf[qb][ks] = __builtin_bit_cast(bf16x8, hdit::pack8(f));
     }
-  }
 
-  const int vt_row = 4 * (lane >> 5) + ((lane & 15) >> 2);
-  const int vt_off = vt_row * ROW + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
-  const int vt_swz = HD == 64 ? ((vt_row >> 1) & 1) : (vt_row & 3);
-  const int k_off = l32 * ROW;
-  const int k_swz = HD == 64 ? ((l32 >> 1) & 7) : (l32 & 15);
-  const bf16x2 ones2 = {(__bf16)1.0f, (__bf16)1.0f};
-  typedef __attribute__((ext_vector_type(8))) short s16x8;
-
-  auto k_frag = [&](const unsigned char* sk, int kb, int ks) -> bf16x8 {
-    return *(const bf16x8*)(sk + k_off + kb * 32 * ROW + (((ks * 2 + lh) ^ k_swz) << 4));
-  };
-  auto v_frag = [&](const unsigned char* sv, int u, int db) -> bf16x8 {
-    const unsigned char* va = sv + vt_off + (u * 16) * ROW + ((db ^ vt_swz) << 6);
-    s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(va));
-    s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(va + 8 * ROW));
-    return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-  };
-
-  f32x16 oacc[DB][2];
-#pragma unroll
-  for (int i = 0; i < DB; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) oacc[i][j][v] = 0.f;
-  float l_run[2] = {0.f, 0.f};
-  f32x16 negm[2];
-  // scores of the tile in work, [key block][query block]; a key block's registers take the next tile's scores as
-  // soon as its probabilities are packed
-  f32x16 s0[2], s1[2];
-
-  auto score_steps = [&](f32x16 (&sn)[2], const unsigned char* sk, int kb, int ks0, int ks1) __attribute__((always_inline)) {
-#pragma unroll
-    for (int ks = ks0; ks < ks1; ks++) {
-      const bf16x8 kf = k_frag(sk, kb, ks);
-#pragma unroll
-      for (int qb = 0; qb < 2; qb++)
-        sn[qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[qb][ks], ks == 0 ? negm[qb] : sn[qb], 0, 0, 0);
-    }
-  };
-
-  // ---- the first 32 keys set the reference: raw scores, column maxima plus the margin, then the scores again
-  // on top of -m
-  {
-#pragma unroll
-    for (int qb = 0; qb < 2; qb++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) negm[qb][v] = 0.f;
-    score_steps(s0, lds, 0, 0, KS);
-#pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
-      float mx = s0[qb][0];
-#pragma unroll
-      for (int v = 1; v < 16; v++) mx = fmaxf(mx, s0[qb][v]);
-      auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(mx), __float_as_int(mx), false, false);
-      const float m = fmaxf(__int_as_float(sw[0]), __int_as_float(sw[1])) + PIPE_MARGIN;
-#pragma unroll
-      for (int v = 0; v < 16; v++) negm[qb][v] = -m;
-    }
-    score_steps(s0, lds, 0, 0, KS);
-  }
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(2 * NCH * (PIPE_LEAD - 2)));  // K1 and V0 have landed
-  __syncthreads();
-
-  // probabilities of a tile: pf[qb][u] holds the 16 keys of P.V k-step u; step 3 is multiplied one iteration late
-  bf16x8 pf[2][4];
-  bf16x8 vf3[DB];  // the V^T fragments of that late step, read before its tile's slot is given away
-  bf16x8 k1c[2];   // the first two K fragments of a tile's keys 32-63, read at the end of the iteration before
-#pragma unroll
-  for (int qb = 0; qb < 2; qb++) pf[qb][3] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-  for (int db = 0; db < DB; db++) vf3[db] = v_frag(lds + PIPE_V_OFF + PIPE_MASK * PIPE_TILE, 3, db);
-#pragma unroll
-  for (int ks = 0; ks < 2; ks++) k1c[ks] = k_frag(lds, 1, ks);
-
-  // exponentials, packs and row sums of the 16 keys of step u: accumulator entries 8*(u%2) .. of key block u/2
-  auto chunk = [&](const f32x16 (&sc)[2], int u) __attribute__((always_inline)) {
-    const int hh = u & 1;
-#pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
-      i32x4 pk;
-      float rs = l_run[qb];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const float p0 = __builtin_amdgcn_exp2f(sc[qb][hh * 8 + 2 * e]);
-        const float p1 = __builtin_amdgcn_exp2f(sc[qb][hh * 8 + 2 * e + 1]);
-        const uint32_t pp = hdit::pack2(p0, p1);
-        pk[e] = (int)pp;
-        rs = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pp), ones2, rs, false);
-      }
-      pf[qb][u] = __builtin_bit_cast(bf16x8, pk);
-      l_run[qb] = rs;
-    }
-  };
-  auto pv_step = [&](const bf16x8 (&vf)[DB], int u) __attribute__((always_inline)) {
-#pragma unroll
-    for (int db = 0; db < DB; db++)
-#pragma unroll
-      for (int qb = 0; qb < 2; qb++) oacc[db][qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[db], pf[qb][u], oacc[db][qb], 0, 0, 0);
-  };
-  auto pv_from = [&](const unsigned char* sv, int u) __attribute__((always_inline)) {
-    bf16x8 vf[DB];
-#pragma unroll
-    for (int db = 0; db < DB; db++) vf[db] = v_frag(sv, u, db);
-    pv_step(vf, u);
-  };
-  auto mask_block = [&](f32x16 (&sc)[2], int kb, int valid) __attribute__((always_inline)) {
-#pragma unroll
-    for (int v = 0; v < 16; v++) {
-      const int key = kb * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-      if (key >= valid) {
-        sc[0][v] = -INFINITY;
-        sc[1][v] = -INFINITY;
-      }
-    }
-  };
-
-  // one pipelined iteration (tile t): s0 holds the scores of its keys 0-31 on entry and those of tile t+1 on exit
-  auto score_mfma = [&](f32x16 (&sn)[2], const bf16x8& kf, int ks) __attribute__((always_inline)) {
-#pragma unroll
-    for (int qb = 0; qb < 2; qb++)
-      sn[qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[qb][ks], ks == 0 ? negm[qb] : sn[qb], 0, 0, 0);
-  };
-  // Lane parts of the fragment addresses (32-bit LDS addresses); an iteration adds the ring slot of its tile, the
-  // rest is an immediate offset of the LDS instruction.
+  // ---- fragments: the lane part of the LDS addresses, the slot of the tile (a scalar), an immediate
   typedef __attribute__((address_space(3))) unsigned char lds_byte;
-  unsigned kaddr[KS], vaddr[DB];  // 32-bit LDS addresses
+  typedef __attribute__((ext_vector_type(8))) short s16x8;
+  const int k_swz = HD == 64 ? ((l16 >> 1) & 7) : l16;
+  const int vt_row = 4 * lg + (l16 >> 2);  // transpose read: key row of this lane's 8 bytes, columns 4*(l16&3)
+  const int vt_swz = HD == 64 ? ((vt_row >> 1) & 3) : (vt_row & 7);
+  unsigned kaddr[KS], vaddr[DB];
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) kaddr[ks] = lds_address(lds) + k_off + (((ks * 2 + lh) ^ k_swz) << 4);
+  for (int ks = 0; ks < KS; ks++) kaddr[ks] = lds_address(lds) + l16 * ROW + (((ks * 4 + lg) ^ k_swz) << 4);
 #pragma unroll
-  for (int db = 0; db < DB; db++) vaddr[db] = lds_address(lds) + PIPE_V_OFF + vt_off + ((db ^ vt_swz) << 6);
-  // slot_off: byte offset of the ring slot (a scalar); the rest of the address is an immediate
-  auto k_frag_s = [&](unsigned slot_off, int kb, int ks) __attribute__((always_inline)) -> bf16x8 {
-    return *(const __attribute__((address_space(3))) bf16x8*)((lds_byte*)(uintptr_t)(kaddr[ks] + slot_off) + kb * 32 * ROW);
+  for (int db = 0; db < DB; db++) vaddr[db] = lds_address(lds) + V_OFF + vt_row * ROW + ((db ^ vt_swz) << 5) + (l16 & 3) * 8;
+  // keys 16*kb .. +15 of a tile, d = 32*ks .. +31
+  auto k_frag = [&](unsigned slot_off, int kb, int ks) __attribute__((always_inline)) -> bf16x8 {
+    return *(const __attribute__((address_space(3))) bf16x8*)((lds_byte*)(uintptr_t)(kaddr[ks] + slot_off) + kb * 16 * ROW);
   };
-  auto v_frag_s = [&](unsigned slot_off, int u, int db) __attribute__((always_inline)) -> bf16x8 {
-    lds_byte* va = (lds_byte*)(uintptr_t)(vaddr[db] + slot_off) + (u * 16) * ROW;
+  // d = 16*db .. +15 of keys 32*half .. +31, in the order of the score accumulators: k-slot 8*lg + j is key 4*lg + j of the
+  // first 16 keys (j < 4) or of the second
+  auto v_frag = [&](unsigned slot_off, int half, int db) __attribute__((always_inline)) -> bf16x8 {
+    lds_byte* va = (lds_byte*)(uintptr_t)(vaddr[db] + slot_off) + half * 32 * ROW;
     s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(va));
-    s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(va + 8 * ROW));
+    s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(va + 16 * ROW));
     return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  for (int t = 0; t < nb; t++) {
-    const unsigned S = (unsigned)(t & PIPE_MASK) * PIPE_TILE, SN = (unsigned)((t + 1) & PIPE_MASK) * PIPE_TILE;  // ring slots of tiles t, t+1
-    dma_k(t + PIPE_LEAD, wave_dst + (unsigned)((t + PIPE_LEAD) & PIPE_MASK) * PIPE_TILE);
-    dma_v(t + PIPE_LEAD - 1, wave_dst + PIPE_V_OFF + (unsigned)((t + PIPE_LEAD - 1) & PIPE_MASK) * PIPE_TILE);
-    __builtin_amdgcn_sched_barrier(0);
-    // fragment reads in the order the MFMAs consume them
-    bf16x8 k1[KS], k0n[KS], vf[3][DB];
-    k1[0] = k1c[0];
-    k1[1] = k1c[1];
+
+  f32x4 oacc[DB][2], negm[2], lsum[2];
+  // scores of the two halves of a tile, [16 keys][query block]; a half's registers take the next tile's scores as
+  // soon as its probabilities are packed
+  f32x4 s0[2][2], s1[2][2];
+  i32x4 pk[2][2];  // probabilities [half][query block], the P^T operand: [2*kb], [2*kb + 1] hold the lane's keys of block kb
 #pragma unroll
-    for (int ks = 2; ks < KS; ks++) k1[ks] = k_frag_s(S, 1, ks);
+  for (int qb = 0; qb < 2; qb++) {
 #pragma unroll
-    for (int db = 0; db < DB; db++) vf[0][db] = v_frag_s(S, 0, db);
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) k0n[ks] = k_frag_s(SN, 0, ks);
-#pragma unroll
-    for (int u = 1; u < 3; u++)
-#pragma unroll
-      for (int db = 0; db < DB; db++) vf[u][db] = v_frag_s(S, u, db);
-    // MFMAs 0-3: the late P.V step of the previous tile; 4-11: scores of keys 32-63
-    pv_step(vf3, 3);
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) score_mfma(s1, k1[ks], ks);
-    chunk(s0, 0);
-    // 12-15: P.V step 0
-    pv_step(vf[0], 0);
-    chunk(s0, 1);
-    // 16-23: scores of the next tile's keys 0-31
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) score_mfma(s0, k0n[ks], ks);
-    chunk(s1, 2);
-    // 24-31: P.V steps 1 and 2
-    pv_step(vf[1], 1);
-    pv_step(vf[2], 2);
-    chunk(s1, 3);
-    // for the next iteration
-#pragma unroll
-    for (int db = 0; db < DB; db++) vf3[db] = v_frag_s(S, 3, db);
-#pragma unroll
-    for (int ks = 0; ks < 2; ks++) k1c[ks] = k_frag_s(SN, 1, ks);
-    // The order above, pinned: every MFMA is followed by a fragment read and its share of the softmax
-    // instructions, so that a fragment is requested a few MFMAs before its use and not much earlier.
-#pragma unroll
-    for (int i = 0; i < NMFMA; i++) {
-      SGB(0x008, 1);
-      if ((i & 3) != 3) SGB(0x100, 1);  // three fragment reads per four MFMAs: the rate they are consumed at
-      SGB(0x402, VALU_PER_MFMA);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    stage_end();
+    for (int db = 0; db < DB; db++) oacc[db][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    negm[qb] = lsum[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    pk[0][qb] = pk[1][qb] = i32x4{0, 0, 0, 0};
   }
+  auto score = [&](f32x4 (&sn)[2][2], const bf16x8& kf, int kb, int ks, int qb) __attribute__((always_inline)) {
+    sn[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[qb][ks], ks == 0 ? negm[qb] : sn[kb][qb], 0, 0, 0);
+  };
+  auto pv = [&](const bf16x8& vf, int half, int db, int qb) __attribute__((always_inline)) {
+    oacc[db][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8, pk[half][qb]), oacc[db][qb], 0, 0, 0);
+  };
+  // pair n: half n / 8, 16 keys (n % 8) / 4, query block (n % 4) / 2, accumulator entries 2 * (n % 2) and the next
+  float pe[2];
+  auto pair_exp = [&](int n, int e) __attribute__((always_inline)) {
+    pe[e] = __builtin_amdgcn_exp2f((n < 8 ? s0 : s1)[(n % 8) / 4][(n % 4) / 2][2 * (n % 2) + e]);
+  };
+  auto pair_pack = [&](int n) __attribute__((always_inline)) {
+    pk[n / 8][(n % 4) / 2][2 * ((n % 8) / 4) + n % 2] = (int)hdit::pack2(pe[0], pe[1]);
+  };
+  // row sums of exactly the bf16 values that enter the P.V product: a lane's own four of pairs n - 1 and n (n odd)
+  auto pair_sum = [&](int n) __attribute__((always_inline)) {
+    const s16x4 ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80};
+    const int qb = (n % 4) / 2, e = 2 * ((n % 8) / 4);
+    const i32x2 p4 = {pk[n / 8][qb][e], pk[n / 8][qb][e + 1]};
+    lsum[qb] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(s16x4, p4), lsum[qb], 0, 0, 0);
+  };
+  auto all_scores = [&](f32x4 (&sn)[2][2], unsigned slot_off, int half) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        const bf16x8 kf = k_frag(slot_off, 2 * half + kb, ks);
+#pragma unroll
+        for (int qb = 0; qb < 2; qb++) score(sn, kf, kb, ks, qb);
+      }
+  };
+  auto all_pv = [&](unsigned slot_off, int half) __attribute__((always_inline)) {
+#pragma unroll
+    for (int db = 0; db < DB; db++) {
+      const bf16x8 vf = v_frag(slot_off, half, db);
+#pragma unroll
+      for (int qb = 0; qb < 2; qb++) pv(vf, half, db, qb);
+    }
+  };
+
+  // ---- the first tile sets the reference: raw scores, column maxima plus the margin, then the scores of its first 32 keys
+  // again on top of -m
+  {
+    all_scores(s0, 0, 0);
+    all_scores(s1, 0, 1);
+#pragma unroll
+    for (int qb = 0; qb < 2; qb++) {
+      float mx = s0[0][qb][0];
+#pragma unroll
+      for (int e = 0; e < 4; e++) mx = fmaxf(fmaxf(fmaxf(fmaxf(mx, s0[0][qb][e]), s0[1][qb][e]), s1[0][qb][e]), s1[1][qb][e]);
+      auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_int(mx), __float_as_int(mx), false, false);
+      mx = fmaxf(__int_as_float(s16[0]), __int_as_float(s16[1]));
+      auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_int(mx), __float_as_int(mx), false, false);
+      mx = fmaxf(__int_as_float(s32[0]), __int_as_float(s32[1]));
+      const float m = mx + PIPE_MARGIN;
+      negm[qb] = f32x4{-m, -m, -m, -m};
+    }
+    all_scores(s0, 0, 0);
+  }
+  stage_end();
+
+  // fragment f of iteration t, in the order of use
+  auto read_frag = [&](int f, unsigned vprev, unsigned cur, unsigned next) __attribute__((always_inline)) -> bf16x8 {
+    if (f < DB) return v_frag(vprev, 1, f);
+    f -= DB;
+    if (f < 2 * KS) return k_frag(cur, 2 + f / KS, f % KS);
+    f -= 2 * KS;
+    if (f < DB) return v_frag(cur, 0, f);
+    f -= DB;
+    return k_frag(next, f / KS, f % KS);
+  };
+  bf16x8 ahead[FRAG_LEAD];  // the first fragments of the next iteration
+#pragma unroll
+  for (int f = 0; f < FRAG_LEAD; f++) ahead[f] = v_frag(MASK * TILE, 1, f);
+  k_ptrs(LEAD);
+  v_ptrs(LEAD - 1);
+  // One iteration; the slots of its tiles are constants (the loop is unrolled over the ring), so that a fragment's address
+  // is a register and an immediate.
+  auto iteration = [&](auto Slot, int t) __attribute__((always_inline)) {
+    constexpr int slot = decltype(Slot)::value;
+    constexpr unsigned prev = ((slot + MASK) & MASK) * TILE, cur = slot * TILE, next = ((slot + 1) & MASK) * TILE;
+    const unsigned kdst = wave_dst + ((slot + LEAD) & MASK) * TILE, vdst = wave_dst + V_OFF + ((slot + LEAD - 1) & MASK) * TILE;
+    // whether the tiles requested next follow these inside one segment
+    const bool next0 = t + LEAD + 1 < full0, next1 = t + LEAD - 1 >= first1 && t + LEAD + 1 < full_all;
+    const unsigned kstep = (next0 ? krow0 : krow1) * BKV, vstep = (next0 ? vrow0 : vrow1) * BKV;
+    __builtin_amdgcn_sched_barrier(0);
+    bf16x8 fr[F];
+#pragma unroll
+    for (int f = 0; f < FRAG_LEAD; f++) fr[f] = ahead[f];
+    static_for<2 * F>([&](auto I) __attribute__((always_inline)) {
+      constexpr int i = decltype(I)::value;
+      constexpr int f = i / 2, qb = (i ^ f) & 1;  // the query block changes with every second MFMA
+      if constexpr (f < DB) pv(fr[f], 1, f, qb);
+      else if constexpr (f < DB + 2 * KS) score(s1, fr[f], (f - DB) / KS, (f - DB) % KS, qb);
+      else if constexpr (f < 2 * DB + 2 * KS) pv(fr[f], 0, f - DB - 2 * KS, qb);
+      else score(s0, fr[f], (f - 2 * DB - 2 * KS) / KS, (f - 2 * DB - 2 * KS) % KS, qb);
+      if constexpr (i % 2 == 0) {
+        if constexpr (f + FRAG_LEAD < F) fr[f + FRAG_LEAD] = read_frag(f + FRAG_LEAD, prev, cur, next);
+        else ahead[f + FRAG_LEAD - F] = v_frag(cur, 1, f + FRAG_LEAD - F);
+      }
+      // softmax: a pair's exponentials in the first and the middle one of its PER slots, its pack in the next (the last of
+      // a half at once: P.V begins)
+      constexpr int n = i / PER;
+      if constexpr (i % PER == 0 && n > 0 && n != 8) pair_pack(n - 1);
+      if constexpr (i % PER == 0) pair_exp(n, 0);
+      if constexpr (i % PER == PER / 2) pair_exp(n, 1);
+      if constexpr (i % PER == PER - 1 && (n == 7 || n == 15)) pair_pack(n);
+      // tile requests
+      constexpr int RSTEP = F / NCH;
+      if constexpr (i % RSTEP == RSTEP / 2) {
+        constexpr int r = i / RSTEP;
+        if constexpr (r < NCH) {
+          dma_k(r, kdst);
+          kp[r] += kstep;
+        } else {
+          dma_v(r - NCH, vdst);
+          vp[r - NCH] += vstep;
+        }
+      }
+      // the row sums last: they wait for the matrix pipe
+      if constexpr (i % PER == 0 && n >= 2 && n % 2 == 0) pair_sum(n - 1);
+      if constexpr (i == 2 * F - 1) pair_sum(15);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if constexpr (SYNC == 1 || slot % 2 == 1) stage_end();
+    if (!(next0 || next1)) {
+      k_ptrs(t + LEAD + 1);
+      v_ptrs(t + LEAD);
+    }
+  };
+  for (int t = 0; t < nb;) {
+    bool more = true;
+    static_for<PL::RING>([&](auto Slot) __attribute__((always_inline)) {
+      if (more) {
+        iteration(Slot, t);
+        more = ++t < nb;
+      }
+    });
+  }
+  if (SYNC == 2) {
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
+    __syncthreads();
+  }
+
   // ---- the last tile: nothing to run ahead for
   {
     const int t = NT - 1;
+    const unsigned prev = (unsigned)((t + MASK) & MASK) * TILE, cur = (unsigned)(t & MASK) * TILE;
     const int valid = P.skv - t * BKV;
-    const unsigned char* sk = lds + (t & PIPE_MASK) * PIPE_TILE;
-    const unsigned char* sv = lds + PIPE_V_OFF + (t & PIPE_MASK) * PIPE_TILE;
-    pv_step(vf3, 3);
-    score_mfma(s1, k1c[0], 0);
-    score_mfma(s1, k1c[1], 1);
-    score_steps(s1, sk, 1, 2, KS);
+    all_pv(prev, 1);
+    all_scores(s1, cur, 1);
     if (valid < BKV) {
-      mask_block(s0, 0, valid);
-      mask_block(s1, 1, valid);
+#pragma unroll
+      for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int key = kb * 16 + 4 * lg + e;
+#pragma unroll
+          for (int qb = 0; qb < 2; qb++) {
+            if (key >= valid) s0[kb][qb][e] = -INFINITY;
+            if (key + 32 >= valid) s1[kb][qb][e] = -INFINITY;
+          }
+        }
     }
-    chunk(s0, 0);
-    pv_from(sv, 0);
-    chunk(s0, 1);
-    pv_from(sv, 1);
-    chunk(s1, 2);
-    pv_from(sv, 2);
-    chunk(s1, 3);
-    pv_from(sv, 3);
+#pragma unroll
+    for (int n = 0; n < 16; n++) {
+      pair_exp(n, 0);
+      pair_exp(n, 1);
+      pair_pack(n);
+      if (n % 2) pair_sum(n);
+    }
+    all_pv(cur, 0);
+    all_pv(cur, 1);
   }
 
-  // ---- did the fixed reference hold?
-  {
-    const bool bad = !(l_run[0] < PIPE_LIMIT) || !(l_run[1] < PIPE_LIMIT);
-    if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *flag = 1;
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
-    __syncthreads();
-    if (*(volatile lds_int*)flag) return true;
-  }
-
-  // ---- normalise and write O[q][d]: lane owns q = qb*32 + l32, d = 32*db + 8*(v/4) + 4*lh + v%4
+  // ---- the row sums: four lanes hold the parts of a row's
+  float total[2];
+  bool held[2];  // compared as bits: above the limit, infinite or not a number
 #pragma unroll
   for (int qb = 0; qb < 2; qb++) {
-    auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(l_run[qb]), __float_as_int(l_run[qb]), false, false);
-    const float inv = 1.0f / (__int_as_float(sw[0]) + __int_as_float(sw[1]));
-    const int r = q0 + qb * 32 + l32;
-    if (r >= P.sq) continue;
+    auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_int(lsum[qb][0]), __float_as_int(lsum[qb][0]), false, false);
+    total[qb] = __int_as_float(s16[0]) + __int_as_float(s16[1]);
+    auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_int(total[qb]), __float_as_int(total[qb]), false, false);
+    total[qb] = __int_as_float(s32[0]) + __int_as_float(s32[1]);
+    held[qb] = __float_as_uint(total[qb]) < __float_as_uint(PIPE_LIMIT);
+    rows |= (unsigned)(__builtin_amdgcn_ballot_w64(!held[qb]) & 0xffffull) << (16 * qb);
+  }
+  if (rows != 0 && lane == 0) *flag = 1;
+
+  // ---- normalise and write O[q][d]: lane owns q = qb*16 + l16, d = 16*db + 4*lg + e
+#pragma unroll
+  for (int qb = 0; qb < 2; qb++) {
+    const float inv = 1.0f / total[qb];
+    const int r = q0 + qb * 16 + l16;
+    if (r >= P.sq || !held[qb]) continue;
     __bf16* op = (__bf16*)row_ptr(P.o, b, h, r);
 #pragma unroll
-    for (int db = 0; db < DB; db++)
-#pragma unroll
-      for (int g = 0; g < 4; g++) {
-        i32x2 out;
-        out[0] = (int)hdit::pack2(oacc[db][qb][g * 4 + 0] * inv, oacc[db][qb][g * 4 + 1] * inv);
-        out[1] = (int)hdit::pack2(oacc[db][qb][g * 4 + 2] * inv, oacc[db][qb][g * 4 + 3] * inv);
-        *(i32x2*)(op + db * 32 + g * 8 + lh * 4) = out;
-      }
+    for (int db = 0; db < DB; db++) {
+      i32x2 out;
+      out[0] = (int)hdit::pack2(oacc[db][qb][0] * inv, oacc[db][qb][1] * inv);
+      out[1] = (int)hdit::pack2(oacc[db][qb][2] * inv, oacc[db][qb][3] * inv);
+      *(i32x2*)(op + db * 16 + lg * 4) = out;
+    }
   }
-  return false;
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));  // nothing may land in LDS after this
+  __syncthreads();
+  return *(volatile lds_int*)flag != 0;
 }
 
 // The second pass.  It takes its arguments from the kernel's parameter block again, through an address the compiler
@@ -1035,7 +1061,7 @@ __device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles,
 // 55.3 -> 52.2; d = 64, 1357 x 1357 28.9 -> 27.9, 333 x 333 13.4 -> 12.8.  Without any second pass the same d = 128
 // times, 26.5 and 12.6.
 template <int HD>
-__device__ __forceinline__ void attn_second_pass(size_t params_at, int q_tiles, unsigned char* lds, int block_id, int nblocks) {
+__device__ __forceinline__ void attn_second_pass(size_t params_at, int q_tiles, unsigned char* lds, int block_id, int nblocks, unsigned rows) {
   typedef const __attribute__((address_space(4))) int64_t* const_ptr;
   uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr() + params_at;
   asm volatile("" : "+s"(at), "+s"(q_tiles), "+s"(block_id), "+s"(nblocks));
@@ -1047,26 +1073,28 @@ __device__ __forceinline__ void attn_second_pass(size_t params_at, int q_tiles, 
   for (unsigned i = 0; i < sizeof(AttnParams) / 8; i++) raw.v[i] = ((const_ptr)at)[i];
   const AttnParams P = __builtin_bit_cast(AttnParams, raw);
   __syncthreads();  // every wave has read the flag, whose bytes this pass may overwrite
-  attn_tracked_body<HD>(P, q_tiles, lds, block_id, nblocks);
+  attn_tracked_body<HD>(P, q_tiles, lds, block_id, nblocks, rows);
 }
 
 template <int HD>
-__global__ void __launch_bounds__(256, 1) attn_fwd_pipe_kernel(const AttnParams P, int q_tiles) {
+__global__ void __launch_bounds__(NTHR, 2) attn_fwd_pipe_kernel(const AttnParams P, int q_tiles) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  if (attn_pipe_body<HD>(P, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x))
-    attn_second_pass<HD>(0, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x);
+  unsigned rows;
+  if (attn_pipe_body<HD>(P, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x, rows))
+    attn_second_pass<HD>(0, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x, rows);
 }
 
 template <int HD>
-__global__ void __launch_bounds__(256, 1) attn_fwd_pipe_multi_kernel(const AttnMulti M) {
+__global__ void __launch_bounds__(NTHR, 2) attn_fwd_pipe_multi_kernel(const AttnMulti M) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   int i = 0;
 #pragma unroll 1
   while (i + 1 < M.count && (int)blockIdx.x >= M.start[i + 1]) i++;
   const int local = (int)blockIdx.x - M.start[i];
   if (local >= M.nblocks[i]) return;
-  if (attn_pipe_body<HD>(M.p[i], M.q_tiles[i], lds, local, M.nblocks[i]))
-    attn_second_pass<HD>(offsetof(AttnMulti, p) + i * sizeof(AttnParams), M.q_tiles[i], lds, local, M.nblocks[i]);
+  unsigned rows;
+  if (attn_pipe_body<HD>(M.p[i], M.q_tiles[i], lds, local, M.nblocks[i], rows))
+    attn_second_pass<HD>(offsetof(AttnMulti, p) + i * sizeof(AttnParams), M.q_tiles[i], lds, local, M.nblocks[i], rows);
 }
 
 // Host side of a multi launch: the table of `count` problems, ranges padded to multiples of 8 workgroups.
@@ -1086,4 +1114,30 @@ inline int fill_multi(AttnMulti& M, const AttnParams* P, const int* q_tiles, con
   return at;
 }
 
+// One grid of `count` problems: a kernel that takes one, or one that takes a table.
+template <class One, class Multi>
+int launch_grid(One one, Multi multi, int lds_bytes, std::atomic<bool>& attr_set, const AttnParams* P, const int* q_tiles,
+                const int* nblocks, int count, hipStream_t stream) {
+  if (lds_bytes > 64 * 1024 && !attr_set.load(std::memory_order_acquire)) {  // setting them twice from two threads is harmless
+    if (hipFuncSetAttribute((const void*)one, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess ||
+        hipFuncSetAttribute((const void*)multi, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
+      return HDIT_ELAUNCH;
+    attr_set.store(true, std::memory_order_release);
+  }
+  if (count == 1) {
+    hipLaunchKernelGGL(one, dim3((unsigned)nblocks[0]), dim3(NTHR), lds_bytes, stream, P[0], q_tiles[0]);
+    return HDIT_OK;
+  }
+  AttnMulti M;
+  const int grid = fill_multi(M, P, q_tiles, nblocks, count);
+  hipLaunchKernelGGL(multi, dim3((unsigned)grid), dim3(NTHR), lds_bytes, stream, M);
+  return HDIT_OK;
+}
+
 }  // namespace
+
+#define HDIT_ATTN_LAUNCH(name, HD, kernel, multi_kernel, lds)                                                              \
+  int name(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream) {                   \
+    static std::atomic<bool> attr_set{false};                                                                              \
+    return launch_grid(kernel<HD>, multi_kernel<HD>, lds<HD>::TOTAL, attr_set, P, q_tiles, nblocks, count, stream);        \
+  }

@@ -424,6 +424,34 @@ def test_attention_image_rows_do_not_depend_on_the_text_queries(hdit, B, ni, nk,
     assert_parity(both[:1, :200], want, what="attention")
 
 
+@pytest.mark.parametrize("hd,B,H,sq,skv", [
+    (64, 1, 2, 200, 192), (64, 1, 3, 129, 193),      # three tiles and one key more, workgroups of 128 rows
+    (64, 1, 80, 256, 513), (64, 1, 86, 640, 640),    # workgroups of 256 rows: one round, and the tail of a second
+    (128, 1, 2, 257, 193), (128, 2, 3, 300, 576),
+])
+def test_attention_rows_do_not_depend_on_rows_that_outgrow(hdit, hd, B, H, sq, skv):
+    """The pipelined kernels leave a row whose sum outgrows the reference fixed after the first tile to the tracked body.
+    That row gets the oracle's numbers and every other row of its wave and workgroup keeps its bits, at every position of
+    the key ring the loop can end on (64 .. 256 keys cut off the end)."""
+    print(f"attention outgrowing rows d={hd} B={B} H={H} {sq}x{skv}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(91)
+    q, k, v = (torch.randn(B, n, H, hd, generator=gen, device=DEV).to(torch.bfloat16) for n in (sq, skv, skv))
+    rows = [0, sq // 2, sq - 1]
+    grown = q.clone()
+    grown[:, rows] = (k[:, -1:] * 12.0).to(torch.bfloat16)  # along the last key: its logit is 12 |k|^2 / sqrt(d)
+    rest = torch.ones(sq, dtype=torch.bool, device=DEV)
+    rest[rows] = False
+    for cut in range(0, min(skv - 129, 449), 64):  # the last key stays: the keys in front of it go
+        kc, vc = (torch.cat([t[:, :skv - 1 - cut], t[:, skv - 1:]], 1).contiguous() for t in (k, v))
+        plain, = hdit.ops.attention([q], [kc], [vc])
+        got, = hdit.ops.attention([grown], [kc], [vc])
+        torch.cuda.synchronize()
+        assert torch.equal(got[:, rest], plain[:, rest]), f"{skv - cut} keys: rows beside the outgrowing ones changed"
+        heads = slice(0, 2)
+        want = O.attention(*(t[:, :, heads].float().cpu().transpose(1, 2) for t in (grown, kc, vc))).transpose(1, 2)
+        assert_parity(got[:, :, heads], want, what=f"attention, outgrowing rows, {skv - cut} keys")
+
+
 # (batch, heads, query rows, key rows, key rows in the second buffer, gap between heads, outgrowing query rows)
 @pytest.mark.parametrize("hd,problems", [
     (128, [(1, 3, 300, 200, 0, 0, ()), (2, 2, 64, 333, 133, 0, (0, 63)), (1, 5, 513, 1000, 77, 64, (512,)), (2, 1, 1, 129, 64, 8, (0,))]),
