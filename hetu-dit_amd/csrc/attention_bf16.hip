@@ -82,9 +82,43 @@ bool is_pipelined(const hdit_attn_args* a, const AttnParams& P) {
   return pipe_env() != '0' && strides_ok && (P.skv + BKV - 1) / BKV >= PIPE_MIN_TILES;
 }
 
+int64_t rows_of(const hdit_attn_args* a) { return a->q[0].len + a->q[1].len; }
+
 int64_t workgroups(const hdit_attn_args* a, int rows_per_workgroup) {
-  const int rows = a->q[0].len + a->q[1].len;
-  return (int64_t)a->batch * a->heads * ((rows + rows_per_workgroup - 1) / rows_per_workgroup);
+  return (int64_t)a->batch * a->heads * ((rows_of(a) + rows_per_workgroup - 1) / rows_per_workgroup);
+}
+
+// A launch of workgroups of eight waves, one per CU: `full` of them with 256 rows and, dealt out behind those, `half` with
+// 128, which take HALF_COST of the time.  Returns the rounds it takes.
+constexpr double HALF_COST = 0.62;
+double rounds(int64_t full, int64_t half, int64_t cus) {
+  const int64_t whole = full / cus, late = full % cus, early = cus - late;  // CUs that are free at `whole`, at `whole` + 1
+  if (half == 0) return (double)(whole + (late > 0));
+  for (int64_t n = 1;; n++) {  // n half tiles one after the other on the early CUs, and what fits beside them on the late ones
+    const double end = n * HALF_COST;
+    const int64_t on_late = end > 1.0 ? (int64_t)((end - 1.0) / HALF_COST + 1e-9) : 0;
+    if (early * n + late * on_late >= half) return (double)whole + (late && end < 1.0 ? 1.0 : end);
+  }
+}
+
+// How many 256-row tiles a (batch, head) of a problem has; the rows behind them go to half tiles.  A launch that ends with
+// a round of few workgroups is over sooner if those are twice as many of half the rows: as many whole tiles as fill whole
+// rounds, or all of them (a last one with more than 128 rows counts as whole), whichever ends first.  24 heads of 16896
+// rows at d = 128 are 1584 workgroups, six rounds and 48: 2845 -> 2725 us, 2854 -> 2789 in another run; 12000 rows (1128) 1439 ->
+// 1360; 512 rows (48) 20.9 -> 15.4.
+struct Tiling {
+  int full;
+  double rounds;
+};
+Tiling tiling(const hdit_attn_args* a, int64_t cus) {
+  const int64_t bh = (int64_t)a->batch * a->heads, rows = rows_of(a), most = rows / 256 + (rows % 256 > 128);
+  auto end = [&](int64_t f) { return rounds(bh * f, rows > 256 * f ? bh * ((rows - 256 * f + 127) / 128) : 0, cus); };
+  Tiling best = {(int)most, end(most)};
+  for (int64_t whole = bh * most / cus; whole >= 0 && whole + 2 > bh * most / cus; whole--) {
+    const int64_t f = whole * cus / bh;
+    if (end(f) < best.rounds - 0.05) best = {(int)f, end(f)};
+  }
+  return best;
 }
 
 // Query rows per workgroup of a pipelined launch at head dim 64, by how the workgroups fill the CUs.  Measured on MI355X,
@@ -105,23 +139,31 @@ int pipe_rows(const hdit_attn_args* const* of, int count) {
   }
   const int cus = hdit_host::num_cus();
   if (cus <= 0) return 256;  // no device to ask: the launch reports it
-  small = (small + cus - 1) / cus, large = (large + cus - 1) / cus;
+  small = (small + cus - 1) / cus;
   const double cost_small = tiles * (0.90 * (double)(small / 2) + 0.55 * (double)(small % 2));
-  return cost_small <= tiles * 0.86 * (double)large + 1.0 ? 128 : 256;
+  const double cost_large = tiles * 0.86 * (count == 1 ? tiling(of[0], cus).rounds : (double)((large + cus - 1) / cus)) + 1.0;
+  return cost_small <= 1.05 * cost_large ? 128 : 256;  // (2 x 4429 rows: modelled 228 / 219, measured 242 / 244)
 }
 
 // The problems of one call that one kernel serves, as one launch.
 int launch_some(const hdit_attn_args* const* of, const AttnParams* P, int count, bool pipelined, hipStream_t s) {
   const int hd = of[0]->head_dim;
   const int rows = pipelined && hd == 64 ? pipe_rows(of, count) : 256;
-  int q_tiles[HDIT_ATTN_MAX_MULTI], nblocks[HDIT_ATTN_MAX_MULTI];
+  const bool eight = pipelined && rows == 256;
+  int q_tiles[HDIT_ATTN_MAX_MULTI], q_full[HDIT_ATTN_MAX_MULTI], nblocks[HDIT_ATTN_MAX_MULTI];
   for (int i = 0; i < count; i++) {
-    q_tiles[i] = (P[i].sq + rows - 1) / rows;
-    nblocks[i] = (int)workgroups(of[i], rows);
+    const int part = eight ? rows / 2 : rows, cus = hdit_host::num_cus();
+    q_full[i] = eight && count == 1 && cus > 0 ? tiling(of[i], cus).full : P[i].sq / rows + (P[i].sq % rows > part);
+    const int left = P[i].sq - q_full[i] * rows;
+    q_tiles[i] = q_full[i] + (left > 0 ? (left + part - 1) / part : 0);
+    nblocks[i] = of[i]->batch * of[i]->heads * q_tiles[i];
   }
-  if (!pipelined) return hd == 64 ? hdit_attn::launch_tracked_d64(P, q_tiles, nblocks, count, s) : hdit_attn::launch_tracked_d128(P, q_tiles, nblocks, count, s);
-  if (hd == 128) return hdit_attn::launch_pipe8_d128(P, q_tiles, nblocks, count, s);
-  return rows == 128 ? hdit_attn::launch_pipe4_d64(P, q_tiles, nblocks, count, s) : hdit_attn::launch_pipe8_d64(P, q_tiles, nblocks, count, s);
+  if (!pipelined)
+    return hd == 64 ? hdit_attn::launch_tracked_d64(P, q_tiles, q_full, nblocks, count, s)
+                    : hdit_attn::launch_tracked_d128(P, q_tiles, q_full, nblocks, count, s);
+  if (hd == 128) return hdit_attn::launch_pipe8_d128(P, q_tiles, q_full, nblocks, count, s);
+  return rows == 128 ? hdit_attn::launch_pipe4_d64(P, q_tiles, q_full, nblocks, count, s)
+                     : hdit_attn::launch_pipe8_d64(P, q_tiles, q_full, nblocks, count, s);
 }
 }  // namespace
 

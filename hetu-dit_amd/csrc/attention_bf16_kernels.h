@@ -61,13 +61,13 @@ struct AttnParams {
 };
 
 // Launch of `count` problems of one head dim, on argument blocks the entry point has validated and converted, as one grid:
-// the tracked kernel (256 query rows per workgroup), the pipelined ones of 128 and 256 rows.  q_tiles and nblocks count
-// workgroups of those rows.
-int launch_tracked_d64(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
-int launch_tracked_d128(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
-int launch_pipe4_d64(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
-int launch_pipe8_d64(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
-int launch_pipe8_d128(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream);
+// the tracked kernel (256 query rows per workgroup), the pipelined ones of 128 and 256 rows.  A (batch, head) is q_tiles
+// workgroups, the first q_full of them with all their rows; nblocks is their number for the whole problem.
+int launch_tracked_d64(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
+int launch_tracked_d128(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
+int launch_pipe4_d64(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
+int launch_pipe8_d64(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
+int launch_pipe8_d128(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
 
 }  // namespace hdit_attn
 
@@ -166,12 +166,39 @@ constexpr int waitcnt_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0
 // accumulator rescale (the most expensive VALU block after the exponentials) is skipped for most tiles.
 constexpr float RESCALE_THRESHOLD = 8.0f;
 
+// Where a workgroup works.  A (batch, head) has q_full tiles of BQ query rows and q_tiles - q_full of HALF rows behind them:
+// in workgroups of eight waves a half tile leaves half of the waves without rows, so that what is over after the full
+// rounds of a launch is spread over twice as many CUs; elsewhere it is the partly filled last tile.
+// Workgroups go to the 8 XCDs round-robin by id, and each XCD has its own L2: all query tiles of one
+// (batch, head) run on one XCD, so that its K and V are fetched into one L2 instead of eight.  Within that,
+// the half tiles come after all full ones: workgroups are placed in id order, one per CU first, so when a launch has a few
+// more workgroups than CUs it is the light ones that share a CU with a full one.
+constexpr int HALF = NWAVE == 8 ? BQ / 2 : BQ;
+struct Place {
+  int b, h, q0, rows;
+};
+__device__ __forceinline__ Place place(const AttnParams& P, int q_tiles, int q_full, int block_id, int nblocks) {
+  const int nbh = nblocks / q_tiles;
+  const bool by_xcd = nbh % 8 == 0;
+  const int slot = by_xcd ? (block_id >> 3) : block_id;
+  const int full = (by_xcd ? nbh / 8 : nbh) * q_full;
+  const bool half = slot >= full;
+  const int of_bh = half ? q_tiles - q_full : q_full, s = half ? slot - full : slot;
+  const int qt = s % of_bh, bhl = s / of_bh;
+  const int bh = by_xcd ? bhl * 8 + (block_id & 7) : bhl;
+  Place at;
+  at.b = bh / P.heads, at.h = bh % P.heads;
+  at.q0 = half ? q_full * BQ + qt * HALF : qt * BQ;
+  at.rows = half ? HALF : BQ;
+  return at;
+}
+
 // The whole kernel for one workgroup: the online softmax with a running reference that follows the column
 // maxima.  Also the second pass of the pipelined kernels, for the rows whose fixed reference did not hold: bit l of
 // `rows` (one query block per wave) stands for the wave's row l, the others have been written.
 template <int HD>
-__device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_tiles, unsigned char* lds, int block_id,
-                                                  int nblocks, unsigned rows = ~0u) {
+__device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_tiles, int q_full, unsigned char* lds,
+                                                  int block_id, int nblocks, unsigned rows = ~0u) {
   using L = Lds<HD>;
   constexpr int KS = HD / 16;       // k-steps of the S^T MFMA (over head dim)
   constexpr int DB = HD / 32;       // 32-wide d blocks of O^T
@@ -184,31 +211,11 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, lh = lane >> 5;
-  // Workgroups go to the 8 XCDs round-robin by id, and each XCD has its own L2: all query tiles of one
-  // (batch, head) run on one XCD, so that its K and V are fetched into one L2 instead of eight.  Within that,
-  // the partly filled last query tiles (some of their waves have no rows and skip the arithmetic) come after
-  // all full ones: workgroups are placed in id order, one per CU first, so when a launch has a few more
-  // workgroups than CUs it is the light ones that share a CU with a full one.
-  const int nbh = nblocks / q_tiles;
-  const bool by_xcd = nbh % 8 == 0;
-  const int slot = by_xcd ? (block_id >> 3) : block_id;
-  const int nbh_loc = by_xcd ? nbh / 8 : nbh;
-  int qt = slot % q_tiles, bhl = slot / q_tiles;
-  if (q_tiles > 1 && P.sq % BQ != 0) {
-    const int heavy = nbh_loc * (q_tiles - 1);
-    if (slot < heavy) {
-      qt = slot % (q_tiles - 1);
-      bhl = slot / (q_tiles - 1);
-    } else {
-      qt = q_tiles - 1;
-      bhl = slot - heavy;
-    }
-  }
-  const int bh = by_xcd ? bhl * 8 + (block_id & 7) : bhl;
-  const int b = bh / P.heads, h = bh % P.heads;
-  const int q0 = qt * BQ + wave * WQ;
-  // a wave past the last query row still stages K/V tiles and meets the barriers, but does no arithmetic
-  const bool active = __builtin_amdgcn_readfirstlane(q0 < P.sq);
+  const Place at = place(P, q_tiles, q_full, block_id, nblocks);
+  const int b = at.b, h = at.h, q0 = at.q0 + wave * WQ;
+  // a wave past the last query row, or past the rows of a half tile, still stages K/V tiles and meets the barriers, but
+  // does no arithmetic
+  const bool active = __builtin_amdgcn_readfirstlane(q0 < P.sq && wave * WQ < at.rows);
 
   // ---- Q fragments: lane holds q row (qb*32 + l32), d = 16*ks + 8*lh .. +7
   bf16x8 qf[QB][L::Q_IN_LDS ? 1 : KS];
@@ -547,9 +554,9 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
 }
 
 template <int HD>
-__global__ void __launch_bounds__(NTHR, HD == 64 ? 2 : 1) attn_fwd_kernel(const AttnParams P, int q_tiles) {
+__global__ void __launch_bounds__(NTHR, HD == 64 ? 2 : 1) attn_fwd_kernel(const AttnParams P, int q_tiles, int q_full) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  attn_tracked_body<HD>(P, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x);
+  attn_tracked_body<HD>(P, q_tiles, q_full, lds, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // Several independent attention problems of one head dim in one grid (the blocks of neighbouring pipeline patches
@@ -558,7 +565,7 @@ __global__ void __launch_bounds__(NTHR, HD == 64 ? 2 : 1) attn_fwd_kernel(const 
 constexpr int ATTN_MAX_MULTI = HDIT_ATTN_MAX_MULTI;
 struct AttnMulti {
   AttnParams p[ATTN_MAX_MULTI];
-  int q_tiles[ATTN_MAX_MULTI];
+  int q_tiles[ATTN_MAX_MULTI], q_full[ATTN_MAX_MULTI];
   int nblocks[ATTN_MAX_MULTI];   // workgroups that have work (the range may be padded beyond them)
   int start[ATTN_MAX_MULTI + 1];
   int count;
@@ -572,7 +579,7 @@ __global__ void __launch_bounds__(NTHR, HD == 64 ? 2 : 1) attn_fwd_multi_kernel(
   while (i + 1 < M.count && (int)blockIdx.x >= M.start[i + 1]) i++;
   const int local = (int)blockIdx.x - M.start[i];
   if (local >= M.nblocks[i]) return;
-  attn_tracked_body<HD>(M.p[i], M.q_tiles[i], lds, local, M.nblocks[i]);
+  attn_tracked_body<HD>(M.p[i], M.q_tiles[i], M.q_full[i], lds, local, M.nblocks[i]);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -650,36 +657,19 @@ constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0f70; }
 
 // true: the fixed reference did not hold for some row of the workgroup; those of this wave are set in `rows`
 template <int HD>
-__device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles, unsigned char* lds, int block_id, int nblocks,
-                                               unsigned& rows) {
+__device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles, int q_full, unsigned char* lds, int block_id,
+                                               int nblocks, unsigned& rows) {
   using PL = PipeLds<HD>;
   constexpr int KS = HD / 32, DB = HD / 16, CPR = HD / 8, NCH = BKV * CPR / NTHR, RPI = 64 / CPR, ROW = PL::ROW;
   constexpr int TILE = PL::TILE, V_OFF = PL::V_OFF, LEAD = PL::LEAD, MASK = PL::MASK, SYNC = PL::SYNC;
   constexpr int F = 2 * DB + 4 * KS;  // fragments per iteration, two MFMAs each
   constexpr int PER = F / 8;          // MFMAs per pair of scores (16 pairs)
-  constexpr int ROWS = 32 * NWAVE;    // query rows per workgroup
+  static_assert(WQ == 32, "written for 32 query rows per wave");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, lg = lane >> 4;
-  // same placement of (batch, head, query tile) on workgroups as the kernel above
-  const int nbh = nblocks / q_tiles;
-  const bool by_xcd = nbh % 8 == 0;
-  const int slot = by_xcd ? (block_id >> 3) : block_id;
-  const int nbh_loc = by_xcd ? nbh / 8 : nbh;
-  int qt = slot % q_tiles, bhl = slot / q_tiles;
-  if (q_tiles > 1 && P.sq % ROWS != 0) {
-    const int heavy = nbh_loc * (q_tiles - 1);
-    if (slot < heavy) {
-      qt = slot % (q_tiles - 1);
-      bhl = slot / (q_tiles - 1);
-    } else {
-      qt = q_tiles - 1;
-      bhl = slot - heavy;
-    }
-  }
-  const int bh = by_xcd ? bhl * 8 + (block_id & 7) : bhl;
-  const int b = bh / P.heads, h = bh % P.heads;
-  const int q0 = qt * ROWS + wave * 32;
-  const bool active = __builtin_amdgcn_readfirstlane(q0 < P.sq);
+  const Place at = place(P, q_tiles, q_full, block_id, nblocks);
+  const int b = at.b, h = at.h, q0 = at.q0 + wave * 32;
+  const bool active = __builtin_amdgcn_readfirstlane(q0 < P.sq && wave * 32 < at.rows);
   const int NT = (P.skv + BKV - 1) / BKV;  // >= PIPE_MIN_TILES (host)
   rows = 0;
 
@@ -1061,10 +1051,11 @@ __device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles,
 // 55.3 -> 52.2; d = 64, 1357 x 1357 28.9 -> 27.9, 333 x 333 13.4 -> 12.8.  Without any second pass the same d = 128
 // times, 26.5 and 12.6.
 template <int HD>
-__device__ __forceinline__ void attn_second_pass(size_t params_at, int q_tiles, unsigned char* lds, int block_id, int nblocks, unsigned rows) {
+__device__ __forceinline__ void attn_second_pass(size_t params_at, int q_tiles, int q_full, unsigned char* lds, int block_id, int nblocks,
+                                                 unsigned rows) {
   typedef const __attribute__((address_space(4))) int64_t* const_ptr;
   uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr() + params_at;
-  asm volatile("" : "+s"(at), "+s"(q_tiles), "+s"(block_id), "+s"(nblocks));
+  asm volatile("" : "+s"(at), "+s"(q_tiles), "+s"(q_full), "+s"(block_id), "+s"(nblocks));
   static_assert(sizeof(AttnParams) % 8 == 0, "copied in 8-byte pieces");
   struct Raw {
     int64_t v[sizeof(AttnParams) / 8];
@@ -1073,15 +1064,15 @@ __device__ __forceinline__ void attn_second_pass(size_t params_at, int q_tiles, 
   for (unsigned i = 0; i < sizeof(AttnParams) / 8; i++) raw.v[i] = ((const_ptr)at)[i];
   const AttnParams P = __builtin_bit_cast(AttnParams, raw);
   __syncthreads();  // every wave has read the flag, whose bytes this pass may overwrite
-  attn_tracked_body<HD>(P, q_tiles, lds, block_id, nblocks, rows);
+  attn_tracked_body<HD>(P, q_tiles, q_full, lds, block_id, nblocks, rows);
 }
 
 template <int HD>
-__global__ void __launch_bounds__(NTHR, 2) attn_fwd_pipe_kernel(const AttnParams P, int q_tiles) {
+__global__ void __launch_bounds__(NTHR, 2) attn_fwd_pipe_kernel(const AttnParams P, int q_tiles, int q_full) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   unsigned rows;
-  if (attn_pipe_body<HD>(P, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x, rows))
-    attn_second_pass<HD>(0, q_tiles, lds, (int)blockIdx.x, (int)gridDim.x, rows);
+  if (attn_pipe_body<HD>(P, q_tiles, q_full, lds, (int)blockIdx.x, (int)gridDim.x, rows))
+    attn_second_pass<HD>(0, q_tiles, q_full, lds, (int)blockIdx.x, (int)gridDim.x, rows);
 }
 
 template <int HD>
@@ -1093,21 +1084,22 @@ __global__ void __launch_bounds__(NTHR, 2) attn_fwd_pipe_multi_kernel(const Attn
   const int local = (int)blockIdx.x - M.start[i];
   if (local >= M.nblocks[i]) return;
   unsigned rows;
-  if (attn_pipe_body<HD>(M.p[i], M.q_tiles[i], lds, local, M.nblocks[i], rows))
-    attn_second_pass<HD>(offsetof(AttnMulti, p) + i * sizeof(AttnParams), M.q_tiles[i], lds, local, M.nblocks[i], rows);
+  if (attn_pipe_body<HD>(M.p[i], M.q_tiles[i], M.q_full[i], lds, local, M.nblocks[i], rows))
+    attn_second_pass<HD>(offsetof(AttnMulti, p) + i * sizeof(AttnParams), M.q_tiles[i], M.q_full[i], lds, local, M.nblocks[i],
+                         rows);
 }
 
 // Host side of a multi launch: the table of `count` problems, ranges padded to multiples of 8 workgroups.
-inline int fill_multi(AttnMulti& M, const AttnParams* P, const int* q_tiles, const int* nblocks, int count) {
+inline int fill_multi(AttnMulti& M, const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count) {
   M.count = count;
   int at = 0;
   for (int i = 0; i < ATTN_MAX_MULTI; i++) {
     M.start[i] = at;
     if (i < count) {
-      M.p[i] = P[i], M.q_tiles[i] = q_tiles[i], M.nblocks[i] = nblocks[i];
+      M.p[i] = P[i], M.q_tiles[i] = q_tiles[i], M.q_full[i] = q_full[i], M.nblocks[i] = nblocks[i];
       at += (nblocks[i] + 7) / 8 * 8;
     } else {
-      M.p[i] = P[0], M.q_tiles[i] = 1, M.nblocks[i] = 0;
+      M.p[i] = P[0], M.q_tiles[i] = 1, M.q_full[i] = 1, M.nblocks[i] = 0;
     }
   }
   M.start[ATTN_MAX_MULTI] = at;
@@ -1117,7 +1109,7 @@ inline int fill_multi(AttnMulti& M, const AttnParams* P, const int* q_tiles, con
 // One grid of `count` problems: a kernel that takes one, or one that takes a table.
 template <class One, class Multi>
 int launch_grid(One one, Multi multi, int lds_bytes, std::atomic<bool>& attr_set, const AttnParams* P, const int* q_tiles,
-                const int* nblocks, int count, hipStream_t stream) {
+                const int* q_full, const int* nblocks, int count, hipStream_t stream) {
   if (lds_bytes > 64 * 1024 && !attr_set.load(std::memory_order_acquire)) {  // setting them twice from two threads is harmless
     if (hipFuncSetAttribute((const void*)one, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess ||
         hipFuncSetAttribute((const void*)multi, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
@@ -1125,11 +1117,11 @@ int launch_grid(One one, Multi multi, int lds_bytes, std::atomic<bool>& attr_set
     attr_set.store(true, std::memory_order_release);
   }
   if (count == 1) {
-    hipLaunchKernelGGL(one, dim3((unsigned)nblocks[0]), dim3(NTHR), lds_bytes, stream, P[0], q_tiles[0]);
+    hipLaunchKernelGGL(one, dim3((unsigned)nblocks[0]), dim3(NTHR), lds_bytes, stream, P[0], q_tiles[0], q_full[0]);
     return HDIT_OK;
   }
   AttnMulti M;
-  const int grid = fill_multi(M, P, q_tiles, nblocks, count);
+  const int grid = fill_multi(M, P, q_tiles, q_full, nblocks, count);
   hipLaunchKernelGGL(multi, dim3((unsigned)grid), dim3(NTHR), lds_bytes, stream, M);
   return HDIT_OK;
 }
@@ -1137,7 +1129,7 @@ int launch_grid(One one, Multi multi, int lds_bytes, std::atomic<bool>& attr_set
 }  // namespace
 
 #define HDIT_ATTN_LAUNCH(name, HD, kernel, multi_kernel, lds)                                                              \
-  int name(const AttnParams* P, const int* q_tiles, const int* nblocks, int count, hipStream_t stream) {                   \
+  int name(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream) {                   \
     static std::atomic<bool> attr_set{false};                                                                              \
-    return launch_grid(kernel<HD>, multi_kernel<HD>, lds<HD>::TOTAL, attr_set, P, q_tiles, nblocks, count, stream);        \
+    return launch_grid(kernel<HD>, multi_kernel<HD>, lds<HD>::TOTAL, attr_set, P, q_tiles, q_full, nblocks, count, stream); \
   }

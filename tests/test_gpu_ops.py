@@ -427,7 +427,7 @@ def test_attention_image_rows_do_not_depend_on_the_text_queries(hdit, B, ni, nk,
 @pytest.mark.parametrize("hd,B,H,sq,skv", [
     (64, 1, 2, 200, 192), (64, 1, 3, 129, 193),      # three tiles and one key more, workgroups of 128 rows
     (64, 1, 80, 256, 513), (64, 1, 86, 640, 640),    # workgroups of 256 rows: one round, and the tail of a second
-    (128, 1, 2, 257, 193), (128, 2, 3, 300, 576),
+    (128, 1, 2, 257, 193), (128, 2, 3, 300, 576), (128, 1, 60, 1100, 200),  # whole tiles and half tiles
 ])
 def test_attention_rows_do_not_depend_on_rows_that_outgrow(hdit, hd, B, H, sq, skv):
     """The pipelined kernels leave a row whose sum outgrows the reference fixed after the first tile to the tracked body.
