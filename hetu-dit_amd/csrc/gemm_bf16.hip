@@ -27,7 +27,7 @@
 // read two quarters ahead; the workgroup barrier sits before the last two
 // quarters of a slab, whose fragments are already in registers, so that the first
 // fragments of the next slab are read under their MFMAs.
-//  * 256-row shapes: direct to LDS (global_load_lds_dwordx4, swizzle applied on
+//  * 256-row shapes, 192x192: direct to LDS (global_load_lds_dwordx4, swizzle applied on
 //    the source side), three A slots and two B slots.  During slab g the A rows
 //    of slab g+2 are requested (quarters 0..5) into the slot slab g-1 vacated;
 //    behind the barrier that ends slab g, the B rows of slab g+2 go into the B
@@ -95,25 +95,26 @@ struct Cfg {
   static constexpr int A_BYTES = BM * ROW_BYTES;
   static constexpr int B_BYTES = BN * ROW_BYTES;
   static constexpr int STAGE_BYTES = (BM + BN) * ROW_BYTES;
-  // DMA: the 256-row shapes take their operand slabs straight from global memory into LDS
+  // DMA: the 256-row shapes and 192x192 take their operand slabs straight from global memory into LDS
   // (global_load_lds_dwordx4: no staging registers, no ds_write).  A has three slots (requested two slabs
   // ahead), B two (requested one slab ahead, first in the queue); the epilogue windows alias the A slot the
-  // tile's last slab vacated, which is exactly as large.
-  static constexpr bool DMA = TM == 4;
+  // tile's last slab vacated, which is exactly as large (192x192: they lie behind the slots).
+  static constexpr bool DMA = TM == 4 || (TM == 3 && TN == 3);
   static constexpr int A_SLOTS = 3, B_SLOTS = 2;
   static constexpr int B_OFF = A_SLOTS * A_BYTES;
-  static constexpr int DMA_BYTES = A_SLOTS * A_BYTES + B_SLOTS * B_BYTES;
+  static constexpr bool EPI_ALIAS = NW * EPI_WAVE_BYTES <= A_BYTES;
+  static constexpr int DMA_BYTES = A_SLOTS * A_BYTES + B_SLOTS * B_BYTES + (EPI_ALIAS ? 0 : NW * EPI_WAVE_BYTES);
   // RING: the shapes with short slabs (8 to 48 MFMAs per wave) take them the same way into a ring of NS stages
   // (A then B), as many as fit beside the epilogue windows: only a lead of several slabs covers the latency of
   // operands that come from HBM.
   static constexpr bool RING = TM * TN <= RING_MAX_MMA;
-  static constexpr int EPI_OFF = 160 * 1024 - NW * EPI_WAVE_BYTES;  // ring shapes: windows of their own behind the stages
+  // windows of their own, behind the stages or slots
+  static constexpr int EPI_OFF = DMA ? DMA_BYTES - NW * EPI_WAVE_BYTES : 160 * 1024 - NW * EPI_WAVE_BYTES;
   static constexpr int NS = RING ? (EPI_OFF / STAGE_BYTES < 8 ? EPI_OFF / STAGE_BYTES : 8) : 2;
   static constexpr bool DIRECT = DMA || RING;
   static constexpr int LDS_BYTES = DMA ? DMA_BYTES : RING ? 160 * 1024 : NS * STAGE_BYTES;
   static_assert(LDS_BYTES <= 160 * 1024, "tile does not fit the LDS");
-  static_assert(RING || (DMA ? NW * EPI_WAVE_BYTES <= A_BYTES : NW * EPI_WAVE_BYTES <= STAGE_BYTES),
-                "the epilogue windows live inside one stage (one A slot)");
+  static_assert(RING || DMA || NW * EPI_WAVE_BYTES <= STAGE_BYTES, "the epilogue windows live inside one stage");
   static_assert(!RING || NS >= 3, "a ring holds the slab being read and at least one on its way");
   static_assert(TN <= 4, "epilogue staging window is 128 columns wide");
 };
@@ -518,9 +519,9 @@ __device__ __forceinline__ void run_tiles(const GemmTable& tab, int total_tiles,
     }
     // staging window of this wave: inside the stage (the A slot) the tile's last slab vacated
     unsigned char* epi = lds + wave * EPI_WAVE_BYTES +
-                         (C::DMA    ? (sa == 0 ? C::A_SLOTS - 1 : sa - 1) * C::A_BYTES
-                          : C::RING ? C::EPI_OFF
-                                    : (stage ^ 1) * C::STAGE_BYTES);
+                         (C::RING || (C::DMA && !C::EPI_ALIAS) ? C::EPI_OFF
+                          : C::DMA                             ? (sa == 0 ? C::A_SLOTS - 1 : sa - 1) * C::A_BYTES
+                                                               : (stage ^ 1) * C::STAGE_BYTES);
 
     // ---- epilogue ---------------------------------------------------------
     auto epilogue = [&](auto mode_tag) {
@@ -859,6 +860,7 @@ using Cfg128x128 = Cfg<2, 2>;
 using Cfg128x192 = Cfg<2, 3>;
 using Cfg64x128 = Cfg<1, 2>;
 using Cfg64x64 = Cfg<1, 1>;
+using Cfg192x192 = Cfg<3, 3>;
 
 std::atomic<int> g_force_cfg{-1};
 
@@ -866,10 +868,11 @@ std::atomic<int> g_force_cfg{-1};
 // A launch deals its tiles to 256 workgroups (one per CU) in rounds; a tile costs (k / 64) slab times plus an epilogue
 // with the fill of the pipeline.  Both depend on how many CUs work: a slab takes `lo` microseconds while at most half of
 // them do (what the CU's requests take to come from the last-level cache) and `hi` while all do (the chip's power budget
-// is shared), in between in between.  All figures fitted to MI355X times with weights that come from HBM: 260 random launches
+// is shared), in between in between.  All figures fitted to MI355X times with weights that come from HBM: 300 random launches
 // of the models' sizes (one or two problems, 64 - 17000 rows, N = 1536 - 21504, K = 1536 - 15360) under every shape; the
-// model reproduces those launches within 4 - 10 % and its choice among the shapes is on average 0.04 % slower than the best
-// of them (at most 3 %).
+// model reproduces those launches within 4 - 10 % and its choice among the shapes is on average 0.1 % slower than the best
+// of them (at most 4 %).  192 x 192 is there for what lies between the others: an eighth of those launches take it and are
+// 5 % faster by it (2333+333 x 6144 x 1536 and 5523+333 x 1536 x 6144 11 %).
 //
 // What a plan has to get right is the last round.  One tile shape for everything wastes most of it: the 666-row text
 // stream of a joint block on the image stream's 256-row tiles adds a nearly empty round, and 17 550 rows x 3072 columns
@@ -882,11 +885,11 @@ struct Shape {
   int bm, bn;
   double lo, hi, epi_lo, epi_hi;
 };
-constexpr int NCFG = 7;
+constexpr int NCFG = 8;
 constexpr Shape kShape[NCFG] = {
-    {256, 192, 0.762, 1.076, 5.1, 5.0}, {128, 256, 0.640, 0.847, 4.1, 4.0}, {128, 128, 0.354, 0.465, 3.1, 3.3},
-    {256, 256, 0.975, 1.357, 5.7, 6.6}, {128, 192, 0.445, 0.617, 4.5, 4.1}, {64, 128, 0.262, 0.323, 1.8, 2.3},
-    {64, 64, 0.195, 0.218, 0.7, 1.3},
+    {256, 192, 0.763, 1.086, 4.7, 5.4}, {128, 256, 0.649, 0.840, 3.5, 4.6}, {128, 128, 0.358, 0.480, 2.9, 3.3},
+    {256, 256, 0.979, 1.369, 5.4, 6.8}, {128, 192, 0.453, 0.638, 3.7, 3.8}, {64, 128, 0.270, 0.329, 1.6, 2.2},
+    {64, 64, 0.211, 0.219, 0.4, 1.3},   {192, 192, 0.625, 0.904, 3.9, 4.5},
 };
 constexpr double kLaunchUs = 4.0;
 constexpr int kSlots = 256;
@@ -972,6 +975,7 @@ int launch_cfg(int cfg, const hdit_gemm_problem* problems, int count, hipStream_
     case 3: return build_and_launch<Cfg256x256>(cfg, problems, count, s);
     case 5: return build_and_launch<Cfg64x128>(cfg, problems, count, s);
     case 6: return build_and_launch<Cfg64x64>(cfg, problems, count, s);
+    case 7: return build_and_launch<Cfg192x192>(cfg, problems, count, s);
     default: return build_and_launch<Cfg128x128>(2, problems, count, s);
   }
 }

@@ -85,6 +85,40 @@ def test_gemm_result_does_not_depend_on_the_tile_shape(hdit, epi):
         assert torch.equal(out, outs[0]), f"shape {cfg} differs from shape 0"
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (191, 200, 128), (193, 192, 192), (400, 392, 1088), (8 * 192 + 1, 33 * 192 + 8, 128)])
+def test_gemm_192x192(hdit, m, n, k):
+    """The 192x192 tiles (epilogue windows behind the operand slots): one slab and several, cut-off rows and columns, more
+    tiles than CUs, two problems of one launch, every epilogue -- against fp32 products and, bit for bit, 256x256 tiles."""
+    print(f"gemm 192x192 {m}x{n}x{k}", flush=True)
+    ops, lib = hdit.ops, hdit._lib.lib()
+    ks = (k, k + 64)
+    a, w = ([g(rnd(rows, kk, scale=s, seed=171 + i)) for i, kk in enumerate(ks)] for rows, s in ((m, 1.0), (n, 0.05)))
+    b = [g(rnd(n, seed=175 + i)) for i in range(2)]
+    res = torch.randn(m, n, generator=torch.Generator(device=DEV).manual_seed(177), device=DEV)
+    gate = torch.randn(1, n, generator=torch.Generator(device=DEV).manual_seed(178), device=DEV)
+
+    def launch(cfg):
+        y = [torch.zeros(m, n + 8, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+        z = torch.zeros(m, n, device=DEV)
+        lib.hdit_gemm_force_config(cfg)
+        try:
+            ops.gemm_launch([ops.gemm_problem(a[0], w[0], y[0][:, :n], b[0], ops.EPI_BIAS),
+                             ops.gemm_problem(a[1], w[1], y[1][:, :n], b[1], ops.EPI_BIAS_GELU)])
+            ops.gemm_launch([ops.gemm_problem(a[0], w[0], z, b[0], ops.EPI_GATE_RESIDUAL, resid=res, gate=gate, rows_per_batch=m)])
+        finally:
+            lib.hdit_gemm_force_config(-1)
+        torch.cuda.synchronize()
+        return y + [z]
+
+    got, want = launch(7), launch(3)
+    for i, (x, y) in enumerate(zip(got, want)):
+        assert torch.equal(x, y), f"output {i} differs from 256x256 tiles"
+    lin = [O.linear(a[i].float().cpu(), w[i].float().cpu(), b[i].float().cpu()) for i in range(2)]
+    assert_parity(got[0][:, :n].float().cpu(), lin[0], what="bias")
+    assert_parity(got[1][:, :n].float().cpu(), O.gelu_tanh(lin[1]), what="gelu")
+    assert_parity(got[2].cpu(), res.cpu() + gate.cpu() * lin[0], what="gated residual")
+
+
 @pytest.mark.parametrize("cfg", [2, 4, 5, 6])
 @pytest.mark.parametrize("m,n,k", [(1, 8, 64), (63, 72, 128), (65, 200, 192), (129, 136, 640), (200, 1544, 1088)])
 def test_gemm_ring_shapes(hdit, cfg, m, n, k):
