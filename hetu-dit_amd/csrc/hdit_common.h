@@ -44,9 +44,23 @@ __device__ __forceinline__ i32x4 pack8(const float (&f)[8]) {
   return r;
 }
 
+// v of the 64 lanes added up, in every lane: the partner of a step is lane ^ 32, ^ 16, ^ 8, ^ 4, ^ 2, ^ 1.  In registers
+// (lane swaps, then rotations inside the rows of 16 lanes, whose values repeat every 2 * n lanes by then): an exchange
+// through LDS costs its latency six times over.  512 rows of 1536 fp32, normalised: 4.44 -> 4.18 us, 1357 rows
+// 5.63 -> 5.42.
+template <int N>
+__device__ __forceinline__ float row_rotate(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xf, 0xf, true));  // row_ror:N
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+  v = __int_as_float(s32[0]) + __int_as_float(s32[1]);
+  auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+  v = __int_as_float(s16[0]) + __int_as_float(s16[1]);
+  v += row_rotate<8>(v);
+  v += row_rotate<4>(v);
+  v += row_rotate<2>(v);
+  v += row_rotate<1>(v);
   return v;
 }
 
