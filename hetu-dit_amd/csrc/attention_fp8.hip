@@ -1,23 +1,29 @@
 // fp8 (OCP e4m3) variant of the joint flash attention for gfx950.
 //
-// Same work split and softmax as the bf16 kernel (S^T = K . Q^T so that a lane
-// owns one query column; O^T = V^T . P^T), but every MFMA is the 64-deep
-// v_mfma_scale_f32_32x32x64_f8f6f4 with unit block scales:
+// Same softmax as the bf16 kernels (S^T = K . Q^T so that a lane owns one query column; O^T = V^T . P^T), but
+// every MFMA is the 64-deep v_mfma_scale_f32_32x32x64_f8f6f4 with unit block scales.
+//
+// Bound: the vector ALU (per tile of 64 keys and 32 queries a wave issues 32 exponentials of 8 cycles, 32 additions,
+// 16 maxima and 16 packs beside 4 MFMAs of 64 cycles at d = 64), and the chain scores -> maximum -> exponentials -> PV
+// of one wave.  A wave therefore takes 32 query rows, which fits d = 64 into 128 registers and d = 128 into 256: four and
+// two waves per SIMD, whose matrix and vector parts run side by side.  With 64 rows per wave, two and one waves, the
+// same loop took (kernel and K / V quantisation, us) 2 x 24 heads of 4429 rows, d = 64: 273, now 226; 48 heads of
+// 17776: 3089, now 2768; 24 heads of 4608, d = 128: 305, now 209; of 16896: 3143, now 2089.  Workgroups of eight waves
+// (258, 2983, 217, 2393) and, at d = 64, three waves per SIMD (230, 2841) were slower.
+//
 //   * Q, K, V are quantised with one scale per (batch, head):
 //     x8 = x * 448 / absmax(x)  (absmax from hdit_attn_absmax, clamped away
 //     from zero).  K and V are quantised ONCE by a pre-pass into a caller
 //     workspace laid out [batch, head, key (padded to 64), d] (every query
 //     tile would otherwise repeat the conversion); Q is quantised as its
 //     fragments are loaded;
-//   * the scores are de-scaled by the MFMA itself.  With d = 64 the Q scale is chosen (within a factor of two
-//     below the full-range one, which costs e4m3 nothing but headroom) so that softmax scale * log2(e) *
-//     de-quantisation factor of q and k is an exact power of two, and that power goes into the block-scale
-//     operand of the score MFMA; the running reference (and the +7 of the next item) is subtracted by letting
-//     the MFMA accumulate onto a vector holding it.  The accumulators then feed exp2 directly: no per-score
-//     multiply-add in a loop whose matrix and vector time add up.  (d = 128 has no registers for that vector and
-//     keeps the multiply-add.)
-//   * P is re-quantised per tile as exp2(s - m + 7): at most 2^8 = 256 < 448
-//     with the running maximum allowed to lag by one power of two, so small
+//   * the scores are de-scaled by the MFMA itself.  The Q scale is chosen (within a factor of two below the
+//     full-range one, which costs e4m3 nothing but headroom) so that softmax scale * log2(e) * de-quantisation
+//     factor of q and k is an exact power of two, and that power goes into the block-scale operand of the score
+//     MFMA; the running reference (and the +7 of the next item) is subtracted by letting the MFMA accumulate onto
+//     a vector holding it.  The accumulators then feed exp2 directly.
+//   * P is re-quantised per tile as exp2(s - m + 7): at most 2^7.5 < 448 with
+//     the running maximum allowed to lag by half a power of two, so small
 //     probabilities keep normal-range e4m3 precision;
 //   * O is de-scaled by absmax_v / 448 when it is normalised.
 // In the 32x32 accumulator layout a lane's 32 score registers are exactly its
@@ -33,12 +39,16 @@ typedef __attribute__((ext_vector_type(8))) int i32x8;
 namespace {
 
 constexpr int BKV = 64;
-constexpr int WQ = 64;
+constexpr int WQ = 32;
 constexpr int NWAVE = 4;
+constexpr int NTHR = 64 * NWAVE;
 constexpr int BQ = WQ * NWAVE;
 constexpr float FP8_MAX = 448.0f;
 constexpr float P_SHIFT = 7.0f;            // P is stored as 2^7 * exp2(s - m)
-constexpr float RESCALE_THRESHOLD = 1.0f;  // running max may lag by 2^1: P <= 2^8
+// The running maximum may lag by 2^0.5 (P <= 2^7.5).  A lag leaves the largest probabilities, which are powers of two
+// otherwise, to be rounded: rms error over random shapes 5.56e-2 with waves of 64 rows and a lag of 1, 5.55e-2 with these.
+// No lag costs 3 - 5 %, a lag of 1 would spare 1 - 3 %.
+constexpr float RESCALE_THRESHOLD = 0.5f;
 
 struct Seg2 {
   const __bf16* p0;
@@ -111,7 +121,7 @@ __device__ __forceinline__ unsigned lds_address(const unsigned char* p) {
 }
 
 template <int HD>
-__global__ void __launch_bounds__(256, (HD == 64 ? 2 : 1)) attn_fp8_kernel(const AttnParams P, int q_tiles) {
+__global__ void __launch_bounds__(NTHR, (HD == 64 ? 4 : 2)) attn_fp8_kernel(const AttnParams P, int q_tiles) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   using L = Lds8<HD>;
   constexpr int KS = HD / 64;  // 64-deep k-steps of the score MFMA
@@ -135,83 +145,76 @@ __global__ void __launch_bounds__(256, (HD == 64 ? 2 : 1)) attn_fp8_kernel(const
   const float amq = fmaxf(P.absmax[bh], 1e-20f);
   const float amk = fmaxf(P.absmax[nbh + bh], 1e-20f);
   const float amv = fmaxf(P.absmax[2 * nbh + bh], 1e-20f);
-  constexpr bool FOLD = HD == 64;
-  // score = f * (q8 . k8), f = softmax scale * log2(e) * amk / (448 * qs).  FOLD: qs = full-range scale * f0 / 2^e
+  // score = f * (q8 . k8), f = softmax scale * log2(e) * amk / (448 * qs); qs = full-range scale * f0 / 2^e
   // with e = ceil(log2 f0), so that f = 2^e exactly and 2^e rides the MFMA's E8M0 block scale of the Q operand.
   float qs = FP8_MAX / amq;
-  float scale_log2 = P.scale * 1.4426950408889634f * (amq / FP8_MAX) * (amk / FP8_MAX);
+  const float scale_log2 = P.scale * 1.4426950408889634f * (amq / FP8_MAX) * (amk / FP8_MAX);
   int q_block_scale = 0x7f7f7f7f;  // E8M0 127 = 2^0 in every byte
-  if constexpr (FOLD) {
+  {
     int e = (int)ceilf(log2f(scale_log2));
     e = max(-126, min(127, e));
     const float pow2 = exp2f((float)e);
     qs *= fminf(scale_log2 / pow2, 1.0f);
-    scale_log2 = pow2;
     q_block_scale = 0x01010101 * (127 + e);
   }
   const float o_descale = amv / FP8_MAX;
 
-  // ---- Q fragments: lane holds q row qb*32 + l32, bytes d = 64*ks + 32*lh .. +31
-  i32x8 qf[2][KS];
-#pragma unroll
-  for (int qb = 0; qb < 2; qb++) {
-    int r = min(q0 + qb * 32 + l32, P.sq - 1);
-    const __bf16* rp = row_ptr(P.q, b, h, r);
+  // ---- Q fragments: lane holds q row l32, bytes d = 64*ks + 32*lh .. +31
+  i32x8 qf[KS];
+  {
+    const __bf16* rp = row_ptr(P.q, b, h, min(q0 + l32, P.sq - 1));
 #pragma unroll
     for (int ks = 0; ks < KS; ks++)
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         i32x2 q8 = quant8(*(const i32x4*)(rp + ks * 64 + lh * 32 + c * 8), qs);
-        qf[qb][ks][2 * c] = q8[0];
-        qf[qb][ks][2 * c + 1] = q8[1];
+        qf[ks][2 * c] = q8[0];
+        qf[ks][2 * c + 1] = q8[1];
       }
   }
 
-  // K/V tiles come from the pre-quantised workspace, 64 rows x HD bytes each: request i of a wave covers rows
-  // RPR * (wave + 4 i) .. + RPR - 1, lane -> (row, slot lane % CPR8); the chunk fetched for a slot is the slot index
-  // XORed with the row's swizzle.  Rows past the last key are zero in the workspace.
+  // K/V tiles come from the pre-quantised workspace, 64 rows x HD bytes each: request j of a tile covers rows
+  // RPR * j .. + RPR - 1 of K, or behind those of V, lane -> (row, slot lane % CPR8); the chunk fetched for a slot is the
+  // slot index XORed with the row's swizzle.  Wave w makes the requests w + NWAVE * i.  Rows past the last key are zero in
+  // the workspace.
   constexpr int CPR8 = HD / 16;        // 16-byte chunks per row
   constexpr int RPR = 64 / CPR8;       // rows per request
-  constexpr int NREQ = BKV / (RPR * NWAVE);
-  const unsigned char* k8 = P.k8 + (size_t)bh * P.skv_pad * HD;
-  const unsigned char* v8 = P.v8 + (size_t)bh * P.skv_pad * HD;
-  unsigned koff[NREQ], voff[NREQ];
+  constexpr int KREQ = BKV / RPR;
+  constexpr int NREQ = 2 * KREQ / NWAVE;
+  static_assert(KREQ * 1024 == L::K_BYTES && 2 * KREQ % NWAVE == 0 && (KREQ % NWAVE == 0 || NWAVE % KREQ == 0));
+  const int uwave = __builtin_amdgcn_readfirstlane(wave);
+  const unsigned char* kv8[NREQ];
+  unsigned off8[NREQ];
 #pragma unroll
   for (int i = 0; i < NREQ; i++) {
-    const int row = RPR * (wave + NWAVE * i) + lane / CPR8, slot = lane % CPR8;
-    koff[i] = (unsigned)(row * HD + ((slot ^ L::xk(row)) << 4));
-    voff[i] = (unsigned)(row * HD + ((slot ^ L::xv(row)) << 4));
+    const int j = uwave + NWAVE * i;
+    const bool is_v = j >= KREQ;
+    const int row = RPR * (is_v ? j - KREQ : j) + lane / CPR8, slot = lane % CPR8;
+    kv8[i] = (is_v ? P.v8 : P.k8) + (size_t)bh * P.skv_pad * HD;
+    off8[i] = (unsigned)(row * HD + ((slot ^ (is_v ? L::xv(row) : L::xk(row))) << 4));
   }
-  const unsigned lds_base_addr = __builtin_amdgcn_readfirstlane(lds_address(lds));
-  const unsigned wave_dst = lds_base_addr + __builtin_amdgcn_readfirstlane(wave) * 1024;
+  const unsigned wave_dst = __builtin_amdgcn_readfirstlane(lds_address(lds)) + uwave * 1024;
   auto dma_tile = [&](int t, int stage) {
-    const unsigned char* kb = k8 + (size_t)t * BKV * HD;
-    const unsigned char* vb = v8 + (size_t)t * BKV * HD;
-    const unsigned kdst = wave_dst + stage * L::STAGE;
 #pragma unroll
-    for (int i = 0; i < NREQ; i++) {
-      lds_dma16(kb, koff[i], kdst + i * NWAVE * 1024);
-      lds_dma16(vb, voff[i], kdst + L::K_BYTES + i * NWAVE * 1024);
-    }
+    for (int i = 0; i < NREQ; i++)
+      lds_dma16(kv8[i] + (size_t)t * BKV * HD, off8[i], wave_dst + stage * L::STAGE + i * NWAVE * 1024);
   };
 
-  f32x16 oacc[DB][2];
+  f32x16 oacc[DB];
 #pragma unroll
   for (int i = 0; i < DB; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int v = 0; v < 16; v++) oacc[i][v] = 0.f;
+  // m_run is the running reference in log2 units (0 until the first tile sets it); the score accumulators start from
+  // negm = P_SHIFT - m_run (one value in all 16 entries: a lane owns one query column)
+  float m_run = 0.f, l_run = 0.f;
+  f32x16 negm;
 #pragma unroll
-      for (int v = 0; v < 16; v++) oacc[i][j][v] = 0.f;
-  // FOLD: m_run is the running reference in log2 units (0 until the first tile sets it); the score accumulators
-  // start from negm = P_SHIFT - m_run (one value in all 16 entries: a lane owns one query column per qb)
-  float m_run[2] = {FOLD ? 0.f : -INFINITY, FOLD ? 0.f : -INFINITY};
-  float l_run[2] = {0.f, 0.f};
-  f32x16 negm[2];
-#pragma unroll
-  for (int qb = 0; qb < 2; qb++)
-#pragma unroll
-    for (int v = 0; v < 16; v++) negm[qb][v] = P_SHIFT;
+  for (int v = 0; v < 16; v++) negm[v] = P_SHIFT;
   bool first = true;
+  // P^T operand, 32 bytes, byte e = 16*kb + v.  d = 128 keeps the registers from tile to tile, which saves clearing them
+  // before the packs (3 %); d = 64 has none to keep.
+  i32x8 pf = {0, 0, 0, 0, 0, 0, 0, 0};
 
   // byte-transpose read of V^T: in a 16-lane group lane x supplies the address of 8 bytes
   // (row = key of slot x>>1, column half x&1) and lane i receives byte i%8 of the rows of lanes 2j + i/8.
@@ -229,8 +232,7 @@ __global__ void __launch_bounds__(256, (HD == 64 ? 2 : 1)) attn_fp8_kernel(const
     constexpr bool MASK = decltype(mask_tag)::value;
     constexpr bool LAST = decltype(last_tag)::value;
     const unsigned char* sv = sk + L::K_BYTES;
-    f32x16 sacc[2][2];
-    const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    f32x16 sacc[2];
 #pragma unroll
     for (int kb = 0; kb < 2; kb++) {
 #pragma unroll
@@ -239,104 +241,63 @@ __global__ void __launch_bounds__(256, (HD == 64 ? 2 : 1)) attn_fp8_kernel(const
         const int c0 = ks * 4 + lh * 2;  // this lane's 32 bytes are chunks c0, c0 + 1 of the row
         i32x4 lo = *(const i32x4*)(ka + ((c0 ^ k_swz) << 4)), hi = *(const i32x4*)(ka + (((c0 + 1) ^ k_swz) << 4));
         i32x8 kf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-#pragma unroll
-        for (int qb = 0; qb < 2; qb++)
-          sacc[kb][qb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-              kf, qf[qb][ks], ks == 0 ? (FOLD ? negm[qb] : zero16) : sacc[kb][qb], 0, 0, 0, unit_scale, 0, q_block_scale);
+        sacc[kb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(kf, qf[ks], ks == 0 ? negm : sacc[kb], 0, 0, 0,
+                                                                   unit_scale, 0, q_block_scale);
       }
     }
+    // Both key blocks start from the reference vector.  Reading it once more here keeps it alive past the second block's
+    // first MFMA, which the compiler otherwise ties to a copy of it.
+    asm volatile("" : : "v"(negm));
     if (MASK) {
 #pragma unroll
       for (int kb = 0; kb < 2; kb++)
 #pragma unroll
         for (int v = 0; v < 16; v++) {
           int key = kb * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-          if (key >= valid) {
-            sacc[kb][0][v] = -INFINITY;
-            sacc[kb][1][v] = -INFINITY;
-          }
+          if (key >= valid) sacc[kb][v] = -INFINITY;
         }
     }
-    if constexpr (FOLD) {
-      // the accumulators hold s - m + P_SHIFT; their column maxima, minus P_SHIFT, are relative to the reference
-      float mrel[2];
+    float mx = fmaxf(sacc[0][0], sacc[1][0]);
 #pragma unroll
-      for (int qb = 0; qb < 2; qb++) {
-        float mx = fmaxf(sacc[0][qb][0], sacc[1][qb][0]);
+    for (int v = 1; v < 16; v++) mx = fmaxf(fmaxf(mx, sacc[0][v]), sacc[1][v]);  // one v_max3 per step
+    auto mx_sw = __builtin_amdgcn_permlane32_swap(__float_as_int(mx), __float_as_int(mx), false, false);
+    mx = fmaxf(__int_as_float(mx_sw[0]), __int_as_float(mx_sw[1]));
+    // The accumulators hold s - m + P_SHIFT; the column maximum, minus P_SHIFT, is relative to the reference.  Where some
+    // column of the wave outgrew the threshold, every column's reference moves up to its maximum.
+    const float mrel = mx - P_SHIFT;
+    if (__builtin_amdgcn_ballot_w64(first || mrel > RESCALE_THRESHOLD) != 0) {
+      const float d = first ? mrel : fmaxf(mrel, 0.f);
+      m_run += d;
+      if (!first) {
+        const float alpha = __builtin_amdgcn_exp2f(-d);
+        l_run *= alpha;
 #pragma unroll
-        for (int v = 1; v < 16; v++) mx = fmaxf(mx, fmaxf(sacc[0][qb][v], sacc[1][qb][v]));
-        auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(mx), __float_as_int(mx), false, false);
-        mrel[qb] = fmaxf(__int_as_float(sw[0]), __int_as_float(sw[1])) - P_SHIFT;
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+          for (int v = 0; v < 16; v++) oacc[db][v] *= alpha;
       }
-      const bool grow = first || mrel[0] > RESCALE_THRESHOLD || mrel[1] > RESCALE_THRESHOLD;
-      if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-#pragma unroll
-        for (int qb = 0; qb < 2; qb++) {
-          const float d = first ? mrel[qb] : fmaxf(mrel[qb], 0.f);
-          m_run[qb] += d;
-          if (!first) {
-            const float alpha = __builtin_amdgcn_exp2f(-d);
-            l_run[qb] *= alpha;
-#pragma unroll
-            for (int db = 0; db < DB; db++)
-#pragma unroll
-              for (int v = 0; v < 16; v++) oacc[db][qb][v] *= alpha;
-          }
-#pragma unroll
-          for (int kb = 0; kb < 2; kb++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) sacc[kb][qb][v] -= d;
-#pragma unroll
-          for (int v = 0; v < 16; v++) negm[qb][v] = P_SHIFT - m_run[qb];
-        }
-        first = false;
-      }
-    } else {
-    float mcand[2];
-#pragma unroll
-      for (int qb = 0; qb < 2; qb++) {
-        float mx = fmaxf(sacc[0][qb][0], sacc[1][qb][0]);
-#pragma unroll
-        for (int v = 1; v < 16; v++) mx = fmaxf(mx, fmaxf(sacc[0][qb][v], sacc[1][qb][v]));
-        auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(mx), __float_as_int(mx), false, false);
-        mx = fmaxf(__int_as_float(sw[0]), __int_as_float(sw[1]));
-        mcand[qb] = fmaxf(m_run[qb], mx * scale_log2);
-      }
-      const bool grow = (mcand[0] - m_run[0] > RESCALE_THRESHOLD) || (mcand[1] - m_run[1] > RESCALE_THRESHOLD);
-      if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-#pragma unroll
-        for (int qb = 0; qb < 2; qb++) {
-          const float alpha = __builtin_amdgcn_exp2f(m_run[qb] - mcand[qb]);
-          m_run[qb] = mcand[qb];
-          l_run[qb] *= alpha;
-#pragma unroll
-          for (int db = 0; db < DB; db++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) oacc[db][qb][v] *= alpha;
-        }
-      }
-    }
-    i32x8 pf[2];  // [qb]: 32 bytes, byte e = 16*kb + v
-#pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
-      const float moff = m_run[qb] - P_SHIFT;
-      float rs = l_run[qb];
 #pragma unroll
       for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-        for (int w4 = 0; w4 < 4; w4++) {
-          float p[4];
+        for (int v = 0; v < 16; v++) sacc[kb][v] -= d;
 #pragma unroll
-          for (int e = 0; e < 4; e++)
-            p[e] = __builtin_amdgcn_exp2f(FOLD ? sacc[kb][qb][w4 * 4 + e] : __builtin_fmaf(sacc[kb][qb][w4 * 4 + e], scale_log2, -moff));
-          int w = 0;
-          w = __builtin_amdgcn_cvt_pk_fp8_f32(p[0], p[1], w, false);
-          w = __builtin_amdgcn_cvt_pk_fp8_f32(p[2], p[3], w, true);
-          pf[qb][kb * 4 + w4] = w;
-          rs += (p[0] + p[1]) + (p[2] + p[3]);
-        }
-      l_run[qb] = rs;
+      for (int v = 0; v < 16; v++) negm[v] = P_SHIFT - m_run;
+      first = false;
     }
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+      for (int w4 = 0; w4 < 4; w4++) {
+        float p[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          p[e] = __builtin_amdgcn_exp2f(sacc[kb][w4 * 4 + e]);
+        int w = HD == 64 ? 0 : pf[kb * 4 + w4];  // both halves are written: what it held does not matter
+        w = __builtin_amdgcn_cvt_pk_fp8_f32(p[0], p[1], w, false);
+        w = __builtin_amdgcn_cvt_pk_fp8_f32(p[2], p[3], w, true);
+        pf[kb * 4 + w4] = w;
+        l_run += (p[0] + p[1]) + (p[2] + p[3]);
+      }
 #pragma unroll
     for (int db = 0; db < DB; db++) {
       i32x8 vf;
@@ -347,10 +308,7 @@ __global__ void __launch_bounds__(256, (HD == 64 ? 2 : 1)) attn_fp8_kernel(const
         vf[2 * r] = t8[0];
         vf[2 * r + 1] = t8[1];
       }
-#pragma unroll
-      for (int qb = 0; qb < 2; qb++)
-        oacc[db][qb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf, pf[qb], oacc[db][qb], 0, 0, 0, unit_scale, 0,
-                                                                       unit_scale);
+      oacc[db] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf, pf, oacc[db], 0, 0, 0, unit_scale, 0, unit_scale);
     }
     if constexpr (LAST) {
       // These PV MFMAs are 16-pass instructions and what follows the last tile reads their accumulators at once
@@ -364,11 +322,9 @@ __global__ void __launch_bounds__(256, (HD == 64 ? 2 : 1)) attn_fp8_kernel(const
       // The other reads of an MFMA result in this kernel (the column maxima behind the score MFMAs, the
       // multiply-add of the d = 128 path) rely on the compiler's own wait states.
       if constexpr (DB == 2)
-        asm volatile("s_nop 15\n\ts_nop 15" : "+v"(oacc[0][0]), "+v"(oacc[0][1]), "+v"(oacc[1][0]), "+v"(oacc[1][1]));
+        asm volatile("s_nop 15\n\ts_nop 15" : "+v"(oacc[0]), "+v"(oacc[1]));
       else
-        asm volatile("s_nop 15\n\ts_nop 15"
-                     : "+v"(oacc[0][0]), "+v"(oacc[0][1]), "+v"(oacc[1][0]), "+v"(oacc[1][1]), "+v"(oacc[2][0]),
-                       "+v"(oacc[2][1]), "+v"(oacc[3][0]), "+v"(oacc[3][1]));
+        asm volatile("s_nop 15\n\ts_nop 15" : "+v"(oacc[0]), "+v"(oacc[1]), "+v"(oacc[2]), "+v"(oacc[3]));
     }
   };
 
@@ -391,23 +347,20 @@ __global__ void __launch_bounds__(256, (HD == 64 ? 2 : 1)) attn_fp8_kernel(const
     if (valid < BKV) tile_compute(lds + (t & 1) * L::STAGE, std::true_type{}, valid, std::true_type{});
     else tile_compute(lds + (t & 1) * L::STAGE, std::false_type{}, BKV, std::true_type{});
   }
+  auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(l_run), __float_as_int(l_run), false, false);
+  const float inv = o_descale / (__int_as_float(sw[0]) + __int_as_float(sw[1]));
+  const int r = q0 + l32;
+  if (r >= P.sq) return;
+  __bf16* op = (__bf16*)row_ptr(P.o, b, h, r);
 #pragma unroll
-  for (int qb = 0; qb < 2; qb++) {
-    auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(l_run[qb]), __float_as_int(l_run[qb]), false, false);
-    const float inv = o_descale / (__int_as_float(sw[0]) + __int_as_float(sw[1]));
-    const int r = q0 + qb * 32 + l32;
-    if (r >= P.sq) continue;
-    __bf16* op = (__bf16*)row_ptr(P.o, b, h, r);
+  for (int db = 0; db < DB; db++)
 #pragma unroll
-    for (int db = 0; db < DB; db++)
-#pragma unroll
-      for (int g = 0; g < 4; g++) {
-        i32x2 out;
-        out[0] = (int)hdit::pack2(oacc[db][qb][g * 4 + 0] * inv, oacc[db][qb][g * 4 + 1] * inv);
-        out[1] = (int)hdit::pack2(oacc[db][qb][g * 4 + 2] * inv, oacc[db][qb][g * 4 + 3] * inv);
-        *(i32x2*)(op + db * 32 + g * 8 + lh * 4) = out;
-      }
-  }
+    for (int g = 0; g < 4; g++) {
+      i32x2 out;
+      out[0] = (int)hdit::pack2(oacc[db][g * 4 + 0] * inv, oacc[db][g * 4 + 1] * inv);
+      out[1] = (int)hdit::pack2(oacc[db][g * 4 + 2] * inv, oacc[db][g * 4 + 3] * inv);
+      *(i32x2*)(op + db * 32 + g * 8 + lh * 4) = out;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -600,7 +553,7 @@ int fwd_fp8_launch(const hdit_attn_args* a, const float* absmax, void* workspace
   else
     hipLaunchKernelGGL(quantize_kv_kernel<128>, qgrid, dim3(256), 0, s, P);
   int q_tiles = (P.sq + BQ - 1) / BQ;
-  dim3 grid((unsigned)(q_tiles * a->batch * a->heads)), block(256);
+  dim3 grid((unsigned)(q_tiles * a->batch * a->heads)), block(NTHR);
   if (a->head_dim == 64)
     hipLaunchKernelGGL(attn_fp8_kernel<64>, grid, block, Lds8<64>::TOTAL, s, P, q_tiles);
   else

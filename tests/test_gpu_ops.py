@@ -641,6 +641,22 @@ def test_attention_fp8(hdit, hd, sq, skv):
 
 
 @pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("sq,skv", [(1, 1), (31, 64), (32, 65), (33, 130), (127, 63), (128, 333), (129, 128), (257, 200)])
+def test_attention_fp8_tile_edges(hdit, hd, sq, skv):
+    """Query counts around the 32 rows of a wave and the 128 of a workgroup, key counts around the 64 of a tile: the same
+    bound as above, and rows that do not exist stay unwritten."""
+    print(f"attention fp8 edges hd={hd} sq={sq} skv={skv}", flush=True)
+    B, H = 2, 2
+    q, k, v = rnd(B, sq, H, hd, seed=41), rnd(B, skv, H, hd, seed=42), rnd(B, skv, H, hd, seed=43)
+    out = torch.full((B, sq + 3, H, hd), 7.0, dtype=torch.bfloat16, device="cuda")
+    hdit.ops.attention([g(q)], [g(k)], [g(v)], out=[out[:, :sq]], fp8=True)
+    torch.cuda.synchronize()
+    want = O.attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)).transpose(1, 2)
+    assert_parity(out[:, :sq], want, rel=FP8_KERNEL_REL, cos=0.998, what="fp8 tile edges")
+    assert bool((out[:, sq:] == 7.0).all())
+
+
+@pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("skv", [77, 333, 64 + 1])
 def test_attention_fp8_masked_last_tile_tail_columns(hdit, hd, skv):
     """Fixed regression case for the distance between the last PV MFMA and the first read of its result: with a
