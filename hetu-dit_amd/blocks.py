@@ -174,9 +174,7 @@ class JointTransformerBlock(nn.Module):
         pipeline patch after the first, ``transformer_sd3.py:131-146``), so the text stream stops after its
         q|k|v projection -- no out-projection, ``norm2_context`` or ``ff_context`` -- and ``None`` is returned
         for it.  With bf16 attention the image output is unchanged bit for bit (the fp8 path scales the queries by
-        their largest value, text rows included) -- for a patch always; for a whole sequence of at most one
-        round of attention workgroups except in rows that share a workgroup with a text row whose logits outgrow those
-        of its first 64 keys by more than 44.
+        their largest value, text rows included).
 
         ``pending`` / ``defer`` (block stacks, f32 streams): the launches of ``hdit_block_sd3`` with
         ``lazy_residual`` -- see ``_forward_lazy``."""

@@ -4,8 +4,10 @@
 // ("B") each run one of: nothing; a loop of independent v_mfma_f32_32x32x16_bf16 (32 per iteration: the matrix
 // work of one 64 x 64 x 64 attention tile); the VALU work of that tile's softmax (64 exponentials, 32 bf16 packs,
 // 32 pair sums, 32 three-way maxima, 64 subtractions per iteration); or both interleaved in one instruction
-// stream.  Every wave reports the shader cycles and the 100 MHz ticks it took.  If the two units overlapped, an
-// MFMA wave and a VALU wave on one SIMD would finish in the time of the longer one; on gfx950 they take the sum.
+// stream.  Every wave reports the shader cycles and the 100 MHz ticks it took.  On gfx950 an
+// MFMA wave and a wave of this mix on one SIMD take the sum of their times, because of the pair sums: dot products
+// (v_dot2*) wait for the matrix pipe.  Additions, fused multiply-adds, exponentials, packs, maxima and lane swaps by
+// themselves run beside the MFMAs of another wave, at a cost of about 8 cycles per MFMA.
 #include "hdit_common.h"
 
 namespace {

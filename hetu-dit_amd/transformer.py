@@ -69,6 +69,9 @@ class _Chain:
 # 3364+333 16.6 / 15.8, 3600+333 17.0 / 16.8, 3844+333 18.5 / 19.2, 4096+333 19.3 / 19.9, 4356+333 21.1 / 21.1.  At B = 3
 # (chains of one and two): 576+333 6.7 / 5.8, 2048+333 14.4 / 12.9, 2398+333 16.5 / 17.1, 3136+333 21.5 / 20.4, 3600+333
 # 24.8 / 25.7; at B = 4: 784+333 9.2 / 8.6, 1444+333 13.9 / 12.7, 2704+333 23.7 / 24.6, 4096+333 36.1 / 37.0.
+# Since then attention and the GEMMs have become faster, the line has stayed: at B = 2 3328+333 14.9 / 14.9, 4096+333 18.4 /
+# 18.8, 4624+333 21.9 / 21.3, 5776+333 26.5 / 27.9, 8100+333 40.5 / 42.6; at B = 3 1920+333 12.9 / 13.0, 4224+333 26.7 / 28.8;
+# at B = 4 2304+333 19.6 / 18.5.
 LANE_ROWS = 4096
 
 
@@ -76,8 +79,7 @@ class SD3TransformerBlocks(nn.Module):
     """The 24 joint blocks of the SD3 transformer with the reference's block loop.
 
     ``use_block_entry_points``: run every block through ``hdit_block_sd3`` (one foreign call per block, the
-    same launches on the same operands as the Python block: results are bit for bit the same; chains of a pass that is
-    divided below the default ``lane_rows`` may get the pipelined attention kernel where the undivided batch does not)
+    same launches on the same operands as the Python block: results are bit for bit the same)
     instead of one foreign call per kernel.  An eager pass is then bound by the GPU and not by the interpreter, which is what
     lets independent work run side by side on several streams:
 
