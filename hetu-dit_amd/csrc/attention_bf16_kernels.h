@@ -444,13 +444,15 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
         mx = fmaxf(__int_as_float(sw[0]), __int_as_float(sw[1]));
         mcand[qb] = fmaxf(m_run[qb], mx * P.scale_log2);
       }
-      // raise the running maxima (and rescale) only if some row outgrew the threshold: wave-uniform branch
+      // raise the running maxima (and rescale) only if some row outgrew the threshold: wave-uniform branch, every column's
+      // own decision, as above (the others are multiplied by 1)
       const bool grow = (mcand[0] - m_run[0] > RESCALE_THRESHOLD) || (mcand[QB - 1] - m_run[QB - 1] > RESCALE_THRESHOLD);
       if (__builtin_amdgcn_ballot_w64(grow) != 0) {
 #pragma unroll
         for (int qb = 0; qb < QB; qb++) {
-          const float alpha = __builtin_amdgcn_exp2f(m_run[qb] - mcand[qb]);
-          m_run[qb] = mcand[qb];
+          const bool move = mcand[qb] - m_run[qb] > RESCALE_THRESHOLD;  // always at the first tile, from -inf
+          const float alpha = move ? __builtin_amdgcn_exp2f(m_run[qb] - mcand[qb]) : 1.0f;
+          m_run[qb] = move ? mcand[qb] : m_run[qb];
           l_run[qb] *= alpha;
 #pragma unroll
           for (int db = 0; db < DB; db++)

@@ -486,6 +486,38 @@ def test_attention_rows_do_not_depend_on_rows_that_outgrow(hdit, hd, B, H, sq, s
         assert_parity(got[:, :, heads], want, what=f"attention, outgrowing rows, {skv - cut} keys")
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("sq,skv", [(64, 100), (333, 128), (64, 333), (300, 640)])  # tracked; pipelined, then the second pass
+def test_attention_rows_do_not_depend_on_neighbours_whose_reference_moves(hdit, hd, sq, skv):
+    """A row keeps its bits whatever the rows beside it hold, also in the kernels whose reference follows the maxima.  Every
+    other row sees its logits jump by hundreds at keys 64.. of a longer sequence (so that the second pass computes it)
+    and by less than the rescale threshold at the last keys, where the reference of its neighbours moves far -- or, in the
+    other launch, does not."""
+    print(f"attention neighbours d={hd} {sq}x{skv}", flush=True)
+    H, half = 2, hd // 2
+    gen = torch.Generator(device=DEV).manual_seed(97)
+    r = lambda n: torch.randn(1, n, H, hd, generator=gen, device=DEV)
+    u, w = torch.zeros(hd, device=DEV), torch.zeros(hd, device=DEV)  # orthogonal
+    u[:half], w[half:] = 1.0, 1.0
+    q, k, v = r(sq) * 0.3, r(skv) * 0.3, r(skv)
+    k[..., half:] = 0.0
+    logit = (40.0 if skv <= 128 else 400.0) / half * math.sqrt(hd)  # q = logit * u against k = u: that many
+    first = 0 if skv <= 128 else 64
+    k[:, first:skv - 20] = u + 0.02 * k[:, first:skv - 20]
+    k[:, skv - 20:] = u * (1.0 + 2.0 / (40.0 if skv <= 128 else 400.0)) + 0.02 * k[:, skv - 20:] + w  # + 2, and w for the others
+    q[:, ::2] += logit * u
+    moving = q.clone()
+    moving[:, 1::2] = logit * w
+    q[:, 1::2] = 0.0
+    q, moving, k, v = (t.to(torch.bfloat16) for t in (q, moving, k, v))
+    a, = hdit.ops.attention([q], [k], [v])
+    b, = hdit.ops.attention([moving], [k], [v])
+    torch.cuda.synchronize()
+    assert torch.equal(a[:, ::2], b[:, ::2]), "rows changed with their neighbours"
+    want = O.attention(*(t.float().cpu().transpose(1, 2) for t in (moving, k, v))).transpose(1, 2)
+    assert_parity(b, want, what="attention, neighbours that move")
+
+
 # (batch, heads, query rows, key rows, key rows in the second buffer, gap between heads, outgrowing query rows)
 @pytest.mark.parametrize("hd,problems", [
     (128, [(1, 3, 300, 200, 0, 0, ()), (2, 2, 64, 333, 133, 0, (0, 63)), (1, 5, 513, 1000, 77, 64, (512,)), (2, 1, 1, 129, 64, 8, (0,))]),
