@@ -20,11 +20,10 @@ HIPCC_FLAGS = [
 ]
 
 
-# Per-file additions.  The attention kernels of one or two waves per SIMD: left alone the compiler keeps every MFMA
+# Per-file additions.  The bf16 attention kernels: left alone the compiler keeps every MFMA
 # accumulator in the AGPR half, and the softmax (VALU) cannot read those without a copy per score.  In the VGPR form the
 # allocator decides per value.
 EXTRA_FLAGS = {
-    "attention_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "attention_bf16_pipe4.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "attention_bf16_pipe8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }

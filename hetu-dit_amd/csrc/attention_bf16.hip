@@ -1,5 +1,5 @@
-// Joint (image + text) flash attention forward for gfx950, bf16 in/out: the C entry point and the head-dim-64
-// kernels (device code and its description: attention_bf16_kernels.h).
+// Joint (image + text) flash attention forward for gfx950, bf16 in/out: the C entry points and the choice of the kernel
+// (device code and its description: attention_bf16_kernels.h).
 #include "attention_bf16_kernels.h"
 
 namespace {
@@ -29,10 +29,6 @@ Seg2 make_seg(const hdit_seq_segment* s) {
 }
 
 }  // namespace
-
-namespace hdit_attn {
-HDIT_ATTN_LAUNCH(launch_tracked_d64, 64, attn_fwd_kernel, attn_fwd_multi_kernel, Lds)
-}  // namespace hdit_attn
 
 namespace hdit_host {
 int attn_validate(const hdit_attn_args* a) {
@@ -65,8 +61,8 @@ bool to_params(const hdit_attn_args* a, AttnParams& P) {
   return true;
 }
 
-// Which kernel serves a problem.  The pipelined ones where there are at least three tiles of keys and a tile's step fits
-// 32 bits; the tracked one otherwise.  That is decided from keys and strides alone, and a row's result depends on the row
+// Which kernel serves a problem.  The pipelined ones where there are enough tiles of keys (pipe_min_tiles) and a tile's step
+// fits 32 bits; the tracked one otherwise.  That is decided from keys and strides alone, and a row's result depends on the row
 // and the keys alone: neither rows that are left out (the text queries of a joint sequence) nor other problems of the
 // launch change a bit.
 // HDIT_ATTN_PIPE=0 keeps every launch on the tracked kernel, =4 and =8 every other one of head dim 64 on workgroups of four
@@ -79,7 +75,7 @@ char pipe_env() {
 bool is_pipelined(const hdit_attn_args* a, const AttnParams& P) {
   const bool strides_ok = a->k[0].stride_s < (1 << 22) && a->k[1].stride_s < (1 << 22) && a->v[0].stride_s < (1 << 22) &&
                           a->v[1].stride_s < (1 << 22);  // a tile step (64 rows, in bytes) fits 32 bits
-  return pipe_env() != '0' && strides_ok && (P.skv + BKV - 1) / BKV >= PIPE_MIN_TILES;
+  return pipe_env() != '0' && strides_ok && (P.skv + BKV - 1) / BKV >= hdit_attn::pipe_min_tiles(a->head_dim);
 }
 
 int64_t rows_of(const hdit_attn_args* a) { return a->q[0].len + a->q[1].len; }
@@ -128,7 +124,7 @@ Tiling tiling(const hdit_attn_args* a, int64_t cus) {
 // Per row the same, so the last round decides, and small workgroups where CUs would be idle.  128 / 256 rows: 333 rows
 // 8.6 / 11.4 us, 2 x 666 15.0 / 16.1, 2 x 1357 37.1 / 39.3, 1024 of 4429 rows 41.0 / 57.5, two of them 63.3 / 60.1, 4470
 // rows 127.9 / 122.4, 2 x 4429 227 / 247, 17776 rows with 48 heads 3443 / 3378.
-int pipe_rows(const hdit_attn_args* const* of, int count) {
+int pipe_rows(const hdit_attn_args* const* of, int count, int cus) {
   if (pipe_env() == '4') return 128;
   if (pipe_env() == '8') return 256;
   int64_t small = 0, large = 0, tiles = 0;
@@ -137,7 +133,6 @@ int pipe_rows(const hdit_attn_args* const* of, int count) {
     const int64_t t = (of[i]->k[0].len + of[i]->k[1].len + BKV - 1) / BKV;
     if (t > tiles) tiles = t;
   }
-  const int cus = hdit_host::num_cus();
   if (cus <= 0) return 256;  // no device to ask: the launch reports it
   small = (small + cus - 1) / cus;
   const double cost_small = tiles * (0.90 * (double)(small / 2) + 0.55 * (double)(small % 2));
@@ -145,27 +140,47 @@ int pipe_rows(const hdit_attn_args* const* of, int count) {
   return cost_small <= 1.05 * cost_large ? 128 : 256;  // (2 x 4429 rows: modelled 228 / 219, measured 242 / 244)
 }
 
+// Query rows per workgroup of a launch.  The tracked kernel serves few keys: d = 64 small workgroups, ahead at every fill
+// (attention_bf16_kernels.h), d = 128 large ones.
+int launch_rows(const hdit_attn_args* const* of, int count, bool pipelined, int cus) {
+  if (of[0]->head_dim == 128) return 256;
+  return pipelined ? pipe_rows(of, count, cus) : 128;
+}
+
 // The problems of one call that one kernel serves, as one launch.
 int launch_some(const hdit_attn_args* const* of, const AttnParams* P, int count, bool pipelined, hipStream_t s) {
-  const int hd = of[0]->head_dim;
-  const int rows = pipelined && hd == 64 ? pipe_rows(of, count) : 256;
-  const bool eight = pipelined && rows == 256;
+  const int hd = of[0]->head_dim, cus = hdit_host::num_cus();
+  const int rows = launch_rows(of, count, pipelined, cus), part = rows == 256 ? rows / 2 : rows;
   int q_tiles[HDIT_ATTN_MAX_MULTI], q_full[HDIT_ATTN_MAX_MULTI], nblocks[HDIT_ATTN_MAX_MULTI];
   for (int i = 0; i < count; i++) {
-    const int part = eight ? rows / 2 : rows, cus = hdit_host::num_cus();
-    q_full[i] = eight && count == 1 && cus > 0 ? tiling(of[i], cus).full : P[i].sq / rows + (P[i].sq % rows > part);
+    const bool tiled = pipelined && rows == 256 && count == 1 && cus > 0;
+    q_full[i] = tiled ? tiling(of[i], cus).full : P[i].sq / rows + (P[i].sq % rows > part);
     const int left = P[i].sq - q_full[i] * rows;
     q_tiles[i] = q_full[i] + (left > 0 ? (left + part - 1) / part : 0);
     nblocks[i] = of[i]->batch * of[i]->heads * q_tiles[i];
   }
   if (!pipelined)
-    return hd == 64 ? hdit_attn::launch_tracked_d64(P, q_tiles, q_full, nblocks, count, s)
-                    : hdit_attn::launch_tracked_d128(P, q_tiles, q_full, nblocks, count, s);
+    return hd == 64 ? hdit_attn::launch_tracked4_d64(P, q_tiles, q_full, nblocks, count, s)
+                    : hdit_attn::launch_tracked8_d128(P, q_tiles, q_full, nblocks, count, s);
   if (hd == 128) return hdit_attn::launch_pipe8_d128(P, q_tiles, q_full, nblocks, count, s);
   return rows == 128 ? hdit_attn::launch_pipe4_d64(P, q_tiles, q_full, nblocks, count, s)
                      : hdit_attn::launch_pipe8_d64(P, q_tiles, q_full, nblocks, count, s);
 }
 }  // namespace
+
+extern "C" __attribute__((visibility("default"))) int hdit_attn_rows(const hdit_attn_args* args, int count, int cus) {
+  if (!args || count <= 0 || count > HDIT_ATTN_MAX_MULTI || cus <= 0) return HDIT_EINVAL;
+  const hdit_attn_args* of[HDIT_ATTN_MAX_MULTI];
+  AttnParams P[HDIT_ATTN_MAX_MULTI];
+  for (int i = 0; i < count; i++) {
+    const int rc = hdit_host::attn_validate(&args[i]);
+    if (rc != HDIT_OK) return rc;
+    if (!to_params(&args[i], P[i]) || args[i].head_dim != args[0].head_dim) return HDIT_EINVAL;
+    if (is_pipelined(&args[i], P[i]) != is_pipelined(&args[0], P[0])) return HDIT_EINVAL;
+    of[i] = &args[i];
+  }
+  return launch_rows(of, count, is_pipelined(args, P[0]), cus);
+}
 
 extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16(const hdit_attn_args* a, void* stream) {
   int rc = hdit_host::attn_validate(a);

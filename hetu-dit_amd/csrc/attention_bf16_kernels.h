@@ -1,16 +1,20 @@
 // Device code of the bf16 flash-attention kernels, shared by the translation units that instantiate them
-// (attention_bf16.hip: head dim 64 and the C entry point; attention_bf16_d128.hip: head dim 128): the two are
-// compiled with different register-allocation options, see build.py.
+// (attention_bf16_pipe4.hip, _pipe8.hip: workgroups of four and of eight waves; the C entry points and the choice between
+// them: attention_bf16.hip).
 //
 // Joint (image + text) flash attention forward for gfx950, bf16 in/out.
 //
-// Two kernels: the pipelined one further down serves everything that has three
-// tiles of keys; the one described here ("tracked") the rest, and the rows for
-// which the pipelined kernel's fixed softmax reference does not hold.
+// Two kernels: the pipelined one further down serves everything that has enough
+// keys (pipe_min_tiles); the one described here ("tracked") the rest, and the rows
+// for which the pipelined kernel's fixed softmax reference does not hold.
 //
-// Work split: one workgroup = 4 waves = 256 query rows of one (batch, head);
-// each wave owns 64 query rows (two 32-row MFMA column blocks; one block inside
-// the pipelined kernels) and walks the keys in tiles of 64.  K and V tiles go straight from global memory into two
+// Work split: one workgroup = 4 or 8 waves = 128 or 256 query rows of one (batch,
+// head); each wave owns 32 query rows (one MFMA column block) and walks the keys in
+// tiles of 64.  (Waves of 64 rows read half the K and V fragments per row, but with
+// few keys what counts is how soon a workgroup is done: 48 heads, d = 64, four waves,
+// 64 / 32 rows per wave: 333 x 128 9.8 / 5.8 us, 4096 x 77 24.0 / 21.9; 192 heads,
+// 1024 x 192 29.6 / 21.9.  d = 128, 24 heads, four waves of 64 / eight of 32 rows:
+// 128 x 128 11.2 / 8.5, 4096 x 77 29.5 / 27.5.)  K and V tiles go straight from global memory into two
 // LDS buffers (direct-to-LDS loads, one barrier per tile).
 //
 // The scores are produced transposed, S^T = K . Q^T, with K rows as the MFMA
@@ -60,11 +64,20 @@ struct AttnParams {
   float scale_log2;
 };
 
+constexpr int BKV = 64;  // keys per tile
+
+// From how many key tiles on the pipelined kernels serve a problem; their loop needs three.  At d = 64 they begin later
+// than the tracked one and are ahead where the loop is long enough.  Tracked / pipelined, 128 rows per workgroup, us:
+//   48 heads   256 x 256 7.0 / 7.4, 2048 x 256 14.0 / 16.2, 384 x 384 8.6 / 8.5, 1024 x 384 12.1 / 12.1, 448 x 448 9.3 / 9.0
+//   192 heads  320 x 320 13.3 / 15.8, 384 x 384 16.2 / 18.7, 1024 x 384 30.8 / 32.6, 448 x 448 18.6 / 19.5
+// At d = 128 they are ahead at once: 24 heads, 192 x 192 14.5 / 10.5.
+constexpr int pipe_min_tiles(int head_dim) { return head_dim == 64 ? 7 : 3; }
+
 // Launch of `count` problems of one head dim, on argument blocks the entry point has validated and converted, as one grid:
-// the tracked kernel (256 query rows per workgroup), the pipelined ones of 128 and 256 rows.  A (batch, head) is q_tiles
-// workgroups, the first q_full of them with all their rows; nblocks is their number for the whole problem.
-int launch_tracked_d64(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
-int launch_tracked_d128(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
+// the tracked and the pipelined kernels, with 128 (four waves) and with 256 query rows per workgroup (eight).  A (batch,
+// head) is q_tiles workgroups, the first q_full of them with all their rows; nblocks is their number for the whole problem.
+int launch_tracked4_d64(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
+int launch_tracked8_d128(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
 int launch_pipe4_d64(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
 int launch_pipe8_d64(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
 int launch_pipe8_d128(const AttnParams* P, const int* q_tiles, const int* q_full, const int* nblocks, int count, hipStream_t stream);
@@ -76,11 +89,8 @@ namespace {
 using hdit_attn::AttnParams;
 using hdit_attn::Seg2;
 
-constexpr int BKV = 64;   // keys per tile
-#ifndef HDIT_ATTN_QUERY_BLOCKS
-#define HDIT_ATTN_QUERY_BLOCKS 2  // 32-row query blocks per wave (the pipelined kernels' units: 1)
-#endif
-constexpr int QB = HDIT_ATTN_QUERY_BLOCKS;
+using hdit_attn::BKV;
+constexpr int QB = 1;        // 32-row query blocks per wave of the tracked kernel
 constexpr int WQ = 32 * QB;  // query rows per wave
 #ifndef HDIT_ATTN_WAVES
 #define HDIT_ATTN_WAVES 4  // waves per workgroup (attention_bf16_pipe8.hip: 8)
@@ -104,9 +114,9 @@ struct Lds {
   static constexpr int K_BYTES = BKV * K_ROW;
   static constexpr int V_BYTES = BKV * V_ROW;
   static constexpr int STAGE = K_BYTES + V_BYTES;
-  // d = 128: the Q fragments (64 registers) live in LDS instead, one private region per wave, rows strided like
+  // d = 128: the Q fragments (32 registers) live in LDS instead, one private region per wave, rows strided like
   // the K rows, and are read per k-step next to the K fragments: the registers they would occupy are what the
-  // loop otherwise spills (and reloads from scratch on every tile, with one wave per SIMD to hide nothing).
+  // loop otherwise spills (and reloads from scratch on every tile, with few waves per SIMD to hide that).
   static constexpr bool Q_IN_LDS = HD == 128;
   static constexpr int Q_ROW = HD * 2 + 16;
   static constexpr int Q_OFF = 2 * STAGE;
@@ -178,6 +188,8 @@ struct Place {
   int b, h, q0, rows;
 };
 __device__ __forceinline__ Place place(const AttnParams& P, int q_tiles, int q_full, int block_id, int nblocks) {
+  // The arguments that are needed next are requested together with those of the divisions, not behind them: 0.2 us.
+  asm volatile("" : "+s"(q_tiles) : "s"(P.q.p0), "s"(P.q.len0), "s"(P.k.p0), "s"(P.k.len0), "s"(P.v.p0), "s"(P.skv));
   const int nbh = nblocks / q_tiles;
   const bool by_xcd = nbh % 8 == 0;
   const int slot = by_xcd ? (block_id >> 3) : block_id;
@@ -195,7 +207,7 @@ __device__ __forceinline__ Place place(const AttnParams& P, int q_tiles, int q_f
 
 // The whole kernel for one workgroup: the online softmax with a running reference that follows the column
 // maxima.  Also the second pass of the pipelined kernels, for the rows whose fixed reference did not hold: bit l of
-// `rows` (one query block per wave) stands for the wave's row l, the others have been written.
+// `rows` stands for the wave's row l, the others have been written.
 template <int HD>
 __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_tiles, int q_full, unsigned char* lds,
                                                   int block_id, int nblocks, unsigned rows = ~0u) {
@@ -221,7 +233,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
   bf16x8 qf[QB][L::Q_IN_LDS ? 1 : KS];
   unsigned char* qlds = lds + L::Q_OFF + wave * L::Q_WAVE_BYTES;
   if constexpr (L::Q_IN_LDS) {
-    // the wave's 64 query rows, 16 lanes per row (coalesced 256-byte rows), into its private LDS region;
+    // the wave's query rows, 16 lanes per row (coalesced 256-byte rows), into its private LDS region;
     // only this wave reads them back, so its own wait for the writes is all the synchronisation needed
     constexpr int RPI = 64 / CPR;  // rows per wave-wide load
 #pragma unroll
@@ -541,7 +553,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(l_run[qb]), __float_as_int(l_run[qb]), false, false);
     const float inv = 1.0f / (__int_as_float(sw[0]) + __int_as_float(sw[1]));
     const int r = q0 + qb * 32 + l32;
-    if (r >= P.sq || (QB == 1 && !((rows >> l32) & 1))) continue;
+    if (r >= P.sq || !((rows >> l32) & 1)) continue;
     __bf16* op = (__bf16*)row_ptr(P.o, b, h, r);
 #pragma unroll
     for (int db = 0; db < DB; db++)
@@ -556,7 +568,7 @@ __device__ __forceinline__ void attn_tracked_body(const AttnParams& P, int q_til
 }
 
 template <int HD>
-__global__ void __launch_bounds__(NTHR, HD == 64 ? 2 : 1) attn_fwd_kernel(const AttnParams P, int q_tiles, int q_full) {
+__global__ void __launch_bounds__(NTHR, HD == 64 ? 3 : 2) attn_fwd_kernel(const AttnParams P, int q_tiles, int q_full) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   attn_tracked_body<HD>(P, q_tiles, q_full, lds, (int)blockIdx.x, (int)gridDim.x);
 }
@@ -574,7 +586,7 @@ struct AttnMulti {
 };
 
 template <int HD>
-__global__ void __launch_bounds__(NTHR, HD == 64 ? 2 : 1) attn_fwd_multi_kernel(const AttnMulti M) {
+__global__ void __launch_bounds__(NTHR, HD == 64 ? 3 : 2) attn_fwd_multi_kernel(const AttnMulti M) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   int i = 0;
 #pragma unroll 1
@@ -643,7 +655,6 @@ struct PipeLds {
 };
 constexpr float PIPE_MARGIN = 24.0f;  // an integer: the exact p's stay exact
 constexpr float PIPE_LIMIT = 0x1p40f;
-constexpr int PIPE_MIN_TILES = 3;
 constexpr int FRAG_LEAD = 3;
 
 template <int... I, class F>
@@ -672,7 +683,7 @@ __device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles,
   const Place at = place(P, q_tiles, q_full, block_id, nblocks);
   const int b = at.b, h = at.h, q0 = at.q0 + wave * 32;
   const bool active = __builtin_amdgcn_readfirstlane(q0 < P.sq && wave * 32 < at.rows);
-  const int NT = (P.skv + BKV - 1) / BKV;  // >= PIPE_MIN_TILES (host)
+  const int NT = (P.skv + BKV - 1) / BKV;  // >= pipe_min_tiles (host)
   rows = 0;
 
   typedef __attribute__((address_space(3))) int lds_int;

@@ -153,6 +153,12 @@ int hdit_attn_fwd_bf16(const hdit_attn_args* args, void* stream);
 #define HDIT_ATTN_MAX_MULTI 4
 int hdit_attn_fwd_bf16_multi(const hdit_attn_args* args, int count, void* stream);
 
+/* Test hook without a counterpart in the reference: the query rows per workgroup
+ * (128 or 256) that a launch of these problems gets on a GPU of `cus` compute
+ * units.  Reads no memory behind the pointers and needs no GPU.  HDIT_EINVAL
+ * where the problems have no rows or go to several launches. */
+int hdit_attn_rows(const hdit_attn_args* args, int count, int cus);
+
 /* Same contract on the fp8-e4m3 (OCP) MFMA path: Q, K, V are quantised with one
  * absmax scale per (batch, head) taken from `absmax` (f32 [3, batch, heads]:
  * q, k, v; written by hdit_attn_absmax), P is re-quantised per tile.  K and V

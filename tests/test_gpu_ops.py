@@ -426,6 +426,23 @@ def test_attention_d64_kernels(hdit, B, H, sq, skv, gain):
     assert_parity(torch.cat(out, 1), want, what="attention d64")
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("sq,skv", [(1, 1), (31, 64), (33, 65), (128, 128), (129, 63), (257, 127), (300, 100)])
+def test_attention_with_few_keys(hdit, hd, sq, skv):
+    """The tracked kernels, workgroups of 128 rows (d = 64) and of 256 (d = 128): edges of waves, workgroups and key tiles, two
+    segments; rows that do not exist stay unwritten."""
+    print(f"attention few keys d={hd} {sq}x{skv}", flush=True)
+    B, H = 2, 3
+    q, k, v = rnd(B, sq, H, hd, seed=61), rnd(B, skv, H, hd, seed=62), rnd(B, skv, H, hd, seed=63)
+    cut = lambda t: [g(t[:, :skv * 2 // 3].contiguous()), g(t[:, skv * 2 // 3:].contiguous())] if skv > 1 else [g(t)]
+    out = torch.full((B, sq + 3, H, hd), 7.0, dtype=torch.bfloat16, device=DEV)
+    hdit.ops.attention([g(q)], cut(k), cut(v), out=[out[:, :sq]])
+    torch.cuda.synchronize()
+    want = O.attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)).transpose(1, 2)
+    assert_parity(out[:, :sq], want, what="attention, few keys")
+    assert bool((out[:, sq:] == 7.0).all())
+
+
 @pytest.mark.parametrize("B,ni,nk,nt", [
     (1, 4096, 4096, 333),  # whole sequence: 256-row workgroups with the text queries
     (1, 1000, 4096, 333),  # patch whose last image rows share their wave with text rows
