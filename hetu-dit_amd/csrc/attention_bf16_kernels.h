@@ -648,8 +648,19 @@ struct PipeLds {
   static constexpr int TILE = BKV * ROW;  // bytes of one K or V tile
   static constexpr int V_OFF = RING * TILE;
   static constexpr int FLAG_OFF = 2 * RING * TILE;
+  // Eight waves: where the query rows of wave w (half a tile) are while the loop has not begun.  In the slots of K tiles
+  // LEAD .. and of V tile LEAD - 1, which iteration 0 and later ones request; where these are not enough (d = 128), behind
+  // the rings, over the flag.
+  static constexpr int K_FREE = RING - LEAD;
+  __device__ static constexpr int q_slot(int w) {
+    const int pair = w / 2;
+    return (pair < K_FREE ? (LEAD + pair) * TILE : pair == K_FREE ? V_OFF + (LEAD - 1) * TILE : FLAG_OFF + (pair - K_FREE - 1) * TILE) +
+           (w % 2) * (TILE / 2);
+  }
+  static constexpr int BEHIND = NWAVE == 8 ? (NWAVE / 2 - K_FREE - 1) * TILE : 0;
+  static constexpr int END = FLAG_OFF + (BEHIND > 16 ? BEHIND : 16);
   // the launch also covers the tracked kernel's layout, which a workgroup falls back to
-  static constexpr int TOTAL = FLAG_OFF + 16 > Lds<HD>::TOTAL ? FLAG_OFF + 16 : Lds<HD>::TOTAL;
+  static constexpr int TOTAL = END > Lds<HD>::TOTAL ? END : Lds<HD>::TOTAL;
   static_assert(TOTAL <= 160 * 1024, "rings do not fit the LDS");
   static_assert(NWAVE != 4 || HD != 64 || TOTAL <= 80 * 1024, "two workgroups per CU");
 };
@@ -757,30 +768,44 @@ __device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles,
     asm volatile("" : : : "memory");
   };
 
-  // ---- prologue: flag, a zero V tile in the last slot (the lagged P.V of iteration 0 multiplies it by P = 0),
+  // ---- prologue: a zero V tile in the last slot (the lagged P.V of iteration 0 multiplies it by P = 0), the query rows,
   // tiles K0 | K1 V0 | K2 V1 .. in request order
-  if (tid == 0) *flag = 0;
   {
     const i32x4 z = {0, 0, 0, 0};
 #pragma unroll
     for (int i = 0; i < TILE / (16 * NTHR); i++) *(i32x4*)(lds + V_OFF + MASK * TILE + i * (16 * NTHR) + tid * 16) = z;
   }
-  // the query rows, requested in front of the tiles: they arrive with the first
+  // The query rows, requested in front of the tiles.  Eight waves: the way K comes, into slots that the first iterations
+  // request -- as loads into registers their first use waits for every tile requested behind them, because the compiler's
+  // count of requests in flight leaves out those of the inline assembly (256 keys, 48 heads: 7.9 us, 7.4 this way; d = 128
+  // 11.9, 10.8).  Four waves have half the tiles in flight and a neighbour on the CU, and lose more by the requests'
+  // addresses than they gain (7.4 us, 7.6 this way).
+  constexpr bool Q_LDS = NWAVE == 8;
+  const unsigned qbase = lds_base_addr + (Q_LDS ? PL::q_slot(__builtin_amdgcn_readfirstlane(wave)) : 0);
   i32x4 qraw[2][KS];
+  if constexpr (!Q_LDS) {
 #pragma unroll
-  for (int qb = 0; qb < 2; qb++) {
-    const __bf16* rp = row_ptr(P.q, b, h, min(q0 + qb * 16 + l16, P.sq - 1));
+    for (int qb = 0; qb < 2; qb++) {
+      const __bf16* rp = row_ptr(P.q, b, h, min(q0 + qb * 16 + l16, P.sq - 1));
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) qraw[qb][ks] = *(const i32x4*)(rp + ks * 32 + lg * 8);
+      for (int ks = 0; ks < KS; ks++) qraw[qb][ks] = *(const i32x4*)(rp + ks * 32 + lg * 8);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  } else if (active) {
+#pragma unroll
+    for (int j = 0; j < 32 / RPI; j++) {
+      const int row = j * RPI + lane / CPR;
+      const int chunk = (lane % CPR) ^ (HD == 64 ? ((row >> 1) & 7) : (row & 15));
+      lds_dma16_ptr<true>((const unsigned char*)(row_ptr(P.q, b, h, min(q0 + row, P.sq - 1)) + chunk * 8), qbase + j * 1024);
+    }
   }
-  __builtin_amdgcn_sched_barrier(0);
   tile_k(0);
 #pragma unroll
   for (int j = 1; j < LEAD; j++) {
     tile_k(j);
     tile_v(j - 1);
   }
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(2 * NCH * (LEAD - 1)));  // K0 has landed
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(2 * NCH * (LEAD - 1)));  // the query rows and K0 have landed
   __syncthreads();
 
   const int nb = NT - 1;  // pipelined iterations
@@ -799,12 +824,15 @@ __device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles,
   }
 
   // ---- Q fragments, softmax scale folded in: lane holds q row (qb*16 + l16), d = 32*ks + 8*lg .. +7
+  const int k_swz = HD == 64 ? ((l16 >> 1) & 7) : l16;
   bf16x8 qf[2][KS];
 #pragma unroll
   for (int qb = 0; qb < 2; qb++)
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
+      typedef const __attribute__((address_space(3))) i32x4 lds_chunk;
       float f[8];
+      if constexpr (Q_LDS) qraw[qb][ks] = *(lds_chunk*)(uintptr_t)(qbase + (qb * 16 + l16) * ROW + (((ks * 4 + lg) ^ k_swz) << 4));
       hdit::unpack8(qraw[qb][ks], f);
 #pragma unroll
       for (int e = 0; e < 8; e++) f[e] *= P.scale_log2;
@@ -814,7 +842,6 @@ __device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles,
   // ---- fragments: the lane part of the LDS addresses, the slot of the tile (a scalar), an immediate
   typedef __attribute__((address_space(3))) unsigned char lds_byte;
   typedef __attribute__((ext_vector_type(8))) short s16x8;
-  const int k_swz = HD == 64 ? ((l16 >> 1) & 7) : l16;
   const int vt_row = 4 * lg + (l16 >> 2);  // transpose read: key row of this lane's 8 bytes, columns 4*(l16&3)
   const int vt_swz = HD == 64 ? ((vt_row >> 1) & 3) : (vt_row & 7);
   unsigned kaddr[KS], vaddr[DB];
@@ -907,6 +934,7 @@ __device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles,
     all_scores(s0, 0, 0);
   }
   stage_end();
+  if (tid == 0) *flag = 0;  // (two barriers and more in front of its next use)
 
   // fragment f of iteration t, in the order of use
   auto read_frag = [&](int f, unsigned vprev, unsigned cur, unsigned next) __attribute__((always_inline)) -> bf16x8 {
