@@ -184,6 +184,7 @@ SIGNATURES = {
     "hdit_attn_fwd_bf16_multi": (C.c_int, [C.POINTER(AttnArgs), C.c_int, C.c_void_p]),
     "hdit_block_sd3_multi": (C.c_int, [C.POINTER(Sd3BlockArgs), C.c_int, C.c_void_p]),
     "hdit_attn_rows": (C.c_int, [C.POINTER(AttnArgs), C.c_int, C.c_int]),
+    "hdit_attn_fwd_bf16_rows": (C.c_int, [C.POINTER(AttnArgs), C.c_int, C.c_int, C.c_void_p]),
     "hdit_attn_absmax": (C.c_int, [C.POINTER(AttnArgs), C.c_void_p, C.c_void_p]),
     "hdit_attn_fp8_workspace_bytes": (C.c_int64, [C.POINTER(AttnArgs)]),
     "hdit_attn_fwd_fp8": (C.c_int, [C.POINTER(AttnArgs), C.c_void_p, C.c_void_p, C.c_void_p]),

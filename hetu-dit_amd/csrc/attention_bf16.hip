@@ -80,28 +80,42 @@ bool is_pipelined(const hdit_attn_args* a, const AttnParams& P) {
 
 int64_t rows_of(const hdit_attn_args* a) { return a->q[0].len + a->q[1].len; }
 
-int64_t workgroups(const hdit_attn_args* a, int rows_per_workgroup) {
-  return (int64_t)a->batch * a->heads * ((rows_of(a) + rows_per_workgroup - 1) / rows_per_workgroup);
-}
-
 // A launch of workgroups of eight waves, one per CU: `full` of them with 256 rows and, dealt out behind those, `half` with
 // 128, which take HALF_COST of the time.  Returns the rounds it takes.
-constexpr double HALF_COST = 0.62;
+//
+// Workgroups go to the XCDs in turn, and there, in order, to four shader engines of eight CUs in turn.  One whose engine
+// has no CU free waits, and everything behind it does, also where another engine has one: with 30 full tiles on an XCD the
+// third half tile runs behind a full one, not on one of the two CUs that are free.  24 heads of 2654 rows in full / half
+// tiles per head, us (rounds by this model): d = 64 10 / 1 68.0 (1.65), 8 / 5 56.7 (1.3), 0 / 21 55.0 (1.3); d = 128
+// 10 / 1 108 (1.65), 0 / 21 88 (1.3); 4000 rows, d = 64, 10 / 12 127.8 (2.3), 16 / 0 109.5 (2).  Over 135 such launches the
+// model's times are off by 4 % rms.  HALF_COST is fitted to them: 0.66 at d = 64, 0.64 at d = 128.
+constexpr double HALF_COST = 0.65;
+constexpr int XCD_CUS = 32, ENGINES = 4;
 double rounds(int64_t full, int64_t half, int64_t cus) {
-  const int64_t whole = full / cus, late = full % cus, early = cus - late;  // CUs that are free at `whole`, at `whole` + 1
-  if (half == 0) return (double)(whole + (late > 0));
-  for (int64_t n = 1;; n++) {  // n half tiles one after the other on the early CUs, and what fits beside them on the late ones
-    const double end = n * HALF_COST;
-    const int64_t on_late = end > 1.0 ? (int64_t)((end - 1.0) / HALF_COST + 1e-9) : 0;
-    if (early * n + late * on_late >= half) return (double)whole + (late && end < 1.0 ? 1.0 : end);
+  const int64_t xcds = cus > XCD_CUS ? cus / XCD_CUS : 1;
+  const int64_t f = (full + xcds - 1) / xcds, n = (full + half + xcds - 1) / xcds;  // on the first XCD, which has most
+  const int64_t whole = f / XCD_CUS;
+  const int late = (int)(f % XCD_CUS);
+  double free_at[ENGINES][XCD_CUS / ENGINES], start = 0.0, end = late > 0;  // from `whole` on
+  for (int e = 0; e < ENGINES; e++)
+    for (int i = 0; i < XCD_CUS / ENGINES; i++) free_at[e][i] = i < late / ENGINES + (e < late % ENGINES) ? 1.0 : 0.0;
+  for (int64_t w = f; w < n; w++) {
+    double* const engine = free_at[w % ENGINES];
+    int cu = 0;
+    for (int i = 1; i < XCD_CUS / ENGINES; i++)
+      if (engine[i] < engine[cu]) cu = i;
+    if (engine[cu] > start) start = engine[cu];
+    engine[cu] = start + HALF_COST;
+    if (engine[cu] > end) end = engine[cu];
   }
+  return (double)whole + end;
 }
 
 // How many 256-row tiles a (batch, head) of a problem has; the rows behind them go to half tiles.  A launch that ends with
 // a round of few workgroups is over sooner if those are twice as many of half the rows: as many whole tiles as fill whole
-// rounds, or all of them (a last one with more than 128 rows counts as whole), whichever ends first.  24 heads of 16896
-// rows at d = 128 are 1584 workgroups, six rounds and 48: 2845 -> 2725 us, 2854 -> 2789 in another run; 12000 rows (1128) 1439 ->
-// 1360; 512 rows (48) 20.9 -> 15.4.
+// rounds, or all of them (a last one with more than 128 rows counts as whole), whichever ends first.  24 heads at d = 128,
+// us: 16896 rows are 1584 workgroups, six rounds and 48: 2823 with all of them whole, 2668 with 64 whole tiles per head;
+// 3830 rows 181.5 -> 153.4; 2654 rows 108 -> 88.
 struct Tiling {
   int full;
   double rounds;
@@ -112,32 +126,39 @@ Tiling tiling(const hdit_attn_args* a, int64_t cus) {
   Tiling best = {(int)most, end(most)};
   for (int64_t whole = bh * most / cus; whole >= 0 && whole + 2 > bh * most / cus; whole--) {
     const int64_t f = whole * cus / bh;
-    if (end(f) < best.rounds - 0.05) best = {(int)f, end(f)};
+    if (f == most) continue;
+    const double e = end(f);
+    if (e < best.rounds - 0.05) best = {(int)f, e};
   }
   return best;
 }
 
-// Query rows per workgroup of a pipelined launch at head dim 64, by how the workgroups fill the CUs.  Measured on MI355X,
-// 24 heads and more, microseconds per tile of 64 keys:
-//   128 rows, four waves, two workgroups per CU   0.55 where a CU has one, 0.90 where it has two
-//   256 rows, eight waves, one per CU             0.86, and 1 us more until it has begun (five tiles ahead, no neighbour)
-// Per row the same, so the last round decides, and small workgroups where CUs would be idle.  128 / 256 rows: 333 rows
-// 8.6 / 11.4 us, 2 x 666 15.0 / 16.1, 2 x 1357 37.1 / 39.3, 1024 of 4429 rows 41.0 / 57.5, two of them 63.3 / 60.1, 4470
-// rows 127.9 / 122.4, 2 x 4429 227 / 247, 17776 rows with 48 heads 3443 / 3378.
+// Query rows per workgroup of a pipelined launch at head dim 64, by how the workgroups fill the CUs.  A CU takes a round of
+// two workgroups of 128 rows (four waves each) or of one with 256 (eight) in about the same time, 0.9 us per tile of 64 keys
+// and 5 us for beginning and end, the eight waves in a little less; one workgroup of 128 alone in 0.56 of it, a half tile of
+// 128 in a workgroup of eight waves in HALF_COST.  So the last round decides, and where it is the same the large workgroups,
+// unless more than half of their waves have no rows (2 x 666 rows 15.1 / 15.7).
+// Measured on MI355X, 128 / 256 rows, us: 24 heads 1357 rows 23.5 / 23.1, 2445 41.9 / 39.1, 2654 45.2 / 52.1, 4470 131.9 /
+// 123.7, 2 x 1357 37.9 / 39.2, 2 x 1024 of 4429 65.6 / 59.9, 2 x 1357 of 4429 99.7 / 102.1, 2 x 4429 235 / 235, 4 x 2637 169 / 178;
+// 48 heads 8000 rows 703 / 676, 13226 1906 / 1826, 17776 3444 / 3428.
+// Over 143 launches of 400 - 13000 keys the choice is 0.5 % slower than the better one on average (always 128: 1.8 %, always 256:
+// 1.7 %), 11 % at most.  Merged launches deal out problem by problem, half tiles in between, and large workgroups lose step with
+// more rounds: of more than two rounds they were level or behind in most launches, up to 15 %; of one or two ahead by 2 - 6 %
+// with the patches of SD3 steps (1357 + 1024 rows of 4429 69.0 / 65.8).
 int pipe_rows(const hdit_attn_args* const* of, int count, int cus) {
   if (pipe_env() == '4') return 128;
   if (pipe_env() == '8') return 256;
-  int64_t small = 0, large = 0, tiles = 0;
-  for (int i = 0; i < count; i++) {
-    small += workgroups(of[i], 128), large += workgroups(of[i], 256);
-    const int64_t t = (of[i]->k[0].len + of[i]->k[1].len + BKV - 1) / BKV;
-    if (t > tiles) tiles = t;
-  }
   if (cus <= 0) return 256;  // no device to ask: the launch reports it
-  small = (small + cus - 1) / cus;
-  const double cost_small = tiles * (0.90 * (double)(small / 2) + 0.55 * (double)(small % 2));
-  const double cost_large = tiles * 0.86 * (count == 1 ? tiling(of[0], cus).rounds : (double)((large + cus - 1) / cus)) + 1.0;
-  return cost_small <= 1.05 * cost_large ? 128 : 256;  // (2 x 4429 rows: modelled 228 / 219, measured 242 / 244)
+  int64_t waves = 0, small = 0, full = 0, half = 0;
+  for (int i = 0; i < count; i++) {
+    const int64_t bh = (int64_t)of[i]->batch * of[i]->heads, rows = rows_of(of[i]), rest = rows % 256;
+    waves += bh * ((rows + 31) / 32), small += bh * ((rows + 127) / 128), full += bh * (rows / 256 + (rest > 128)), half += bh * (rest > 0 && rest <= 128);
+  }
+  const int64_t rest = small % (2 * cus);
+  const double rounds_small = (double)(small / (2 * cus)) + (rest == 0 ? 0.0 : rest <= cus ? 0.56 : 1.0);
+  const double rounds_large = count == 1 ? tiling(of[0], cus).rounds : rounds(full, half, cus);
+  if ((count > 1 && rounds_large > 2.0) || (double)waves < 0.5 * rounds_large * 8 * cus) return 128;
+  return rounds_small <= 0.99 * rounds_large ? 128 : 256;
 }
 
 // Query rows per workgroup of a launch.  The tracked kernel serves few keys: d = 64 small workgroups, ahead at every fill
@@ -147,10 +168,12 @@ int launch_rows(const hdit_attn_args* const* of, int count, bool pipelined, int 
   return pipelined ? pipe_rows(of, count, cus) : 128;
 }
 
-// The problems of one call that one kernel serves, as one launch.
-int launch_some(const hdit_attn_args* const* of, const AttnParams* P, int count, bool pipelined, hipStream_t s) {
+// The problems of one call that one kernel serves, as one launch; `pinned` rows per workgroup where there is a choice and
+// it is not 0.
+int launch_some(const hdit_attn_args* const* of, const AttnParams* P, int count, bool pipelined, int pinned, hipStream_t s) {
   const int hd = of[0]->head_dim, cus = hdit_host::num_cus();
-  const int rows = launch_rows(of, count, pipelined, cus), part = rows == 256 ? rows / 2 : rows;
+  const int rows = pinned && pipelined && hd == 64 ? pinned : launch_rows(of, count, pipelined, cus);
+  const int part = rows == 256 ? rows / 2 : rows;
   int q_tiles[HDIT_ATTN_MAX_MULTI], q_full[HDIT_ATTN_MAX_MULTI], nblocks[HDIT_ATTN_MAX_MULTI];
   for (int i = 0; i < count; i++) {
     const bool tiled = pipelined && rows == 256 && count == 1 && cus > 0;
@@ -182,19 +205,9 @@ extern "C" __attribute__((visibility("default"))) int hdit_attn_rows(const hdit_
   return launch_rows(of, count, is_pipelined(args, P[0]), cus);
 }
 
-extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16(const hdit_attn_args* a, void* stream) {
-  int rc = hdit_host::attn_validate(a);
-  if (rc != HDIT_OK) return rc;
-  AttnParams P;
-  if (!to_params(a, P)) return HDIT_OK;
-  rc = launch_some(&a, &P, 1, is_pipelined(a, P), (hipStream_t)stream);
-  if (rc != HDIT_OK) return rc;
-  return hdit_host::check_launch("hdit_attn_fwd_bf16");
-}
-
-extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16_multi(const hdit_attn_args* args, int count, void* stream) {
+namespace {
+int attn_fwd(const hdit_attn_args* args, int count, int pinned, hipStream_t stream, const char* what) {
   if (!args || count <= 0 || count > HDIT_ATTN_MAX_MULTI) return HDIT_EINVAL;
-  if (count == 1) return hdit_attn_fwd_bf16(args, stream);
   for (int i = 0; i < count; i++) {
     const int rc = hdit_host::attn_validate(&args[i]);
     if (rc != HDIT_OK) return rc;
@@ -210,9 +223,23 @@ extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16_multi(c
       of[n++] = &args[i];
     }
     if (n == 0) continue;
-    int rc = launch_some(of, P, n, pass == 0, (hipStream_t)stream);
+    int rc = launch_some(of, P, n, pass == 0, pinned, stream);
     if (rc != HDIT_OK) return rc;
-    if ((rc = hdit_host::check_launch("hdit_attn_fwd_bf16_multi")) != HDIT_OK) return rc;
+    if ((rc = hdit_host::check_launch(what)) != HDIT_OK) return rc;
   }
   return HDIT_OK;
+}
+}  // namespace
+
+extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16(const hdit_attn_args* a, void* stream) {
+  return attn_fwd(a, 1, 0, (hipStream_t)stream, "hdit_attn_fwd_bf16");
+}
+
+extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16_multi(const hdit_attn_args* args, int count, void* stream) {
+  return attn_fwd(args, count, 0, (hipStream_t)stream, "hdit_attn_fwd_bf16_multi");
+}
+
+extern "C" __attribute__((visibility("default"))) int hdit_attn_fwd_bf16_rows(const hdit_attn_args* args, int count, int rows, void* stream) {
+  if (rows != 128 && rows != 256) return HDIT_EINVAL;
+  return attn_fwd(args, count, rows, (hipStream_t)stream, "hdit_attn_fwd_bf16_rows");
 }

@@ -159,6 +159,11 @@ int hdit_attn_fwd_bf16_multi(const hdit_attn_args* args, int count, void* stream
  * where the problems have no rows or go to several launches. */
 int hdit_attn_rows(const hdit_attn_args* args, int count, int cus);
 
+/* Test hook without a counterpart in the reference: hdit_attn_fwd_bf16_multi with
+ * the rows per workgroup pinned to 128 or 256 where the library chooses between
+ * them (head dim 64, more than 384 keys).  Same bits. */
+int hdit_attn_fwd_bf16_rows(const hdit_attn_args* args, int count, int rows, void* stream);
+
 /* Same contract on the fp8-e4m3 (OCP) MFMA path: Q, K, V are quantised with one
  * absmax scale per (batch, head) taken from `absmax` (f32 [3, batch, heads]:
  * q, k, v; written by hdit_attn_absmax), P is re-quantised per tile.  K and V

@@ -535,6 +535,42 @@ def test_attention_rows_do_not_depend_on_neighbours_whose_reference_moves(hdit, 
     assert_parity(b, want, what="attention, neighbours that move")
 
 
+# (batch, heads, query rows, key rows, key rows in the second buffer, outgrowing query rows)
+@pytest.mark.parametrize("problems", [
+    [(1, 2, 1, 385, 0, ())], [(2, 3, 129, 448, 100, (0, 128))], [(1, 3, 257, 500, 0, (255, 256))],
+    [(1, 24, 2654, 390, 6, (1000, 2653))],  # half tiles only where the workgroups are large
+    [(1, 24, 3068, 450, 0, (2816,))],       # whole tiles and two half tiles per head
+    [(1, 3, 300, 400, 0, ()), (2, 2, 64, 777, 133, (0, 63)), (1, 5, 513, 1000, 77, (512,)), (2, 1, 1, 449, 64, (0,))],
+    [(1, 2, 640, 410, 0, (639, 5)), (1, 2, 40, 100, 0, ()), (2, 5, 513, 513, 13, (512,))],  # one of them goes its own way
+])
+def test_attention_workgroup_sizes_agree(hdit, problems):
+    """Workgroups of 128 and of 256 query rows give the same bits, alone and merged, for keys that end at every position of
+    the key ring (64 .. 512 cut off), and rows whose logits outgrow the first tile get the oracle's numbers in both."""
+    print(f"attention workgroup sizes {problems}", flush=True)
+    lib, gen = hdit._lib.lib(), torch.Generator(device=DEV).manual_seed(85)
+    cuts = range(0, 512, 64) if len(problems) == 1 and problems[0][2] < 1000 else (0,)
+    for more in cuts:  # `more` keys in front
+        args, outs, want = [], [], []
+        for B, H, sq, skv, second, grown in problems:
+            r = lambda n: torch.randn(B, n, H, 64, generator=gen, device=DEV).to(torch.bfloat16)
+            q, k, v = r(sq), r(skv + more), r(skv + more)
+            for i, row in enumerate(grown):  # a late key along the row: its logit is 12 or 52 |q|^2 / 8, 96 or 416
+                k[:, -1 - i] = (12.0 + 40.0 * (i % 2)) * q[:, row]
+            cut = lambda t: [t[:, :t.shape[1] - second], t[:, t.shape[1] - second:].clone()] if second else [t]
+            outs.append([torch.zeros(B, sq, H, 64, dtype=torch.bfloat16, device=DEV) for _ in range(3)])
+            args.append([hdit.ops.attention_args([q], cut(k), cut(v), [o], 0.0) for o in outs[-1]])
+            heads = slice(0, 2)
+            want.append(O.attention(*(t[:, :, heads].float().cpu().transpose(1, 2) for t in (q, k, v))).transpose(1, 2))
+        arr = [(hdit._lib.AttnArgs * len(args))(*(a[f] for a in args)) for f in range(3)]
+        assert lib.hdit_attn_fwd_bf16_rows(arr[0], len(args), 128, hdit.ops._stream()) == 0
+        assert lib.hdit_attn_fwd_bf16_rows(arr[1], len(args), 256, hdit.ops._stream()) == 0
+        assert lib.hdit_attn_fwd_bf16_multi(arr[2], len(args), hdit.ops._stream()) == 0
+        torch.cuda.synchronize()
+        for i, ((small, large, chosen), w) in enumerate(zip(outs, want)):
+            assert torch.equal(small, large) and torch.equal(small, chosen), f"problem {i}, {more} more keys: workgroup sizes differ"
+            assert_parity(small[:, :, :2], w, what=f"attention, problem {i}, {more} more keys")
+
+
 # (batch, heads, query rows, key rows, key rows in the second buffer, gap between heads, outgrowing query rows)
 @pytest.mark.parametrize("hd,problems", [
     (128, [(1, 3, 300, 200, 0, 0, ()), (2, 2, 64, 333, 133, 0, (0, 63)), (1, 5, 513, 1000, 77, 64, (512,)), (2, 1, 1, 129, 64, 8, (0,))]),

@@ -371,3 +371,20 @@ def test_attention_rows_of_a_launch_are_refused_where_there_is_none():
     assert attention_rows(64, [(1, 24, 100, 100), (1, 24, 100, 1000)]) == -1  # two launches
     assert attention_rows(96, [(1, 24, 100, 100)]) == -2
     assert attention_rows(128, [(1, 24, 100, 100)]) == attention_rows(128, [(1, 24, 100, 1000)]) == 256
+
+
+LONG = (1, 24, 1024, 4429)  # a patch of an SD3 sequence
+
+
+@pytest.mark.parametrize("rows,problems", [
+    # sizes measured in favour of one form by 3 % and more
+    (256, [(1, 24, 2445, 2445)]), (256, [(1, 24, 4470, 4470)]), (256, [(2, 24, 1024, 4429)]), (256, [(1, 48, 1000, 1000)]),
+    (256, [(1, 48, 8000, 8000)]), (256, [(1, 48, 13226, 13226)]),
+    (256, [(1, 24, 1357, 4429), LONG]), (256, [(1, 24, 1357, 4429), LONG, LONG, LONG]),
+    (128, [(1, 24, 2654, 2654)]), (128, [(1, 24, 4000, 4000)]), (128, [(2, 24, 1357, 1357)]), (128, [(2, 24, 666, 666)]), (128, [(4, 24, 2637, 2637)]),
+    (128, [(8, 24, 1357, 1357)]), (128, [(2, 24, 1357, 4429)] + [(2, 24, 1024, 4429)] * 3), (128, [(2, 24, 904, 3154), (2, 24, 750, 3154)]),
+    (128, [(1, 24, 410, 1178)] + [(1, 24, 256, 1178)] * 3),
+])
+def test_attention_workgroups_are_chosen_as_measured(rows, problems):
+    """Head dim 64: 128 or 256 query rows per workgroup by how they fill 256 CUs; either is chosen where it was ahead."""
+    assert attention_rows(64, problems) == rows
