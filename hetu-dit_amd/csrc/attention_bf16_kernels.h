@@ -799,11 +799,29 @@ __device__ __forceinline__ bool attn_pipe_body(const AttnParams& P, int q_tiles,
     }
     __builtin_amdgcn_sched_barrier(0);
   } else if (active) {
+    auto chunk = [&](int row) __attribute__((always_inline)) { return (lane % CPR) ^ (HD == 64 ? ((row >> 1) & 7) : (row & 15)); };
+    const int uq0 = __builtin_amdgcn_readfirstlane(q0);
+    const uint64_t qb0 = (uint64_t)(P.q.p0 + b * P.q.sb0 + h * P.q.sh0), qb1 = (uint64_t)(P.q.p1 + b * P.q.sb1 + h * P.q.sh1);
+    int64_t ss0 = P.q.ss0 * 2, ss1 = P.q.ss1 * 2;
+    int qlen0 = P.q.len0;
+    asm volatile("" : "+s"(ss0), "+s"(ss1), "+s"(qlen0));  // values: selected below, not loaded from a selected address
+    const bool in0 = uq0 < qlen0;
+    const int64_t ss = in0 ? ss0 : ss1;
+    if (uq0 + 32 <= (in0 ? qlen0 : P.sq) && ss >= 0 && ss < (1 << 26)) {  // 32 rows of one segment: a base and 32-bit offsets
+      const uint64_t base = (in0 ? qb0 : qb1) + (in0 ? uq0 : uq0 - qlen0) * ss;
 #pragma unroll
-    for (int j = 0; j < 32 / RPI; j++) {
-      const int row = j * RPI + lane / CPR;
-      const int chunk = (lane % CPR) ^ (HD == 64 ? ((row >> 1) & 7) : (row & 15));
-      lds_dma16_ptr<true>((const unsigned char*)(row_ptr(P.q, b, h, min(q0 + row, P.sq - 1)) + chunk * 8), qbase + j * 1024);
+      for (int j = 0; j < 32 / RPI; j++) {
+        const int row = j * RPI + lane / CPR;
+        lds_dma16<true>((const unsigned char*)base, (unsigned)(row * (int)ss + chunk(row) * 16), qbase + j * 1024);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 32 / RPI; j++) {
+        const int row = j * RPI + lane / CPR, r = min(q0 + row, P.sq - 1);
+        const bool first = r < qlen0;
+        const uint64_t rp = (first ? qb0 : qb1) + (uint64_t)((first ? r : r - qlen0) * (first ? ss0 : ss1));
+        lds_dma16_ptr<true>((const unsigned char*)rp + chunk(row) * 16, qbase + j * 1024);
+      }
     }
   }
   tile_k(0);

@@ -571,6 +571,34 @@ def test_attention_workgroup_sizes_agree(hdit, problems):
             assert_parity(small[:, :, :2], w, what=f"attention, problem {i}, {more} more keys")
 
 
+@pytest.mark.parametrize("hd,skv", [(64, 450), (128, 200)])
+@pytest.mark.parametrize("first,second,gap", [(64, 32, 0), (40, 333, 0), (0, 100, 8), (300, 0, 64), (31, 1, 8), (256, 129, 0)])
+def test_attention_query_segments(hdit, hd, skv, first, second, gap):
+    """Query rows of two buffers, the boundary at the edge of a wave's 32 rows and inside them, rows with gaps: the pipelined
+    kernels take a wave's rows with one base or row by row.  Alone and as the second problem of a merged launch."""
+    print(f"attention query segments d={hd} {first}+{second} gap {gap}", flush=True)
+    B, H = 2, 3
+    gen = torch.Generator(device=DEV).manual_seed(93)
+    r = lambda n: torch.randn(B, n, H, hd + gap, generator=gen, device=DEV).to(torch.bfloat16)[..., :hd]
+    q, k, v = [r(n) for n in (first, second) if n], r(skv), r(skv)
+    o = lambda: [torch.zeros(t.shape, dtype=torch.bfloat16, device=DEV) for t in q]
+    alone, merged, other = o(), o(), o()
+    hdit.ops.attention(q, [k], [v], out=alone)
+    args = [hdit.ops.attention_args(q, [k], [v], x, 0.0) for x in (other, merged)]
+    lib = hdit._lib.lib()
+    assert lib.hdit_attn_fwd_bf16_multi((hdit._lib.AttnArgs * 2)(*args), 2, hdit.ops._stream()) == 0
+    outs = [alone, merged]
+    if hd == 64:
+        for rows in (128, 256):
+            outs.append(o())
+            assert lib.hdit_attn_fwd_bf16_rows(hdit.ops.attention_args(q, [k], [v], outs[-1], 0.0), 1, rows, hdit.ops._stream()) == 0
+    torch.cuda.synchronize()
+    for x in outs[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(x, alone)), "launches differ"
+    want = O.attention(*(t.float().cpu().transpose(1, 2) for t in (torch.cat(q, 1), k, v))).transpose(1, 2)
+    assert_parity(torch.cat(alone, 1), want, what="attention, query segments")
+
+
 # (batch, heads, query rows, key rows, key rows in the second buffer, gap between heads, outgrowing query rows)
 @pytest.mark.parametrize("hd,problems", [
     (128, [(1, 3, 300, 200, 0, 0, ()), (2, 2, 64, 333, 133, 0, (0, 63)), (1, 5, 513, 1000, 77, 64, (512,)), (2, 1, 1, 129, 64, 8, (0,))]),
