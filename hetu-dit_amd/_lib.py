@@ -227,6 +227,7 @@ SIGNATURES = {
     "hdit_clock_sample": (C.c_int, [C.c_void_p, C.c_int, C.c_void_p]),
     "hdit_probe_coissue": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p]),
     "hdit_gemm_force_config": (None, [C.c_int]),
+    "hdit_gemm_plan": (C.c_int, [C.POINTER(GemmProblem), C.c_int]),
     "hdit_rope_table": (
         C.c_int,
         [C.c_void_p, C.c_int, C.POINTER(C.c_int), C.c_int, C.c_double, C.c_void_p, C.c_void_p, C.c_void_p],

@@ -900,8 +900,18 @@ int tiles_of(const hdit_gemm_problem& p, int c) {
 
 struct Load {  // the tiles of some problems under one shape
   int tiles = 0;
-  double slabs = 0;  // per tile, on average
+  double slabs = 0;    // per tile, on average
+  double cold_us = 0;  // per tile, on average: what its slabs take longer because few tiles share the weights
 };
+
+// Weights that one or two rows of tiles read come from HBM for a single CU or two, and every slab waits for that where no
+// helper has fetched them: measured 0.2 - 0.3 us and 0.1 us more per slab, whatever the shape.  Merged patches of few rows,
+// 4 x 146 rows x 6144 x 1536 with weights of their own: 128 tiles of 192 x 192, priced at 22.9 us, take 30.7, 256 tiles of 128 x
+// 192 26.1; 2 x 162 x 12288 x 3072 53.0 and 44.0.
+constexpr double kColdUs[2] = {0.20, 0.08};
+constexpr int kHelpedTiles = 240;  // ring shapes, up to this many tiles: helpers fetch the weights (fetch_weights)
+
+bool is_ring(int c) { return kShape[c].bm * kShape[c].bn <= RING_MAX_MMA * 64 * 64; }
 
 Load load_of(const hdit_gemm_problem* ps, int count, int c) {
   Load l;
@@ -909,8 +919,13 @@ Load load_of(const hdit_gemm_problem* ps, int count, int c) {
     const int t = tiles_of(ps[i], c);
     l.tiles += t;
     l.slabs += (double)t * (ps[i].k / BK);
+    int sharing = 0;  // rows of tiles that read these weights
+    for (int j = 0; j < count; j++)
+      if (ps[j].b == ps[i].b) sharing += (ps[j].m + kShape[c].bm - 1) / kShape[c].bm;
+    if (sharing > 0 && sharing <= 2) l.cold_us += (double)t * (ps[i].k / BK) * kColdUs[sharing - 1];
   }
-  if (l.tiles) l.slabs /= l.tiles;
+  if (l.tiles) l.slabs /= l.tiles, l.cold_us /= l.tiles;
+  if (is_ring(c) && l.tiles <= kHelpedTiles) l.cold_us = 0;
   return l;
 }
 
@@ -920,13 +935,13 @@ double tile_us(int c, double slabs, int busy) {
   const Shape& s = kShape[c];
   return slabs * (s.lo + (s.hi - s.lo) * f) + s.epi_lo + (s.epi_hi - s.epi_lo) * f;
 }
+double tile_us(int c, const Load& l, int busy) { return tile_us(c, l.slabs, busy) + l.cold_us; }
 
 // A partial round behind full ones has no helpers beside it, and without them the slabs of the ring shapes take as long as
 // on a full chip (274 + 295 rows x 12288 x 3072: 384 tiles of 128 x 192 76 us, priced at 66 with `lo`; 256 of 256 x 192 61).
 double single_us(const Load& l, int c) {
   const int full = l.tiles / kSlots, rem = l.tiles % kSlots;
-  const bool ring = kShape[c].bm * kShape[c].bn <= RING_MAX_MMA * 64 * 64;
-  return full * tile_us(c, l.slabs, kSlots) + (rem ? tile_us(c, l.slabs, full && ring ? kSlots : rem) : 0.0);
+  return full * tile_us(c, l, kSlots) + (rem ? tile_us(c, l, full && is_ring(c) ? kSlots : rem) : 0.0);
 }
 
 // Tiles of c1, then tiles of c2 in the same launch: the small tiles go first to the workgroups that have one large tile
@@ -938,8 +953,8 @@ double two_us(const Load& l1, int c1, const Load& l2, int c2) {
   const int idle = rem ? kSlots - rem : 0;  // workgroups without a tile of the last large round
   const int base = l2.tiles / kSlots, extra = l2.tiles % kSlots;
   const int busy = rem + l2.tiles;  // CUs at work in the last round
-  const double t1 = full * tile_us(c1, l1.slabs, kSlots), t1_last = rem ? tile_us(c1, l1.slabs, busy) : 0.0;
-  const double t2 = tile_us(c2, l2.slabs, busy);
+  const double t1 = full * tile_us(c1, l1, kSlots), t1_last = rem ? tile_us(c1, l1, busy) : 0.0;
+  const double t2 = tile_us(c2, l2, busy);
   const double of_idle = t1 + (base + (extra > 0 ? 1 : 0)) * t2;
   const double of_rest = t1 + t1_last + (base + (extra > idle ? 1 : 0)) * t2;
   return idle && of_idle > of_rest ? of_idle : of_rest;
@@ -980,14 +995,10 @@ int launch_cfg(int cfg, const hdit_gemm_problem* problems, int count, hipStream_
   }
 }
 
-}  // namespace
-
-extern "C" __attribute__((visibility("default"))) void hdit_gemm_force_config(int cfg) { g_force_cfg.store(cfg, std::memory_order_relaxed); }
-
-extern "C" __attribute__((visibility("default"))) int hdit_gemm_bf16(const hdit_gemm_problem* problems, int count, void* stream) {
+// The problems of a call that have rows, checked.
+int live_problems(const hdit_gemm_problem* problems, int count, hdit_gemm_problem* live, int& nlive) {
   if (!problems || count < 0 || count > HDIT_GEMM_MAX_PROBLEMS) return HDIT_EINVAL;
-  hdit_gemm_problem live[HDIT_GEMM_MAX_PROBLEMS];
-  int nlive = 0;
+  nlive = 0;
   for (int i = 0; i < count; i++) {
     const hdit_gemm_problem& p = problems[i];
     if (p.m < 0 || p.n <= 0 || p.k <= 0) return HDIT_EINVAL;
@@ -1012,22 +1023,24 @@ extern "C" __attribute__((visibility("default"))) int hdit_gemm_bf16(const hdit_
     }
     live[nlive++] = p;
   }
-  if (nlive == 0) return HDIT_OK;
-  hipStream_t s = (hipStream_t)stream;
-  const int forced = g_force_cfg.load(std::memory_order_relaxed);
-  if (forced >= 0) return launch_cfg(forced, live, nlive, s);
+  return HDIT_OK;
+}
 
-  // one shape for everything
-  int single = 0;
-  double single_cost = 1e30;
+struct Plan {  // one shape for everything, or (two_cost < single_cost) two: large tiles and small ones
+  int single = 0, big_cfg = 3, small_cfg = 2, nb = 0, ns = 0;
+  double single_cost = 1e30, two_cost = 1e30;
+  hdit_gemm_problem big[HDIT_GEMM_MAX_PROBLEMS + 1], small[HDIT_GEMM_MAX_PROBLEMS + 1];
+};
+
+void make_plan(const hdit_gemm_problem* live, int nlive, Plan& plan) {
+  int &single = plan.single, &big_cfg = plan.big_cfg, &small_cfg = plan.small_cfg, &nb = plan.nb, &ns = plan.ns;
+  double &single_cost = plan.single_cost, &two_cost = plan.two_cost;
+  hdit_gemm_problem *const big = plan.big, *const small = plan.small;
   for (int c = 0; c < NCFG; c++) {
     const double t = single_us(load_of(live, nlive, c), c);
     if (t < single_cost) single_cost = t, single = c;
   }
   // two shapes, large tiles of 256 rows (c1) and small ones of 128 (c2)
-  hdit_gemm_problem big[HDIT_GEMM_MAX_PROBLEMS + 1], small[HDIT_GEMM_MAX_PROBLEMS + 1];
-  int nb = 0, ns = 0, big_cfg = 3, small_cfg = 2;
-  double two_cost = 1e30;
   for (const int c1 : {3, 0}) {
     for (const int c2 : {2, 1}) {
       // (a) every problem where it is cheaper on its own
@@ -1092,11 +1105,40 @@ extern "C" __attribute__((visibility("default"))) int hdit_gemm_bf16(const hdit_
             single_cost + kLaunchUs, big_cfg, load_of(big, nb, big_cfg).tiles, small_cfg, load_of(small, ns, small_cfg).tiles,
             two_cost + kLaunchUs);
   }
-  if (two_cost < single_cost) {
-    if (big_cfg == 0 && small_cfg == 2) return launch2<Cfg256x192, Cfg128x128>(big, nb, small, ns, s);
-    if (big_cfg == 0) return launch2<Cfg256x192, Cfg128x256>(big, nb, small, ns, s);
-    if (small_cfg == 2) return launch2<Cfg256x256, Cfg128x128>(big, nb, small, ns, s);
+}
+
+}  // namespace
+
+extern "C" __attribute__((visibility("default"))) void hdit_gemm_force_config(int cfg) { g_force_cfg.store(cfg, std::memory_order_relaxed); }
+
+extern "C" __attribute__((visibility("default"))) int hdit_gemm_plan(const hdit_gemm_problem* problems, int count) {
+  hdit_gemm_problem live[HDIT_GEMM_MAX_PROBLEMS];
+  int nlive = 0;
+  const int rc = live_problems(problems, count, live, nlive);
+  if (rc != HDIT_OK) return rc;
+  if (nlive == 0) return HDIT_EINVAL;
+  Plan plan;
+  make_plan(live, nlive, plan);
+  return plan.two_cost < plan.single_cost ? 16 * (1 + plan.big_cfg) + plan.small_cfg : plan.single;
+}
+
+extern "C" __attribute__((visibility("default"))) int hdit_gemm_bf16(const hdit_gemm_problem* problems, int count, void* stream) {
+  hdit_gemm_problem live[HDIT_GEMM_MAX_PROBLEMS];
+  int nlive = 0;
+  const int rc = live_problems(problems, count, live, nlive);
+  if (rc != HDIT_OK || nlive == 0) return rc;
+  hipStream_t s = (hipStream_t)stream;
+  const int forced = g_force_cfg.load(std::memory_order_relaxed);
+  if (forced >= 0) return launch_cfg(forced, live, nlive, s);
+  Plan plan;
+  make_plan(live, nlive, plan);
+  if (plan.two_cost < plan.single_cost) {
+    const hdit_gemm_problem *big = plan.big, *small = plan.small;
+    const int nb = plan.nb, ns = plan.ns;
+    if (plan.big_cfg == 0 && plan.small_cfg == 2) return launch2<Cfg256x192, Cfg128x128>(big, nb, small, ns, s);
+    if (plan.big_cfg == 0) return launch2<Cfg256x192, Cfg128x256>(big, nb, small, ns, s);
+    if (plan.small_cfg == 2) return launch2<Cfg256x256, Cfg128x128>(big, nb, small, ns, s);
     return launch2<Cfg256x256, Cfg128x256>(big, nb, small, ns, s);
   }
-  return launch_cfg(single, live, nlive, s);
+  return launch_cfg(plan.single, live, nlive, s);
 }

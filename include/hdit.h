@@ -112,6 +112,11 @@ int hdit_gemm_bf16(const hdit_gemm_problem* problems, int count, void* stream);
  * back to the planner). */
 void hdit_gemm_force_config(int cfg);
 
+/* Test hook without a counterpart in the reference: the tile shape the planner
+ * gives these problems (numbered as above), or 16 * (1 + large) + small for a
+ * launch of two shapes.  Reads no memory behind the pointers and needs no GPU. */
+int hdit_gemm_plan(const hdit_gemm_problem* problems, int count);
+
 /* ------------------------------------------------------------------------
  * Joint (image + text) flash attention, non-causal, no mask, bf16 in/out,
  * fp32 online softmax on MFMA.

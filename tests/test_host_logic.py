@@ -388,3 +388,26 @@ LONG = (1, 24, 1024, 4429)  # a patch of an SD3 sequence
 def test_attention_workgroups_are_chosen_as_measured(rows, problems):
     """Head dim 64: 128 or 256 query rows per workgroup by how they fill 256 CUs; either is chosen where it was ahead."""
     assert attention_rows(64, problems) == rows
+
+
+def gemm_plan(problems, n, k, shared=False):
+    """Tile shape of one call of (rows of each problem) x n x k; nothing is read or launched."""
+    from hetu_dit_amd import _lib
+
+    arr = (_lib.GemmProblem * len(problems))()
+    for i, (p, m) in enumerate(zip(arr, problems)):
+        p.a, p.b, p.c = 4096, 4096 * (1 if shared else 1 + i), 4096
+        p.lda, p.ldb, p.ldc, p.m, p.n, p.k = k, k, n, m, n, k
+    return _lib.lib().hdit_gemm_plan(arr, len(problems))
+
+
+@pytest.mark.parametrize("rows,n,k", [([144] * 4, 6144, 1536), ([146] * 4, 6144, 1536), ([162] * 2, 12288, 3072)])
+def test_gemm_plan_prices_weights_that_few_tiles_share(rows, n, k):
+    """Merged patches of few rows, each with weights of its own: 192 x 192 tiles (7) read every weight panel from one CU and
+    were 15 - 25 % slower than the 128 x 192 tiles (4) the planner has to choose."""
+    assert gemm_plan(rows, n, k) == 4
+
+
+def test_gemm_plan_of_calls_that_are_refused():
+    assert gemm_plan([0], 64, 64) == -1 and gemm_plan([64], 64, 65) == -2
+    assert gemm_plan([8192], 8192, 8192) in range(8) or gemm_plan([8192], 8192, 8192) >= 16
