@@ -21,7 +21,7 @@ def rnd(*shape, scale=1.0, seed=None):
     return bf16_round(torch.randn(*shape, generator=gen) * scale)
 
 
-@pytest.mark.parametrize("cfg", [-1, 0, 1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("cfg", [-1, 0, 1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("m,n,k", [(256, 256, 64), (300, 384, 128), (666, 1536, 1536), (1, 128, 64), (1024, 512, 256)])
 def test_gemm_bias(hdit, m, n, k, cfg):
     print(f"gemm_bias m={m} n={n} k={k} cfg={cfg}", flush=True)
@@ -35,7 +35,7 @@ def test_gemm_bias(hdit, m, n, k, cfg):
         hdit._lib.lib().hdit_gemm_force_config(-1)
 
 
-@pytest.mark.parametrize("cfg", [0, 1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("cfg", [0, 1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("m", [666, 154, 40])
 def test_gemm_ragged_tile_with_operands_out_of_the_caches(hdit, m, cfg):
     """The out-of-range rows of a ragged tile all read the problem's last row.  Served from the CU's L1, such
@@ -72,7 +72,7 @@ def test_gemm_result_does_not_depend_on_the_tile_shape(hdit, epi):
     a, w, b = g(rnd(m, k, seed=1)), g(rnd(n, k, scale=0.05, seed=2)), g(rnd(n, seed=3))
     outs = []
     try:
-        for cfg in (0, 1, 2, 3, 4, 5, 6):
+        for cfg in (0, 1, 2, 3, 4, 5, 6, 7):
             lib.hdit_gemm_force_config(cfg)
             out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
             hdit.ops.gemm_launch([hdit.ops.gemm_problem(a, w, out, None if epi == "nobias" else b,
@@ -252,7 +252,7 @@ def test_gemm_gelu_and_gate_residual_grouped(hdit):
     assert_parity(res, want, what="gate residual")
 
 
-@pytest.mark.parametrize("cfg", [0, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("cfg", [0, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("m,n,k", [(4096, 4608, 64), (2500, 3000, 192), (5000, 2056, 320)])
 @pytest.mark.parametrize("epi", ["bias", "nobias", "gate"])
 def test_gemm_many_short_tiles_per_workgroup(hdit, m, n, k, cfg, epi):
@@ -384,8 +384,8 @@ def test_attention_large_logits_and_scale(hdit):
 @pytest.mark.parametrize("gain", [4.0, 40.0, 400.0])
 @pytest.mark.parametrize("skv", [256, 300, 1000])
 def test_attention_logits_outgrow_the_first_tile(hdit, gain, skv):
-    """The d = 64 kernel fixes its softmax reference after the first keys and starts over with a tracked reference
-    if a row sum overflows.  Keys placed behind the first tile get logits far above everything the first tile
+    """From 385 keys on the d = 64 kernel fixes its softmax reference after the first keys and starts over with a tracked
+    reference if a row sum outgrows it; below the reference is tracked anyway.  Keys placed behind the first tile get logits far above everything the first tile
     holds: a few tens of nats (inside the fixed reference's range), hundreds (overflow, second pass), for every
     row or only for some, in a full or a masked last tile."""
     print(f"attention outgrow gain={gain} skv={skv}", flush=True)
@@ -405,12 +405,13 @@ def test_attention_logits_outgrow_the_first_tile(hdit, gain, skv):
 
 @pytest.mark.parametrize("gain", [0.0, 40.0])
 @pytest.mark.parametrize("B,H,sq,skv", [
-    (1, 96, 320, 256), (1, 96, 320, 300),                       # one round of 256-row workgroups: pipelined
-    (4, 100, 200, 65), (4, 100, 200, 128), (4, 100, 256, 200),  # between one and two: tracked, 256 rows
-    (1, 2, 1, 1), (2, 2, 31, 64), (1, 3, 33, 63), (1, 2, 127, 65), (2, 1, 128, 300), (1, 2, 129, 130), (1, 2, 257, 577),  # 128 rows
+    (1, 96, 320, 256), (1, 96, 320, 300), (4, 100, 200, 65), (4, 100, 200, 128), (4, 100, 256, 200),  # tracked, a round and more
+    (1, 2, 1, 1), (2, 2, 31, 64), (1, 3, 33, 63), (1, 2, 127, 65), (2, 1, 128, 300), (1, 2, 129, 130), (1, 2, 127, 384),
+    (1, 2, 257, 577), (1, 96, 320, 500), (1, 3, 33, 385),       # pipelined, 128 rows per workgroup
+    (4, 100, 200, 450),                                         # pipelined, 256 rows
 ])
 def test_attention_d64_kernels(hdit, B, H, sq, skv, gain):
-    """The three kernels of head dim 64, each at sizes that the choice gives to it (on 256 CUs): cut-off query and key
+    """The kernels of head dim 64, each at sizes that the choice gives to it (on 256 CUs): cut-off query and key
     tiles, joint sequences of two buffers whose boundary lies inside a tile, logits that outgrow the first tile's."""
     print(f"attention d64 B={B} H={H} {sq}x{skv} gain={gain}", flush=True)
     q, k, v = rnd(B, sq, H, 64, seed=71), rnd(B, skv, H, 64, seed=72), rnd(B, skv, H, 64, seed=73)
@@ -444,13 +445,14 @@ def test_attention_with_few_keys(hdit, hd, sq, skv):
 
 
 @pytest.mark.parametrize("B,ni,nk,nt", [
-    (1, 4096, 4096, 333),  # whole sequence: 256-row workgroups with the text queries
+    (1, 4096, 4096, 333),  # whole sequence
     (1, 1000, 4096, 333),  # patch whose last image rows share their wave with text rows
-    (2, 5184, 5184, 333),  # other workgroups for one batch element than for two
+    (2, 5184, 5184, 333),  # 128 rows per workgroup with the text queries, 256 without
     (2, 1024, 4096, 77),
     (2, 648, 5184, 333),   # few workgroups without the text queries, on a long sequence
-    (1, 1024, 1024, 333),  # pipelined with the text queries
+    (1, 1024, 1024, 333),  # 256 rows with the text queries, 128 without
     (1, 512, 512, 50),
+    (2, 200, 200, 77),     # tracked
 ])
 def test_attention_image_rows_do_not_depend_on_the_text_queries(hdit, B, ni, nk, nt):
     """Dropping the text queries of a joint problem, or a batch element, leaves the image rows' bits alone, whatever
@@ -476,14 +478,15 @@ def test_attention_image_rows_do_not_depend_on_the_text_queries(hdit, B, ni, nk,
 
 
 @pytest.mark.parametrize("hd,B,H,sq,skv", [
-    (64, 1, 2, 200, 192), (64, 1, 3, 129, 193),      # three tiles and one key more, workgroups of 128 rows
-    (64, 1, 80, 256, 513), (64, 1, 86, 640, 640),    # workgroups of 256 rows: one round, and the tail of a second
+    (64, 1, 2, 200, 192), (64, 1, 3, 129, 193),      # tracked
+    (64, 1, 80, 256, 513), (64, 1, 86, 640, 640),    # workgroups of 128 rows, the shortest cuts tracked
+    (64, 4, 100, 200, 896),                          # workgroups of 256 rows
     (128, 1, 2, 257, 193), (128, 2, 3, 300, 576), (128, 1, 60, 1100, 200),  # whole tiles and half tiles
 ])
 def test_attention_rows_do_not_depend_on_rows_that_outgrow(hdit, hd, B, H, sq, skv):
     """The pipelined kernels leave a row whose sum outgrows the reference fixed after the first tile to the tracked body.
-    That row gets the oracle's numbers and every other row of its wave and workgroup keeps its bits, at every position of
-    the key ring the loop can end on (64 .. 256 keys cut off the end)."""
+    That row gets the oracle's numbers and every other row of its wave and workgroup keeps its bits, at several positions of
+    the key ring (64, 128 .. keys cut off the end)."""
     print(f"attention outgrowing rows d={hd} B={B} H={H} {sq}x{skv}", flush=True)
     gen = torch.Generator(device=DEV).manual_seed(91)
     q, k, v = (torch.randn(B, n, H, hd, generator=gen, device=DEV).to(torch.bfloat16) for n in (sq, skv, skv))
@@ -603,9 +606,9 @@ def test_attention_query_segments(hdit, hd, skv, first, second, gap):
 @pytest.mark.parametrize("hd,problems", [
     (128, [(1, 3, 300, 200, 0, 0, ()), (2, 2, 64, 333, 133, 0, (0, 63)), (1, 5, 513, 1000, 77, 64, (512,)), (2, 1, 1, 129, 64, 8, (0,))]),
     (128, [(1, 2, 256, 193, 0, 0, (255,)), (1, 2, 40, 100, 0, 0, (3,))]),  # the second: two key tiles, tracked
-    # one round of 256-row workgroups that small tiles would overfill: pipelined
+    # tracked and, the third, pipelined
     (64, [(1, 96, 320, 256, 0, 0, ()), (1, 100, 300, 260, 60, 8, (299, 5)), (2, 45, 513, 513, 13, 0, (512,))]),
-    (64, [(4, 100, 200, 65, 0, 0, (1,)), (4, 100, 255, 130, 2, 8, (0, 254))]),  # between one and two rounds: 256 rows, tracked
+    (64, [(4, 100, 200, 65, 0, 0, (1,)), (4, 100, 255, 130, 2, 8, (0, 254))]),  # tracked, more than a round
     (64, [(1, 2, 31, 64, 0, 0, (30,)), (2, 3, 200, 333, 77, 8, (0, 199)), (1, 1, 1, 1, 0, 0, ()), (1, 96, 320, 256, 56, 0, (319,))]),
 ])
 def test_attention_merged_launches(hdit, hd, problems):
@@ -942,7 +945,7 @@ def test_attention_random_shapes(hdit):
 # fp32 residual stream: gated-residual epilogue with f32 residual and / or f32 output, LayerNorm on f32 rows
 # ---------------------------------------------------------------------------
 
-@pytest.mark.parametrize("cfg", [-1, 0, 1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("cfg", [-1, 0, 1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("resid_f32,out_f32", [(True, True), (False, True), (True, False)])
 @pytest.mark.parametrize("m,n,k", [(666, 1536, 128), (1000, 520, 64), (4100, 1536, 192)])
 def test_gemm_gate_residual_fp32_stream(hdit, m, n, k, resid_f32, out_f32, cfg):

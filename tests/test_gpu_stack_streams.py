@@ -245,7 +245,8 @@ def test_patch_steps_with_unchanged_inputs_repeat_the_whole_pass(hdit, B):
     """PipeFusion steps whose patches are those of the whole-sequence pass before them: every key and value row is written
     again with what the buffer holds, so the outputs are the rows of the whole pass and stay so step after step -- bit for
     bit, although rows share waves and workgroups with other rows than in the whole pass, and with weights that make
-    logits outgrow those of the first key tile.  (384 rows and more per patch, 24 heads: no pipelined kernel on either side.)"""
+    logits outgrow those of the first key tile.  (With two batch
+    elements the whole pass and the patches get workgroups of different sizes.)"""
     from hetu_dit_amd.runtime_state import get_runtime_state
 
     D, H, L, Nt = 1536, 24, 2, 77
