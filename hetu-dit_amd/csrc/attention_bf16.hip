@@ -87,7 +87,7 @@ int64_t rows_of(const hdit_attn_args* a) { return a->q[0].len + a->q[1].len; }
 // has no CU free waits, and everything behind it does, also where another engine has one: with 30 full tiles on an XCD the
 // third half tile runs behind a full one, not on one of the two CUs that are free.  24 heads of 2654 rows in full / half
 // tiles per head, us (rounds by this model): d = 64 10 / 1 68.0 (1.65), 8 / 5 56.7 (1.3), 0 / 21 55.0 (1.3); d = 128
-// 10 / 1 108 (1.65), 0 / 21 88 (1.3); 4000 rows, d = 64, 10 / 12 127.8 (2.3), 16 / 0 109.5 (2).  Over 135 such launches the
+// 10 / 1 108 (1.65), 0 / 21 88 (1.3); 4000 rows, d = 64, 10 / 12 127.8 (2.3), 16 / 0 109.5 (2).  Over 180 such launches the
 // model's times are off by 4 % rms.  HALF_COST is fitted to them: 0.66 at d = 64, 0.64 at d = 128.
 constexpr double HALF_COST = 0.65;
 constexpr int XCD_CUS = 32, ENGINES = 4;
@@ -95,18 +95,21 @@ double rounds(int64_t full, int64_t half, int64_t cus) {
   const int64_t xcds = cus > XCD_CUS ? cus / XCD_CUS : 1;
   const int64_t f = (full + xcds - 1) / xcds, n = (full + half + xcds - 1) / xcds;  // on the first XCD, which has most
   const int64_t whole = f / XCD_CUS;
-  const int late = (int)(f % XCD_CUS);
-  double free_at[ENGINES][XCD_CUS / ENGINES], start = 0.0, end = late > 0;  // from `whole` on
-  for (int e = 0; e < ENGINES; e++)
-    for (int i = 0; i < XCD_CUS / ENGINES; i++) free_at[e][i] = i < late / ENGINES + (e < late % ENGINES) ? 1.0 : 0.0;
+  const int late = (int)(f % XCD_CUS);  // CUs that are free at `whole` + 1, the others at `whole`
+  constexpr int SLOTS = XCD_CUS / ENGINES;
+  // Per engine: CUs that have begun a half tile, those ended and followed by another, and the ends of all, in order (a ring).
+  int taken[ENGINES] = {}, ended[ENGINES] = {};
+  double ends[ENGINES][SLOTS];
+  double start = 0.0, end = late > 0;
   for (int64_t w = f; w < n; w++) {
-    double* const engine = free_at[w % ENGINES];
-    int cu = 0;
-    for (int i = 1; i < XCD_CUS / ENGINES; i++)
-      if (engine[i] < engine[cu]) cu = i;
-    if (engine[cu] > start) start = engine[cu];
-    engine[cu] = start + HALF_COST;
-    if (engine[cu] > end) end = engine[cu];
+    const int e = (int)(w % ENGINES), first_late = SLOTS - (late / ENGINES + (e < late % ENGINES));
+    const double fresh = taken[e] < first_late ? 0.0 : taken[e] < SLOTS ? 1.0 : 1e30;
+    const bool again = taken[e] > 0 && ends[e][ended[e] % SLOTS] < fresh;
+    const double at = again ? ends[e][ended[e] % SLOTS] : fresh;
+    if (at > start) start = at;
+    (again ? ended : taken)[e]++;
+    ends[e][(taken[e] + ended[e] - 1) % SLOTS] = start + HALF_COST;
+    if (start + HALF_COST > end) end = start + HALF_COST;
   }
   return (double)whole + end;
 }
@@ -145,7 +148,7 @@ Tiling tiling(const hdit_attn_args* a, int64_t cus) {
 // 1.7 %), 11 % at most.  Merged launches deal out problem by problem, half tiles in between, and large workgroups lose step with
 // more rounds: of more than two rounds they were level or behind in most launches, up to 15 %; of one or two ahead by 2 - 6 %
 // with the patches of SD3 steps (1357 + 1024 rows of 4429 69.0 / 65.8).
-int pipe_rows(const hdit_attn_args* const* of, int count, int cus) {
+int pipe_rows(const hdit_attn_args* const* of, int count, int cus, Tiling& tiles) {
   if (pipe_env() == '4') return 128;
   if (pipe_env() == '8') return 256;
   if (cus <= 0) return 256;  // no device to ask: the launch reports it
@@ -156,28 +159,31 @@ int pipe_rows(const hdit_attn_args* const* of, int count, int cus) {
   }
   const int64_t rest = small % (2 * cus);
   const double rounds_small = (double)(small / (2 * cus)) + (rest == 0 ? 0.0 : rest <= cus ? 0.56 : 1.0);
-  const double rounds_large = count == 1 ? tiling(of[0], cus).rounds : rounds(full, half, cus);
+  if (count == 1) tiles = tiling(of[0], cus);
+  const double rounds_large = count == 1 ? tiles.rounds : rounds(full, half, cus);
   if ((count > 1 && rounds_large > 2.0) || (double)waves < 0.5 * rounds_large * 8 * cus) return 128;
   return rounds_small <= 0.99 * rounds_large ? 128 : 256;
 }
 
 // Query rows per workgroup of a launch.  The tracked kernel serves few keys: d = 64 small workgroups, ahead at every fill
-// (attention_bf16_kernels.h), d = 128 large ones.
-int launch_rows(const hdit_attn_args* const* of, int count, bool pipelined, int cus) {
+// (attention_bf16_kernels.h), d = 128 large ones.  `tiles`: of a single problem, where the choice needed it.
+int launch_rows(const hdit_attn_args* const* of, int count, bool pipelined, int cus, Tiling& tiles) {
   if (of[0]->head_dim == 128) return 256;
-  return pipelined ? pipe_rows(of, count, cus) : 128;
+  return pipelined ? pipe_rows(of, count, cus, tiles) : 128;
 }
 
 // The problems of one call that one kernel serves, as one launch; `pinned` rows per workgroup where there is a choice and
 // it is not 0.
 int launch_some(const hdit_attn_args* const* of, const AttnParams* P, int count, bool pipelined, int pinned, hipStream_t s) {
   const int hd = of[0]->head_dim, cus = hdit_host::num_cus();
-  const int rows = pinned && pipelined && hd == 64 ? pinned : launch_rows(of, count, pipelined, cus);
+  Tiling tiles = {-1, 0.0};
+  const int rows = pinned && pipelined && hd == 64 ? pinned : launch_rows(of, count, pipelined, cus, tiles);
   const int part = rows == 256 ? rows / 2 : rows;
   int q_tiles[HDIT_ATTN_MAX_MULTI], q_full[HDIT_ATTN_MAX_MULTI], nblocks[HDIT_ATTN_MAX_MULTI];
   for (int i = 0; i < count; i++) {
     const bool tiled = pipelined && rows == 256 && count == 1 && cus > 0;
-    q_full[i] = tiled ? tiling(of[i], cus).full : P[i].sq / rows + (P[i].sq % rows > part);
+    if (tiled && tiles.full < 0) tiles = tiling(of[i], cus);
+    q_full[i] = tiled ? tiles.full : P[i].sq / rows + (P[i].sq % rows > part);
     const int left = P[i].sq - q_full[i] * rows;
     q_tiles[i] = q_full[i] + (left > 0 ? (left + part - 1) / part : 0);
     nblocks[i] = of[i]->batch * of[i]->heads * q_tiles[i];
@@ -202,7 +208,8 @@ extern "C" __attribute__((visibility("default"))) int hdit_attn_rows(const hdit_
     if (is_pipelined(&args[i], P[i]) != is_pipelined(&args[0], P[0])) return HDIT_EINVAL;
     of[i] = &args[i];
   }
-  return launch_rows(of, count, is_pipelined(args, P[0]), cus);
+  Tiling tiles;
+  return launch_rows(of, count, is_pipelined(args, P[0]), cus, tiles);
 }
 
 namespace {
