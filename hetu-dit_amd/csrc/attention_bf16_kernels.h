@@ -618,14 +618,14 @@ __global__ void __launch_bounds__(NTHR, HD == 64 ? 3 : 2) attn_fwd_multi_kernel(
 // Operands: fragment f (two MFMAs) is read FRAG_LEAD fragments ahead, across the barrier too; the tile requests are
 // dealt over the slots and have a pointer per lane that moves on from tile to tile.
 //
-// Measured on one box, the better of the kernel above and a former pipelined one (64 rows per wave, one wave per SIMD, dot
-// products, 32x32x16 MFMAs, requests in one piece) -> this one.  d = 64, 24 heads: 333 rows 8.9 -> 8.6 us, 2 x 666 18.1 ->
-// 15.0, 1357 27.2 -> 24.0, 4470 130 -> 122, 1024 of 4429 rows 52.3 -> 41.0, two of them 75 -> 60, 2 x 4429 255 -> 227; 17776 rows
-// with 48 heads 3573 -> 3378 (1.15 PFLOP/s).  d = 128, 24 heads: 1536 rows 50.5 -> 42.1, 4608 258 -> 214, 9728 1062 -> 903 (1.29
-// PFLOP/s), 16896 3420 -> 2880.  Of the steps, at 2 x 4429 rows: this layout 244, the loop unrolled over the ring 241 (a
+// Measured on one box, former kernels (64 rows per wave: tracked as above, or pipelined with one wave per SIMD, dot products,
+// 32x32x16 MFMAs, requests in one piece; the better of them) -> this one, us.  d = 64, 24 heads: 2 x 666 rows 17.7 -> 15.2, 1357
+// 27.1 -> 23.0, 4470 131 -> 122, 1024 of 4429 rows 53.0 -> 40.7, two of them 74.7 -> 58.5, 2 x 4429 258 -> 231; 17776 rows with 48
+// heads 3544 -> 3309 (1.17 PFLOP/s).  d = 128, 24 heads: 333 rows 21.1 -> 12.3, 1536 50.2 -> 41.2, 4608 261 -> 217, 9728 1078 -> 911
+// (1.28 PFLOP/s), 16896 3316 -> 2660 (1.32).  Of the steps, at 2 x 4429 rows: this layout 244, the loop unrolled over the ring 241 (a
 // fragment's address needs no addition), one exponential per MFMA in place of two in turn with none 235, the query rows
-// requested in front of the tiles 1 us (at 333 rows 9.3 -> 8.6).  With 32x32x16 MFMAs a SIMD's tile takes fewer cycles (each
-// MFMA holds the issue port) but the clock falls by more: 2 x 4429 rows 244 us at 1.92 GHz against 244 at 2.15.
+// requested in front of the tiles 1 us.  With 32x32x16 MFMAs a SIMD's tile takes fewer cycles (each MFMA holds the issue
+// port) but the clock falls by more: 2 x 4429 rows 244 us at 1.92 GHz against 244 at 2.15.
 //
 // For the block to have no branch the reference of the online softmax is fixed after the first tile (its column
 // maxima plus a margin: p = 2^(s - m) may then grow to PIPE_LIMIT and shrink to nothing without any loss

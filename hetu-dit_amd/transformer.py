@@ -64,14 +64,18 @@ class _Chain:
 
 # Rows (image + text) per chain, on average over the chains, from which a pass of several batch elements runs as chains
 # on side streams: the default of ``SD3TransformerBlocks.lane_rows``.  Below, one chain of all elements is faster: half
-# the launches and half the host time, weights fetched once, launches that fill more of the GPU.  SD3 step at B = 2 on
-# two streams / one, ms: 256+77 rows per element 4.4 / 3.4, 784+333 6.7 / 5.4, 1024+333 6.6 / 6.5, 2112+333 11.4 / 10.1,
-# 3364+333 16.6 / 15.8, 3600+333 17.0 / 16.8, 3844+333 18.5 / 19.2, 4096+333 19.3 / 19.9, 4356+333 21.1 / 21.1.  At B = 3
-# (chains of one and two): 576+333 6.7 / 5.8, 2048+333 14.4 / 12.9, 2398+333 16.5 / 17.1, 3136+333 21.5 / 20.4, 3600+333
-# 24.8 / 25.7; at B = 4: 784+333 9.2 / 8.6, 1444+333 13.9 / 12.7, 2704+333 23.7 / 24.6, 4096+333 36.1 / 37.0.
-# Since then attention and the GEMMs have become faster, the line has stayed: at B = 2 3328+333 14.9 / 14.9, 4096+333 18.4 /
-# 18.8, 4624+333 21.9 / 21.3, 5776+333 26.5 / 27.9, 8100+333 40.5 / 42.6; at B = 3 1920+333 12.9 / 13.0, 4224+333 26.7 / 28.8;
-# at B = 4 2304+333 19.6 / 18.5.
+# the launches and half the host time, weights fetched once, launches that fill more of the GPU (256+77 rows per element
+# at B = 2: 4.4 ms on two streams, 3.4 on one).  SD3 step on two streams / one, ms, two runs on two boxes within 1 % (on
+# faster boxes, whose clock falls less, one stream gains more: 4096+333 17.7 / 17.3 at 2.17 GHz, 18.9 / 19.0 at 2.0):
+# B = 2: 3328+333 14.9 / 14.5, 3584+333 16.3 / 15.1, 3840+333 16.8 / 17.4, 4096+333 18.1 / 18.3, 4356+333 19.4 / 19.3,
+#   4624+333 20.8 / 20.5, 4900+333 22.1 / 21.5, 5184+333 23.7 / 24.9, 5776+333 26.5 / 27.3, 6400+333 29.9 / 30.6, 8100+333
+#   40.1 / 42.0
+# B = 3 (chains of one and two): 1536+333 10.6 / 10.7, 2304+333 14.8 / 14.1, 3072+333 19.6 / 18.8, 3584+333 23.0 / 23.1,
+#   4224+333 26.6 / 28.3
+# B = 4: 768+333 8.6 / 8.5, 1280+333 11.6 / 11.4, 1600+333 14.5 / 13.6, 2304+333 18.4 / 18.3, 2704+333 21.9 / 22.9, 4096+333
+#   33.6 / 35.2; B = 6: 1024+333 14.1 / 13.3, 1600+333 19.8 / 20.5; B = 8: 1024+333 18.3 / 18.3, 2304+333 34.7 / 36.0
+# What decides is how full the last rounds of the GEMMs are, on one stream and on two, and rows alone do not tell: above
+# the line two streams are ahead by up to 6 %, except between 4600 and 5300 rows per chain, where one is by up to 4 %.
 LANE_ROWS = 4096
 
 
